@@ -256,3 +256,46 @@ def test_conv2d_forward_from_fp32_reports_a_bad_range(ctx, hipq):
     assert p.status == hipq.INVALID_ARGUMENT and p.scale != p.scale
     with pytest.raises(hipq.HipqError):
         ctx.conv2d_dynamic_packed(x[:, :31].contiguous(), packed, sums, (3, 3), sw, None, 0.05, 0, (1, 1))
+
+
+WINDOW_GEOMS = [
+    # nb, c, h, w, oc, (kh, kw), stride, pad, zp: strides and channel counts of the window kernel
+    (2, 3, 32, 30, 64, (7, 7), (2, 2), (3, 3), 5),       # the first layer of an image network: pitch 4
+    (1, 1, 5, 5, 1, (5, 5), (1, 1), (0, 0), 0),          # a single window, channel and filter
+    (5, 1, 7, 7, 33, (3, 2), (1, 2), (1, 0), 255),       # planes smaller than a run of 16 windows; 33 filters
+    (3, 33, 9, 11, 65, (3, 3), (2, 1), (1, 1), 77),      # two channel groups of 20 bytes
+    (2, 31, 6, 6, 32, (1, 1), (2, 2), (0, 0), 128),      # one group, one k block, 1 x 1 with stride 2
+    (2, 100, 12, 13, 129, (3, 3), (2, 2), (1, 1), 9),    # four groups, two filter tiles with one filter in the last
+    (1, 5, 300, 260, 40, (3, 3), (1, 1), (1, 1), 200),   # enough windows for a wave on its own windows, K short
+    (4, 64, 120, 121, 80, (3, 3), (2, 2), (1, 1), 3),    # the same with more than 64 filters and several groups
+    (3, 40, 20, 21, 16, (5, 3), (3, 2), (2, 1), 60),     # few filters: one filter block, four window fragments
+]
+
+
+@pytest.mark.parametrize("nb,c,h,w,oc,k,stride,pad,zp", WINDOW_GEOMS)
+def test_conv_any_stride_and_channel_count(ctx, hipq, oracle, nb, c, h, w, oc, k, stride, pad, zp):
+    """The window kernel: int32 accumulators, the dequantized and the requantized outputs, all bit for bit."""
+    rng = np.random.default_rng(nb + c * 3 + h * 5 + oc)
+    x = rng.integers(0, 256, size=(nb, c, h, w), dtype=np.uint8)
+    wq = rng.integers(-128, 128, size=(oc, c) + k, dtype=np.int8)
+    sw = rng.uniform(1e-4, 1e-3, oc).astype(np.float32)
+    bias = (rng.standard_normal(oc) * 0.01).astype(np.float32)
+    acc = oracle.backend_conv2d_i32(x, zp, wq, stride, pad)
+    xd, wd, swd, bd = dev(x), dev(wq), dev(sw), dev(bias)
+    np.testing.assert_array_equal(host(ctx.conv2d_i32(xd, zp, wd, stride, pad)), acc)
+    acc2d = acc.reshape(nb * oc, -1)
+    s_in = np.float32(0.02)
+    want = (acc2d.astype(np.float32) * np.tile(s_in * sw, nb)[:, None]) + np.tile(bias, nb)[:, None]
+    got = host(ctx.conv2d_f32(xd, zp, float(s_in), wd, swd, bd, stride, pad))
+    np.testing.assert_array_equal(got.reshape(acc2d.shape), want)
+    s_out = float(np.abs(want).max() / 100)
+    for mode, rm in ((hipq.ROUND_HALF_AWAY, 0), (hipq.ROUND_HALF_EVEN, 1)):
+        oracle.set_round_mode(rm)
+        try:
+            codes = [oracle.requantize_epilogue(acc2d, float(s_in), sw, b, s_out, -2, channel_axis_is_row=True, inner=oc)
+                     for b in (bias, None)]
+        finally:
+            oracle.set_round_mode(0)
+        for b, q in zip((bd, None), codes):
+            got = host(ctx.conv2d_i8(xd, zp, float(s_in), wd, swd, b, s_out, -2, stride, pad, mode))
+            np.testing.assert_array_equal(got.reshape(acc2d.shape), q)

@@ -1,70 +1,19 @@
 // Quantized Conv2d forward: u8 activations (NCHW) x per-channel int8 filters ->
 // int32 accumulators -> requantized int8 (NCHW), bias fused.
 //
-// Fast path (stride 1, channels a multiple of 32): an im2col-free implicit GEMM on the
-// fragment-packed MFMA kernel (hipq_gemm_packed.h, CONV).  The activations are rewritten
-// once as signed bytes (x - 128) in a zero-point-padded image stored as
-// [channel block of 32][pixel][32 bytes]: consecutive pixels of one channel block are 32
-// bytes apart, so the 32 windows of an MFMA fragment, shifted by any filter tap, are one
-// contiguous KiB that a wave loads with a single coalesced instruction, straight into the
-// operand registers (no LDS, no gather).  The filters are packed once in the GEMM's
-// fragment order with K = (tap, channel).  Shifting by 128 lets the signed int8 MFMA
-// multiply unsigned activations; the shift and the zero point are undone in the epilogue
-// with the per-filter weight sum:  sum (x - zp) w = sum (x - 128) w + (128 - zp) sum w,
-// and a border pixel holds exactly zp so padded taps contribute nothing.
-// Everything else runs through a direct per-output kernel (correct, not fast).
+// The convolution is an implicit GEMM on the matrix cores (hipq_conv_window.h): a layout pass rewrites the input as
+// signed bytes x - 128 with the zero point as border, and the product's window fragments come straight out of that
+// image.  Shifting by 128 lets the signed int8 MFMA multiply unsigned activations; the shift and the zero point are
+// undone in the epilogue with the per-filter weight sum:  sum (x - zp) w = sum (x - 128) w + (128 - zp) sum w,
+// and a border pixel holds exactly zp so padded taps contribute nothing.  Prepared filters (and the forward from fp32)
+// take stride 1 and channels a multiple of 32.
+#include "hipq_conv_window.h"
 #include "hipq_gemm_kernels.h"
 #include "hipq_meeting.h"
 
 namespace hipq {
 
 constexpr int kConvThreads = 256;
-
-// u8 NCHW -> i8 [channel block][padded pixel][32] with a border of `pad` pixels holding (zp - 128); pixel
-// index = (n * hp + y) * wp + x, `pixels` of them per channel block (the real ones, then zeroed slack that
-// the last windows read into).  One thread per (channel block, padded pixel): it reads its pixel's byte from
-// each of the block's 32 channel planes (consecutive lanes are consecutive pixels: consecutive bytes of a
-// plane row), all 32 loads in flight at once, and writes the 32 bytes as two 16-byte stores (a wave writes
-// 2 KiB contiguous).  x - 128 on a byte is a flip of its top bit.  No LDS.  The last cbs workgroups clear
-// the slack.  C % 32 == 0.
-__global__ __launch_bounds__(kConvThreads) void conv_pack_image_kernel(const uint8_t *__restrict__ x, int C, int H, int W,
-                                                                         int pad_h, int pad_w, int zp,
-                                                                         const int32_t *__restrict__ zp_dev, int nb,
-                                                                         int groups_per_cb, int8_t *__restrict__ out,
-                                                                         int pixels) {
-    if (zp_dev) zp = *zp_dev;  // the zero point a dynamic quantize has left on the device
-    const int hp = H + 2 * pad_h, wp = W + 2 * pad_w, cbs = C / 32;
-    const int real_pixels = nb * hp * wp;
-    const int work = cbs * groups_per_cb;
-    if (static_cast<int>(blockIdx.x) >= work) {
-        const int cb = blockIdx.x - work;
-        uint4 *tail = reinterpret_cast<uint4 *>(out + (size_t(cb) * pixels + real_pixels) * 32);
-        for (int i = threadIdx.x; i < (pixels - real_pixels) * 2; i += kConvThreads) tail[i] = make_uint4(0, 0, 0, 0);
-        return;
-    }
-    const int cb = blockIdx.x / groups_per_cb;
-    const int p = (blockIdx.x % groups_per_cb) * kConvThreads + threadIdx.x;  // padded pixel of the whole batch
-    if (p >= real_pixels) return;
-    const int n = p / (hp * wp), rem = p % (hp * wp);
-    const int h = rem / wp - pad_h, w = rem % wp - pad_w;
-    const uint32_t border4 = static_cast<uint32_t>(static_cast<uint8_t>(zp - 128)) * 0x01010101u;
-    uint32_t d[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) d[i] = border4;
-    if (h >= 0 && h < H && w >= 0 && w < W) {
-        const size_t plane = size_t(H) * W;
-        const uint8_t *src = x + ((size_t(n) * C + cb * 32) * H + h) * W + w;
-        uint32_t b[32];
-#pragma unroll
-        for (int c = 0; c < 32; ++c) b[c] = src[size_t(c) * plane];
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-            d[i] = (b[4 * i] | (b[4 * i + 1] << 8) | (b[4 * i + 2] << 16) | (b[4 * i + 3] << 24)) ^ 0x80808080u;
-    }
-    uint4 *dst = reinterpret_cast<uint4 *>(out + (size_t(cb) * pixels + p) * 32);
-    dst[0] = make_uint4(d[0], d[1], d[2], d[3]);
-    dst[1] = make_uint4(d[4], d[5], d[6], d[7]);
-}
 
 // The same image from fp32 activations, quantized on the way: per-tensor uint8 with parameters from the
 // tensor's own range (flavor; codes 0..255).  A thread keeps the 32 channel values of its pixel in registers
@@ -75,18 +24,16 @@ __global__ __launch_bounds__(kConvThreads) void conv_pack_image_kernel(const uin
 template <bool DIV, int RND>
 __global__ __launch_bounds__(kConvThreads, 4) void conv_quantize_pack_image_kernel(
     const float *__restrict__ x, int C, int H, int W, int pad_h, int pad_w, int flavor, int nb, int groups_per_cb,
-    hipq_qparams *out_params, uint32_t *words, int spin_limit, int8_t *__restrict__ out, int pixels,
+    hipq_qparams *out_params, uint32_t *words, int spin_limit, int8_t *__restrict__ out,
     const uint32_t *__restrict__ touch, uint32_t touch_lines) {
     __shared__ float lds[kMeetingLdsFloats];
     const int hp = H + 2 * pad_h, wp = W + 2 * pad_w, cbs = C / 32;
-    const int real_pixels = nb * hp * wp;
-    const int work = cbs * groups_per_cb;
-    const bool slack = static_cast<int>(blockIdx.x) >= work;
-    const int cb = slack ? blockIdx.x - work : blockIdx.x / groups_per_cb;
+    const int pixels = nb * hp * wp, work = cbs * groups_per_cb;
+    const int cb = blockIdx.x / groups_per_cb;
     const int p = (blockIdx.x % groups_per_cb) * kConvThreads + threadIdx.x;  // padded pixel of the whole batch
     bool inside = false;
     float v[32];
-    if (!slack && p < real_pixels) {
+    if (p < pixels) {
         const int n = p / (hp * wp), rem = p % (hp * wp);
         const int h = rem / wp - pad_h, w = rem % wp - pad_w;
         if (h >= 0 && h < H && w >= 0 && w < W) {
@@ -107,14 +54,6 @@ __global__ __launch_bounds__(kConvThreads, 4) void conv_quantize_pack_image_kern
         }
     }
     const MinMax r = block_minmax(m, lds);
-    if (slack) {
-        // These workgroups only clear the slack behind the image: they take part in the meeting with a range
-        // that changes nothing and do not wait for its result.
-        meeting_publish_range(words, gen, r);
-        uint4 *tail = reinterpret_cast<uint4 *>(out + (size_t(cb) * pixels + real_pixels) * 32);
-        for (int i = threadIdx.x; i < (pixels - real_pixels) * 2; i += kConvThreads) tail[i] = make_uint4(0, 0, 0, 0);
-        return;
-    }
     // While the grid agrees on the range: one load per 128-byte line of the prepared filters, which every die's
     // workgroups of the convolution kernel read first thing (workgroups are dealt to the dies in turn, there as
     // here), by the waves that do not poll.  The values are not used.
@@ -126,7 +65,7 @@ __global__ __launch_bounds__(kConvThreads, 4) void conv_quantize_pack_image_kern
     }
     const MeetingParams agreed = meet_on_range(words, gen, r, flavor, 0, 255, /*poison=*/true, spin_limit, lds, out_params);
     asm volatile("" ::"v"(touched));
-    if (p >= real_pixels) return;
+    if (p >= pixels) return;
     const bool bad = agreed.scale != agreed.scale;
     const float scale = bad ? INFINITY : agreed.scale;  // x / inf: every code is the zero point
     const int zp = agreed.zero_point;
@@ -234,20 +173,14 @@ static int32_t check_geom(const char *fn, const ConvGeom &g) {
     return HIPQ_SUCCESS;
 }
 
-// Pixels per channel block of the packed image: the padded grid, what the last windows' taps reach past it,
-// and the 32 windows of a fragment that starts at the last one.
-static size_t image_pixels(const ConvGeom &g) {
-    const size_t hp = g.h + 2 * g.ph, wp = g.w + 2 * g.pw;
-    const size_t reach = size_t(g.kh - 1) * wp + g.kw + 32;
-    return (size_t(g.nb) * hp * wp + reach + 31) / 32 * 32;
-}
+// Bytes of an image or a filter operand that the 32-bit offsets of the window kernel reach.
+constexpr size_t kConvOperandLimit = 0x7ffffc00;
 
-static bool fast_path_ok(const ConvGeom &g) {
-    const size_t k = size_t(g.c) * g.kh * g.kw;
-    // offsets into the packed image and the packed filters are 32-bit
-    return g.sh == 1 && g.sw == 1 && g.c % 32 == 0 && g.oc >= 1 &&
-           size_t(g.c / 32) * image_pixels(g) * 32 < (size_t(1) << 31) &&
-           packed_operand_bytes(g.oc, k) < (size_t(1) << 31);
+// What the entry points on prepared filters take.
+static bool prepared_ok(const ConvGeom &g) {
+    const size_t pixels = size_t(g.nb) * (g.h + 2 * g.ph) * (g.w + 2 * g.pw);
+    return g.sh == 1 && g.sw == 1 && g.c % 32 == 0 && g.oc >= 1 && size_t(g.c) * pixels < kConvOperandLimit &&
+           packed_operand_bytes(g.oc, size_t(g.c) * g.kh * g.kw) < kConvOperandLimit;
 }
 
 static size_t align256(size_t v) { return (v + 255) & ~size_t(255); }
@@ -270,14 +203,77 @@ struct ConvDynamicInput {
     hipq_qparams *params = nullptr;
 };
 
+// Geometry of the image layout of hipq_conv_window.h; false where its 32-bit offsets do not reach.
+static bool window_geometry(const ConvGeom &g, ConvWindow *cw) {
+    const size_t cgs = (size_t(g.c) + 31) / 32, pitch = ((size_t(g.c) + cgs - 1) / cgs + 3) / 4 * 4;
+    const size_t segs = (size_t(g.kw) * pitch + 31) / 32, kblocks = size_t(g.kh) * segs * cgs;
+    const size_t hp = size_t(g.h) + 2 * g.ph, wp = size_t(g.w) + 2 * g.pw;
+    const size_t plane = size_t(g.nb) * hp * wp * pitch, KB = (kblocks + 3) / 4 * 4;
+    const size_t windows = size_t(g.nb) * g.ho * g.wo;
+    if (cgs * plane >= kConvOperandLimit || (size_t(g.oc) + 31) / 32 * KB * 1024 >= kConvOperandLimit ||
+        windows >= (size_t(1) << 31) - 1024)
+        return false;
+    *cw = ConvWindow{g.oc, static_cast<int>(windows), static_cast<int>(KB), static_cast<int>(kblocks), static_cast<int>(cgs),
+                     static_cast<int>(segs), static_cast<int>(pitch), static_cast<int>(wp * pitch), static_cast<int>(plane),
+                     static_cast<int>(cgs * plane), static_cast<int>(hp), static_cast<int>(wp), g.sh, g.sw, g.ho, g.wo};
+    return true;
+}
+
+template <int EPI, bool EVEN>
+static int32_t launch_conv_window(hipq_ctx *ctx, const int8_t *filters, const int8_t *image, const ConvWindow &cw,
+                                  const GemmEpilogue &ep) {
+    // Waves on different windows while there are enough of them for two per SIMD, else K split between four.
+    const size_t waves = (size_t(cw.N) + 63) / 64 * ((size_t(cw.M) + 127) / 128);
+    if (waves >= size_t(ctx->num_cus) * 8 || cw.kblocks < 8) {
+        if (cw.M <= 32) return launch_conv_window_form<1, 4, 3, false, EPI, EVEN>(ctx, filters, image, cw, ep);
+        if (cw.M <= 64) return launch_conv_window_form<2, 2, 4, false, EPI, EVEN>(ctx, filters, image, cw, ep);
+        return launch_conv_window_form<4, 2, 2, false, EPI, EVEN>(ctx, filters, image, cw, ep);
+    }
+    if (cw.M <= 32) return launch_conv_window_form<1, 4, 3, true, EPI, EVEN>(ctx, filters, image, cw, ep);
+    if (cw.M <= 64) return launch_conv_window_form<2, 2, 4, true, EPI, EVEN>(ctx, filters, image, cw, ep);
+    return launch_conv_window_form<4, 2, 2, true, EPI, EVEN>(ctx, filters, image, cw, ep);
+}
+
+// Layout pass of a u8 input, and of the filters when `f` has any, in one launch.
+static int32_t launch_window_pack(const char *fn, hipq_ctx *ctx, const uint8_t *x, int zp, const int32_t *zp_dev,
+                                  const ConvGeom &g, const ConvWindow &cw, int8_t *image, const ConvWindowFilters &f) {
+    const int groups = static_cast<int>((size_t(g.nb) * cw.hp * cw.wp + 255) / 256);
+    const dim3 grid(cw.cgs * groups + (f.w ? g.oc : 0));
+#define HIPQ_PACK_WINDOWS(DW)                                                                                         \
+    case DW:                                                                                                          \
+        hipLaunchKernelGGL((conv_window_pack_kernel<DW>), grid, dim3(256), 0, ctx->stream, x, g.c, g.h, g.w, g.ph, g.pw, \
+                           zp, zp_dev, g.nb, groups, image, cw, f);                                                   \
+        break
+    switch (cw.pitch / 4) {
+        HIPQ_PACK_WINDOWS(1);
+        HIPQ_PACK_WINDOWS(2);
+        HIPQ_PACK_WINDOWS(3);
+        HIPQ_PACK_WINDOWS(4);
+        HIPQ_PACK_WINDOWS(5);
+        HIPQ_PACK_WINDOWS(6);
+        HIPQ_PACK_WINDOWS(7);
+        HIPQ_PACK_WINDOWS(8);
+    }
+#undef HIPQ_PACK_WINDOWS
+    return check_launch(fn);
+}
+
+// The forward from u8 (or, with dyn, fp32) activations, on filters as the caller stores them (w) or prepared ones
+// (wpacked, wsum: prepared_ok geometries only).
 template <int EPI, bool EVEN>
 static int32_t conv_forward(const char *fn, hipq_ctx *ctx, const uint8_t *x, int zp_in, float s_in, const int8_t *w,
                             const int8_t *wpacked, const int32_t *wsum, const float *sw, const float *bias,
                             const ConvGeom &g, float s_out, int zp_out, void *out,
                             const ConvDynamicInput &dyn = ConvDynamicInput{}) {
-    if (!fast_path_ok(g)) {
-        if (dyn.x) return fail(HIPQ_INVALID_ARGUMENT, "%s: needs stride 1 and channels a multiple of 32", fn);
-        if (!w) return fail(HIPQ_INVALID_ARGUMENT, "%s: this geometry needs the unpacked filters", fn);
+    const int taps = g.kh * g.kw;
+    const size_t k = size_t(g.c) * taps, elems = size_t(g.nb) * g.c * g.h * g.w;
+    GemmEpilogue ep{nullptr, 0, sw, bias, s_out, zp_out, out};
+    ep.s_out_inv = host_recip_for_div(s_out);
+    ep.sa_scalar = s_in;
+    ep.cv_corr_mul = 128 - zp_in;
+    ConvWindow cw;
+    if (!window_geometry(g, &cw)) {
+        if (dyn.x || !w) return fail(HIPQ_SHAPE_ERROR, "%s: image or filters too large", fn);
         const size_t total = size_t(g.nb) * g.oc * g.ho * g.wo;
         size_t blocks = (total + kConvThreads - 1) / kConvThreads;
         const size_t cap = size_t(ctx->num_cus) * 32;
@@ -286,70 +282,57 @@ static int32_t conv_forward(const char *fn, hipq_ctx *ctx, const uint8_t *x, int
                            ctx->stream, x, zp_in, w, g, s_in, sw, bias, s_out, zp_out, out);
         return check_launch(fn);
     }
-    const int hp = g.h + 2 * g.ph, wp = g.w + 2 * g.pw, taps = g.kh * g.kw, cbs = g.c / 32;
     // One launch, the image gathered by the convolution kernel itself (hipq_conv_patch.h): built, bit-exact, and
     // measured no faster than the two launches below on the shape it was built for (13.3 against 13.4 us at
     // [32, 256, 14, 14] x [256, 256, 3, 3]: the gather costs what the layout launch did, and the window fragments
     // leave LDS no faster than they leave the L2), so it runs only under test hook 14.
-    if (!dyn.x && ctx->gemm_variant == 14 && conv_patch_applicable(g.nb, g.c, g.h, g.w, hp, wp, g.kh, g.kw) &&
-        size_t(g.nb) * g.c * g.h * g.w < (size_t(1) << 31) && !(reinterpret_cast<uintptr_t>(x) & 3u)) {
-        const size_t kk = size_t(g.c) * taps;
-        int32_t rc;
-        if (!wpacked) {
-            void *s = nullptr;
-            const size_t need = kScratchHeader + align256(size_t(g.oc) * kk) + align256(packed_operand_bytes(g.oc, kk)) +
-                                align256(size_t(g.oc) * 4);
-            if ((rc = scratch(ctx, need, &s))) return rc;
-            int8_t *staging = reinterpret_cast<int8_t *>(static_cast<char *>(s) + kScratchHeader);
-            int8_t *pbuf = staging + align256(size_t(g.oc) * kk);
-            int32_t *wsbuf = reinterpret_cast<int32_t *>(pbuf + align256(packed_operand_bytes(g.oc, kk)));
-            if ((rc = pack_filters(ctx, w, g.oc, g.c, taps, staging, pbuf, wsbuf))) return rc;
-            wpacked = pbuf;
-            wsum = wsbuf;
-        }
-        GemmEpilogue ep{nullptr, 0, sw, bias, s_out, zp_out, out};
-        ep.s_out_inv = host_recip_for_div(s_out);
-        ep.sa_scalar = s_in;
+    if (wpacked && !dyn.x && ctx->gemm_variant == 14 && elems < (size_t(1) << 31) && !(reinterpret_cast<uintptr_t>(x) & 3u) &&
+        conv_patch_applicable(g.nb, g.c, g.h, g.w, cw.hp, cw.wp, g.kh, g.kw)) {
         ep.cv_kw = g.kw;
-        ep.cv_wp = wp;
-        ep.cv_hp = hp;
+        ep.cv_wp = cw.wp;
+        ep.cv_hp = cw.hp;
         ep.cv_c = g.c;
         ep.cv_ho = g.ho;
         ep.cv_wo = g.wo;
         ep.cv_oc = g.oc;
         ep.cv_nb = g.nb;
         ep.cv_wsum = wsum;
-        ep.cv_corr_mul = 128 - zp_in;
-        ep.cv_kblocks = taps * cbs;
-        return conv_gemm_patch(ctx, wpacked, x, size_t(g.nb) * g.c * g.h * g.w, zp_in, g.h, g.w, g.ph, g.pw, g.kh, g.oc,
-                               g.nb * hp * wp, static_cast<int>(kk), ep, EPI, EVEN);
+        ep.cv_kblocks = cw.kblocks;
+        return conv_gemm_patch(ctx, wpacked, x, elems, zp_in, g.h, g.w, g.ph, g.pw, g.kh, g.oc, g.nb * cw.hp * cw.wp,
+                               static_cast<int>(k), ep, EPI, EVEN);
     }
-    const size_t pixels = image_pixels(g);
-    const size_t img_bytes = size_t(cbs) * pixels * 32;
-    const size_t k = size_t(g.c) * taps;
-    const size_t w_bytes = wpacked ? 0 : align256(size_t(g.oc) * k) + align256(packed_operand_bytes(g.oc, k)) +
-                                             align256(size_t(g.oc) * 4);
-    const int groups_per_cb = (g.nb * hp * wp + kConvThreads - 1) / kConvThreads;
-    const size_t pack_grid = size_t(cbs) * groups_per_cb + cbs;
+    const size_t img_bytes = align256(size_t(cw.image_bytes));
+    const size_t f_bytes = wpacked ? 0 : align256((size_t(cw.M) + 31) / 32 * cw.KB * 1024);
+    const size_t w_bytes = wpacked ? 0 : f_bytes + align256(size_t(cw.M) * 4);
     // Dynamic input: in one launch with the image pack when its grid can be resident at once (the kernel holds 32
     // floats a lane: four workgroups per compute unit), else quantized to a uint8 copy first.
+    const int groups_per_cb = static_cast<int>((size_t(g.nb) * cw.hp * cw.wp + kConvThreads - 1) / kConvThreads);
+    const size_t pack_grid = size_t(cw.cgs) * groups_per_cb;
     const bool fused_input = dyn.x && ctx->gemm_variant != 6 && pack_grid <= resident_workgroups(ctx, true);
-    const size_t u8_bytes = (dyn.x && !fused_input) ? align256(size_t(g.nb) * g.c * g.h * g.w) : 0;
+    const size_t u8_bytes = (dyn.x && !fused_input) ? align256(elems) : 0;
     void *s = nullptr;
-    int32_t rc = scratch(ctx, kScratchHeader + align256(img_bytes) + w_bytes + u8_bytes, &s);
+    int32_t rc = scratch(ctx, kScratchHeader + img_bytes + w_bytes + u8_bytes, &s);
     if (rc) return rc;
-    int8_t *ximg = reinterpret_cast<int8_t *>(static_cast<char *>(s) + kScratchHeader);
+    int8_t *image = reinterpret_cast<int8_t *>(static_cast<char *>(s) + kScratchHeader);
+    ConvWindowFilters f{nullptr, nullptr, nullptr, g.c, g.kh, g.kw};
+    if (!wpacked) {
+        f.w = w;
+        f.packed = image + img_bytes;
+        f.wsum = reinterpret_cast<int32_t *>(f.packed + f_bytes);
+        wpacked = f.packed;
+        wsum = f.wsum;
+    }
     if (fused_input) {
         const bool qdiv = (dyn.quant_mode & HIPQ_FORM_DIV) != 0, qeven = (dyn.quant_mode & HIPQ_ROUND_HALF_EVEN) != 0;
         // Prepared filters of at most 1 MiB: touched by the quantizer while it waits (variant 11 switches it off).
         const size_t filter_bytes = packed_operand_bytes(g.oc, k);
-        const bool touching = wpacked && ctx->gemm_variant != 11 && filter_bytes <= (size_t(1) << 20);
+        const bool touching = ctx->gemm_variant != 11 && filter_bytes <= (size_t(1) << 20);
         const uint32_t *touch = touching ? reinterpret_cast<const uint32_t *>(wpacked) : nullptr;
         const uint32_t touch_lines = touching ? static_cast<uint32_t>(filter_bytes / 128) : 0u;
 #define HIPQ_LAUNCH_CQ(D, E)                                                                                          \
     hipLaunchKernelGGL((conv_quantize_pack_image_kernel<D, E>), dim3(static_cast<int>(pack_grid)), dim3(kConvThreads), 0, \
                        ctx->stream, dyn.x, g.c, g.h, g.w, g.ph, g.pw, dyn.flavor, g.nb, groups_per_cb, dyn.params,    \
-                       ctx->wait_error, ctx->wait_spin_limit, ximg, static_cast<int>(pixels), touch, touch_lines)
+                       ctx->wait_error, ctx->wait_spin_limit, image, touch, touch_lines)
         if (qdiv && qeven)
             HIPQ_LAUNCH_CQ(true, 1);
         else if (qdiv)
@@ -359,52 +342,27 @@ static int32_t conv_forward(const char *fn, hipq_ctx *ctx, const uint8_t *x, int
         else
             HIPQ_LAUNCH_CQ(false, 0);
 #undef HIPQ_LAUNCH_CQ
+        rc = check_launch(fn);
+    } else if (dyn.x) {
+        uint8_t *xq = reinterpret_cast<uint8_t *>(image + img_bytes + w_bytes);
+        rc = quantize_dynamic_per_tensor(ctx, dyn.x, elems, dyn.flavor, HIPQ_DTYPE_U8, dyn.quant_mode, xq, dyn.params,
+                                         nullptr, 0);
+        if (rc) return rc;
+        // the call above may have grown (moved) the scratch
+        if ((rc = scratch(ctx, kScratchHeader + img_bytes + w_bytes + u8_bytes, &s))) return rc;
+        if (static_cast<char *>(s) + kScratchHeader != reinterpret_cast<char *>(image))
+            return fail(HIPQ_DEVICE_ERROR, "%s: scratch moved under a pending kernel", fn);
+        rc = launch_window_pack(fn, ctx, xq, 0, &dyn.params->zero_point, g, cw, image, f);
     } else {
-        if (dyn.x) {
-            uint8_t *xq = reinterpret_cast<uint8_t *>(ximg + align256(img_bytes) + w_bytes);
-            rc = quantize_dynamic_per_tensor(ctx, dyn.x, size_t(g.nb) * g.c * g.h * g.w, dyn.flavor, HIPQ_DTYPE_U8,
-                                             dyn.quant_mode, xq, dyn.params, nullptr, 0);
-            if (rc) return rc;
-            // the call above may have grown (moved) the scratch
-            if ((rc = scratch(ctx, kScratchHeader + align256(img_bytes) + w_bytes + u8_bytes, &s))) return rc;
-            if (static_cast<char *>(s) + kScratchHeader != reinterpret_cast<char *>(ximg))
-                return fail(HIPQ_DEVICE_ERROR, "%s: scratch moved under a pending kernel", fn);
-            x = xq;
-        }
-        hipLaunchKernelGGL(conv_pack_image_kernel, dim3(static_cast<int>(pack_grid)), dim3(kConvThreads), 0, ctx->stream,
-                           x, g.c, g.h, g.w, g.ph, g.pw, zp_in, dyn.x ? &dyn.params->zero_point : nullptr, g.nb,
-                           groups_per_cb, ximg, static_cast<int>(pixels));
+        rc = launch_window_pack(fn, ctx, x, zp_in, nullptr, g, cw, image, f);
     }
-    if ((rc = check_launch(fn))) return rc;
-    if (!wpacked) {
-        int8_t *staging = ximg + align256(img_bytes);
-        int8_t *pbuf = staging + align256(size_t(g.oc) * k);
-        int32_t *wsbuf = reinterpret_cast<int32_t *>(pbuf + align256(packed_operand_bytes(g.oc, k)));
-        if ((rc = pack_filters(ctx, w, g.oc, g.c, taps, staging, pbuf, wsbuf))) return rc;
-        wpacked = pbuf;
-        wsum = wsbuf;
-    }
-    GemmEpilogue ep{nullptr, 0, sw, bias, s_out, zp_out, out};
-    ep.s_out_inv = host_recip_for_div(s_out);
-    ep.sa_scalar = s_in;
-    ep.cv_kw = g.kw;
-    ep.cv_wp = wp;
-    ep.cv_hp = hp;
-    ep.cv_c = g.c;
-    ep.cv_ho = g.ho;
-    ep.cv_wo = g.wo;
-    ep.cv_oc = g.oc;
-    ep.cv_nb = g.nb;
+    if (rc) return rc;
     ep.cv_wsum = wsum;
-    ep.cv_corr_mul = 128 - zp_in;
     if (dyn.x) {
         ep.sa = &dyn.params->scale;  // NaN for a range that is not finite: the outputs then carry no information
         ep.cv_zp_in = &dyn.params->zero_point;
     }
-    ep.cv_pixels = static_cast<int>(pixels);
-    ep.cv_kblocks = taps * cbs;
-    ep.fresh_activations = 1;  // the image was written by the kernel just before
-    return conv_gemm_packed(ctx, wpacked, ximg, g.oc, g.nb * hp * wp, static_cast<int>(k), ep, EPI, EVEN);
+    return launch_conv_window<EPI, EVEN>(ctx, wpacked, image, cw, ep);
 }
 
 static int32_t make_geom(const char *fn, size_t nb, size_t c, size_t h, size_t w, size_t oc, size_t kh, size_t kw,
@@ -527,7 +485,7 @@ int32_t hipq_conv2d_u8i8_i8_packed(hipq_ctx *ctx, const uint8_t *x, int32_t zp_i
     ConvGeom g;
     int32_t rc = make_geom(__func__, nb, c, h, wd, oc, kh, kw, 1, 1, pad_h, pad_w, &g);
     if (rc) return rc;
-    if (!fast_path_ok(g))
+    if (!prepared_ok(g))
         return fail(HIPQ_INVALID_ARGUMENT, "%s: packed filters need stride 1 and channels a multiple of 32", __func__);
     if (nb != 0 && oc != 0) {
         HIPQ_REQUIRE_PTR(w_packed);
@@ -546,7 +504,7 @@ int32_t hipq_conv2d_dynamic_f32_i8_packed(hipq_ctx *ctx, const float *x, int32_t
     ConvGeom g;
     int32_t rc = make_geom(__func__, nb, c, h, wd, oc, kh, kw, 1, 1, pad_h, pad_w, &g);
     if (rc) return rc;
-    if (!fast_path_ok(g))
+    if (!prepared_ok(g))
         return fail(HIPQ_INVALID_ARGUMENT, "%s: packed filters need stride 1 and channels a multiple of 32", __func__);
     if (flavor < HIPQ_PARAMS_SYMMETRIC || flavor > HIPQ_PARAMS_NN_ASYMMETRIC)
         return fail(HIPQ_INVALID_ARGUMENT, "%s: unknown flavor %d", __func__, flavor);

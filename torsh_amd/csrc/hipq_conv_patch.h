@@ -23,13 +23,118 @@
 // its share with LDS byte reads at immediate offsets: lanes are consecutive pixels, consecutive bytes of a raw row.
 //
 // M = filters, N = padded pixels (n * hp * wp), K = taps * channels, tap-major.  Geometries taken: see
-// conv_patch_fits; all others run the two-launch form.  Epilogue: conv_store_block (hipq_gemm_packed.h).
+// conv_patch_fits; all others run the two-launch form.  Epilogue: conv_store_block.
 // Included by hipq_gemm_packed.hip.
 #pragma once
 
 #include "hipq_gemm_packed.h"
 
 namespace hipq {
+
+// Convolution epilogue of one 32-row block (rows = output channels from `row0`, a lane = one window per column
+// block): accumulator + (128 - zp_in) * sum of the filter's weights, then the Linear's dequantize / requantize
+// arithmetic, stored to NCHW (consecutive lanes are consecutive ow: consecutive bytes).  c_l / s_l / b_l: the
+// correction, combined scale and bias of row row0 + lane % 32, handed round by shuffles.
+//
+// With one wave per SIMD the epilogue is bound by instruction issue, so the common case - the whole row block
+// inside the output channels, the output below 2 GiB - has no branch and no 64-bit address per element: the
+// stores are buffer stores whose per-lane offset (the window's place in its image plus the lane half's four
+// rows; beyond the buffer for a window of the padded grid that is not an output, which makes the hardware drop
+// the store) is formed once, and whose row offset is scalar.
+template <int TNB, int EPI, bool EVEN>
+__device__ __forceinline__ void conv_store_block(v16i (&own)[1][TNB], const GemmEpilogue &ep, int M, int row0, int lane,
+                                                 const size_t (&out_base)[TNB], const bool (&valid)[TNB], int c_l,
+                                                 float s_l, float b_l) {
+    constexpr int ES = EPI == EPI_I8 ? 1 : 4;  // bytes per output element
+    const float zpf = static_cast<float>(ep.zp_out);
+    const bool has_bias = ep.bias != nullptr;
+    const size_t plane = size_t(ep.cv_ho) * ep.cv_wo;
+    wait_vmcnt<0>();
+    float s_row[16], b_row[16];
+    int c_row[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const int src = 8 * (r / 4) + 4 * (lane / 32) + (r % 4);  // row of the block = lane that holds its operands
+        c_row[r] = __shfl(c_l, src, kWave);
+        s_row[r] = __shfl(s_l, src, kWave);
+        b_row[r] = __shfl(b_l, src, kWave);
+    }
+    // The element's bits (int8 in the low byte for EPI_I8).  FAST_DIV / BIAS are hoisted out of the element loop
+    // so that its body is straight-line code the compiler can interleave across the 32 outputs of a lane.
+    auto value = [&](int r, int j, auto fast_div, auto with_bias) -> int {
+        const int a = own[0][j][r] + c_row[r];
+        if constexpr (EPI == EPI_I32) {
+            return a;
+        } else {
+            float v = static_cast<float>(a) * s_row[r];
+            if constexpr (decltype(with_bias)::value) v = v + b_row[r];
+            if constexpr (EPI == EPI_F32) {
+                return __builtin_bit_cast(int, v);
+            } else {
+                float q;
+                if constexpr (decltype(fast_div)::value) {
+                    const float q0 = v * ep.s_out_inv;  // div_rn with a usable reciprocal
+                    const float rem = fmaf(-q0, ep.s_out, v);
+                    const float q1 = fmaf(rem, ep.s_out_inv, q0);
+                    q = (rem == rem) ? q1 : q0;
+                } else {
+                    q = v / ep.s_out;
+                }
+                return clamp_to_int(round_mode<EVEN>(q) + zpf, -128, 127);  // NaN -> 0, as `as i8` after the clamp
+            }
+        }
+    };
+    const size_t out_bytes = size_t(ep.cv_nb) * ep.cv_oc * plane * ES;
+    const bool whole = row0 + 32 <= M && out_bytes < (size_t(1) << 31);
+    const __amdgpu_buffer_rsrc_t ro =
+        __builtin_amdgcn_make_buffer_rsrc(ep.out, 0, whole ? static_cast<int>(out_bytes) : 0, 0x00020000);
+    int voff[TNB];
+#pragma unroll
+    for (int j = 0; j < TNB; ++j)
+        voff[j] = valid[j] ? static_cast<int>((out_base[j] + size_t(4 * (lane / 32)) * plane) * ES) : 0x7fffffff;
+    const int plane_bytes = static_cast<int>(plane) * ES;
+    auto emit = [&](auto fast_div, auto with_bias) {
+        if (whole) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int soff = (row0 + 8 * (r / 4) + (r % 4)) * plane_bytes;
+#pragma unroll
+                for (int j = 0; j < TNB; ++j) {
+                    const int bits = value(r, j, fast_div, with_bias);
+                    if constexpr (EPI == EPI_I8)
+                        __builtin_amdgcn_raw_buffer_store_b8(static_cast<char>(bits), ro, voff[j], soff, 0);
+                    else
+                        __builtin_amdgcn_raw_buffer_store_b32(bits, ro, voff[j], soff, 0);
+                }
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int m = row0 + 8 * (r / 4) + 4 * (lane / 32) + (r % 4);
+                if (m >= M) continue;
+#pragma unroll
+                for (int j = 0; j < TNB; ++j) {
+                    if (!valid[j]) continue;
+                    const size_t off = out_base[j] + size_t(m) * plane;
+                    const int bits = value(r, j, fast_div, with_bias);
+                    if constexpr (EPI == EPI_I8)
+                        static_cast<int8_t *>(ep.out)[off] = static_cast<int8_t>(bits);
+                    else
+                        static_cast<int32_t *>(ep.out)[off] = bits;
+                }
+            }
+        }
+    };
+    const bool fast = ep.s_out_inv != 0.0f;
+    if (fast && has_bias)
+        emit(std::true_type{}, std::true_type{});
+    else if (fast)
+        emit(std::true_type{}, std::false_type{});
+    else if (has_bias)
+        emit(std::false_type{}, std::true_type{});
+    else
+        emit(std::false_type{}, std::false_type{});
+}
 
 struct ConvPatch {
     const uint8_t *x;  // [nb, c, h, w]

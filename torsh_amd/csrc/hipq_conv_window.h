@@ -1,0 +1,405 @@
+// Quantized Conv2d of any stride and any channel count as an implicit GEMM on the matrix cores: rows of the product
+// are the output positions ("windows", in output order: no padded grid), columns the output channels.
+//
+// Image layout.  The u8 NCHW input is rewritten once as signed bytes (x - 128) in
+//   [channel group][image][padded row][padded pixel][pitch]
+// with the channels cut into ceil(C / 32) groups of `pitch` bytes (the group's channels, rounded up to 4) and a border
+// of the zero point.  One row of a filter's taps then covers kw * pitch CONSECUTIVE bytes, whatever the stride, so K is
+// cut into k blocks of 32 bytes along (tap row, 32-byte piece of the row, channel group): a window's slice of a k block
+// is two 16-byte pieces at (address of its first pixel) + (an offset that is the same for every window), which is
+// exactly what a lane of v_mfma_i32_32x32x32_i8 holds.  A wave loads 32 windows' slice with one instruction whose
+// per-lane offset never changes and whose k block is a scalar: no im2col, no gather, no LDS.  Windows overlap in
+// memory; the vector-memory path and L1 see that, HBM does not.  Three channels (pitch 4, 7 taps: 28 of 32 bytes
+// used) waste an eighth of the multiply, 32 channels nothing.  What a slice reads beyond its row of taps are other
+// pixels' bytes; the packed filters hold zeros there.
+//
+// The filters are packed in the fragment order of hipq_gemm_packed.h with the same K order, and
+// sum (x - zp) w = sum (x - 128) w + (128 - zp) sum w is undone per output channel in the epilogue.
+//
+// Measured against what it replaced, u8 in, filters as rows (us per forward): [32,3,224,224] x [64,3,7,7] stride 2
+// 2288 -> 31 (a thread per output); [32,64,56,56] x [64,64,3,3] 63 -> 24, [32,128,28,28] x [128,128,3,3] 26.4 -> 20.4,
+// [32,256,14,14] x [256,256,3,3] 20.9 -> 17.5, [32,512,7,7] x [512,512,3,3] 28.0 -> 25.9, [32,256,56,56] x [64,256,1,1] 50 -> 33
+// (the packed GEMM over the padded grid, which always split K: its 128 x 64 tiles spend more on the sum of the partial
+// products than on short K, compute the windows of the border, and store single bytes).  What bounds it now: at long K
+// the vector-memory path, 6 KiB per 8 MFMAs; at short K (the first layer) instruction issue, ~1100 vector instructions
+// per wave of which 700 are the requantize of its 64 x 64 outputs, and the misaligned 16-byte pieces (34 L1 accesses
+// per load of overlapping windows, 16 where they are a contiguous KiB).
+//
+// Waves.  A workgroup's four waves either take different windows (SPLIT = false: FM x FN accumulator blocks each, the
+// filters' fragments coming out of L1 for three of the four) or split K and sum through LDS (SPLIT = true), which keeps
+// all SIMDs busy when there are fewer tiles than that.  A lane of the accumulators holds ONE output channel and 16
+// windows: its scale, bias and zero-point correction are one register each, and after one exchange between the halves
+// of the wave it owns 16 consecutive outputs of a channel's plane: one 16-byte store.
+#pragma once
+
+#include <type_traits>
+
+#include "hipq_gemm_kernels.h"
+
+namespace hipq {
+
+struct ConvWindow {
+    int M, N;             // output channels; windows = images * ho * wo
+    int KB, kblocks;      // k blocks per filter row block as stored; those that hold data
+    int cgs, segs;        // channel groups; 32-byte pieces per row of taps
+    int pitch;            // bytes per pixel and channel group
+    int row_bytes;        // wp * pitch
+    int plane_bytes;      // bytes per channel group (nb * hp * wp * pitch)
+    int image_bytes;      // cgs * plane_bytes
+    int hp, wp, sh, sw, ho, wo;
+};
+
+// u8 NCHW -> the layout above.  One thread per (channel group, padded pixel), DW dwords of four channels each
+// (consecutive lanes are consecutive pixels: consecutive bytes of every channel plane).  Workgroups past the image
+// pack the filters: one output channel each, a thread per 16-byte piece.
+struct ConvWindowFilters {
+    const int8_t *w;  // [OC, IC, KH, KW]
+    int8_t *packed;
+    int32_t *wsum;
+    int ic, kh, kw;
+};
+
+template <int DW>
+__global__ __launch_bounds__(256) void conv_window_pack_kernel(const uint8_t *__restrict__ x, int C, int H, int W, int pad_h,
+                                                                 int pad_w, int zp, const int32_t *__restrict__ zp_dev,
+                                                                 int nb, int groups_per_cg, int8_t *__restrict__ image,
+                                                                 ConvWindow cw, ConvWindowFilters f) {
+    const int work = cw.cgs * groups_per_cg;
+    if (static_cast<int>(blockIdx.x) >= work) {
+        __shared__ int part[4];
+        const int oc = blockIdx.x - work;
+        const int8_t *w = f.w + size_t(oc) * f.ic * f.kh * f.kw;
+        int sum = 0;
+        for (int piece = threadIdx.x; piece < cw.KB * 2; piece += 256) {
+            const int kb = piece / 2, half = piece % 2;
+            const int cg = kb % cw.cgs, seg = (kb / cw.cgs) % cw.segs, ty = kb / (cw.cgs * cw.segs);
+            uint32_t d[4] = {0, 0, 0, 0};
+            if (kb < cw.kblocks) {
+                int p = seg * 32 + half * 16;  // byte within the row of taps
+                int tx = p / cw.pitch, c = p % cw.pitch;
+#pragma unroll
+                for (int b = 0; b < 16; ++b) {
+                    const int ch = cg * cw.pitch + c;
+                    if (tx < f.kw && ch < f.ic) {
+                        const int8_t v = w[(size_t(ch) * f.kh + ty) * f.kw + tx];
+                        sum += v;
+                        d[b / 4] |= static_cast<uint32_t>(static_cast<uint8_t>(v)) << (8 * (b % 4));
+                    }
+                    if (++c == cw.pitch) {
+                        c = 0;
+                        ++tx;
+                    }
+                }
+            }
+            *reinterpret_cast<uint4 *>(f.packed + (size_t(oc / 32) * cw.KB + kb) * 1024 + (oc % 32 + 32 * half) * 16) =
+                make_uint4(d[0], d[1], d[2], d[3]);
+        }
+#pragma unroll
+        for (int o = kWave / 2; o > 0; o >>= 1) sum += __shfl_xor(sum, o, kWave);
+        if (threadIdx.x % kWave == 0) part[threadIdx.x / kWave] = sum;
+        __syncthreads();
+        if (threadIdx.x == 0) f.wsum[oc] = part[0] + part[1] + part[2] + part[3];
+        return;
+    }
+    if (zp_dev) zp = *zp_dev;  // the zero point a dynamic quantize has left on the device
+    const int cg = blockIdx.x / groups_per_cg;
+    const int p = (blockIdx.x % groups_per_cg) * 256 + threadIdx.x;
+    if (p >= nb * cw.hp * cw.wp) return;
+    const int n = p / (cw.hp * cw.wp), rem = p % (cw.hp * cw.wp);
+    const int h = rem / cw.wp - pad_h, v = rem % cw.wp - pad_w;
+    uint32_t d[DW];
+    const uint32_t border = static_cast<uint32_t>(static_cast<uint8_t>(zp ^ 0x80)) * 0x01010101u;
+#pragma unroll
+    for (int i = 0; i < DW; ++i) d[i] = border;
+    if (h >= 0 && h < H && v >= 0 && v < W) {
+        const size_t plane = size_t(H) * W;
+        const int c0 = cg * DW * 4;
+        const uint8_t *src = x + ((size_t(n) * C + c0) * H + h) * W + v;
+        uint32_t b[4 * DW];
+#pragma unroll
+        for (int c = 0; c < 4 * DW; ++c) b[c] = c0 + c < C ? src[size_t(c) * plane] : 0u;
+#pragma unroll
+        for (int i = 0; i < DW; ++i)
+            d[i] = (b[4 * i] | (b[4 * i + 1] << 8) | (b[4 * i + 2] << 16) | (b[4 * i + 3] << 24)) ^ 0x80808080u;
+    }
+    uint32_t *dst = reinterpret_cast<uint32_t *>(image + size_t(cg) * cw.plane_bytes + size_t(p) * (4 * DW));
+    if constexpr (DW % 4 == 0) {
+#pragma unroll
+        for (int i = 0; i < DW; i += 4) *reinterpret_cast<uint4 *>(dst + i) = make_uint4(d[i], d[i + 1], d[i + 2], d[i + 3]);
+    } else {
+#pragma unroll
+        for (int i = 0; i < DW; ++i) dst[i] = d[i];
+    }
+}
+
+// 16 and 4 x 4 bytes to an address that need not be aligned (global memory takes it; the outputs of a channel's plane
+// start wherever ho * wo puts them).
+struct __attribute__((packed, aligned(1))) ConvBytes16 {
+    v4i v;
+};
+struct __attribute__((packed, aligned(4))) ConvWords4 {
+    v4i v;
+};
+
+template <int FM, int FN, int D, bool SPLIT, int EPI, bool EVEN>
+__global__ __launch_bounds__(256, FM * FN < 8 ? 3 : (SPLIT ? 1 : 2)) void conv_i8_window_kernel(const int8_t *__restrict__ filters,
+                                                               const int8_t *__restrict__ image, ConvWindow cw,
+                                                               GemmEpilogue ep) {
+    constexpr int NBLK = FM * FN;
+    constexpr int OWN = SPLIT ? NBLK / 4 : NBLK;  // accumulator blocks a wave finishes
+    static_assert(!SPLIT || (NBLK % 4 == 0 && FN % OWN == 0), "the K-split waves share the blocks of one channel block each");
+    constexpr int COLS = SPLIT ? 1 : FM;          // channel blocks among them
+    extern __shared__ __attribute__((aligned(16))) int8_t lds[];
+    const int lane = threadIdx.x % kWave, half = lane / 32;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int plane = cw.ho * cw.wo;
+    // An XCD (workgroups b, b + 8, ...) takes a contiguous run of windows and, inside it, all channel tiles of a
+    // window tile one after the other: the image rows are fetched into its L2 once.
+    constexpr int kTileN = (SPLIT ? 1 : 4) * FN * 32;
+    const int tiles_m = ((cw.M + 31) / 32 + FM - 1) / FM, tiles_n = (cw.N + kTileN - 1) / kTileN;
+    const int per_xcd = (tiles_n + 7) / 8, slot = blockIdx.x / 8;
+    const int tile_m = slot % tiles_m, tile_n = static_cast<int>(blockIdx.x % 8) * per_xcd + slot / tiles_m;
+    if (slot / tiles_m >= per_xcd || tile_n >= tiles_n) return;
+    const int q0 = tile_n * kTileN + (SPLIT ? 0 : wave * FN * 32);  // first window of this wave
+    const int rb0 = tile_m * FM;
+
+    // Operands of the epilogue, ahead of the main loop: one channel per lane and channel block.
+    const int own0 = SPLIT ? wave * OWN : 0;  // first block (channel block own0 / FN, window fragment own0 % FN)
+    int corr[COLS];
+    float sc[COLS], bias[COLS];
+#pragma unroll
+    for (int j = 0; j < COLS; ++j) {
+        const int oc = (rb0 + own0 / FN + j) * 32 + lane % 32;
+        const int occ = oc < cw.M ? oc : cw.M - 1;
+        corr[j] = (ep.cv_zp_in ? 128 - *ep.cv_zp_in : ep.cv_corr_mul) * ep.cv_wsum[occ];
+        sc[j] = 1.0f;
+        bias[j] = -0.0f;  // (v + -0.0f is v, bit for bit)
+        if constexpr (EPI != EPI_I32) {
+            sc[j] = (ep.sa ? ep.sa[0] : ep.sa_scalar) * ep.sw[occ];
+            if (ep.bias) bias[j] = ep.bias[occ];
+        }
+    }
+
+    const __amdgpu_buffer_rsrc_t rf = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<int8_t *>(filters), 0, ((cw.M + 31) / 32) * cw.KB * 1024, 0x00020000);
+    const __amdgpu_buffer_rsrc_t ri =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t *>(image), 0, cw.image_bytes, 0x00020000);
+    int sof[FM];
+#pragma unroll
+    for (int j = 0; j < FM; ++j) {
+        const int rb = rb0 + j < (cw.M + 31) / 32 ? rb0 + j : (cw.M + 31) / 32 - 1;  // (repeated: not stored)
+        sof[j] = rb * cw.KB * 1024;
+    }
+    int voi[FN];
+#pragma unroll
+    for (int i = 0; i < FN; ++i) {
+        int q = q0 + i * 32 + lane % 32;
+        q = q < cw.N ? q : cw.N - 1;
+        const int n = q / plane, rem = q % plane;
+        const int oh = rem / cw.wo, ow = rem % cw.wo;
+        voi[i] = ((n * cw.hp + oh * cw.sh) * cw.wp + ow * cw.sw) * cw.pitch + 16 * half;
+    }
+    // This wave's next k block as (tap row, piece, channel group) and its offset in the image.
+    constexpr int STEP = SPLIT ? 4 : 1;
+    int kb = 0, cg = 0, seg = 0, ty = 0;
+    auto advance = [&](int by) {
+        kb += by;
+        cg += by;
+        while (cg >= cw.cgs) {
+            cg -= cw.cgs;
+            if (++seg == cw.segs) {
+                seg = 0;
+                ++ty;
+            }
+        }
+    };
+    if constexpr (SPLIT) advance(wave);
+    v4i ff[D][FM], fi[D][FN];
+    auto issue = [&](int s) {
+        // k blocks past the last lie beyond both buffers: zeros, no memory access
+        const bool real = kb < cw.kblocks;
+        const int kof = real ? kb * 1024 : 0x7fffff00;
+        const int koi = real ? cg * cw.plane_bytes + ty * cw.row_bytes + seg * 32 : 0x7fffff00;
+#pragma unroll
+        for (int j = 0; j < FM; ++j)
+            ff[s][j] = __builtin_bit_cast(
+                v4i, __builtin_amdgcn_raw_buffer_load_b128(rf, lane * 16, real ? sof[j] + kof : kof, 0));
+#pragma unroll
+        for (int i = 0; i < FN; ++i)
+            fi[s][i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(ri, voi[i], koi, 0));
+        advance(STEP);
+    };
+    v16i acc[FM][FN];
+#pragma unroll
+    for (int j = 0; j < FM; ++j)
+#pragma unroll
+        for (int i = 0; i < FN; ++i)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[j][i][r] = SPLIT ? 0 : corr[j];
+    auto compute = [&](int s) {
+#pragma unroll
+        for (int j = 0; j < FM; ++j)
+#pragma unroll
+            for (int i = 0; i < FN; ++i)
+                acc[j][i] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fi[s][i], ff[s][j], acc[j][i], 0, 0, 0);
+    };
+    const int steps = (cw.kblocks + STEP - 1) / STEP, rounds_end = (steps + D - 1) / D * D;
+#pragma unroll
+    for (int u = 0; u < D; ++u) issue(u);
+    for (int s0 = D; s0 < rounds_end; s0 += D) {
+#pragma unroll
+        for (int u = 0; u < D; ++u) {
+            compute(u);
+            issue(u);
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < D; ++u) compute(u);
+
+    // Outputs of one accumulator block: channel block column j of this wave's constants, first window q.
+    const float zpf = static_cast<float>(ep.zp_out);
+    const uint32_t offset2 = static_cast<uint32_t>(ep.zp_out + 128) * 0x10001u;
+    auto emit_block = [&](const v16i &a, int j, int oc, int q, auto plain) {
+        auto dequant = [&](int r) { return static_cast<float>(a[r]) * sc[j] + bias[j]; };
+        if constexpr (EPI == EPI_I8) {
+            // register 4 g + i of half h is window 8 g + 4 h + i; after the exchange half h holds windows 16 h .. + 15
+            uint32_t w[4];
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const float v[4] = {dequant(4 * g), dequant(4 * g + 1), dequant(4 * g + 2), dequant(4 * g + 3)};
+                if constexpr (decltype(plain)::value) {
+                    w[g] = requant_pack4<EVEN>(v, ep.s_out, ep.s_out_inv, offset2);
+                } else {
+                    auto code = [&](float f) {  // NaN -> 0
+                        return clamp_to_int(round_mode<EVEN>(div_rn(f, ep.s_out, ep.s_out_inv)) + zpf, -128, 127);
+                    };
+                    w[g] = pack4(code(v[0]), code(v[1]), code(v[2]), code(v[3]));
+                }
+            }
+            const auto lo = __builtin_amdgcn_permlane32_swap(w[0], w[2], false, false);
+            const auto hi = __builtin_amdgcn_permlane32_swap(w[1], w[3], false, false);
+            const v4i bytes = {static_cast<int>(lo[0]), static_cast<int>(lo[1]), static_cast<int>(hi[0]),
+                               static_cast<int>(hi[1])};
+            const int first = q + 16 * half;
+            if (oc >= cw.M || first >= cw.N) return;
+            const int n = first / plane, pos = first % plane;
+            int8_t *o = static_cast<int8_t *>(ep.out) + (size_t(n) * cw.M + oc) * plane + pos;
+            if (pos + 16 <= plane) {
+                reinterpret_cast<ConvBytes16 *>(o)->v = bytes;
+            } else {  // the run crosses into the next image (or the end)
+                const size_t skip = size_t(cw.M - 1) * plane;  // from the end of this plane to the next image's
+                int at = pos;
+#pragma unroll
+                for (int k = 0; k < 16; ++k) {
+                    if (first + k < cw.N) *o = static_cast<int8_t>(bytes[k / 4] >> (8 * (k % 4)));
+                    ++o;
+                    if (++at == plane) {
+                        at = 0;
+                        o += skip;
+                    }
+                }
+            }
+        } else {
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                auto bits = [&](int r) {
+                    if constexpr (EPI == EPI_I32) return a[r];
+                    return __builtin_bit_cast(int, dequant(r));
+                };
+                const v4i four = {bits(4 * g), bits(4 * g + 1), bits(4 * g + 2), bits(4 * g + 3)};
+                const int first = q + 8 * g + 4 * half;
+                if (oc >= cw.M || first >= cw.N) continue;
+                const int n = first / plane, pos = first % plane;
+                int32_t *o = static_cast<int32_t *>(ep.out) + (size_t(n) * cw.M + oc) * plane + pos;
+                if (pos + 4 <= plane) {
+                    reinterpret_cast<ConvWords4 *>(o)->v = four;
+                } else {
+                    const size_t skip = size_t(cw.M - 1) * plane;
+                    int at = pos;
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        if (first + k < cw.N) *o = four[k];
+                        ++o;
+                        if (++at == plane) {
+                            at = 0;
+                            o += skip;
+                        }
+                    }
+                }
+            }
+        }
+    };
+    bool all_plain = true;
+    if constexpr (EPI == EPI_I8) {
+#pragma unroll
+        for (int j = 0; j < COLS; ++j) all_plain = all_plain && requant_is_plain(sc[j], bias[j], ep.s_out_inv);
+    }
+    auto with_division = [&](auto finish) {
+        if constexpr (EPI == EPI_I8) {
+            if (!all_plain) return finish(std::false_type{});
+        }
+        finish(std::true_type{});
+    };
+    if constexpr (!SPLIT) {
+        with_division([&](auto plain) {
+#pragma unroll
+            for (int j = 0; j < FM; ++j)
+#pragma unroll
+                for (int i = 0; i < FN; ++i) emit_block(acc[j][i], j, (rb0 + j) * 32 + lane % 32, q0 + i * 32, plain);
+        });
+    } else {
+        // Block b = j * FN + i belongs to wave b / OWN; the other three park their partial sums of it in LDS.
+        v4i *red = reinterpret_cast<v4i *>(lds);
+#pragma unroll
+        for (int b = 0; b < NBLK; ++b) {
+            const int owner = b / OWN;
+            if (owner == wave) continue;
+            v4i *dst = red + (((wave - owner + 3) % 4) * NBLK + b) * 4 * kWave + lane;
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+                dst[g * kWave] = v4i{acc[b / FN][b % FN][4 * g], acc[b / FN][b % FN][4 * g + 1],
+                                     acc[b / FN][b % FN][4 * g + 2], acc[b / FN][b % FN][4 * g + 3]};
+        }
+        v16i own[OWN];
+#pragma unroll
+        for (int b = 0; b < NBLK; ++b)
+            if (b / OWN == wave) own[b % OWN] = acc[b / FN][b % FN];
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < OWN; ++k) {
+            v4i part[3][4];
+#pragma unroll
+            for (int s = 0; s < 3; ++s)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) part[s][g] = red[((s * NBLK + own0 + k) * 4 + g) * kWave + lane];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) own[k][r] += corr[0] + part[0][r / 4][r % 4] + part[1][r / 4][r % 4] + part[2][r / 4][r % 4];
+        }
+        with_division([&](auto plain) {
+#pragma unroll
+            for (int k = 0; k < OWN; ++k)
+                emit_block(own[k], 0, (rb0 + own0 / FN) * 32 + lane % 32, q0 + ((own0 + k) % FN) * 32, plain);
+        });
+    }
+}
+
+template <int FM, int FN, int D, bool SPLIT, int EPI, bool EVEN>
+static int32_t launch_conv_window_form(hipq_ctx *ctx, const int8_t *filters, const int8_t *image, const ConvWindow &cw,
+                                       const GemmEpilogue &ep) {
+    constexpr int kLds = SPLIT ? FM * FN * 3 * 4096 : 0;
+    auto kernel = conv_i8_window_kernel<FM, FN, D, SPLIT, EPI, EVEN>;
+    static bool configured[16] = {false};  // per device: raise the dynamic LDS limit once
+    if (SPLIT && ctx->device < 16 && !configured[ctx->device]) {
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
+        if (e != hipSuccess)
+            return fail(HIPQ_DEVICE_ERROR, "conv2d: cannot reserve %d bytes of LDS: %s", kLds, hipGetErrorString(e));
+        configured[ctx->device] = true;
+    }
+    constexpr int kTileN = (SPLIT ? 1 : 4) * FN * 32;
+    const int tiles_m = ((cw.M + 31) / 32 + FM - 1) / FM, tiles_n = (cw.N + kTileN - 1) / kTileN;
+    hipLaunchKernelGGL(kernel, dim3((tiles_n + 7) / 8 * 8 * tiles_m), dim3(256), kLds, ctx->stream, filters, image, cw, ep);
+    return check_launch("conv2d (windows)");
+}
+
+}  // namespace hipq

@@ -22,15 +22,13 @@ struct GemmEpilogue {
     int zp_out;
     void *out;  // int32 / float / int8 [M,N]
     const float *residual = nullptr;  // fp32 epilogue only: added after the bias, [M,N]; may alias out
-    // Implicit-GEMM convolution (packed kernel, CONV): the row operand holds the packed filters, the column
-    // operand is the padded int8 image as [channel block of 32][pixel][32 bytes]; column q is the window whose
-    // top-left tap is padded pixel q = (n * hp + y) * wp + x, and K runs over (tap, channel).
+    // Convolution.  The one-launch form (hipq_conv_patch.h) numbers its windows over the padded image: window q has
+    // its top-left tap at padded pixel q = (n * hp + y) * wp + x, and K runs over (tap, channel).
     int cv_kw = 0, cv_wp = 0, cv_hp = 0, cv_c = 0;
     int cv_ho = 0, cv_wo = 0, cv_oc = 0, cv_nb = 0;
     const int32_t *cv_wsum = nullptr;  // [oc] sum of the filter's int8 weights
     int cv_corr_mul = 0;               // 128 - zp_in: accumulator += cv_corr_mul * cv_wsum[oc]
     const int32_t *cv_zp_in = nullptr; // when set: the input zero point on the device, used instead of cv_corr_mul
-    int cv_pixels = 0;                 // pixels per channel block of the image buffer (with slack)
     int cv_kblocks = 0;                // taps * (c / 32): the k blocks that hold data
     float sa_scalar = 1.0f;            // activation scale used when sa is null
     float s_out_inv = 0.0f;            // recip_for_div(s_out), or 0 to divide directly (requantize only)
@@ -55,11 +53,7 @@ constexpr int kTracePoints = 6, kTraceWords = 8;
 // Row-major int8 [rows, k] -> fragment-packed operand (packed_operand_bytes(rows, k) bytes at dst).
 int32_t pack_rows(hipq_ctx *ctx, const int8_t *src, size_t rows, size_t k, int8_t *dst);
 size_t packed_operand_bytes(size_t rows, size_t k);
-// Implicit-GEMM convolution: `filters` packed [M = output channels, K = taps x channels], `image` in
-// [channel block][pixel][32] order, N = padded pixels; ep carries the cv_* geometry.  epi: EPI_I32 / _F32 / _I8.
-int32_t conv_gemm_packed(hipq_ctx *ctx, const int8_t *filters, const int8_t *image, int M, int N, int K,
-                         const GemmEpilogue &ep, int epi, bool even);
-// The same convolution in one launch, from the u8 NCHW input itself (hipq_conv_patch.h): `fits` says whether
+// The convolution in one launch, from the u8 NCHW input itself (hipq_conv_patch.h): `applicable` says whether
 // that form takes the geometry (c channels, padded width wp, kh x kw taps).
 bool conv_patch_applicable(int nb, int c, int h, int w, int hp, int wp, int kh, int kw);
 int32_t conv_gemm_patch(hipq_ctx *ctx, const int8_t *filters, const uint8_t *x, size_t x_bytes, int zp_in, int h, int w,

@@ -181,6 +181,36 @@ __device__ __forceinline__ uint32_t pack4(int a, int b, int c, int d) {
     return lo | hi;
 }
 
+// Four requantized bytes clamp(round(v / s) + zp, -128, 127) in one dword, for values whose quotient is finite
+// (requant_is_plain).  inv = recip_for_div(s), not 0; offset2 holds zp + 128 in both halves.  Division as div_rn
+// without its guards; the clamp by the saturating packs: to i16, + offset saturating, to u8, then the top bits flipped
+// (11 instructions per value where the guards and min / max per value made 18).
+template <bool EVEN>
+__device__ __forceinline__ uint32_t requant_pack4(const float (&v)[4], float s, float inv, uint32_t offset2) {
+    int q[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float q0 = v[i] * inv;
+        const float d = fmaf(fmaf(-q0, s, v[i]), inv, q0);
+        // v_cvt_i32_f32 truncates: the trunc of round_mode<0> is its own
+        q[i] = cvt_i32_sat(EVEN ? rintf(d) : d + copysignf(0x1.fffffep-2f, d));
+    }
+    uint32_t h[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        uint32_t t;
+        asm("v_cvt_pk_i16_i32 %0, %1, %2" : "=v"(t) : "v"(q[2 * i]), "v"(q[2 * i + 1]));
+        asm("v_pk_add_i16 %0, %1, %2 clamp" : "=v"(t) : "v"(t), "v"(offset2));
+        asm("v_sat_pk_u8_i16 %0, %1" : "=v"(h[i]) : "v"(t));
+    }
+    return ((h[1] << 16) | h[0]) ^ 0x80808080u;
+}
+// Whether requant_pack4 may take every value acc * scale + bias (|acc| < 2^31) of this wave.
+__device__ __forceinline__ bool requant_is_plain(float scale, float bias, float inv) {
+    const float most = (fabsf(scale) * 2147483648.0f + fabsf(bias)) * fabsf(inv);
+    return inv != 0.0f && __all(most < 1e37f);
+}
+
 // 4 x 4 byte transpose inside a quad of lanes: lane q holds bytes (row 0..3) of column q and ends with the bytes
 // (column 0..3) of row q.  Two butterfly steps - swap with lane q ^ 1 and interleave bytes, swap with lane q ^ 2 and
 // interleave halves - each a data-parallel move and a byte permute whose selector depends on the lane:
