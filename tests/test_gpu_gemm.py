@@ -376,3 +376,27 @@ def test_output_larger_than_four_gib(ctx, hipq, oracle):
     out = ctx.linear_i8_f32(a, dev(sa0).repeat(reps), w, dev(sw0).repeat(reps), dev(b0).repeat(reps))
     torch.cuda.synchronize()
     assert bool((out.view(reps, blk, reps, blk) == dev(out0)[None, :, None, :]).all())
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 17, 16), (16, 40, 17), (5, 33, 65), (3, 100, 1001), (17, 64, 31), (64, 65, 127), (65, 130, 129),
+                                   (130, 4200, 143), (33, 90, 257), (300, 200, 1023), (2, 50, 4099)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_gemm_any_k_and_alignment(ctx, oracle, m, n, k, shift):
+    """K that is no multiple of 16 and operands at odd addresses: rows are read in 16-byte pieces at any alignment and
+    the piece over a row's end is shifted down, so the last row must not be read past its end (the operands end where
+    their allocation ends, in a guard of other values)."""
+    rng = np.random.default_rng(m * 31 + n * 7 + k)
+    a, w = rand_i8(rng, (m, k)), rand_i8(rng, (n, k))
+
+    def placed(v):
+        buf = torch.full((v.size + shift + 64,), 77, dtype=torch.int8, device="cuda")
+        part = buf[shift:shift + v.size].view(v.shape)
+        part.copy_(torch.from_numpy(v))
+        return part
+
+    acc = oracle.gemm_i8_nk(a, w)
+    np.testing.assert_array_equal(host(ctx.gemm_i8_i32(placed(a), placed(w))), acc)
+    sa, sw = rng.uniform(1e-3, 1e-2, m).astype(np.float32), rng.uniform(1e-4, 1e-3, n).astype(np.float32)
+    bias = rng.standard_normal(n).astype(np.float32)
+    got = host(ctx.linear_i8_f32(placed(a), dev(sa), placed(w), dev(sw), dev(bias)))
+    np.testing.assert_array_equal(got, acc.astype(np.float32) * (sa[:, None] * sw[None, :]) + bias[None, :])

@@ -79,7 +79,8 @@ __device__ __forceinline__ void gemv_store(const GemmEpilogue &ep, v4i sum, int 
 // MFMAs then run off registers while the next batch is already in flight.  The
 // four partial 16x16 accumulators are summed through LDS (integer adds: order
 // independent).
-template <int G, int EPI, bool EVEN>
+// ANYK: operands of any alignment and any K >= 16, the steps dealt to the waves in four runs.
+template <int G, int EPI, bool EVEN, bool ANYK = false>
 __global__ __launch_bounds__(kGemmThreads) void gemv_i8_kernel(const int8_t *__restrict__ A,
                                                                const int8_t *__restrict__ W, int M, int N, int K,
                                                                GemmEpilogue ep) {
@@ -89,8 +90,9 @@ __global__ __launch_bounds__(kGemmThreads) void gemv_i8_kernel(const int8_t *__r
     const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
     const int n0 = blockIdx.x * (16 * G);
     const int frow = lane % 16, g = lane / 16;
-    const int kw = K / NW;  // bytes of K per wave, a multiple of 64
-    const int kbeg = wave * kw;
+    const int per = ANYK ? ((K + 63) / 64 + NW - 1) / NW * 64 : K / NW;  // bytes of K per wave, a multiple of 64
+    const int kbeg = wave * per;
+    const int kw = ANYK ? (K - kbeg < per ? K - kbeg : per) : per;  // (ANYK: the last waves' runs may be short or empty)
     const int mrow = frow < M ? frow : M - 1;
     const int8_t *ap = A + size_t(mrow) * K + kbeg + g * 16;
     const int8_t *wp[G];
@@ -117,17 +119,23 @@ __global__ __launch_bounds__(kGemmThreads) void gemv_i8_kernel(const int8_t *__r
     v4i acc[G];
 #pragma unroll
     for (int r = 0; r < G; ++r) acc[r] = v4i{0, 0, 0, 0};
+    auto piece = [&](const int8_t *row, int k) {  // k: bytes from kbeg + g * 16
+        if constexpr (ANYK) {
+            if (kbeg + k + 64 > K) return load_row_piece<true>(row, kbeg + k + g * 16, K);
+        }
+        return load_row_piece<false>(row, kbeg + k + g * 16, K);
+    };
     for (int k0 = 0; k0 < kw; k0 += BATCH * 64) {
         v4i fa[BATCH];
 #pragma unroll
         for (int u = 0; u < BATCH; ++u)
-            if (k0 + u * 64 < kw) fa[u] = *reinterpret_cast<const v4i *>(ap + k0 + u * 64);
+            if (k0 + u * 64 < kw) fa[u] = piece(ap - kbeg - g * 16, k0 + u * 64);
 #pragma unroll
         for (int r = 0; r < G; ++r) {
             v4i fw[BATCH];
 #pragma unroll
             for (int u = 0; u < BATCH; ++u)
-                if (k0 + u * 64 < kw) fw[u] = *reinterpret_cast<const v4i *>(wp[r] + k0 + u * 64);
+                if (k0 + u * 64 < kw) fw[u] = piece(wp[r] - kbeg - g * 16, k0 + u * 64);
 #pragma unroll
             for (int u = 0; u < BATCH; ++u)
                 if (k0 + u * 64 < kw) acc[r] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fw[u], fa[u], acc[r], 0, 0, 0);
@@ -246,8 +254,7 @@ static int32_t launch_gemv(hipq_ctx *ctx, const int8_t *a, const int8_t *w, int 
     return check_launch("gemv_i8 (LDS staged)");
 }
 
-// Any shape, any alignment: one thread per output, plain integer dot product.
-// Used when K is not a multiple of 16 or an operand is not 16-byte aligned.
+// Any shape: one thread per output, plain integer dot product.  Used when K is below 16.
 template <int EPI, bool EVEN>
 __global__ __launch_bounds__(kGemmThreads) void gemm_i8_generic_kernel(const int8_t *__restrict__ A,
                                                                         const int8_t *__restrict__ W, int M, int N,
@@ -277,13 +284,13 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_i8_generic_kernel(const int
     }
 }
 
-template <int BM, int BN, int WM, int WN, int EPI, bool EVEN>
+template <int BM, int BN, int WM, int WN, int EPI, bool EVEN, bool ANYK = false>
 static void launch_tile(hipq_ctx *ctx, const int8_t *a, const int8_t *w, int M, int N, int K,
                         const GemmEpilogue &ep) {
     const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
     GemmEpilogue placed = ep;
     pick_xcd_rectangle(tiles_m, tiles_n, BM, BN, &placed.xcd_gm, &placed.xcd_gn);
-    hipLaunchKernelGGL((gemm_i8_mfma_kernel<BM, BN, WM, WN, EPI, EVEN>), dim3(tiles_m * tiles_n), dim3(kGemmThreads), 0,
+    hipLaunchKernelGGL((gemm_i8_mfma_kernel<BM, BN, WM, WN, EPI, EVEN, ANYK>), dim3(tiles_m * tiles_n), dim3(kGemmThreads), 0,
                        ctx->stream, a, w, M, N, K, placed);
 }
 
@@ -298,6 +305,21 @@ static int32_t launch_gemm(hipq_ctx *ctx, const int8_t *a, const int8_t *w, size
     const int M = static_cast<int>(m), N = static_cast<int>(n), K = static_cast<int>(k);
     const bool fast = (K % 16 == 0) && ((reinterpret_cast<uintptr_t>(a) & 15u) == 0) &&
                       ((reinterpret_cast<uintptr_t>(w) & 15u) == 0);
+    if (!fast && K >= 16) {
+        // Rows at any alignment (load_row_piece).  Instead of a thread per output, us: M = 300, N = 1000, K = 1001
+        // 1206 -> 11; 1 x 11008 x 4001 19, 64 x 4096 x 4097 26, 512 x 4096 x 4097 43.  The four waves of a
+        // workgroup split K up to 16 rows; what bounds it from there on is the register-staged tile's one stage in flight.
+        if (M <= 16) {
+            hipLaunchKernelGGL((gemv_i8_kernel<1, EPI, EVEN, true>), dim3((N + 15) / 16), dim3(kGemmThreads), 0, ctx->stream, a,
+                               w, M, N, K, ep);
+            return check_launch("gemv_i8 (any K)");
+        }
+        if (((m + 127) / 128) * ((n + 63) / 64) >= size_t(ctx->num_cus))
+            launch_tile<128, 64, 2, 2, EPI, EVEN, true>(ctx, a, w, M, N, K, ep);
+        else
+            launch_tile<64, 64, 2, 2, EPI, EVEN, true>(ctx, a, w, M, N, K, ep);
+        return check_launch("gemm_i8 (any K)");
+    }
     if (!fast) {
         size_t blocks = (m * n + kGemmThreads - 1) / kGemmThreads;
         const size_t cap = size_t(ctx->num_cus) * 8;

@@ -3,6 +3,7 @@
 #pragma once
 
 #include <cstdlib>
+#include <type_traits>
 
 #include "hipq_internal.h"
 #include "hipq_math.h"
@@ -180,9 +181,36 @@ static inline void pick_xcd_rectangle(int tiles_m, int tiles_n, int bm, int bn, 
     }
 }
 
+// 16 bytes of a row of K >= 16 bytes at any alignment, from byte k on; bytes past the row's end are zero.  Reads inside
+// the row only: a piece that runs over the end is taken from the row's last 16 bytes and shifted down.  TAIL = false:
+// the caller knows that k + 16 <= K.  (Global loads of any alignment are one instruction; only the last K-tile of a row
+// pays for the shift.)
+struct __attribute__((packed, aligned(1))) AnyBytes16 {
+    v4i v;
+};
+template <bool TAIL>
+__device__ __forceinline__ v4i load_row_piece(const int8_t *row, int k, int K) {
+    if constexpr (!TAIL) return reinterpret_cast<const AnyBytes16 *>(row + k)->v;
+    const int at = k < K - 16 ? k : K - 16, drop = k - at;  // bytes of the loaded piece that lie before k
+    const v4i v = reinterpret_cast<const AnyBytes16 *>(row + at)->v;
+    uint64_t lo = static_cast<uint32_t>(v[0]) | uint64_t(static_cast<uint32_t>(v[1])) << 32;
+    uint64_t hi = static_cast<uint32_t>(v[2]) | uint64_t(static_cast<uint32_t>(v[3])) << 32;
+    if (drop >= 8) {
+        lo = hi;
+        hi = 0;
+    }
+    const int s = 8 * (drop & 7);
+    if (s) {
+        lo = lo >> s | hi << (64 - s);
+        hi >>= s;
+    }
+    if (drop >= 16) lo = hi = 0;
+    return v4i{static_cast<int>(lo), static_cast<int>(lo >> 32), static_cast<int>(hi), static_cast<int>(hi >> 32)};
+}
+
 // BM x BN output tile per workgroup, BK = 128 bytes of K per stage, WM x WN
-// waves each owning a (BM/WM) x (BN/WN) sub-tile.
-template <int BM, int BN, int WM, int WN, int EPI, bool EVEN>
+// waves each owning a (BM/WM) x (BN/WN) sub-tile.  ANYK: operands of any alignment and any K >= 16.
+template <int BM, int BN, int WM, int WN, int EPI, bool EVEN, bool ANYK = false>
 __global__ __launch_bounds__(kGemmThreads) void gemm_i8_mfma_kernel(const int8_t *__restrict__ A,
                                                                      const int8_t *__restrict__ W, int M, int N,
                                                                      int K, GemmEpilogue ep) {
@@ -214,21 +242,28 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_i8_mfma_kernel(const int8_t
     v4i ra[A_PER_T], rw[W_PER_T];
     const v4i zero = v4i{0, 0, 0, 0};
 
-    auto load_global = [&](int k0) {
+    auto load_pieces = [&](int k0, auto tail) {
+        constexpr bool kTail = decltype(tail)::value;
 #pragma unroll
         for (int i = 0; i < A_PER_T; ++i) {
             const int c = tid + i * kGemmThreads;
             const int row = c / CPR, col = c % CPR;
             const int gm = m0 + row, gk = k0 + col * 16;
-            ra[i] = (gm < M && gk < K) ? *reinterpret_cast<const v4i *>(A + size_t(gm) * K + gk) : zero;
+            ra[i] = (gm < M && gk < K) ? load_row_piece<kTail>(A + size_t(gm) * K, gk, K) : zero;
         }
 #pragma unroll
         for (int i = 0; i < W_PER_T; ++i) {
             const int c = tid + i * kGemmThreads;
             const int row = c / CPR, col = c % CPR;
             const int gn = n0 + row, gk = k0 + col * 16;
-            rw[i] = (gn < N && gk < K) ? *reinterpret_cast<const v4i *>(W + size_t(gn) * K + gk) : zero;
+            rw[i] = (gn < N && gk < K) ? load_row_piece<kTail>(W + size_t(gn) * K, gk, K) : zero;
         }
+    };
+    auto load_global = [&](int k0) {
+        if constexpr (ANYK) {
+            if (k0 + BK > K) return load_pieces(k0, std::true_type{});
+        }
+        load_pieces(k0, std::false_type{});
     };
     auto store_lds = [&](int stage) {
         int8_t *sa = lds + stage * STAGE;
