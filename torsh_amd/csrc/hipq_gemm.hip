@@ -284,13 +284,13 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_i8_generic_kernel(const int
     }
 }
 
-template <int BM, int BN, int WM, int WN, int EPI, bool EVEN, bool ANYK = false>
+template <int BM, int BN, int WM, int WN, int EPI, bool EVEN>
 static void launch_tile(hipq_ctx *ctx, const int8_t *a, const int8_t *w, int M, int N, int K,
                         const GemmEpilogue &ep) {
     const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
     GemmEpilogue placed = ep;
     pick_xcd_rectangle(tiles_m, tiles_n, BM, BN, &placed.xcd_gm, &placed.xcd_gn);
-    hipLaunchKernelGGL((gemm_i8_mfma_kernel<BM, BN, WM, WN, EPI, EVEN, ANYK>), dim3(tiles_m * tiles_n), dim3(kGemmThreads), 0,
+    hipLaunchKernelGGL((gemm_i8_mfma_kernel<BM, BN, WM, WN, EPI, EVEN>), dim3(tiles_m * tiles_n), dim3(kGemmThreads), 0,
                        ctx->stream, a, w, M, N, K, placed);
 }
 
@@ -305,22 +305,7 @@ static int32_t launch_gemm(hipq_ctx *ctx, const int8_t *a, const int8_t *w, size
     const int M = static_cast<int>(m), N = static_cast<int>(n), K = static_cast<int>(k);
     const bool fast = (K % 16 == 0) && ((reinterpret_cast<uintptr_t>(a) & 15u) == 0) &&
                       ((reinterpret_cast<uintptr_t>(w) & 15u) == 0);
-    if (!fast && K >= 16) {
-        // Rows at any alignment (load_row_piece).  Instead of a thread per output, us: M = 300, N = 1000, K = 1001
-        // 1206 -> 11; 1 x 11008 x 4001 19, 64 x 4096 x 4097 26, 512 x 4096 x 4097 43.  The four waves of a
-        // workgroup split K up to 16 rows; what bounds it from there on is the register-staged tile's one stage in flight.
-        if (M <= 16) {
-            hipLaunchKernelGGL((gemv_i8_kernel<1, EPI, EVEN, true>), dim3((N + 15) / 16), dim3(kGemmThreads), 0, ctx->stream, a,
-                               w, M, N, K, ep);
-            return check_launch("gemv_i8 (any K)");
-        }
-        if (((m + 127) / 128) * ((n + 63) / 64) >= size_t(ctx->num_cus))
-            launch_tile<128, 64, 2, 2, EPI, EVEN, true>(ctx, a, w, M, N, K, ep);
-        else
-            launch_tile<64, 64, 2, 2, EPI, EVEN, true>(ctx, a, w, M, N, K, ep);
-        return check_launch("gemm_i8 (any K)");
-    }
-    if (!fast) {
+    if (!fast && K < 16) {
         size_t blocks = (m * n + kGemmThreads - 1) / kGemmThreads;
         const size_t cap = size_t(ctx->num_cus) * 8;
         if (blocks > cap) blocks = cap;
@@ -332,9 +317,20 @@ static int32_t launch_gemm(hipq_ctx *ctx, const int8_t *a, const int8_t *w, size
     auto tiles = [&](size_t bm, size_t bn) { return ((m + bm - 1) / bm) * ((n + bn - 1) / bn); };
     int variant = gemm_variant_override(ctx);
     if (variant == 9 || variant == 11) variant = 0;  // switches of the packed forms only
-    if (variant == 0 && M <= 16 && K % 256 == 0) return launch_gemv<EPI, EVEN>(ctx, a, w, M, N, K, ep);
-    const bool pipe_ok = (K % 128 == 0) && K >= 256;
-    if (variant == 0 && pipe_ok) {
+    // Rows at any alignment (load_row_piece): up to 16 of them the K-split kernel, else the register-staged tile.  Instead
+    // of a thread per output, us: M = 300, N = 1000, K = 1001 1206 -> 11; 1 x 11008 x 4001 19, 64 x 4096 x 4097 26,
+    // 512 x 4096 x 4097 43.
+    if (!fast) variant = M <= 16 ? 0 : 10;
+    if (variant == 0 && M <= 16) {
+        if (fast && K % 256 == 0) return launch_gemv<EPI, EVEN>(ctx, a, w, M, N, K, ep);
+        hipLaunchKernelGGL((gemv_i8_kernel<1, EPI, EVEN, true>), dim3((N + 15) / 16), dim3(kGemmThreads), 0, ctx->stream, a, w,
+                           M, N, K, ep);
+        return check_launch("gemv_i8 (any K)");
+    }
+    // The LDS-pipelined kernels for every K that is a multiple of 16 (a last K-tile that runs over the rows is filled
+    // with zeros).  Against the register-staged tile, us: 512 x 4096 x 4112 37 / 20, 300 x 1000 x 1008 14.6 / 7.6,
+    // 8192 x 3072 x 320 73 / 29, x 64 66 / 25, 100 x 1408 x 192 10.5 / 6.1, 50 x 300 x 64 6.0 / 5.7.
+    if (variant == 0) {
         variant = 2;
         if (tiles(128, 64) >= 2 * cus) {
             // Many more tiles than CUs: the persistent kernel.  Its tile shape is picked with a
@@ -344,7 +340,7 @@ static int32_t launch_gemm(hipq_ctx *ctx, const int8_t *a, const int8_t *w, size
             // a workgroup runs ceil(tiles / CUs) tiles.  Bigger tiles move fewer LDS bytes per MAC
             // but quantise worse.  The 256x128 and 128x192 forms have no room for residual values
             // in registers.
-            const double nk = double(K / 128), out_scale = (EPI == EPI_I8) ? 0.25 : 1.0;
+            const double nk = double((K + 127) / 128), out_scale = (EPI == EPI_I8) ? 0.25 : 1.0;
             auto cost = [&](size_t bm, size_t bn, double L, double E) {
                 const size_t t = tiles(bm, bn);
                 return double((t + cus - 1) / cus) * (nk * L + E * out_scale);
@@ -357,7 +353,6 @@ static int32_t launch_gemm(hipq_ctx *ctx, const int8_t *a, const int8_t *w, size
             variant = (c7 <= c6 && c7 <= c5 && c7 <= c8) ? 7 : (c8 <= c6 && c8 <= c5 ? 8 : (c6 <= c5 ? 6 : 5));
         }
     }
-    if (variant == 0 || (variant != 10 && !pipe_ok)) variant = 10;
     switch (variant) {
     case 1: return launch_pipe<128, 64, 6, 4, 1, 1, 4, EPI, EVEN>(ctx, a, w, M, N, K, ep);
     case 2: return launch_pipe<128, 64, 6, 4, 2, 1, 2, EPI, EVEN>(ctx, a, w, M, N, K, ep);
@@ -372,10 +367,10 @@ static int32_t launch_gemm(hipq_ctx *ctx, const int8_t *a, const int8_t *w, size
         return launch_persist<128, 128, 4, 4, 2, 2, 2, EPI, EVEN>(ctx, a, w, M, N, K, ep);
     default: break;
     }
-    // Register-staged kernel: any K that is a multiple of 16.
+    // Register-staged kernel: any K from 16 on, any alignment.
     if (tiles(128, 128) >= 2 * cus)
         launch_tile<128, 128, 2, 2, EPI, EVEN>(ctx, a, w, M, N, K, ep);
-    else if (tiles(128, 64) >= cus || m > 64)
+    else if (tiles(128, 64) >= cus)
         launch_tile<128, 64, 2, 2, EPI, EVEN>(ctx, a, w, M, N, K, ep);
     else
         launch_tile<64, 64, 2, 2, EPI, EVEN>(ctx, a, w, M, N, K, ep);

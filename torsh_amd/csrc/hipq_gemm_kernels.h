@@ -209,8 +209,8 @@ __device__ __forceinline__ v4i load_row_piece(const int8_t *row, int k, int K) {
 }
 
 // BM x BN output tile per workgroup, BK = 128 bytes of K per stage, WM x WN
-// waves each owning a (BM/WM) x (BN/WN) sub-tile.  ANYK: operands of any alignment and any K >= 16.
-template <int BM, int BN, int WM, int WN, int EPI, bool EVEN, bool ANYK = false>
+// waves each owning a (BM/WM) x (BN/WN) sub-tile.  Operands of any alignment and any K >= 16.
+template <int BM, int BN, int WM, int WN, int EPI, bool EVEN>
 __global__ __launch_bounds__(kGemmThreads) void gemm_i8_mfma_kernel(const int8_t *__restrict__ A,
                                                                      const int8_t *__restrict__ W, int M, int N,
                                                                      int K, GemmEpilogue ep) {
@@ -260,10 +260,10 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_i8_mfma_kernel(const int8_t
         }
     };
     auto load_global = [&](int k0) {
-        if constexpr (ANYK) {
-            if (k0 + BK > K) return load_pieces(k0, std::true_type{});
-        }
-        load_pieces(k0, std::false_type{});
+        if (k0 + BK > K)
+            load_pieces(k0, std::true_type{});
+        else
+            load_pieces(k0, std::false_type{});
     };
     auto store_lds = [&](int stage) {
         int8_t *sa = lds + stage * STAGE;
@@ -333,8 +333,12 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_i8_mfma_kernel(const int8_t
     }
 }
 
+// What the fills of a last K-tile that runs over the end of the rows (K % 128 != 0) read instead: zeros, which add
+// nothing.
+static __device__ const v4i kZeroPiece = {0, 0, 0, 0};
+
 // ---------------------------------------------------------------------------
-// Deep-pipelined kernel for K % 128 == 0 (the shapes that matter).
+// Deep-pipelined kernel for K % 16 == 0 (the shapes that matter).
 //
 // Occupancy for the headline shape is one workgroup per CU (256 tiles on 256
 // CUs), so all latency hiding happens inside the workgroup:
@@ -573,16 +577,18 @@ __global__ __launch_bounds__((PW + WM * WN * WK) * kWave) void gemm_i8_pipe_kern
     tile_of_block((M + BM - 1) / BM, (N + BN - 1) / BN, ep.xcd_gm, ep.xcd_gn, &tile_m, &tile_n);
     const int m0 = tile_m * BM, n0 = tile_n * BN;
     const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
-    const int nk = K / BK;
+    const int nk = (K + BK - 1) / BK;
 
     if (wave < PW) {
         // ---------------- producer ----------------
         const int8_t *src[IPW];
+        bool past_end[IPW];  // the piece lies past the end of the rows in the last K-tile
 #pragma unroll
         for (int j = 0; j < IPW; ++j) {
             const int q = wave * IPW + j;
             const int trow = q * RPI + lane / CPR;  // row in the stacked [A rows | W rows] tile
             const int col = (lane % CPR) ^ ((trow >> 1) & 7);
+            past_end[j] = (nk - 1) * BK + col * 16 >= K;
             if (trow < BM) {
                 int gm = m0 + trow;
                 gm = gm < M ? gm : M - 1;  // rows past the edge are computed and discarded
@@ -596,11 +602,14 @@ __global__ __launch_bounds__((PW + WM * WN * WK) * kWave) void gemm_i8_pipe_kern
         auto issue_stage = [&](int kt, int buf) {
             int8_t *base = lds + buf * STAGE + wave * (IPW * 1024);
             const size_t koff_row = size_t(kt) * BK;
+            const bool last = kt == nk - 1;
 #pragma unroll
-            for (int j = 0; j < IPW; ++j)
-                __builtin_amdgcn_global_load_lds(
-                    (const __attribute__((address_space(1))) void *)(src[j] + koff_row),
-                    (__attribute__((address_space(3))) void *)(base + j * 1024), 16, 0, 0);
+            for (int j = 0; j < IPW; ++j) {
+                const int8_t *from = src[j] + koff_row;
+                if (last && past_end[j]) from = reinterpret_cast<const int8_t *>(&kZeroPiece);
+                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)from,
+                                                 (__attribute__((address_space(3))) void *)(base + j * 1024), 16, 0, 0);
+            }
         };
         // Two stages before the first barrier so the consumers start after one memory
         // latency; the remaining buffers are requested while they work on stage 0.

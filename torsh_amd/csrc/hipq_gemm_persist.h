@@ -109,7 +109,7 @@ __global__ __launch_bounds__((PW + WM * WN) * kWave) void gemm_i8_persist_kernel
 
     const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
     const int ntiles = tiles_m * tiles_n;
-    const int nk = K / BK;  // >= 1
+    const int nk = (K + BK - 1) / BK;  // >= 1
     const int my_tiles = (ntiles - static_cast<int>(blockIdx.x) + static_cast<int>(gridDim.x) - 1) /
                          static_cast<int>(gridDim.x);
     const int T = my_tiles * nk;  // K-tiles this workgroup streams, in consumption order
@@ -122,6 +122,12 @@ __global__ __launch_bounds__((PW + WM * WN) * kWave) void gemm_i8_persist_kernel
     if (wave < PW) {
         // ---------------- producer ----------------
         const int8_t *src[IPW];
+        bool past_end[IPW];  // the piece lies past the end of the rows in the last K-tile
+#pragma unroll
+        for (int j = 0; j < IPW; ++j) {
+            const int trow = (wave * IPW + j) * RPI + lane / CPR;
+            past_end[j] = (nk - 1) * BK + ((lane % CPR) ^ ((trow >> 1) & 7)) * 16 >= K;
+        }
         auto set_tile = [&](int ti) {
             const int t = static_cast<int>(blockIdx.x) + ti * static_cast<int>(gridDim.x);
             const int m0 = (t % tiles_m) * BM, n0 = (t / tiles_m) * BN;
@@ -163,9 +169,12 @@ __global__ __launch_bounds__((PW + WM * WN) * kWave) void gemm_i8_persist_kernel
             int8_t *base = lds + buf * STAGE + wave * (IPW * 1024);
             const size_t koff = size_t(kt_issue) * BK;
 #pragma unroll
-            for (int j = 0; j < IPW; ++j)
-                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(src[j] + koff),
+            for (int j = 0; j < IPW; ++j) {
+                const int8_t *from = src[j] + koff;
+                if (kt_issue == nk - 1 && past_end[j]) from = reinterpret_cast<const int8_t *>(&kZeroPiece);
+                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)from,
                                                  (__attribute__((address_space(3))) void *)(base + j * 1024), 16, 0, 0);
+            }
             ++unreported;
             if (++buf == STAGES) {
                 buf = 0;
@@ -568,7 +577,7 @@ static int32_t launch_persist(hipq_ctx *ctx, const int8_t *a, const int8_t *w, i
             return fail(HIPQ_DEVICE_ERROR, "gemm_i8: cannot reserve %d bytes of LDS: %s", kLds, hipGetErrorString(e));
         configured[ctx->device][with_residual] = true;
     }
-    if (K % 128 != 0 || K < 128) return fail(HIPQ_INVALID_ARGUMENT, "gemm_i8 (persistent): K must be a multiple of 128");
+    if (K % 16 != 0) return fail(HIPQ_INVALID_ARGUMENT, "gemm_i8 (persistent): K must be a multiple of 16");
     if (EPI != EPI_I32 && (!ep.sa || !ep.sw)) return fail(HIPQ_INVALID_ARGUMENT, "gemm_i8 (persistent): scales must be given");
     const int tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
     const int grid = tiles < ctx->num_cus ? tiles : ctx->num_cus;
