@@ -490,6 +490,44 @@ def test_prepared_stack_small_against_the_oracle(ctx, oracle, tokens, d, dff, la
     assert rel_plain < 2e-3
 
 
+@pytest.mark.parametrize("tokens,d,dff,layers", [(1, 768, 3072, 2), (2, 128, 384, 3), (31, 256, 256, 2), (33, 768, 3072, 2), (77, 1152, 2304, 2),
+                                                 (300, 1664, 1792, 1)])
+def test_prepared_stack_few_tokens(hipq, tokens, d, dff, layers):
+    """Few tokens run as products split over their columns; test hook 15 runs the row panels.  Both within the drift of
+    the LayerNorm sums (their order differs) of the stack on row-major weights, for both roundings."""
+    c = hipq.Context(0)
+    try:
+        g = torch.Generator(device="cuda").manual_seed(tokens + d)
+        blocks = []
+        for _ in range(layers):
+            blk = {}
+            for name, (o, i) in {"qkv": (3 * d, d), "out": (d, d), "fc1": (dff, d), "fc2": (d, dff)}.items():
+                q, sc, _, _ = c.quantize_per_row(torch.randn(o, i, generator=g, device="cuda") * 0.02)
+                blk["w_" + name], blk["s_" + name] = q, sc
+                blk["b_" + name] = torch.randn(o, generator=g, device="cuda") * 0.01
+            for ln in ("ln1", "ln2"):
+                blk[ln + "_gamma"] = torch.rand(d, generator=g, device="cuda") + 0.5
+                blk[ln + "_beta"] = torch.randn(d, generator=g, device="cuda") * 0.1
+            blocks.append(blk)
+        prepared = c.stack_prepare(blocks)
+        x0 = torch.randn(tokens, d, generator=g, device="cuda")
+        for mode in (0, hipq.ROUND_HALF_EVEN):
+            run = lambda: c.stack_forward(prepared, x0.clone(), dff, c.stack_workspace_prepared(tokens, d, dff), mode=mode,
+                                          prepared=True)
+            got = run()
+            c.set_gemm_kernel_variant(15)
+            panels = run()
+            c.set_gemm_kernel_variant(0)
+            plain = c.stack_forward(blocks, x0.clone(), dff, c.stack_workspace(tokens, d, dff), mode=mode)
+            torch.cuda.synchronize()
+            assert torch.isfinite(got).all()
+            for other in (panels, plain):
+                assert float((got - other).norm() / plain.norm()) < 2e-3
+    finally:
+        torch.cuda.synchronize()
+        c.close()
+
+
 def test_prepared_stack_full_size_equals_its_parts(ctx, hipq):
     """Config 5 at its real size (8192 tokens, d = 768, d_ff = 3072; 3 layers keep the test short): the one call is
     bit-identical to the same layers composed from the entry points tested above, and stays within the drift bound

@@ -70,6 +70,17 @@ bool pairs_share_an_xcd(hipq_ctx *ctx) {
     return known[ctx->device] > 0;
 }
 
+int32_t linear_packed_rows_f32(hipq_ctx *ctx, const int8_t *a_packed, const float *a_scales, const int8_t *w_packed,
+                               const float *w_scales, const float *bias, const float *residual, size_t m, size_t n, size_t k,
+                               float *out) {
+    int32_t rc = check_packed_shape("linear (packed)", m, n, k);
+    if (rc) return rc;
+    GemmEpilogue ep{a_scales, 1, w_scales, bias, 1.0f, 0, out};
+    ep.residual = residual;
+    ep.fresh_activations = 1;
+    return launch_gemm_packed<EPI_F32, false>(ctx, a_packed, w_packed, m, n, k, ep);
+}
+
 bool conv_patch_applicable(int nb, int c, int h, int w, int hp, int wp, int kh, int kw) {
     int patch = 0, lds_bytes = 0;
     return conv_patch_fits(c, h, w, hp, wp, kh, kw, static_cast<long long>(nb) * hp * wp, &patch, &lds_bytes);

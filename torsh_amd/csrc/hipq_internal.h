@@ -119,6 +119,17 @@ int32_t quantize_activations_per_row(hipq_ctx *ctx, const float *x, size_t rows,
 // The same for rows that lie `ld` floats apart (a column slice of a wider matrix).
 int32_t quantize_activations_per_row_strided(hipq_ctx *ctx, const float *x, size_t rows, size_t cols, size_t ld,
                                              int32_t mode, int8_t *out, float *out_scales, bool packed);
+// The row operations of the transformer stack with their codes in the packed operand layout (cols a multiple of 128; the
+// rows that pad the last row block are not written: products of them are discarded).  delta: x += delta first.
+int32_t layer_norm_quantize_packed(hipq_ctx *ctx, float *x, const float *delta, size_t rows, size_t cols, const float *gamma,
+                                   const float *beta, float eps, int32_t mode, int8_t *out_packed, float *out_scales);
+int32_t gelu_quantize_packed(hipq_ctx *ctx, const float *x, size_t rows, size_t cols, int32_t mode, int8_t *out_packed,
+                             float *out_scales);
+// hipq_linear_packed_i8_f32 on per-row scales and activations that the kernel just before wrote; residual (may be null,
+// may be out) is added after the bias.
+int32_t linear_packed_rows_f32(hipq_ctx *ctx, const int8_t *a_packed, const float *a_scales, const int8_t *w_packed,
+                               const float *w_scales, const float *bias, const float *residual, size_t m, size_t n, size_t k,
+                               float *out);
 // Looks up, once per device, the address of the static device array behind
 // hipq_linear_dynamic_f32_noalloc; called by hipq_ctx_create with the device current.
 int32_t linear_noalloc_setup(int device);

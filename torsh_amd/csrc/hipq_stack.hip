@@ -11,6 +11,36 @@
 
 namespace {
 size_t align256(size_t v) { return (v + 255) & ~size_t(255); }
+
+// Parts of the workspace of the forward on prepared weights.
+struct StackBuffers {
+    int8_t *qa, *qb;  // packed int8 activations
+    float *sa, *sb;   // their per-token scales
+    float *qkv;
+};
+
+// Few tokens: every product split over its columns (the packed tiled kernels), the row operations between them in
+// kernels of their own that write packed codes.  hidden: [tokens, d_ff] fp32.
+int32_t stack_tiled(hipq_ctx *ctx, const hipq_block_weights *blocks, size_t n_layers, size_t tokens, size_t d_model,
+                    size_t d_ff, float eps, int32_t mode, float *x, const StackBuffers &b, float *hidden) {
+    using namespace hipq;
+    for (size_t l = 0; l < n_layers; ++l) {
+        const hipq_block_weights &w = blocks[l];
+        int32_t rc;
+        if ((rc = layer_norm_quantize_packed(ctx, x, nullptr, tokens, d_model, w.ln1_gamma, w.ln1_beta, eps, mode, b.qa, b.sa)) ||
+            (rc = linear_packed_rows_f32(ctx, b.qa, b.sa, w.w_qkv, w.s_qkv, w.b_qkv, nullptr, tokens, 3 * d_model, d_model,
+                                         b.qkv)) ||
+            (rc = quantize_activations_per_row_strided(ctx, b.qkv + 2 * d_model, tokens, d_model, 3 * d_model, mode, b.qb, b.sb,
+                                                       /*packed=*/true)) ||
+            (rc = linear_packed_rows_f32(ctx, b.qb, b.sb, w.w_out, w.s_out, w.b_out, x, tokens, d_model, d_model, x)) ||
+            (rc = layer_norm_quantize_packed(ctx, x, nullptr, tokens, d_model, w.ln2_gamma, w.ln2_beta, eps, mode, b.qa, b.sa)) ||
+            (rc = linear_packed_rows_f32(ctx, b.qa, b.sa, w.w_fc1, w.s_fc1, w.b_fc1, nullptr, tokens, d_ff, d_model, hidden)) ||
+            (rc = gelu_quantize_packed(ctx, hidden, tokens, d_ff, mode, b.qb, b.sb)) ||
+            (rc = linear_packed_rows_f32(ctx, b.qb, b.sb, w.w_fc2, w.s_fc2, w.b_fc2, x, tokens, d_model, d_ff, x)))
+            return rc;
+    }
+    return HIPQ_SUCCESS;
+}
 }  // namespace
 
 extern "C" {
@@ -86,7 +116,7 @@ int32_t hipq_transformer_stack_forward_f32(hipq_ctx *ctx, const hipq_block_weigh
     return HIPQ_SUCCESS;
 }
 
-// ---- the same forward on prepared (fragment-packed) weights: five kernels per layer ---------------------------
+// ---- the same forward on prepared (fragment-packed) weights ---------------------------
 // Every Linear that feeds a row operation runs as a row-panel GEMM with that operation in its epilogue
 // (hipq_gemm_rows.h): out-proj + skip + LayerNorm 2 + quantize, fc1 + GELU + quantize, fc2 + skip + the next
 // layer's LayerNorm 1 + quantize.  Activations travel between them as packed int8; the only fp32 tensors that
@@ -138,8 +168,23 @@ int32_t hipq_transformer_stack_forward_prepared_f32(hipq_ctx *ctx, const hipq_bl
     float *qkv = reinterpret_cast<float *>(p);
     const int32_t round_bits = mode & HIPQ_ROUND_HALF_EVEN;
 
+    const StackBuffers buf{qa, qb, sa, sb, qkv};
+    int32_t rc;
+    // Row panels are 32 (or 64) rows of one workgroup (or pair), so a forward of few tokens leaves compute units idle and
+    // every busy one streams the whole weight matrices: 1.5-1.65 ms for 12 layers at d 768, d_ff 3072 whatever the
+    // number of tokens, up to 8192.  The separate tiled products and row kernels grow with it instead, us (panels / tiled):
+    //   d 768, d_ff 3072:  77 1510 / 530, 1000 1590 / 690, 4096 1660 / 1270, 8192 1835 / 2120
+    //   d 256, d_ff 1024:  77 635 / 480, 4096 660 / 630, 8192 705 / 860;   d 1024: 77 2425 / 590, 8192 2730 / 2700
+    // so the panels are taken when they fill five eighths of the device.  (Test hook 15: panels always.)
+    if (tokens <= size_t(ctx->num_cus) * 20 && ctx->gemm_variant != 15) {
+        void *s = nullptr;
+        if (hipq::scratch(ctx, hipq::kScratchHeader + tokens * d_ff * sizeof(float), &s) == HIPQ_SUCCESS)
+            return stack_tiled(ctx, blocks, n_layers, tokens, d_model, d_ff, eps, round_bits, x, buf,
+                               reinterpret_cast<float *>(static_cast<char *>(s) + hipq::kScratchHeader));
+        hipq::clear_error();  // (no memory, or a first call under stream capture: the panels need none)
+    }
     // quant(LN1(x)) of the first layer: the row kernel, then the packing pass (row-major codes parked in qb)
-    int32_t rc = hipq_layer_norm_quantize_f32_i8(ctx, x, tokens, d_model, blocks[0].ln1_gamma, blocks[0].ln1_beta, eps,
+    rc = hipq_layer_norm_quantize_f32_i8(ctx, x, tokens, d_model, blocks[0].ln1_gamma, blocks[0].ln1_beta, eps,
                                                  round_bits, qb, sa);
     if (rc) return rc;
     if ((rc = hipq_pack_rows_i8(ctx, qb, tokens, d_model, qa))) return rc;
