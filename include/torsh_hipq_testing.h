@@ -24,7 +24,8 @@ extern "C" {
  * the forms of the GEMM that are picked by occupancy - two workgroups per compute unit, the
  * weight-streaming kernel for 33..128 rows - (9) and the touching of weight / filter lines by the
  * one-launch activation quantizers of the dynamic Linear and Conv2d forwards while their grids wait
- * for the range (11); 12 runs shapes of whole 128 x 128 tiles that fill the device once as one tile
+ * for the range (11); on prepared operands 7 and 8 force the tiles of 256 x 128 and 128 x 256 that are
+ * staged through LDS; 12 runs shapes of whole 128 x 128 tiles that fill the device once as one tile
  * per PAIR of compute units, K halved between the two, partial sums exchanged through their XCD's L2
  * (measured slower than the default forms; kept as a measured alternative); 14 runs a Conv2d
  * forward on a uint8 input of 128 or 256 channels and small planes as ONE launch whose workgroups

@@ -782,3 +782,37 @@ def test_scratch_growth_under_capture_is_refused_not_attempted(hipq):
         finally:
             torch.cuda.synchronize()
             c.close()
+
+
+@pytest.mark.parametrize("tall", [7, 8])
+@pytest.mark.parametrize("m,n,k", [(33, 40, 16), (256, 256, 128), (257, 129, 130), (129, 257, 256), (40, 700, 4100), (255, 127, 600),
+                                   (600, 300, 1000), (128, 512, 384), (700, 1100, 260)])
+def test_gemm_tiles_staged_through_lds(hipq, oracle, m, n, k, tall):
+    """The 256 x 128 and 128 x 256 tiles (forced): ragged edges, K from one stage of the pipeline to more than its ring
+    holds, every epilogue: int32, fp32 (per-row and per-tensor scales, with and without bias), requantized int8."""
+    c = hipq.Context(0)
+    try:
+        rng = np.random.default_rng(m * 5 + n * 3 + k)
+        a, w = rand_i8(rng, (m, k)), rand_i8(rng, (n, k))
+        acc = oracle.gemm_i8_nk(a, w)
+        pa, pw = c.pack_rows(dev(a)), c.pack_rows(dev(w))
+        sa, sw = rng.uniform(1e-3, 1e-2, m).astype(np.float32), rng.uniform(1e-4, 1e-3, n).astype(np.float32)
+        bias = rng.standard_normal(n).astype(np.float32)
+        c.set_gemm_kernel_variant(tall)
+        np.testing.assert_array_equal(host(c.gemm_packed_i8_i32(pa, pw, m, n, k)), acc)
+        for scale, b in ((sa, bias), (sa[:1], None)):
+            got = host(c.linear_packed_i8_f32(pa, dev(scale), pw, dev(sw), None if b is None else dev(b), m, n, k))
+            want = acc.astype(np.float32) * ((scale[:, None] if scale.size > 1 else scale[0]) * sw[None, :])
+            np.testing.assert_array_equal(got, want if b is None else want + b[None, :])
+        s_out = float(np.abs(acc).max() * sa[0] * sw.max() / 90)
+        for mode, rm in ((hipq.ROUND_HALF_AWAY, 0), (hipq.ROUND_HALF_EVEN, 1)):
+            oracle.set_round_mode(rm)
+            try:
+                want = oracle.requantize_epilogue(acc, float(sa[0]), sw, bias, s_out, 3)
+            finally:
+                oracle.set_round_mode(0)
+            got = host(c.linear_packed_i8_i8(pa, dev(sa[:1]), pw, dev(sw), dev(bias), m, n, k, s_out, 3, mode))
+            np.testing.assert_array_equal(got, want)
+    finally:
+        torch.cuda.synchronize()
+        c.close()

@@ -54,6 +54,9 @@ constexpr int kTracePoints = 6, kTraceWords = 8;
 // Row-major int8 [rows, k] -> fragment-packed operand (packed_operand_bytes(rows, k) bytes at dst).
 int32_t pack_rows(hipq_ctx *ctx, const int8_t *src, size_t rows, size_t k, int8_t *dst);
 size_t packed_operand_bytes(size_t rows, size_t k);
+// The packed GEMM in large tiles staged through LDS (hipq_gemm_big.hip): 256 x 128 (tall) or 128 x 256.
+int32_t gemm_packed_lds(hipq_ctx *ctx, bool tall, const int8_t *pa, const int8_t *pw, int M, int N, int K,
+                        const GemmEpilogue &ep, int epi, bool even);
 // The convolution in one launch, from the u8 NCHW input itself (hipq_conv_patch.h): `applicable` says whether
 // that form takes the geometry (c channels, padded width wp, kh x kw taps).
 bool conv_patch_applicable(int nb, int c, int h, int w, int hp, int wp, int kh, int kw);
@@ -539,6 +542,75 @@ __device__ __forceinline__ void store_tile(v16i (&acc)[FM][FN], const GemmEpilog
                     }
                 }
             }
+        }
+    }
+}
+
+// ---- fragment-packed operands (layout: hipq_gemm_packed.h) ----------------------------------------------------
+constexpr int kPackKbAlign = 4;  // k blocks per row block are padded to a multiple of the K-split
+
+__host__ __device__ inline size_t packed_row_blocks(size_t rows) { return (rows + 31) / 32; }
+__host__ __device__ inline size_t packed_k_blocks(size_t k) {
+    return ((k + 31) / 32 + kPackKbAlign - 1) / kPackKbAlign * kPackKbAlign;
+}
+__host__ __device__ inline size_t packed_bytes(size_t rows, size_t k) {
+    return packed_row_blocks(rows) * packed_k_blocks(k) * 1024;
+}
+
+// fp32 / int32 epilogue of one 32-row block that lies wholly inside the output (first row `row0`, first
+// column `n0`): the same arithmetic as store_tile, without per-element bounds checks and with buffer
+// stores whose row and column-block offsets are scalar, so that an output costs a convert, a multiply,
+// an add and a store instead of a predicate, a branch and a 64-bit address as well.
+template <int TNB, int EPI>
+__device__ __forceinline__ void store_block_interior(v16i (&own)[1][TNB], const GemmEpilogue &ep, int N, int row0,
+                                                     int n0, int lane, const float (&swv)[TNB],
+                                                     const float (&bv)[TNB], float sa0) {
+    static_assert(EPI == EPI_F32 || EPI == EPI_I32, "interior epilogue: fp32 or int32 output");
+    // 4-byte elements: a row block spans at most (31 * N + 64) * 4 bytes from its first element, far below
+    // the 2 GiB a buffer offset can hold for any N the entry points accept.
+    char *base = static_cast<char *>(ep.out) + (size_t(row0) * N + n0) * 4;
+    const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(base, 0, 0x7fffffff, 0x00020000);
+    const int voff = (4 * (lane / 32) * N + lane % 32) * 4;
+    const int row_bytes = N * 4;
+    auto put = [&](int r, int j, int bits) {
+        __builtin_amdgcn_raw_buffer_store_b32(bits, ro, voff, (8 * (r / 4) + (r % 4)) * row_bytes + j * 128, /*nt*/ 2);
+    };
+    if constexpr (EPI == EPI_I32) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+#pragma unroll
+            for (int j = 0; j < TNB; ++j) put(r, j, own[0][j][r]);
+    } else {
+        const bool has_bias = ep.bias != nullptr;
+        auto emit = [&](auto scale_of, auto with_bias) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+#pragma unroll
+                for (int j = 0; j < TNB; ++j) {
+                    float v = static_cast<float>(own[0][j][r]) * scale_of(r, j);
+                    if constexpr (decltype(with_bias)::value) v = v + bv[j];
+                    put(r, j, __builtin_bit_cast(int, v));
+                }
+        };
+        if (ep.sa_per_row) {
+            float s_row[16];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s_row[r] = ep.sa[row0 + 8 * (r / 4) + 4 * (lane / 32) + (r % 4)];
+            wait_vmcnt<0>();
+            auto sc = [&](int r, int j) { return s_row[r] * swv[j]; };
+            if (has_bias)
+                emit(sc, std::true_type{});
+            else
+                emit(sc, std::false_type{});
+        } else {
+            float s_comb[TNB];
+#pragma unroll
+            for (int j = 0; j < TNB; ++j) s_comb[j] = sa0 * swv[j];
+            auto sc = [&](int, int j) { return s_comb[j]; };
+            if (has_bias)
+                emit(sc, std::true_type{});
+            else
+                emit(sc, std::false_type{});
         }
     }
 }

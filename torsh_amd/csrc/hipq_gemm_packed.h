@@ -23,74 +23,6 @@
 
 namespace hipq {
 
-constexpr int kPackKbAlign = 4;  // k blocks per row block are padded to a multiple of the K-split
-
-__host__ __device__ inline size_t packed_row_blocks(size_t rows) { return (rows + 31) / 32; }
-__host__ __device__ inline size_t packed_k_blocks(size_t k) {
-    return ((k + 31) / 32 + kPackKbAlign - 1) / kPackKbAlign * kPackKbAlign;
-}
-__host__ __device__ inline size_t packed_bytes(size_t rows, size_t k) {
-    return packed_row_blocks(rows) * packed_k_blocks(k) * 1024;
-}
-
-// fp32 / int32 epilogue of one 32-row block that lies wholly inside the output (first row `row0`, first
-// column `n0`): the same arithmetic as store_tile, without per-element bounds checks and with buffer
-// stores whose row and column-block offsets are scalar, so that an output costs a convert, a multiply,
-// an add and a store instead of a predicate, a branch and a 64-bit address as well.
-template <int TNB, int EPI>
-__device__ __forceinline__ void store_block_interior(v16i (&own)[1][TNB], const GemmEpilogue &ep, int N, int row0,
-                                                     int n0, int lane, const float (&swv)[TNB],
-                                                     const float (&bv)[TNB], float sa0) {
-    static_assert(EPI == EPI_F32 || EPI == EPI_I32, "interior epilogue: fp32 or int32 output");
-    // 4-byte elements: a row block spans at most (31 * N + 64) * 4 bytes from its first element, far below
-    // the 2 GiB a buffer offset can hold for any N the entry points accept.
-    char *base = static_cast<char *>(ep.out) + (size_t(row0) * N + n0) * 4;
-    const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(base, 0, 0x7fffffff, 0x00020000);
-    const int voff = (4 * (lane / 32) * N + lane % 32) * 4;
-    const int row_bytes = N * 4;
-    auto put = [&](int r, int j, int bits) {
-        __builtin_amdgcn_raw_buffer_store_b32(bits, ro, voff, (8 * (r / 4) + (r % 4)) * row_bytes + j * 128, /*nt*/ 2);
-    };
-    if constexpr (EPI == EPI_I32) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-#pragma unroll
-            for (int j = 0; j < TNB; ++j) put(r, j, own[0][j][r]);
-    } else {
-        const bool has_bias = ep.bias != nullptr;
-        auto emit = [&](auto scale_of, auto with_bias) {
-#pragma unroll
-            for (int r = 0; r < 16; ++r)
-#pragma unroll
-                for (int j = 0; j < TNB; ++j) {
-                    float v = static_cast<float>(own[0][j][r]) * scale_of(r, j);
-                    if constexpr (decltype(with_bias)::value) v = v + bv[j];
-                    put(r, j, __builtin_bit_cast(int, v));
-                }
-        };
-        if (ep.sa_per_row) {
-            float s_row[16];
-#pragma unroll
-            for (int r = 0; r < 16; ++r) s_row[r] = ep.sa[row0 + 8 * (r / 4) + 4 * (lane / 32) + (r % 4)];
-            wait_vmcnt<0>();
-            auto sc = [&](int r, int j) { return s_row[r] * swv[j]; };
-            if (has_bias)
-                emit(sc, std::true_type{});
-            else
-                emit(sc, std::false_type{});
-        } else {
-            float s_comb[TNB];
-#pragma unroll
-            for (int j = 0; j < TNB; ++j) s_comb[j] = sa0 * swv[j];
-            auto sc = [&](int, int j) { return s_comb[j]; };
-            if (has_bias)
-                emit(sc, std::true_type{});
-            else
-                emit(sc, std::false_type{});
-        }
-    }
-}
-
 // TMB x TNB row blocks of 32 per workgroup tile; D register stages of (TMB + TNB) KiB per wave in
 // flight.  Loads are buffer loads with a constant per-lane offset and scalar (SGPR) fragment
 // offsets, so the loop spends no vector instruction on addressing.
@@ -866,9 +798,26 @@ static int32_t launch_gemm_packed(hipq_ctx *ctx, const int8_t *pa, const int8_t 
         int32_t rc = HIPQ_SUCCESS;
         if (launch_pair_if_fits<EPI, EVEN>(ctx, pa, pw, m, n, k, ep, &rc)) return rc;
     }
-    if (ctx->gemm_variant != 9 && !ctx->trace) {  // (the phase stamps are the 128 x 64 kernel's)
+    if (ctx->gemm_variant != 7 && ctx->gemm_variant != 8 && ctx->gemm_variant != 9 &&
+        !ctx->trace) {  // (the phase stamps are the 128 x 64 kernel's)
         const size_t tiles64 = ((packed_row_blocks(m) + 1) / 2) * ((packed_row_blocks(n) + 1) / 2);
         if (M <= 64 || tiles64 <= size_t(ctx->num_cus)) return launch_skinny_packed<EPI, EVEN>(ctx, pa, pw, M, N, K, ep);
+    }
+    {
+        // Tiles of 128 x 256 or 256 x 128 staged through LDS (hipq_gemm_big.hip; the shape that covers the matrix with
+        // fewer of them) once the 128 x 64 tiles make four rounds over the compute units, or three with K <= 1024.
+        // 128 x 64 tiles / LDS in us: four rounds: 2048 x 4096 x 4096 43 / 38, 1800 x 4096 x 4096 45 / 36, 600 x 11008 x 4096
+        // 49 / 33, 8192 x 1024 x 128 10.8 / 8.6, 2816 x 2304 x 768 13.4 / 11.5; three: 2000 x 3072 x 768 14.5 / 11.7,
+        // 20000 x 256 x 256 9.8 / 7.7, but 1536 x 4096 x 4096 31.8 / 33.7, 768 x 8192 x 2048 18.4 / 19.1, 8192 x 768 x 3072
+        // 24.5 / 26.6; two: 4096 x 1024 x 1024 8.7 / 11.4, 1024 x 4096 x 4096 22.3 / 31.6.  (Hooks 7 and 8 force them.)
+        const size_t rbA = packed_row_blocks(m), rbW = packed_row_blocks(n), cus = size_t(ctx->num_cus);
+        const size_t rounds = (((rbA + 3) / 4) * ((rbW + 1) / 2) + cus - 1) / cus;
+        const bool forced = ctx->gemm_variant == 7 || ctx->gemm_variant == 8;
+        if (forced || (ctx->gemm_variant != 9 && !ctx->trace && (rounds >= 4 || (rounds == 3 && K <= 1024)))) {
+            const bool tall = forced ? ctx->gemm_variant == 7
+                                     : ((rbA + 7) / 8) * ((rbW + 3) / 4) < ((rbA + 3) / 4) * ((rbW + 7) / 8);
+            return gemm_packed_lds(ctx, tall, pa, pw, M, N, K, ep, EPI, EVEN);
+        }
     }
     if constexpr (EPI == EPI_F32 && !EVEN) {
         // Phase stamps (hipq_ctx_set_trace_buffer): the depth-2 fp32 form only, and only when the buffer holds
