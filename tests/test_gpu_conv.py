@@ -269,6 +269,9 @@ WINDOW_GEOMS = [
     (1, 5, 300, 260, 40, (3, 3), (1, 1), (1, 1), 200),   # enough windows for a wave on its own windows, K short
     (4, 64, 120, 121, 80, (3, 3), (2, 2), (1, 1), 3),    # the same with more than 64 filters and several groups
     (3, 40, 20, 21, 16, (5, 3), (3, 2), (2, 1), 60),     # few filters: one filter block, four window fragments
+    (2, 3, 6, 4, 20, (3, 3), (1, 1), (5, 5), 31),        # rows of one run of four pixels, runs wholly inside the border
+    (3, 70, 4, 3, 8, (3, 1), (1, 1), (1, 2), 12),        # rows shorter than a run: a pixel per thread
+    (2, 32, 5, 9, 32, (1, 3), (1, 2), (0, 1), 250),      # a whole group of 32 channels, rows of 2 1/4 runs
 ]
 
 

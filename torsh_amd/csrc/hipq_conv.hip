@@ -215,7 +215,8 @@ static bool window_geometry(const ConvGeom &g, ConvWindow *cw) {
         return false;
     *cw = ConvWindow{g.oc, static_cast<int>(windows), static_cast<int>(KB), static_cast<int>(kblocks), static_cast<int>(cgs),
                      static_cast<int>(segs), static_cast<int>(pitch), static_cast<int>(wp * pitch), static_cast<int>(plane),
-                     static_cast<int>(cgs * plane), static_cast<int>(hp), static_cast<int>(wp), g.sh, g.sw, g.ho, g.wo};
+                     static_cast<int>(cgs * plane), static_cast<int>(hp), static_cast<int>(wp), g.sh, g.sw, g.ho, g.wo,
+                     FastDiv::by(static_cast<uint32_t>(g.ho) * g.wo), FastDiv::by(g.wo)};
     return true;
 }
 
@@ -237,12 +238,19 @@ static int32_t launch_conv_window(hipq_ctx *ctx, const int8_t *filters, const in
 // Layout pass of a u8 input, and of the filters when `f` has any, in one launch.
 static int32_t launch_window_pack(const char *fn, hipq_ctx *ctx, const uint8_t *x, int zp, const int32_t *zp_dev,
                                   const ConvGeom &g, const ConvWindow &cw, int8_t *image, const ConvWindowFilters &f) {
-    const int groups = static_cast<int>((size_t(g.nb) * cw.hp * cw.wp + 255) / 256);
-    const dim3 grid(cw.cgs * groups + (f.w ? g.oc : 0));
-#define HIPQ_PACK_WINDOWS(DW)                                                                                         \
-    case DW:                                                                                                          \
-        hipLaunchKernelGGL((conv_window_pack_kernel<DW>), grid, dim3(256), 0, ctx->stream, x, g.c, g.h, g.w, g.ph, g.pw, \
-                           zp, zp_dev, g.nb, groups, image, cw, f);                                                   \
+    const int v = g.w >= 4 ? 4 : 1, runs = (cw.wp + v - 1) / v;
+    const size_t items = size_t(g.nb) * cw.hp * runs;
+    const ConvPackWalk walk{f.w ? g.oc : 0, static_cast<int>((items + 255) / 256), static_cast<int>(items), FastDiv::by(runs), FastDiv::by(cw.hp)};
+    const dim3 grid(walk.filters + cw.cgs * walk.groups_per_cg);
+#define HIPQ_PACK_WINDOWS_V(DW, V)                                                                                         \
+    hipLaunchKernelGGL((conv_window_pack_kernel<DW, V>), grid, dim3(256), 0, ctx->stream, x, g.c, g.h, g.w, g.ph, g.pw, zp, \
+                       zp_dev, walk, image, cw, f)
+#define HIPQ_PACK_WINDOWS(DW)           \
+    case DW:                            \
+        if (v == 4)                     \
+            HIPQ_PACK_WINDOWS_V(DW, 4); \
+        else                            \
+            HIPQ_PACK_WINDOWS_V(DW, 1); \
         break
     switch (cw.pitch / 4) {
         HIPQ_PACK_WINDOWS(1);
@@ -255,6 +263,7 @@ static int32_t launch_window_pack(const char *fn, hipq_ctx *ctx, const uint8_t *
         HIPQ_PACK_WINDOWS(8);
     }
 #undef HIPQ_PACK_WINDOWS
+#undef HIPQ_PACK_WINDOWS_V
     return check_launch(fn);
 }
 

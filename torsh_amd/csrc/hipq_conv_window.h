@@ -17,7 +17,7 @@
 // sum (x - zp) w = sum (x - 128) w + (128 - zp) sum w is undone per output channel in the epilogue.
 //
 // Measured against what it replaced, u8 in, filters as rows (us per forward): [32,3,224,224] x [64,3,7,7] stride 2
-// 2288 -> 31 (a thread per output); [32,64,56,56] x [64,64,3,3] 63 -> 24, [32,128,28,28] x [128,128,3,3] 26.4 -> 20.4,
+// 2288 -> 27 (a thread per output); [32,64,56,56] x [64,64,3,3] 63 -> 24, [32,128,28,28] x [128,128,3,3] 26.4 -> 20.4,
 // [32,256,14,14] x [256,256,3,3] 20.9 -> 17.5, [32,512,7,7] x [512,512,3,3] 28.0 -> 25.9, [32,256,56,56] x [64,256,1,1] 50 -> 33
 // (the packed GEMM over the padded grid, which always split K: its 128 x 64 tiles spend more on the sum of the partial
 // products than on short K, compute the windows of the border, and store single bytes).  What bounds it now: at long K
@@ -47,11 +47,27 @@ struct ConvWindow {
     int plane_bytes;      // bytes per channel group (nb * hp * wp * pitch)
     int image_bytes;      // cgs * plane_bytes
     int hp, wp, sh, sw, ho, wo;
+    FastDiv by_plane, by_wo;  // window -> (image, position), position -> (row, column)
 };
 
-// u8 NCHW -> the layout above.  One thread per (channel group, padded pixel), DW dwords of four channels each
-// (consecutive lanes are consecutive pixels: consecutive bytes of every channel plane).  Workgroups past the image
-// pack the filters: one output channel each, a thread per 16-byte piece.
+// 16, 4 x 4 and 4 bytes at an address that need not be aligned (global memory takes it; the outputs of a channel's plane
+// start wherever ho * wo puts them).
+struct __attribute__((packed, aligned(1))) ConvBytes16 {
+    v4i v;
+};
+struct __attribute__((packed, aligned(4))) ConvWords4 {
+    v4i v;
+};
+struct __attribute__((packed, aligned(1))) ConvWord {
+    uint32_t v;
+};
+
+// u8 NCHW -> the layout above.  One thread per (channel group, V consecutive padded pixels of a row), DW dwords of four
+// channels each (consecutive lanes are consecutive pixels: consecutive bytes of every channel plane).  V = 4: a channel's
+// four pixels are one dword at any alignment, loaded from inside the image row and shifted where the run reaches over
+// its end, and 4 x 4 bytes are transposed by eight permutes: a quarter of the loads and of the address arithmetic, which
+// is what bounded the pass ([32,3,224,224] pad 3: 11.1 -> 5.5 us, filters included; 12 MB moved).  V = 1: rows of fewer than four pixels.
+// Further workgroups pack the filters: one output channel each, a thread per 16-byte piece.
 struct ConvWindowFilters {
     const int8_t *w;  // [OC, IC, KH, KW]
     int8_t *packed;
@@ -59,37 +75,50 @@ struct ConvWindowFilters {
     int ic, kh, kw;
 };
 
-template <int DW>
+// How the image part of the grid is walked: runs of V pixels, `runs` to a padded row.
+struct ConvPackWalk {
+    int filters;        // workgroups that pack filters, ahead of the image's
+    int groups_per_cg;  // workgroups per channel group
+    int items;          // runs per channel group
+    FastDiv by_runs, by_hp;
+};
+
+template <int DW, int V>
 __global__ __launch_bounds__(256) void conv_window_pack_kernel(const uint8_t *__restrict__ x, int C, int H, int W, int pad_h,
                                                                  int pad_w, int zp, const int32_t *__restrict__ zp_dev,
-                                                                 int nb, int groups_per_cg, int8_t *__restrict__ image,
+                                                                 ConvPackWalk walk, int8_t *__restrict__ image,
                                                                  ConvWindow cw, ConvWindowFilters f) {
-    const int work = cw.cgs * groups_per_cg;
-    if (static_cast<int>(blockIdx.x) >= work) {
+    static_assert(V == 1 || V == 4, "pixels per thread");
+    // The filters' workgroups come first: their chain (16 gathered bytes, a sum over the workgroup) is the longer one.
+    if (static_cast<int>(blockIdx.x) < walk.filters) {
         __shared__ int part[4];
-        const int oc = blockIdx.x - work;
-        const int8_t *w = f.w + size_t(oc) * f.ic * f.kh * f.kw;
+        const int oc = blockIdx.x, taps = f.kh * f.kw;
+        const int8_t *w = f.w + size_t(oc) * f.ic * taps;
         int sum = 0;
         for (int piece = threadIdx.x; piece < cw.KB * 2; piece += 256) {
             const int kb = piece / 2, half = piece % 2;
             const int cg = kb % cw.cgs, seg = (kb / cw.cgs) % cw.segs, ty = kb / (cw.cgs * cw.segs);
-            uint32_t d[4] = {0, 0, 0, 0};
-            if (kb < cw.kblocks) {
-                int p = seg * 32 + half * 16;  // byte within the row of taps
-                int tx = p / cw.pitch, c = p % cw.pitch;
+            const int p = seg * 32 + half * 16;  // byte within the row of taps
+            int tx = p / cw.pitch, c = p % cw.pitch;
+            // All 16 requested before the first is used; a byte that is not a weight reads the first one and counts 0.
+            int8_t v[16];
+            bool real[16];
 #pragma unroll
-                for (int b = 0; b < 16; ++b) {
-                    const int ch = cg * cw.pitch + c;
-                    if (tx < f.kw && ch < f.ic) {
-                        const int8_t v = w[(size_t(ch) * f.kh + ty) * f.kw + tx];
-                        sum += v;
-                        d[b / 4] |= static_cast<uint32_t>(static_cast<uint8_t>(v)) << (8 * (b % 4));
-                    }
-                    if (++c == cw.pitch) {
-                        c = 0;
-                        ++tx;
-                    }
+            for (int b = 0; b < 16; ++b) {
+                const int ch = cg * cw.pitch + c;
+                real[b] = kb < cw.kblocks && tx < f.kw && ch < f.ic;
+                v[b] = w[real[b] ? ch * taps + ty * f.kw + tx : 0];
+                if (++c == cw.pitch) {
+                    c = 0;
+                    ++tx;
                 }
+            }
+            uint32_t d[4] = {0, 0, 0, 0};
+#pragma unroll
+            for (int b = 0; b < 16; ++b) {
+                const int value = real[b] ? v[b] : 0;
+                sum += value;
+                d[b / 4] |= static_cast<uint32_t>(static_cast<uint8_t>(value)) << (8 * (b % 4));
             }
             *reinterpret_cast<uint4 *>(f.packed + (size_t(oc / 32) * cw.KB + kb) * 1024 + (oc % 32 + 32 * half) * 16) =
                 make_uint4(d[0], d[1], d[2], d[3]);
@@ -101,45 +130,80 @@ __global__ __launch_bounds__(256) void conv_window_pack_kernel(const uint8_t *__
         if (threadIdx.x == 0) f.wsum[oc] = part[0] + part[1] + part[2] + part[3];
         return;
     }
+    const int block = blockIdx.x - walk.filters, groups_per_cg = walk.groups_per_cg;
     if (zp_dev) zp = *zp_dev;  // the zero point a dynamic quantize has left on the device
-    const int cg = blockIdx.x / groups_per_cg;
-    const int p = (blockIdx.x % groups_per_cg) * 256 + threadIdx.x;
-    if (p >= nb * cw.hp * cw.wp) return;
-    const int n = p / (cw.hp * cw.wp), rem = p % (cw.hp * cw.wp);
-    const int h = rem / cw.wp - pad_h, v = rem % cw.wp - pad_w;
-    uint32_t d[DW];
+    const int cg = block / groups_per_cg;
+    const int item = (block % groups_per_cg) * 256 + threadIdx.x;
+    if (item >= walk.items) return;
+    uint32_t run, row;
+    const uint32_t line = walk.by_runs.quotient(item, &run);  // padded row of the whole batch
+    const uint32_t n = walk.by_hp.quotient(line, &row);
+    const int h = static_cast<int>(row) - pad_h, v = static_cast<int>(run) * V - pad_w;
+    const int pixels = cw.wp - static_cast<int>(run) * V < V ? cw.wp - static_cast<int>(run) * V : V;
     const uint32_t border = static_cast<uint32_t>(static_cast<uint8_t>(zp ^ 0x80)) * 0x01010101u;
+    const size_t plane = size_t(H) * W;
+    const int c0 = cg * DW * 4;
+    uint32_t d[V][DW];
+    if constexpr (V == 1) {
 #pragma unroll
-    for (int i = 0; i < DW; ++i) d[i] = border;
-    if (h >= 0 && h < H && v >= 0 && v < W) {
-        const size_t plane = size_t(H) * W;
-        const int c0 = cg * DW * 4;
-        const uint8_t *src = x + ((size_t(n) * C + c0) * H + h) * W + v;
+        for (int i = 0; i < DW; ++i) d[0][i] = border;
+        if (h >= 0 && h < H && v >= 0 && v < W) {
+            const uint8_t *src = x + ((size_t(n) * C + c0) * H + h) * W + v;
+            uint32_t b[4 * DW];
+#pragma unroll
+            for (int c = 0; c < 4 * DW; ++c) b[c] = c0 + c < C ? src[size_t(c) * plane] : 0u;
+#pragma unroll
+            for (int i = 0; i < DW; ++i)
+                d[0][i] = (b[4 * i] | (b[4 * i + 1] << 8) | (b[4 * i + 2] << 16) | (b[4 * i + 3] << 24)) ^ 0x80808080u;
+        }
+    } else {
+        // The run's pixels v .. v + 3 from the dword at `at`, which lies inside the image row (W >= 4).
+        const int hc = h < 0 ? 0 : (h < H ? h : H - 1);
+        const int at = v < 0 ? 0 : (v < W - 4 ? v : W - 4);
+        const uint8_t *src = x + ((size_t(n) * C + c0) * H + hc) * W + at;
         uint32_t b[4 * DW];
 #pragma unroll
-        for (int c = 0; c < 4 * DW; ++c) b[c] = c0 + c < C ? src[size_t(c) * plane] : 0u;
+        for (int c = 0; c < 4 * DW; ++c) b[c] = c0 + c < C ? reinterpret_cast<const ConvWord *>(src + size_t(c) * plane)->v : 0u;
+        const uint32_t left = 8 * (at - v), right = 8 * (v - at);  // one of them 0; from 32 on no pixel is inside
 #pragma unroll
-        for (int i = 0; i < DW; ++i)
-            d[i] = (b[4 * i] | (b[4 * i + 1] << 8) | (b[4 * i + 2] << 16) | (b[4 * i + 3] << 24)) ^ 0x80808080u;
+        for (int c = 0; c < 4 * DW; ++c) b[c] = v < at ? b[c] << (left & 31) : b[c] >> (right & 31);
+        bool inside[V];
+#pragma unroll
+        for (int p = 0; p < V; ++p) inside[p] = h == hc && v + p >= 0 && v + p < W;
+#pragma unroll
+        for (int i = 0; i < DW; ++i) {
+            const uint32_t lo0 = __builtin_amdgcn_perm(b[4 * i + 1], b[4 * i], 0x05010400u);  // c0p0 c1p0 c0p1 c1p1
+            const uint32_t lo1 = __builtin_amdgcn_perm(b[4 * i + 1], b[4 * i], 0x07030602u);  // ... p2, p3
+            const uint32_t hi0 = __builtin_amdgcn_perm(b[4 * i + 3], b[4 * i + 2], 0x05010400u);
+            const uint32_t hi1 = __builtin_amdgcn_perm(b[4 * i + 3], b[4 * i + 2], 0x07030602u);
+            const uint32_t t[4] = {__builtin_amdgcn_perm(hi0, lo0, 0x05040100u), __builtin_amdgcn_perm(hi0, lo0, 0x07060302u),
+                                   __builtin_amdgcn_perm(hi1, lo1, 0x05040100u), __builtin_amdgcn_perm(hi1, lo1, 0x07060302u)};
+#pragma unroll
+            for (int p = 0; p < V; ++p) d[p][i] = inside[p] ? t[p] ^ 0x80808080u : border;
+        }
     }
-    uint32_t *dst = reinterpret_cast<uint32_t *>(image + size_t(cg) * cw.plane_bytes + size_t(p) * (4 * DW));
-    if constexpr (DW % 4 == 0) {
+    uint32_t *dst = reinterpret_cast<uint32_t *>(image + size_t(cg) * cw.plane_bytes +
+                                                 (size_t(line) * cw.wp + size_t(run) * V) * (4 * DW));
+    if constexpr (V == 4 && DW == 1) {
+        if (pixels == V) {
+            reinterpret_cast<ConvWords4 *>(dst)->v = v4i{static_cast<int>(d[0][0]), static_cast<int>(d[1][0]),
+                                                         static_cast<int>(d[2][0]), static_cast<int>(d[3][0])};
+            return;
+        }
+    }
 #pragma unroll
-        for (int i = 0; i < DW; i += 4) *reinterpret_cast<uint4 *>(dst + i) = make_uint4(d[i], d[i + 1], d[i + 2], d[i + 3]);
-    } else {
+    for (int p = 0; p < V; ++p) {
+        if (p >= pixels) break;
+        if constexpr (DW % 4 == 0) {
 #pragma unroll
-        for (int i = 0; i < DW; ++i) dst[i] = d[i];
+            for (int i = 0; i < DW; i += 4)
+                *reinterpret_cast<uint4 *>(dst + p * DW + i) = make_uint4(d[p][i], d[p][i + 1], d[p][i + 2], d[p][i + 3]);
+        } else {
+#pragma unroll
+            for (int i = 0; i < DW; ++i) dst[p * DW + i] = d[p][i];
+        }
     }
 }
-
-// 16 and 4 x 4 bytes to an address that need not be aligned (global memory takes it; the outputs of a channel's plane
-// start wherever ho * wo puts them).
-struct __attribute__((packed, aligned(1))) ConvBytes16 {
-    v4i v;
-};
-struct __attribute__((packed, aligned(4))) ConvWords4 {
-    v4i v;
-};
 
 template <int FM, int FN, int D, bool SPLIT, int EPI, bool EVEN>
 __global__ __launch_bounds__(256, FM * FN < 8 ? 3 : (SPLIT ? 1 : 2)) void conv_i8_window_kernel(const int8_t *__restrict__ filters,
@@ -195,8 +259,8 @@ __global__ __launch_bounds__(256, FM * FN < 8 ? 3 : (SPLIT ? 1 : 2)) void conv_i
     for (int i = 0; i < FN; ++i) {
         int q = q0 + i * 32 + lane % 32;
         q = q < cw.N ? q : cw.N - 1;
-        const int n = q / plane, rem = q % plane;
-        const int oh = rem / cw.wo, ow = rem % cw.wo;
+        uint32_t rem, ow;
+        const uint32_t n = cw.by_plane.quotient(q, &rem), oh = cw.by_wo.quotient(rem, &ow);
         voi[i] = ((n * cw.hp + oh * cw.sh) * cw.wp + ow * cw.sw) * cw.pitch + 16 * half;
     }
     // This wave's next k block as (tap row, piece, channel group) and its offset in the image.
@@ -282,13 +346,14 @@ __global__ __launch_bounds__(256, FM * FN < 8 ? 3 : (SPLIT ? 1 : 2)) void conv_i
                                static_cast<int>(hi[1])};
             const int first = q + 16 * half;
             if (oc >= cw.M || first >= cw.N) return;
-            const int n = first / plane, pos = first % plane;
+            uint32_t pos;
+            const uint32_t n = cw.by_plane.quotient(first, &pos);
             int8_t *o = static_cast<int8_t *>(ep.out) + (size_t(n) * cw.M + oc) * plane + pos;
-            if (pos + 16 <= plane) {
+            if (static_cast<int>(pos) + 16 <= plane) {
                 reinterpret_cast<ConvBytes16 *>(o)->v = bytes;
             } else {  // the run crosses into the next image (or the end)
                 const size_t skip = size_t(cw.M - 1) * plane;  // from the end of this plane to the next image's
-                int at = pos;
+                int at = static_cast<int>(pos);
 #pragma unroll
                 for (int k = 0; k < 16; ++k) {
                     if (first + k < cw.N) *o = static_cast<int8_t>(bytes[k / 4] >> (8 * (k % 4)));
@@ -309,13 +374,14 @@ __global__ __launch_bounds__(256, FM * FN < 8 ? 3 : (SPLIT ? 1 : 2)) void conv_i
                 const v4i four = {bits(4 * g), bits(4 * g + 1), bits(4 * g + 2), bits(4 * g + 3)};
                 const int first = q + 8 * g + 4 * half;
                 if (oc >= cw.M || first >= cw.N) continue;
-                const int n = first / plane, pos = first % plane;
+                uint32_t pos;
+                const uint32_t n = cw.by_plane.quotient(first, &pos);
                 int32_t *o = static_cast<int32_t *>(ep.out) + (size_t(n) * cw.M + oc) * plane + pos;
-                if (pos + 4 <= plane) {
+                if (static_cast<int>(pos) + 4 <= plane) {
                     reinterpret_cast<ConvWords4 *>(o)->v = four;
                 } else {
                     const size_t skip = size_t(cw.M - 1) * plane;
-                    int at = pos;
+                    int at = static_cast<int>(pos);
 #pragma unroll
                     for (int k = 0; k < 4; ++k) {
                         if (first + k < cw.N) *o = four[k];

@@ -234,6 +234,27 @@ __device__ __forceinline__ float wave_max(float v) {
     return v;
 }
 
+// n / d for 0 <= n < 2^31 by a multiply-high and a shift, where the compiler's division of a lane's value by a launch
+// argument is some thirty instructions, a third of them at quarter rate.  With L = ceil(log2 d) the multiplier is
+// m = floor(2^(31 + L) / d) + 1 <= 2^32 - 1, so m d = 2^(31 + L) + e with 0 < e <= d <= 2^L, and n m / 2^(31 + L)
+// exceeds n / d by n e / (d 2^(31 + L)) < 1 / d: the floor is the quotient.
+struct FastDiv {
+    uint32_t d, m;
+    int shift;
+    __host__ static FastDiv by(uint32_t d) {  // 1 <= d < 2^31
+        if (d <= 1) return FastDiv{1, 0, 0};
+        int l = 0;
+        while ((uint64_t(1) << l) < d) ++l;
+        return FastDiv{d, static_cast<uint32_t>((uint64_t(1) << (31 + l)) / d + 1), l - 1};
+    }
+    __device__ __forceinline__ uint32_t quotient(uint32_t n) const { return d == 1 ? n : __umulhi(n, m) >> shift; }
+    __device__ __forceinline__ uint32_t quotient(uint32_t n, uint32_t *rem) const {
+        const uint32_t q = quotient(n);
+        *rem = n - q * d;
+        return q;
+    }
+};
+
 // (min,max) -> (scale, zero_point) with the reference formula `flavor` selects.
 // Returns HIPQ_SUCCESS or HIPQ_INVALID_ARGUMENT.
 //   HIPQ_PARAMS_SYMMETRIC          crates/torsh-quantization/src/algorithms.rs:397-422
