@@ -262,6 +262,30 @@ def test_non_finite_range_sets_status_and_skips(ctx, hipq, n):
     assert bool((out == 77).all())
 
 
+@pytest.mark.parametrize("n", [1, 2, 3, 5, 4095, 4096 + 1, 3 * 4096 + 2, (1 << 22) + 1, 6 * (1 << 20) + 3])
+def test_dynamic_quantize_one_launch_of_any_length(hipq, n):
+    """Lengths that are no multiple of four (the last elements alone in a workgroup, or behind its last whole float4) in
+    one launch against the two-launch path (variant 6): codes with nothing written behind them, and the whole record."""
+    c = hipq.Context(0)
+    try:
+        g = torch.Generator(device="cuda").manual_seed(n % 977)
+        x = torch.randn(n, generator=g, device="cuda") * 3.0 + 0.5
+        x[-1] = 19.0  # the range is made by the last element
+        for dtype, tdt in ((hipq.DTYPE_I8, torch.int8), (hipq.DTYPE_U8, torch.uint8)):
+            got, want = [], []
+            for res, variant in ((got, 0), (want, 6)):
+                c.set_gemm_kernel_variant(variant)
+                out = torch.full((n + 8,), 77, dtype=tdt, device="cuda")
+                params = torch.full((32,), 255, dtype=torch.uint8, device="cuda")
+                c.quantize_dynamic_per_tensor(x, hipq.PARAMS_AFFINE, dtype, hipq.FORM_DIV, out=out, params=params)
+                res += [out, params]
+            c.synchronize()
+            assert torch.equal(got[0], want[0]) and bool((got[0][n:] == 77).all())
+            assert torch.equal(got[1], want[1]) and bool((got[1][20:] == 0).all())
+    finally:
+        c.close()
+
+
 @pytest.mark.parametrize("n", [1000, 6 * (1 << 20) + 4])
 @pytest.mark.parametrize("dtype_name", ["i8", "u8"])
 def test_dynamic_quantize_one_launch_matches_two_launches(hipq, n, dtype_name):

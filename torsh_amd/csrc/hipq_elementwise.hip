@@ -192,6 +192,7 @@ __device__ __forceinline__ bool resolve_quantize_params(const DynamicRange &dyn,
             dyn.out_params->min_val = r.mn;
             dyn.out_params->max_val = r.mx;
             dyn.out_params->status = st;
+            clear_reserved(dyn.out_params);
         }
         if (bad) {  // the reference errors before quantizing
             if (!dyn.poison) return false;
@@ -209,6 +210,7 @@ __device__ __forceinline__ bool resolve_quantize_params(const DynamicRange &dyn,
         dyn.out_params->min_val = 0.0f;
         dyn.out_params->max_val = 0.0f;
         dyn.out_params->status = HIPQ_SUCCESS;
+        clear_reserved(dyn.out_params);
     }
     return true;
 }
@@ -428,7 +430,8 @@ __global__ __launch_bounds__(kBlock, 4) void quantize_packed_one_launch_kernel(c
 // 64 registers of data per lane: with four workgroups per compute unit the chip's register files hold 16 Mi
 // floats, so even a 4096 x 4096 tensor is read from memory once (29.5 -> ~20 us).  The launch bound keeps the
 // kernel at 128 registers, which is what lets four workgroups share a compute unit: the grid has to be resident
-// at once.  n is a multiple of 4, x is 16-byte and out 4-byte aligned.  `poison`: what a bad range leaves behind,
+// at once.  x is 16-byte and out 4-byte aligned; the up to three elements behind the last whole float4 are loaded and
+// stored one by one by the thread whose turn that float4 would be.  `poison`: what a bad range leaves behind,
 // see meet_on_range; without it no code is written, as in the two-launch path.
 template <typename OutT, bool DIV, int RND, int VPT>
 __global__ __launch_bounds__(kBlock, 4) void quantize_flat_one_launch_kernel(const float *__restrict__ x, size_t n,
@@ -439,6 +442,7 @@ __global__ __launch_bounds__(kBlock, 4) void quantize_flat_one_launch_kernel(con
     static_assert(sizeof(OutT) == 1, "int8 or uint8 codes");
     __shared__ float lds[kMeetingLdsFloats];
     const size_t nvec = n / 4;
+    const int tail = static_cast<int>(n % 4);
     const float4 *x4 = reinterpret_cast<const float4 *>(x);
     const size_t base = size_t(blockIdx.x) * (size_t(kBlock) * VPT) + threadIdx.x;
     const bool whole = (size_t(blockIdx.x) + 1) * (size_t(kBlock) * VPT) <= nvec;
@@ -451,7 +455,13 @@ __global__ __launch_bounds__(kBlock, 4) void quantize_flat_one_launch_kernel(con
         for (int i = 0; i < VPT; ++i) {
             // past the end: a value that changes neither the minimum nor the maximum (NaN is skipped by both)
             v[i] = make_float4(NAN, NAN, NAN, NAN);
-            if (base + size_t(i) * kBlock < nvec) v[i] = x4[base + size_t(i) * kBlock];
+            if (base + size_t(i) * kBlock < nvec) {
+                v[i] = x4[base + size_t(i) * kBlock];
+            } else if (base + size_t(i) * kBlock == nvec && tail) {
+                v[i].x = x[nvec * 4];
+                if (tail > 1) v[i].y = x[nvec * 4 + 1];
+                if (tail > 2) v[i].z = x[nvec * 4 + 2];
+            }
         }
     }
     const uint32_t gen = meeting_number(words);  // behind the data in program order: returned after it
@@ -472,13 +482,19 @@ __global__ __launch_bounds__(kBlock, 4) void quantize_flat_one_launch_kernel(con
     const float zpf = static_cast<float>(agreed.zero_point);
     uint32_t *out4 = reinterpret_cast<uint32_t *>(out);
 #pragma unroll
-    for (int i = 0; i < VPT; ++i)
-        if (whole || base + size_t(i) * kBlock < nvec)
-            store_stream(out4 + base + size_t(i) * kBlock,
-                         pack4(quantize_int<DIV, RND>(v[i].x, scale, inv, zpf, qmin, qmax),
-                               quantize_int<DIV, RND>(v[i].y, scale, inv, zpf, qmin, qmax),
-                               quantize_int<DIV, RND>(v[i].z, scale, inv, zpf, qmin, qmax),
-                               quantize_int<DIV, RND>(v[i].w, scale, inv, zpf, qmin, qmax)));
+    for (int i = 0; i < VPT; ++i) {
+        const size_t at = base + size_t(i) * kBlock;
+        if (!whole && at > nvec) continue;
+        const uint32_t codes = pack4(quantize_int<DIV, RND>(v[i].x, scale, inv, zpf, qmin, qmax),
+                                     quantize_int<DIV, RND>(v[i].y, scale, inv, zpf, qmin, qmax),
+                                     quantize_int<DIV, RND>(v[i].z, scale, inv, zpf, qmin, qmax),
+                                     quantize_int<DIV, RND>(v[i].w, scale, inv, zpf, qmin, qmax));
+        if (whole || at < nvec) {
+            store_stream(out4 + at, codes);
+        } else {
+            for (int b = 0; b < tail; ++b) out[nvec * 4 + b] = static_cast<OutT>(codes >> (8 * b));
+        }
+    }
 }
 
 // The one-launch quantizers that hold 64 floats a lane need four workgroups per compute unit resident: what the
@@ -504,13 +520,13 @@ bool four_wide_workgroups_fit(const hipq_ctx *ctx) {
 template <typename OutT>
 static bool launch_flat_one_launch(hipq_ctx *ctx, const float *x, size_t n, int flavor, int qmin, int qmax, int mode,
                                    bool poison, hipq_qparams *out_params, OutT *out, int32_t *rc) {
-    if (ctx->gemm_variant == 6 || n % 4 != 0 || (reinterpret_cast<uintptr_t>(x) & 15u) ||
+    if (ctx->gemm_variant == 6 || (reinterpret_cast<uintptr_t>(x) & 15u) ||
         (reinterpret_cast<uintptr_t>(out) & 3u) || (mode & ~(HIPQ_FORM_DIV | HIPQ_ROUND_HALF_EVEN)))
         return false;
     // The torsh-nn flavours do not clamp their zero point to the code range (min = 2, max = 5 gives -170), and the
     // word the meeting ends with has room for -128..895 only: they take the two launches, whatever the size.
     if (flavor > HIPQ_PARAMS_ZERO_INCLUDED) return false;
-    const size_t nvec = n / 4;
+    const size_t nvec = (n + 3) / 4;
     const int vpt = nvec <= resident_workgroups(ctx, false) * kBlock * 4 ? 4 : 16;
     const size_t blocks = (nvec + size_t(kBlock) * vpt - 1) / (size_t(kBlock) * vpt);
     if (blocks > resident_workgroups(ctx, vpt == 16)) return false;

@@ -255,6 +255,12 @@ struct FastDiv {
     }
 };
 
+// A kernel that writes a parameter record writes all of it, so that the record needs no fill before.
+__device__ __forceinline__ void clear_reserved(hipq_qparams *p) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) p->reserved[i] = 0;
+}
+
 // (min,max) -> (scale, zero_point) with the reference formula `flavor` selects.
 // Returns HIPQ_SUCCESS or HIPQ_INVALID_ARGUMENT.
 //   HIPQ_PARAMS_SYMMETRIC          crates/torsh-quantization/src/algorithms.rs:397-422

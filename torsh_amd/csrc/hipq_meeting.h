@@ -195,6 +195,7 @@ __device__ __forceinline__ MeetingParams meet_on_range(uint32_t *words, uint32_t
             out_params->zero_point = bad ? zp : p.zero_point;
             out_params->min_val = t.mn;
             out_params->max_val = t.mx;
+            clear_reserved(out_params);
             // A workgroup that stopped waiting for the word above has marked the context; the record says so as
             // well (it writes the status itself too, in case this store is the later one).
             const bool lost = __hip_atomic_load(words + kCtxFlagWord, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;

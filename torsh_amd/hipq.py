@@ -49,6 +49,9 @@ class QParams(C.Structure):
                 ("status", C.c_int32), ("reserved", C.c_int32 * 3)]
 
 
+_QPARAMS_BYTES = C.sizeof(QParams)
+
+
 class QuantMetrics(C.Structure):
     """hipq_quant_metrics: the fields of the reference's QuantizationMetrics, in its order."""
     _fields_ = [(n, C.c_float) for n in ("mse", "psnr", "snr", "mae", "max_error", "zero_error_percentage",
@@ -226,6 +229,7 @@ class Context:
         self._lib = load()
         self.handle = _vp()
         self.device = device
+        self._device = torch.device("cuda", device)
         if own_stream:
             _check(self._lib.hipq_ctx_create(device, C.byref(self.handle)))
         else:
@@ -276,7 +280,7 @@ class Context:
 
     # ---- convenience wrappers over torch tensors (device memory only) -------------
     def _dev(self):
-        return torch.device("cuda", self.device)
+        return self._device
 
     def minmax(self, x: torch.Tensor) -> torch.Tensor:
         out = torch.empty(2, dtype=torch.float32, device=self._dev())
@@ -287,6 +291,10 @@ class Context:
         out = torch.empty(1, dtype=torch.float32, device=self._dev())
         self.call("hipq_absmax_f32", _ptr(x), x.numel(), _ptr(out))
         return out
+
+    def _unset_qparams(self) -> torch.Tensor:
+        """A record for a call that writes every field of it (a zeroed one costs a launch of its own)."""
+        return torch.empty(_QPARAMS_BYTES, dtype=torch.uint8, device=self._device)
 
     def new_qparams(self) -> torch.Tensor:
         return torch.zeros(C.sizeof(QParams), dtype=torch.uint8, device=self._dev())
@@ -391,7 +399,7 @@ class Context:
     def quantize_dynamic_per_tensor(self, x, flavor=PARAMS_SYMMETRIC, dtype=DTYPE_I8, mode=0, out=None, params=None):
         tdt = torch.int8 if dtype == DTYPE_I8 else torch.uint8
         out = out if out is not None else torch.empty(x.shape, dtype=tdt, device=self._dev())
-        params = params if params is not None else self.new_qparams()
+        params = params if params is not None else self._unset_qparams()
         self.call("hipq_quantize_dynamic_per_tensor_f32", _ptr(x), x.numel(), flavor, dtype, mode, _ptr(out),
                   _ptr(params))
         return out, params
@@ -732,7 +740,7 @@ class Context:
         ho = h + 2 * padding[0] - kh + 1
         wo = wd + 2 * padding[1] - kw + 1
         out = out if out is not None else torch.empty((nb, oc, ho, wo), dtype=torch.int8, device=self._dev())
-        params = params if params is not None else self.new_qparams()
+        params = params if params is not None else self._unset_qparams()
         self.call("hipq_conv2d_dynamic_f32_i8_packed", _ptr(x), flavor, quant_mode, _ptr(w_packed), _ptr(w_sums),
                   _ptr(w_scales), _ptr(bias), nb, c, h, wd, oc, kh, kw, padding[0], padding[1], float(s_out),
                   int(zp_out), mode, _ptr(out), _ptr(params))
