@@ -323,21 +323,26 @@ __global__ __launch_bounds__(256, FM * FN < 8 ? 3 : (SPLIT ? 1 : 2)) void conv_i
     // Outputs of one accumulator block: channel block column j of this wave's constants, first window q.
     const float zpf = static_cast<float>(ep.zp_out);
     const uint32_t offset2 = static_cast<uint32_t>(ep.zp_out + 128) * 0x10001u;
+    RequantFast fast[COLS];
     auto emit_block = [&](const v16i &a, int j, int oc, int q, auto plain) {
         auto dequant = [&](int r) { return static_cast<float>(a[r]) * sc[j] + bias[j]; };
         if constexpr (EPI == EPI_I8) {
             // register 4 g + i of half h is window 8 g + 4 h + i; after the exchange half h holds windows 16 h .. + 15
             uint32_t w[4];
+            bool done = false;
+            if constexpr (decltype(plain)::value) done = requant_fast16(a, fast[j], offset2, w);
+            if (!done) {
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const float v[4] = {dequant(4 * g), dequant(4 * g + 1), dequant(4 * g + 2), dequant(4 * g + 3)};
-                if constexpr (decltype(plain)::value) {
-                    w[g] = requant_pack4<EVEN>(v, ep.s_out, ep.s_out_inv, offset2);
-                } else {
-                    auto code = [&](float f) {  // NaN -> 0
-                        return clamp_to_int(round_mode<EVEN>(div_rn(f, ep.s_out, ep.s_out_inv)) + zpf, -128, 127);
-                    };
-                    w[g] = pack4(code(v[0]), code(v[1]), code(v[2]), code(v[3]));
+                for (int g = 0; g < 4; ++g) {
+                    const float v[4] = {dequant(4 * g), dequant(4 * g + 1), dequant(4 * g + 2), dequant(4 * g + 3)};
+                    if constexpr (decltype(plain)::value) {
+                        w[g] = requant_pack4<EVEN>(v, ep.s_out, ep.s_out_inv, offset2);
+                    } else {
+                        auto code = [&](float f) {  // NaN -> 0
+                            return clamp_to_int(round_mode<EVEN>(div_rn(f, ep.s_out, ep.s_out_inv)) + zpf, -128, 127);
+                        };
+                        w[g] = pack4(code(v[0]), code(v[1]), code(v[2]), code(v[3]));
+                    }
                 }
             }
             const auto lo = __builtin_amdgcn_permlane32_swap(w[0], w[2], false, false);
@@ -395,8 +400,10 @@ __global__ __launch_bounds__(256, FM * FN < 8 ? 3 : (SPLIT ? 1 : 2)) void conv_i
             }
         }
     };
-    bool all_plain = true;
+    bool all_plain = ep.zp_out >= -32000 && ep.zp_out <= 32000;  // (zp + 128 has 16 bits in the packed clamp)
     if constexpr (EPI == EPI_I8) {
+#pragma unroll
+        for (int j = 0; j < COLS; ++j) fast[j] = RequantFast(sc[j], bias[j], ep.s_out_inv, ep.zp_out);
 #pragma unroll
         for (int j = 0; j < COLS; ++j) all_plain = all_plain && requant_is_plain(sc[j], bias[j], ep.s_out_inv);
     }
@@ -411,7 +418,9 @@ __global__ __launch_bounds__(256, FM * FN < 8 ? 3 : (SPLIT ? 1 : 2)) void conv_i
 #pragma unroll
             for (int j = 0; j < FM; ++j)
 #pragma unroll
-                for (int i = 0; i < FN; ++i) emit_block(acc[j][i], j, (rb0 + j) * 32 + lane % 32, q0 + i * 32, plain);
+                for (int i = 0; i < FN; ++i)
+                    if ((rb0 + j) * 32 < cw.M)  // (a channel block past the last has no outputs)
+                        emit_block(acc[j][i], j, (rb0 + j) * 32 + lane % 32, q0 + i * 32, plain);
         });
     } else {
         // Block b = j * FN + i belongs to wave b / OWN; the other three park their partial sums of it in LDS.

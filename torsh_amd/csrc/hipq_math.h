@@ -181,6 +181,19 @@ __device__ __forceinline__ uint32_t pack4(int a, int b, int c, int d) {
     return lo | hi;
 }
 
+// Four bytes clamp(q + zp, -128, 127) in one dword; offset2 holds zp + 128 in both halves.  To i16 with saturation, +
+// offset with saturation, to u8 with saturation, then the top bits flipped.
+__device__ __forceinline__ uint32_t saturate_pack4(int q0, int q1, int q2, int q3, uint32_t offset2) {
+    uint32_t h[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        uint32_t t;
+        asm("v_cvt_pk_i16_i32 %0, %1, %2" : "=v"(t) : "v"(i ? q2 : q0), "v"(i ? q3 : q1));
+        asm("v_pk_add_i16 %0, %1, %2 clamp" : "=v"(t) : "v"(t), "v"(offset2));
+        asm("v_sat_pk_u8_i16 %0, %1" : "=v"(h[i]) : "v"(t));
+    }
+    return ((h[1] << 16) | h[0]) ^ 0x80808080u;
+}
 // Four requantized bytes clamp(round(v / s) + zp, -128, 127) in one dword, for values whose quotient is finite
 // (requant_is_plain).  inv = recip_for_div(s), not 0; offset2 holds zp + 128 in both halves.  Division as div_rn
 // without its guards; the clamp by the saturating packs: to i16, + offset saturating, to u8, then the top bits flipped
@@ -195,15 +208,41 @@ __device__ __forceinline__ uint32_t requant_pack4(const float (&v)[4], float s, 
         // v_cvt_i32_f32 truncates: the trunc of round_mode<0> is its own
         q[i] = cvt_i32_sat(EVEN ? rintf(d) : d + copysignf(0x1.fffffep-2f, d));
     }
-    uint32_t h[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        uint32_t t;
-        asm("v_cvt_pk_i16_i32 %0, %1, %2" : "=v"(t) : "v"(q[2 * i]), "v"(q[2 * i + 1]));
-        asm("v_pk_add_i16 %0, %1, %2 clamp" : "=v"(t) : "v"(t), "v"(offset2));
-        asm("v_sat_pk_u8_i16 %0, %1" : "=v"(h[i]) : "v"(t));
+    return saturate_pack4(q[0], q[1], q[2], q[3], offset2);
+}
+// The codes of 16 accumulators in one fused multiply-add each, where that is provably the same: with A = sc / s and
+// B = bias / s + 1/2 + eps in f32, U = fma(acc, A, B) is within eps of (the quotient the exact chain rounds) + 1/2 + eps,
+// so floor(U) is the code unless U lies less than 2 eps above an integer; which way ties go never matters.  With u = 2^-24,
+// b = |bias / s| and |quotient| <= T: the chain's multiply, add and divide are off by u (T + b) + u T + u T, A by 2 u, B by
+// 2 u b + u |B| and the fma by u |U|, together at most u (6 T + 6 b + 2); codes beyond T = 129 + |zp| saturate either way.
+// A lane that has such a value (once in ten blocks of 1024 at T = 129) sends the wave to the exact form: 6.5 instructions
+// per value instead of 11 where it does not.
+struct RequantFast {
+    float a, b, limit;
+    __device__ __forceinline__ RequantFast() {}
+    __device__ __forceinline__ RequantFast(float sc, float bias, float inv, int zp) {
+        const float t = 129.0f + fabsf(static_cast<float>(zp)), bq = bias * inv;
+        const float eps = (6.0f * t + 6.0f * fabsf(bq) + 4.0f) * 0x1.02p-24f;
+        a = sc * inv;
+        b = bq + (0.5f + eps);
+        limit = 2.0f * eps;
     }
-    return ((h[1] << 16) | h[0]) ^ 0x80808080u;
+};
+// w[g]: the bytes of accumulators 4 g .. 4 g + 3, valid where it returns true (the same for all lanes of the wave).
+// For values that requant_is_plain has cleared.
+template <typename Acc>
+__device__ __forceinline__ bool requant_fast16(const Acc &acc, const RequantFast &f, uint32_t offset2, uint32_t (&w)[4]) {
+    int q[16];
+    float low = 1.0f;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const float v = fmaf(static_cast<float>(acc[r]), f.a, f.b);
+        low = fminf(low, __builtin_amdgcn_fractf(v));
+        asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(q[r]) : "v"(v));
+    }
+#pragma unroll
+    for (int g = 0; g < 4; ++g) w[g] = saturate_pack4(q[4 * g], q[4 * g + 1], q[4 * g + 2], q[4 * g + 3], offset2);
+    return !__any(!(low >= f.limit));
 }
 // Whether requant_pack4 may take every value acc * scale + bias (|acc| < 2^31) of this wave.
 __device__ __forceinline__ bool requant_is_plain(float scale, float bias, float inv) {
@@ -222,16 +261,39 @@ __device__ __forceinline__ uint32_t quad_byte_transpose(uint32_t d, uint32_t sel
     return __builtin_amdgcn_perm(p2, t, sel2);
 }
 
+// Butterfly over the 64 lanes in the order lane ^ 32, 16, 8, 4, 2, 1, all lanes ending with the result; op commutes.  The
+// two wide steps are the half and the row swap, the others moves inside a row of 16: a rotation by 8, by 4 (equal to
+// lane ^ 4, since lanes 8 apart agree by then) and two quad permutes.  A step is two dependent vector instructions instead
+// of a trip through LDS, which is what a kernel of one row per wave waits for (LayerNorm + quantize of 77 x 768: three such
+// reductions one after the other).
+template <int CTRL>
+__device__ __forceinline__ float lane_move(float v) {
+    const int b = __builtin_bit_cast(int, v);
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(b, b, CTRL, 0xf, 0xf, true));
+}
+template <typename Op>
+__device__ __forceinline__ float wave_butterfly(float v, Op op) {
+    uint32_t b = __builtin_bit_cast(uint32_t, v);
+    const auto halves = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+    // (through scalars: a bit cast of a vector's element takes its first one)
+    const uint32_t h0 = halves[0], h1 = halves[1];
+    v = op(__builtin_bit_cast(float, h0), __builtin_bit_cast(float, h1));
+    b = __builtin_bit_cast(uint32_t, v);
+    const auto rows = __builtin_amdgcn_permlane16_swap(b, b, false, false);
+    const uint32_t r0 = rows[0], r1 = rows[1];
+    v = op(__builtin_bit_cast(float, r0), __builtin_bit_cast(float, r1));
+    v = op(v, lane_move<0x128>(v));  // row_ror:8
+    v = op(v, lane_move<0x124>(v));  // row_ror:4
+    v = op(v, lane_move<0x4E>(v));   // quad_perm [2, 3, 0, 1]
+    return op(v, lane_move<0xB1>(v));  // quad_perm [1, 0, 3, 2]
+}
+
 __device__ __forceinline__ float wave_min(float v) {
-#pragma unroll
-    for (int o = kWave / 2; o > 0; o >>= 1) v = fminf(v, __shfl_xor(v, o, kWave));
-    return v;
+    return wave_butterfly(v, [](float a, float b) { return fminf(a, b); });
 }
 
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int o = kWave / 2; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, kWave));
-    return v;
+    return wave_butterfly(v, [](float a, float b) { return fmaxf(a, b); });
 }
 
 // n / d for 0 <= n < 2^31 by a multiply-high and a shift, where the compiler's division of a lane's value by a launch
