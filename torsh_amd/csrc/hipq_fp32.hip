@@ -12,9 +12,7 @@ constexpr int kRowBlock = 256;
 constexpr int kRowCacheMax = 12;  // most float4 a thread keeps in registers (RC template parameter)
 
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int o = kWave / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
-    return v;
+    return wave_butterfly(v, [](float a, float b) { return a + b; });
 }
 
 template <int TPR>
@@ -71,6 +69,30 @@ __device__ __forceinline__ float gelu_tanh(float x) {
 
 enum { ROW_LAYERNORM = 0, ROW_GELU = 1 };
 
+// Gain and offset of a LayerNorm (either may be null).  Held: requested together with the row instead of behind its sums -
+// a trip to memory less where a wave has a single row.
+template <int TPR, int RC>
+struct RowAffine {
+    const float *gamma = nullptr, *beta = nullptr;
+    bool held = false;
+    float4 g[RC], b[RC];
+    __device__ __forceinline__ void hold(int lane, size_t nvec) {
+        held = true;
+#pragma unroll
+        for (int i = 0; i < RC; ++i) {
+            const size_t idx = size_t(lane) + size_t(i) * TPR;
+            if (gamma && idx < nvec) g[i] = reinterpret_cast<const float4 *>(gamma)[idx];
+            if (beta && idx < nvec) b[i] = reinterpret_cast<const float4 *>(beta)[idx];
+        }
+    }
+    __device__ __forceinline__ float4 gamma_at(int i, size_t idx) const {
+        return held ? g[i] : reinterpret_cast<const float4 *>(gamma)[idx];
+    }
+    __device__ __forceinline__ float4 beta_at(int i, size_t idx) const {
+        return held ? b[i] : reinterpret_cast<const float4 *>(beta)[idx];
+    }
+};
+
 // OP: LayerNorm over the row (biased variance, eps inside the square root) or GELU.
 // QUANT: write the row as per-token symmetric int8 (scale = absmax/127,
 // q = clamp(round(y / scale)), the division form of
@@ -80,8 +102,7 @@ enum { ROW_LAYERNORM = 0, ROW_GELU = 1 };
 // so both streams bypass the caches.
 template <int TPR, int RC, int OP, bool QUANT, bool EVEN>
 __device__ __forceinline__ void row_op_body(float4 (&v)[RC], size_t row, bool active, int lane, size_t cols,
-                                            const float *__restrict__ gamma, const float *__restrict__ beta,
-                                            float eps, float *__restrict__ out_f, int8_t *__restrict__ out_q,
+                                            const RowAffine<TPR, RC> &affine, float eps, float *__restrict__ out_f, int8_t *__restrict__ out_q,
                                             float *__restrict__ out_scales, int packed, float *lds) {
     const size_t nvec = cols / 4;
     if constexpr (OP == ROW_LAYERNORM) {
@@ -100,19 +121,18 @@ __device__ __forceinline__ void row_op_body(float4 (&v)[RC], size_t row, bool ac
         }
         const float var = row_sum<TPR>(sq, lds) / static_cast<float>(cols);
         const float rstd = 1.0f / sqrtf(var + eps);
-        const float4 *g4 = reinterpret_cast<const float4 *>(gamma), *b4 = reinterpret_cast<const float4 *>(beta);
 #pragma unroll
         for (int i = 0; i < RC; ++i) {
             const size_t idx = size_t(lane) + size_t(i) * TPR;
             if (idx < nvec) {
                 float4 y = make_float4((v[i].x - mean) * rstd, (v[i].y - mean) * rstd, (v[i].z - mean) * rstd,
                                        (v[i].w - mean) * rstd);
-                if (gamma) {
-                    const float4 g = g4[idx];
+                if (affine.gamma) {
+                    const float4 g = affine.gamma_at(i, idx);
                     y = make_float4(y.x * g.x, y.y * g.y, y.z * g.z, y.w * g.w);
                 }
-                if (beta) {
-                    const float4 b = b4[idx];
+                if (affine.beta) {
+                    const float4 b = affine.beta_at(i, idx);
                     y = make_float4(y.x + b.x, y.y + b.y, y.z + b.z, y.w + b.w);
                 }
                 v[i] = y;
@@ -214,11 +234,15 @@ __global__ __launch_bounds__(kRowBlock) void row_op_kernel(const float *x, const
     float4 v[RC], d[RD];
     size_t g = blockIdx.x;
     if (g >= groups) return;
+    RowAffine<TPR, RC> affine;
+    affine.gamma = gamma;
+    affine.beta = beta;
     load_row(g, v, d);
     if constexpr (!STRIDE) {
         const size_t row = g * kRowsPerBlock + sub;
+        if constexpr (OP == ROW_LAYERNORM && RC <= 4) affine.hold(lane, nvec);
         add_row(g, v, d);
-        row_op_body<TPR, RC, OP, QUANT, EVEN>(v, row, row < rows, lane, cols, gamma, beta, eps, out_f, out_q, out_scales,
+        row_op_body<TPR, RC, OP, QUANT, EVEN>(v, row, row < rows, lane, cols, affine, eps, out_f, out_q, out_scales,
                                               packed, lds);
     } else {
         float4 nx[RC], nd[RD];
@@ -227,7 +251,7 @@ __global__ __launch_bounds__(kRowBlock) void row_op_kernel(const float *x, const
             if (gn < groups) load_row(gn, nx, nd);
             const size_t row = g * kRowsPerBlock + sub;
             add_row(g, v, d);
-            row_op_body<TPR, RC, OP, QUANT, EVEN>(v, row, row < rows, lane, cols, gamma, beta, eps, out_f, out_q,
+            row_op_body<TPR, RC, OP, QUANT, EVEN>(v, row, row < rows, lane, cols, affine, eps, out_f, out_q,
                                                   out_scales, packed, lds);
 #pragma unroll
             for (int i = 0; i < RC; ++i) v[i] = nx[i];

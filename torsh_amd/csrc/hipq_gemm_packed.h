@@ -245,6 +245,35 @@ __global__ __launch_bounds__(256) void gemm_i8_packed_kernel(const int8_t *__res
     }
 }
 
+// fp32 epilogue of one 32 x 32 block in a kernel that lives for a few microseconds: the row scales and the residual are
+// requested before the main loop, so that no trip to memory is left behind it, and the results are ordinary stores, which
+// leave them where the next kernel finds them sooner.  The arithmetic is store_tile's.
+struct BlockOperands {
+    float scale[16], residual[16];
+    __device__ __forceinline__ void request(const GemmEpilogue &ep, int M, int N, int row0, int n, int lane, float sa0) {
+        const int nc = n < N ? n : N - 1;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int m = row0 + 8 * (r / 4) + 4 * (lane / 32) + (r % 4), mc = m < M ? m : M - 1;
+            scale[r] = ep.sa_per_row ? ep.sa[mc] : sa0;
+            residual[r] = ep.residual ? ep.residual[size_t(mc) * N + nc] : 0.0f;
+        }
+    }
+    __device__ __forceinline__ void store(const v16i &acc, const GemmEpilogue &ep, int M, int N, int row0, int n, int lane,
+                                          float sw, float bias) const {
+        if (n >= N) return;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int m = row0 + 8 * (r / 4) + 4 * (lane / 32) + (r % 4);
+            if (m >= M) continue;
+            float v = static_cast<float>(acc[r]) * (scale[r] * sw);
+            if (ep.bias) v = v + bias;
+            if (ep.residual) v = v + residual[r];
+            static_cast<float *>(ep.out)[size_t(m) * N + n] = v;
+        }
+    }
+};
+
 // Skinny product on packed operands (M <= 32: decode-shaped Linear).  The weight matrix is read exactly once and
 // nothing else matters: one 32-row block of weights per workgroup, K split between the four waves, D stages of
 // one weight fragment (1 KiB, contiguous in HBM) and one activation fragment (L2 resident) per wave in flight.
@@ -297,6 +326,9 @@ __global__ __launch_bounds__(256) void gemv_i8_packed_kernel(const int8_t *__res
     for (int r = 0; r < 16; ++r) acc[r] = 0;
 #pragma unroll
     for (int u = 0; u < D; ++u) issue(u, u);
+    BlockOperands operands;
+    if constexpr (EPI == EPI_F32)
+        if (wave == 0) operands.request(ep, M, N, 0, nn[0], lane, sa0);
     for (int s0 = D; s0 < rounds_end; s0 += D) {
 #pragma unroll
         for (int u = 0; u < D; ++u) {
@@ -319,7 +351,10 @@ __global__ __launch_bounds__(256) void gemv_i8_packed_kernel(const int8_t *__res
 #pragma unroll
         for (int c = 0; c < 4; ++c) own[0][0][4 * g + c] = acc[4 * g + c] + t[c];
     }
-    store_tile<1, 1, 1, EPI, EVEN>(own, ep, M, N, 0, 0, lane, nn, swv, bv, sa0);
+    if constexpr (EPI == EPI_F32)
+        operands.store(own[0][0], ep, M, N, 0, nn[0], lane, swv[0], bv[0]);
+    else
+        store_tile<1, 1, 1, EPI, EVEN>(own, ep, M, N, 0, 0, lane, nn, swv, bv, sa0);
 }
 
 // The same with RB = 1 or 2 activation row blocks and TNB = 1 or 2 32-row blocks of weights per workgroup (a batch of
@@ -400,6 +435,10 @@ __global__ __launch_bounds__(256) void skinny_i8_packed_kernel(const int8_t *__r
     };
 #pragma unroll
     for (int u = 0; u < D; ++u) issue(u, u);
+    const int row0 = (rb0 + wave / TNB) * 32;  // of the block this wave will own
+    BlockOperands operands;
+    if constexpr (EPI == EPI_F32)
+        if (wave < NBLK) operands.request(ep, M, N, row0, nn[0], lane, sa0);
     for (int s0 = D; s0 < rounds_end; s0 += D) {
 #pragma unroll
         for (int u = 0; u < D; ++u) {
@@ -431,7 +470,10 @@ __global__ __launch_bounds__(256) void skinny_i8_packed_kernel(const int8_t *__r
             for (int c = 0; c < 4; ++c) own[0][0][4 * g + c] = acc[b][4 * g + c] + t[c];
         }
     }
-    store_tile<1, 1, 1, EPI, EVEN>(own, ep, M, N, (rb0 + wave / TNB) * 32, 0, lane, nn, swv, bv, sa0);
+    if constexpr (EPI == EPI_F32)
+        operands.store(own[0][0], ep, M, N, row0, nn[0], lane, swv[0], bv[0]);
+    else
+        store_tile<1, 1, 1, EPI, EVEN>(own, ep, M, N, row0, 0, lane, nn, swv, bv, sa0);
 }
 
 // The same product straight from fp32 activations of at most four rows (decode), per-row dynamic int8: one launch
