@@ -21,7 +21,7 @@ extern "C" {
  * Linear forwards run as two launches (range partials, then a quantizer that folds them) where it
  * would run as one, and the per-token forward of one or two rows as a quantizer and a product where
  * it would be one kernel; 9 and 11 leave the choice automatic and switch off, on prepared operands,
- * the forms of the GEMM that are picked by occupancy - two workgroups per compute unit, the
+ * the forms of the GEMM that are picked by occupancy - two workgroups per compute unit, K split between the waves of few blocks, the
  * weight-streaming kernel for 33..128 rows - (9) and the touching of weight / filter lines by the
  * one-launch activation quantizers of the dynamic Linear and Conv2d forwards while their grids wait
  * for the range (11); on prepared operands 7 and 8 force the tiles of 256 x 128 and 128 x 256 that are

@@ -816,3 +816,33 @@ def test_gemm_tiles_staged_through_lds(hipq, oracle, m, n, k, tall):
     finally:
         torch.cuda.synchronize()
         c.close()
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 1, 1), (1, 768, 768), (32, 33, 129), (33, 31, 512), (40, 65, 513), (31, 200, 1024), (77, 768, 3072),
+                                   (65, 64, 1025), (9, 513, 4097), (300, 64, 12480), (1000, 1000, 96), (129, 250, 640)])
+def test_products_of_few_blocks(hipq, m, n, k):
+    """K split between 4, 8 or 16 waves (one or several rounds of steps, waves without any): int32 sums against float64
+    (|sum| < 2^53), the fp32 forward with and without per-row scales and bias against the forms of variant 9, bit for bit,
+    and nothing written outside the matrix."""
+    c = hipq.Context(0)
+    try:
+        g = torch.Generator(device="cuda").manual_seed(m * 7 + n + k)
+        a = torch.randint(-128, 128, (m, k), generator=g, device="cuda", dtype=torch.int8)
+        w = torch.randint(-128, 128, (n, k), generator=g, device="cuda", dtype=torch.int8)
+        pa, pw = c.pack_rows(a), c.pack_rows(w)
+        want = (a.double().cpu() @ w.double().cpu().t()).to(torch.int32)
+        out = torch.full((m + 1, n), 77, dtype=torch.int32, device="cuda")
+        c.gemm_packed_i8_i32(pa, pw, m, n, k, out=out)
+        c.synchronize()
+        assert torch.equal(out[:m].cpu(), want) and bool((out[m] == 77).all())
+        sw, bias = torch.rand(n, generator=g, device="cuda"), torch.randn(n, generator=g, device="cuda")
+        for sa in (torch.rand(m, generator=g, device="cuda"), torch.rand(1, generator=g, device="cuda")):
+            for b in (bias, None):
+                got = []
+                for variant in (0, 9):
+                    c.set_gemm_kernel_variant(variant)
+                    got.append(c.linear_packed_i8_f32(pa, sa, pw, sw, b, m, n, k))
+                c.synchronize()
+                assert torch.equal(got[0], got[1])
+    finally:
+        c.close()

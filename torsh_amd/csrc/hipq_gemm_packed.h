@@ -757,6 +757,116 @@ static int32_t launch_gemv_packed(hipq_ctx *ctx, const int8_t *pa, const int8_t 
     }
 }
 
+// Products of few 32 x 32 output blocks: a workgroup per block and K split between all of its WK waves, so that even a few
+// dozen blocks keep many loads in flight and a wave's share of K is a handful of steps, all requested at once (D of them;
+// further ones, if any, a round behind).  What bounds such a product is latency - a trip to memory for the fragments and
+// the sum of the partial blocks - not the operand bytes.  All waves park their partial block in LDS; waves 0 .. 3 sum
+// four of its 16 registers each (rows 8 wave + 4 half + 0 .. 3) and store them.
+template <int WK, int D, int EPI>
+__global__ __launch_bounds__(64 * WK) void split_i8_packed_kernel(const int8_t *__restrict__ PA, const int8_t *__restrict__ PW,
+                                                                  int M, int N, int K, GemmEpilogue ep) {
+    static_assert(EPI == EPI_F32 || EPI == EPI_I32, "4-byte results");
+    __shared__ __attribute__((aligned(16))) v4i part[WK][4][kWave];
+    const int KB = static_cast<int>(packed_k_blocks(K));
+    const int lane = threadIdx.x % kWave;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int row0 = static_cast<int>(blockIdx.y) * 32, n = static_cast<int>(blockIdx.x) * 32 + lane % 32;
+    const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t *>(PA), 0, 0x7ffffffe, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t *>(PW), 0, 0x7fffffff, 0x00020000);
+    const int soa = static_cast<int>(blockIdx.y) * KB * 1024, sow = static_cast<int>(blockIdx.x) * KB * 1024;
+    const int voff = lane * 16, voffa = row0 + lane % 32 < M ? voff : 0x7fffffff;  // rows past M: zeros, no memory access
+    v4i fa[D], fw[D];
+    auto issue = [&](int s, int slot) {
+        const int kb = wave + WK * s;
+        const bool real = kb < KB;
+        fa[slot] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(ra, real ? voffa : 0x7fffffff,
+                                                                                 real ? soa + kb * 1024 : 0, 0));
+        fw[slot] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rw, real ? voff : 0x7fffffff,
+                                                                                 real ? sow + kb * 1024 : 0, 0));
+    };
+#pragma unroll
+    for (int u = 0; u < D; ++u) issue(u, u);
+    float scale[4], residual[4], bias = 0.0f;
+    if constexpr (EPI == EPI_F32) {
+        if (wave < 4) {
+            const int nc = n < N ? n : N - 1;
+            const float sw = ep.sw[nc], sa0 = ep.sa_per_row ? 1.0f : (ep.sa ? ep.sa[0] : ep.sa_scalar);
+            if (ep.bias) bias = ep.bias[nc];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const int m = row0 + 8 * wave + 4 * (lane / 32) + c, mc = m < M ? m : M - 1;
+                scale[c] = (ep.sa_per_row ? ep.sa[mc] : sa0) * sw;
+                residual[c] = ep.residual ? ep.residual[size_t(mc) * N + nc] : 0.0f;
+            }
+        }
+    }
+    v16i acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0;
+    const int steps = (KB + WK - 1) / WK, rounds_end = (steps + D - 1) / D * D;
+    for (int s0 = D; s0 < rounds_end; s0 += D) {
+#pragma unroll
+        for (int u = 0; u < D; ++u) {
+            acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[u], fw[u], acc, 0, 0, 0);
+            issue(s0 + u, u);
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < D; ++u) acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[u], fw[u], acc, 0, 0, 0);
+#pragma unroll
+    for (int g = 0; g < 4; ++g) part[wave][g][lane] = v4i{acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]};
+    __syncthreads();
+    if (wave >= 4) return;
+    v4i sum = part[0][wave][lane];
+#pragma unroll
+    for (int w = 1; w < WK; ++w) sum += part[w][wave][lane];
+    if (n >= N) return;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        const int m = row0 + 8 * wave + 4 * (lane / 32) + c;
+        if (m >= M) continue;
+        const size_t at = size_t(m) * N + n;
+        if constexpr (EPI == EPI_I32) {
+            static_cast<int32_t *>(ep.out)[at] = sum[c];
+        } else {
+            float v = static_cast<float>(sum[c]) * scale[c];
+            if (ep.bias) v = v + bias;
+            if (ep.residual) v = v + residual[c];
+            static_cast<float *>(ep.out)[at] = v;
+        }
+    }
+}
+
+// Whether a product is one of few blocks.  The split form against the weight-streaming and tiled ones that take over
+// beyond these lines, us (other / split), weights from beyond the L2:
+//   up to 32 rows: N = K = 768 M = 1 2.95 / 2.43, 32 3.50 / 2.68; N = 768, K = 3072 4.3-5.2 / 4.1-4.4; N = K = 4096 M = 8
+//     5.4 / 4.9, 32 6.3 / 5.3; N = 4096, K = 11008 M = 16 10.3 / 10.0, 32 11.6 / 11.0, but M = 1 9.63 / 9.80; N = 320,
+//     K = 1984 M = 16 3.72 / 3.86; N = 9000, K = 4096 M = 24 9.6 / 10.1 (288 blocks: the weights' stream is the time)
+//   more rows, up to one block per compute unit: 77 x 768 x 768 5.2 / 2.7, 77 x 768 x 3072 7.6 / 4.4, 300 x 64 x 12480
+//     18.9 / 10.2, 64 x 4096 x 4096 7.4 / 5.5, 500 x 500 x 8000 14.4 / 7.9
+//   up to four with K <= 1024: 1000 x 1000 x 256 5.8 / 4.4, 300 x 3072 x 768 5.9 / 5.1, 1000 x 1000 x 1000 6.0 / 5.5; up to
+//     64 rows 33 x 8000 x 512 4.0 / 3.9 but 64 x 8000 x 1024 4.7 / 4.9; 512 x 3072 x 768 (1536 blocks) 6.2 / 6.6
+//   past them: 64 x 5000 x 2048 5.5 / 7.7, 400 x 1200 x 2048 7.4 / 7.5, 4239 x 64 x 12480 20.3 / 24.9
+static bool few_blocks(const hipq_ctx *ctx, int M, int N, int K) {
+    const size_t cus = size_t(ctx->num_cus), KB = packed_k_blocks(size_t(K)), rbW = packed_row_blocks(size_t(N));
+    if (M <= 32) return rbW <= cus && (KB <= 32 || M > 16 || (rbW >= 16 && (M > 8 || KB <= 128)));
+    const size_t blocks = packed_row_blocks(size_t(M)) * rbW;
+    return blocks <= cus || (blocks <= 4 * cus && KB <= size_t(M <= 64 ? 16 : 32));
+}
+
+template <int EPI>
+static int32_t launch_split_packed(hipq_ctx *ctx, const int8_t *pa, const int8_t *pw, int M, int N, int K, const GemmEpilogue &ep) {
+    const int KB = static_cast<int>(packed_k_blocks(size_t(K)));
+    const dim3 grid((N + 31) / 32, (M + 31) / 32);
+    if (KB <= 16)
+        hipLaunchKernelGGL((split_i8_packed_kernel<4, 4, EPI>), grid, dim3(256), 0, ctx->stream, pa, pw, M, N, K, ep);
+    else if (KB <= 32)
+        hipLaunchKernelGGL((split_i8_packed_kernel<8, 4, EPI>), grid, dim3(512), 0, ctx->stream, pa, pw, M, N, K, ep);
+    else
+        hipLaunchKernelGGL((split_i8_packed_kernel<16, 8, EPI>), grid, dim3(1024), 0, ctx->stream, pa, pw, M, N, K, ep);
+    return check_launch("gemm_i8 (packed, split)");
+}
+
 // Row-major int8 [rows, k] -> packed.  One wave per fragment: a lane copies the 16 bytes of its
 // (row, half k block); rows and k past the matrix become zero.
 __global__ __launch_bounds__(256) void pack_rows_i8_kernel(const int8_t *__restrict__ src, size_t rows, size_t k,
@@ -821,6 +931,11 @@ static int32_t launch_gemm_packed(hipq_ctx *ctx, const int8_t *pa, const int8_t 
                                   const GemmEpilogue &ep) {
     const int M = static_cast<int>(m), N = static_cast<int>(n), K = static_cast<int>(k);
     const int steps = static_cast<int>(packed_k_blocks(k)) / 4;
+    if constexpr (EPI != EPI_I8) {
+        const bool forced = ctx->gemm_variant == 7 || ctx->gemm_variant == 8 || ctx->gemm_variant == 9 ||
+                            ctx->gemm_variant == 12 || ctx->trace;
+        if (!forced && few_blocks(ctx, M, N, K)) return launch_split_packed<EPI>(ctx, pa, pw, M, N, K, ep);
+    }
     if (M <= 32) {  // one row block of activations
         if ((N + 31) / 32 >= kTwoBlockRowBlocks && ctx->gemm_variant != 9)
             return launch_skinny_packed<EPI, EVEN>(ctx, pa, pw, M, N, K, ep);
