@@ -659,12 +659,17 @@ HIPQ_API int32_t hipq_transformer_stack_forward_f32(hipq_ctx *ctx, const hipq_bl
                                                     size_t tokens, size_t d_model, size_t d_ff, float eps,
                                                     int32_t mode, float *x, void *workspace, size_t workspace_bytes);
 /* The same forward on PREPARED weights: every w_* of `blocks` points to the packed form of the [out, in] matrix
- * (hipq_pack_rows_i8, once, when the model is converted).  Four kernels per layer: each Linear that feeds a row
- * operation applies it in its epilogue (hipq_linear_residual_layer_norm_quantize_packed_i8,
- * hipq_linear_gelu_quantize_packed_i8), the out-projection quantizes the fp32 value slice itself
- * (hipq_linear_from_f32_residual_layer_norm_quantize_packed_i8), and int8 activations stay packed between them.  x is what
- * hipq_transformer_stack_forward_f32 computes up to the fold order of the LayerNorm sums (see those entry
- * points).  d_model and d_ff: multiples of 128, at most 3072 (else HIPQ_SHAPE_ERROR: use the form above). */
+ * (hipq_pack_rows_i8, once, when the model is converted).  Beyond 5120 tokens (20 per compute unit) four kernels per
+ * layer: each Linear that feeds a row operation applies it in its epilogue
+ * (hipq_linear_residual_layer_norm_quantize_packed_i8, hipq_linear_gelu_quantize_packed_i8), the out-projection
+ * quantizes the fp32 value slice itself (hipq_linear_from_f32_residual_layer_norm_quantize_packed_i8), and int8
+ * activations stay packed between them.  Up to there the products are split over their columns and the row operations
+ * are kernels of their own (eight kernels per layer), with the same bits.  x is what hipq_transformer_stack_forward_f32
+ * computes up to the fold order of the LayerNorm sums (see those entry points).  d_model and d_ff: multiples of 128, at
+ * most 3072 (else HIPQ_SHAPE_ERROR: use the form above).  The forward uses no memory but the workspace (and, where panels
+ * of rows are shared by two workgroups, their exchange area).  A workspace that holds the packed activations, the scales
+ * and the qkv product but not, for up to 5120 tokens and d_ff > 3 d_model, fc1's fp32 output in its place is taken too:
+ * the four kernels per layer then run at any number of tokens. */
 HIPQ_API size_t hipq_transformer_stack_prepared_workspace_bytes(size_t tokens, size_t d_model, size_t d_ff);
 HIPQ_API int32_t hipq_transformer_stack_forward_prepared_f32(hipq_ctx *ctx, const hipq_block_weights *blocks,
                                                              size_t n_layers, size_t tokens, size_t d_model,

@@ -490,42 +490,138 @@ def test_prepared_stack_small_against_the_oracle(ctx, oracle, tokens, d, dff, la
     assert rel_plain < 2e-3
 
 
-@pytest.mark.parametrize("tokens,d,dff,layers", [(1, 768, 3072, 2), (2, 128, 384, 3), (31, 256, 256, 2), (33, 768, 3072, 2), (77, 1152, 2304, 2),
-                                                 (300, 1664, 1792, 1)])
+def _random_blocks(c, g, d, dff, layers, offset=0):
+    """Blocks with row-major weights; the LayerNorm vectors start `offset` floats into their storage."""
+    blocks = []
+    for _ in range(layers):
+        blk = {}
+        for name, (o, i) in {"qkv": (3 * d, d), "out": (d, d), "fc1": (dff, d), "fc2": (d, dff)}.items():
+            q, sc, _, _ = c.quantize_per_row(torch.randn(o, i, generator=g, device="cuda") * 0.02)
+            blk["w_" + name], blk["s_" + name] = q, sc
+            blk["b_" + name] = torch.randn(o, generator=g, device="cuda") * 0.01
+        for ln in ("ln1", "ln2"):
+            blk[ln + "_gamma"] = (torch.rand(d + offset, generator=g, device="cuda") + 0.5)[offset:]
+            blk[ln + "_beta"] = (torch.randn(d + offset, generator=g, device="cuda") * 0.1)[offset:]
+        blocks.append(blk)
+    return blocks
+
+
+def _stack_of_its_parts(c, prepared, x, d, dff, mode=0):
+    """The prepared stack composed from the row-panel entry points, x in place."""
+    tokens, last = x.shape[0], len(prepared) - 1
+    q, s = c.layer_norm_quantize(x, prepared[0]["ln1_gamma"], prepared[0]["ln1_beta"], 1e-5, mode)
+    qa = c.pack_rows(q)
+    for i, blk in enumerate(prepared):
+        qkv = c.linear_packed_i8_f32(qa, s, blk["w_qkv"], blk["s_qkv"], blk["b_qkv"], tokens, 3 * d, d)
+        ln2 = dict(gamma=blk["ln2_gamma"], beta=blk["ln2_beta"], mode=mode)
+        if d <= 1536:
+            qa, s = c.linear_from_f32_residual_layer_norm_quantize_packed(qkv[:, 2 * d:], blk["w_out"], blk["s_out"],
+                                                                          blk["b_out"], d, x, **ln2)
+        else:
+            q, s = c.quantize_per_row_strided(qkv, tokens, d, 3 * d, elem_offset=2 * d, mode=mode)
+            qa, s = c.linear_residual_layer_norm_quantize_packed(c.pack_rows(q), s, blk["w_out"], blk["s_out"], blk["b_out"],
+                                                                 tokens, d, d, x, **ln2)
+        qb, sb = c.linear_gelu_quantize_packed(qa, s, blk["w_fc1"], blk["s_fc1"], blk["b_fc1"], tokens, dff, d, mode=mode)
+        nxt = {} if i == last else dict(gamma=prepared[i + 1]["ln1_gamma"], beta=prepared[i + 1]["ln1_beta"])
+        qa, s = c.linear_residual_layer_norm_quantize_packed(qb, sb, blk["w_fc2"], blk["s_fc2"], blk["b_fc2"], tokens, d, dff,
+                                                             x, normalize=i != last, mode=mode, **nxt)
+    return x
+
+
+# One and two column blocks per panel wave, panel waves without columns; d >= 1536 with enough rows: shared panels.
+@pytest.mark.parametrize("tokens,d,dff,layers", [(1, 768, 3072, 2), (2, 128, 384, 3), (31, 256, 256, 2), (33, 768, 3072, 2),
+                                                 (77, 1152, 2304, 2), (300, 1664, 1792, 1), (45, 896, 512, 3),
+                                                 (40, 1536, 1792, 2), (70, 2048, 1024, 2), (20, 2432, 1280, 2),
+                                                 (33, 3072, 768, 2)])
 def test_prepared_stack_few_tokens(hipq, tokens, d, dff, layers):
-    """Few tokens run as products split over their columns; test hook 15 runs the row panels.  Both within the drift of
-    the LayerNorm sums (their order differs) of the stack on row-major weights, for both roundings."""
+    """Few tokens run as products split over their columns with the row operations in kernels of their own: the bits of the
+    row panels (composed from their entry points; the one call under test hook 15, where that has the same panels; a
+    workspace without room for the split form), for both roundings, and within the drift of the LayerNorm sums (their order
+    differs) of the stack on row-major weights."""
     c = hipq.Context(0)
     try:
         g = torch.Generator(device="cuda").manual_seed(tokens + d)
-        blocks = []
-        for _ in range(layers):
-            blk = {}
-            for name, (o, i) in {"qkv": (3 * d, d), "out": (d, d), "fc1": (dff, d), "fc2": (d, dff)}.items():
-                q, sc, _, _ = c.quantize_per_row(torch.randn(o, i, generator=g, device="cuda") * 0.02)
-                blk["w_" + name], blk["s_" + name] = q, sc
-                blk["b_" + name] = torch.randn(o, generator=g, device="cuda") * 0.01
-            for ln in ("ln1", "ln2"):
-                blk[ln + "_gamma"] = torch.rand(d, generator=g, device="cuda") + 0.5
-                blk[ln + "_beta"] = torch.randn(d, generator=g, device="cuda") * 0.1
-            blocks.append(blk)
+        blocks = _random_blocks(c, g, d, dff, layers)
         prepared = c.stack_prepare(blocks)
         x0 = torch.randn(tokens, d, generator=g, device="cuda")
+        ws = c.stack_workspace_prepared(tokens, d, dff)
         for mode in (0, hipq.ROUND_HALF_EVEN):
-            run = lambda: c.stack_forward(prepared, x0.clone(), dff, c.stack_workspace_prepared(tokens, d, dff), mode=mode,
-                                          prepared=True)
-            got = run()
-            c.set_gemm_kernel_variant(15)
-            panels = run()
-            c.set_gemm_kernel_variant(0)
+            run = lambda w: c.stack_forward(prepared, x0.clone(), dff, w, mode=mode, prepared=True)
+            got = run(ws)
+            assert torch.isfinite(got).all()
+            assert torch.equal(got, _stack_of_its_parts(c, prepared, x0.clone(), d, dff, mode)), mode
+            if dff > 3 * d:  # room for the qkv product only
+                up = lambda v: (v + 255) // 256 * 256
+                small = 4 * tokens * (dff - 3 * d) // 256 * 256
+                least = ws[:up(c.packed_size(tokens, d)) + up(c.packed_size(tokens, dff)) + 2 * up(4 * tokens) +
+                           up(12 * tokens * d)]
+                assert least.numel() <= ws.numel() - small
+                assert torch.equal(got, run(least)), mode
+                with pytest.raises(hipq.HipqError) as e:
+                    run(least[:-1])
+                assert e.value.code == hipq.INVALID_ARGUMENT
+            if d < 1536:
+                c.set_gemm_kernel_variant(15)
+                assert torch.equal(got, run(ws)), mode
+                c.set_gemm_kernel_variant(0)
             plain = c.stack_forward(blocks, x0.clone(), dff, c.stack_workspace(tokens, d, dff), mode=mode)
             torch.cuda.synchronize()
-            assert torch.isfinite(got).all()
-            for other in (panels, plain):
-                assert float((got - other).norm() / plain.norm()) < 2e-3
+            assert float((got - plain).norm() / plain.norm()) < 2e-3
     finally:
         torch.cuda.synchronize()
         c.close()
+
+
+def test_prepared_stack_few_tokens_layer_norm_vectors_at_any_float(hipq):
+    """Gain and offset of every LayerNorm behind a Linear are taken at the alignment of a float, as the row panels take
+    them (the first layer's ln1 is the row kernel's: 16 bytes)."""
+    c = hipq.Context(0)
+    try:
+        tokens, d, dff = 33, 384, 1280
+        g = torch.Generator(device="cuda").manual_seed(5)
+        blocks = _random_blocks(c, g, d, dff, 2, offset=1)
+        for name in ("ln1_gamma", "ln1_beta"):
+            blocks[0][name] = blocks[0][name].clone()
+        assert blocks[1]["ln1_gamma"].data_ptr() % 16 == 4
+        x0 = torch.randn(tokens, d, generator=g, device="cuda")
+        got = [c.stack_forward(c.stack_prepare(b), x0.clone(), dff, c.stack_workspace_prepared(tokens, d, dff), prepared=True)
+               for b in (blocks, [{k: v.clone() for k, v in blk.items()} for blk in blocks])]
+        torch.cuda.synchronize()
+        assert torch.equal(got[0], got[1])
+    finally:
+        torch.cuda.synchronize()
+        c.close()
+
+
+def test_prepared_stack_first_call_in_a_graph(hipq):
+    """The stack needs no memory of the context: its first call may be captured, and every replay gives the eager call's
+    bits."""
+    tokens, d, dff = 77, 256, 1024
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        maker, c = hipq.Context(0), hipq.Context(0)
+        try:
+            g = torch.Generator(device="cuda").manual_seed(9)
+            prepared = maker.stack_prepare(_random_blocks(maker, g, d, dff, 2))
+            ws, x = maker.stack_workspace_prepared(tokens, d, dff), torch.zeros(tokens, d, device="cuda")
+            side.synchronize()
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph, stream=side):
+                c.stack_forward(prepared, x, dff, ws, prepared=True)
+            for rep in range(4):
+                x0 = torch.randn(tokens, d, generator=g, device="cuda")
+                x.copy_(x0)
+                side.synchronize()
+                graph.replay()
+                torch.cuda.synchronize()
+                eager = maker.stack_forward(prepared, x0, dff, maker.stack_workspace_prepared(tokens, d, dff), prepared=True)
+                side.synchronize()
+                assert torch.equal(x, eager), rep
+            c.synchronize()
+        finally:
+            torch.cuda.synchronize()
+            c.close()
+            maker.close()
 
 
 def test_prepared_stack_full_size_equals_its_parts(ctx, hipq):

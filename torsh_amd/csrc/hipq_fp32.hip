@@ -348,14 +348,126 @@ static int32_t launch_row_op(const char *fn, hipq_ctx *ctx, const float *x, size
     return check_launch(fn);
 }
 
-int32_t layer_norm_quantize_packed(hipq_ctx *ctx, float *x, const float *delta, size_t rows, size_t cols, const float *gamma,
+// Four floats at an address that is a multiple of four bytes only.
+struct __attribute__((packed, aligned(4))) AnyFloat4 {
+    float x, y, z, w;
+};
+
+// LayerNorm + per-token int8 of whole rows with the bits of the row-panel GEMM's epilogue (hipq_gemm_rows.h): its sums run
+// over a lane's column blocks first, then over the 32 columns of a block (neighbours first), then over the eight waves in
+// pairs, and in the pair form over the two halves of the columns last.  Eight lanes stand for a panel wave here, four
+// neighbouring columns each, so the panel's fold is this wave's butterfly in ascending order and a load is 16 bytes a lane.
+// One wave per row, RC float4 a lane; PAIR: the first RC / 2 of them belong to the first half of the columns.
+template <int RC, bool PAIR, bool EVEN>
+__global__ __launch_bounds__(kRowBlock) void panel_layer_norm_kernel(const float *__restrict__ x, size_t rows, int nblocks,
+                                                                      const float *__restrict__ gamma,
+                                                                      const float *__restrict__ beta, float eps,
+                                                                      int8_t *__restrict__ out_q,
+                                                                      float *__restrict__ out_scales) {
+    constexpr int H = PAIR ? 2 : 1, PER = RC / H;
+    const size_t row = size_t(blockIdx.x) * (kRowBlock / kWave) + threadIdx.x / kWave;
+    if (row >= rows) return;
+    const int lane = threadIdx.x % kWave, wave = lane / 8, part = lane % 8;  // panel wave, columns 4 part .. of its blocks
+    const int cols = nblocks * 32, half_blocks = nblocks / H;
+    int block[RC];
+    bool real[RC];
+#pragma unroll
+    for (int i = 0; i < RC; ++i) {
+        const int b = PAIR ? wave + 8 * (i % PER) : wave * RC + i;
+        real[i] = b < half_blocks;
+        block[i] = b + (i / PER) * half_blocks;
+    }
+    const float *xr = x + row * cols;
+    float4 v[RC], g[RC], b[RC];
+#pragma unroll
+    for (int i = 0; i < RC; ++i) v[i] = real[i] ? *reinterpret_cast<const float4 *>(xr + block[i] * 32 + part * 4) : float4{};
+    auto affine = [&](const float *p, int i, float missing) {
+        if (!p || !real[i]) return make_float4(missing, missing, missing, missing);
+        const AnyFloat4 t = *reinterpret_cast<const AnyFloat4 *>(p + block[i] * 32 + part * 4);
+        return make_float4(t.x, t.y, t.z, t.w);
+    };
+#pragma unroll
+    for (int i = 0; i < RC; ++i) {  // (y * 1.0f and y + -0.0f are y, bit for bit)
+        g[i] = affine(gamma, i, 1.0f);
+        b[i] = affine(beta, i, -0.0f);
+    }
+    auto total = [&](auto term) {
+        float half[H];
+#pragma unroll
+        for (int h = 0; h < H; ++h) {
+            float4 s = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll
+            for (int i = h * PER; i < (h + 1) * PER; ++i)
+                if (real[i]) {
+                    const float4 t = term(v[i]);
+                    s = make_float4(s.x + t.x, s.y + t.y, s.z + t.z, s.w + t.w);
+                }
+            half[h] = wave_sum_ascending((s.x + s.y) + (s.z + s.w));
+        }
+        return PAIR ? half[0] + half[H - 1] : half[0];
+    };
+    const float cols_f = static_cast<float>(cols);
+    const float mean = total([](const float4 &t) { return t; }) / cols_f;
+    const float var = total([&](const float4 &t) {
+        const float p = t.x - mean, q = t.y - mean, r = t.z - mean, s = t.w - mean;
+        return make_float4(p * p, q * q, r * r, s * s);
+    }) / cols_f;
+    const float rstd = 1.0f / sqrtf(var + eps);
+    float am = 0.0f;
+#pragma unroll
+    for (int i = 0; i < RC; ++i) {
+        if (!real[i]) continue;
+        v[i] = make_float4((v[i].x - mean) * rstd * g[i].x + b[i].x, (v[i].y - mean) * rstd * g[i].y + b[i].y,
+                           (v[i].z - mean) * rstd * g[i].z + b[i].z, (v[i].w - mean) * rstd * g[i].w + b[i].w);
+        am = fmaxf(fmaxf(am, fmaxf(fabsf(v[i].x), fabsf(v[i].y))), fmaxf(fabsf(v[i].z), fabsf(v[i].w)));
+    }
+    am = wave_max(am);
+    float scale = am < FLT_EPSILON ? 1.0f : am / 127.0f;
+    if (!(fabsf(am) <= FLT_MAX)) scale = NAN;
+    if (lane == 0) out_scales[row] = scale;
+    const float inv = recip_for_div(scale);
+    uint32_t *q4 = reinterpret_cast<uint32_t *>(out_q + (row / 32) * cols * 32 + (row % 32) * 16) + (part / 4) * 128 + part % 4;
+#pragma unroll
+    for (int i = 0; i < RC; ++i)
+        if (real[i])
+            q4[block[i] * 256] = pack4(quantize_int_sym<EVEN>(v[i].x, scale, inv), quantize_int_sym<EVEN>(v[i].y, scale, inv),
+                                       quantize_int_sym<EVEN>(v[i].z, scale, inv), quantize_int_sym<EVEN>(v[i].w, scale, inv));
+}
+
+int32_t layer_norm_quantize_packed(hipq_ctx *ctx, const float *x, size_t rows, size_t cols, const float *gamma,
                                    const float *beta, float eps, int32_t mode, int8_t *out_packed, float *out_scales) {
-    const char *fn = "layer_norm_quantize (packed)";
-    if (delta)
-        return launch_row_op<ROW_LAYERNORM, true, true>(fn, ctx, x, rows, cols, gamma, beta, eps, mode, nullptr, out_packed,
-                                                        out_scales, delta, x, true);
-    return launch_row_op<ROW_LAYERNORM, true>(fn, ctx, x, rows, cols, gamma, beta, eps, mode, nullptr, out_packed, out_scales,
-                                              nullptr, nullptr, true);
+    return launch_row_op<ROW_LAYERNORM, true>("layer_norm_quantize (packed)", ctx, x, rows, cols, gamma, beta, eps, mode, nullptr,
+                                              out_packed, out_scales, nullptr, nullptr, true);
+}
+
+int32_t panel_layer_norm_quantize_packed(hipq_ctx *ctx, const float *x, size_t rows, size_t cols, const float *gamma,
+                                         const float *beta, float eps, int32_t mode, PanelFold fold, int8_t *out_packed,
+                                         float *out_scales) {
+    const char *fn = "layer_norm_quantize (panel order)";
+    const int nblocks = static_cast<int>(cols / 32), wave_blocks = fold.pair ? (nblocks / 2 + 7) / 8 * 2 : fold.wave_blocks;
+    if (cols % 128 != 0 || wave_blocks > 12 || (!fold.pair && wave_blocks * 8 < nblocks) || (reinterpret_cast<uintptr_t>(x) & 15u))
+        return fail(HIPQ_SHAPE_ERROR, "%s: rows of %zu floats", fn, cols);
+    const dim3 grid(static_cast<unsigned>((rows + kRowBlock / kWave - 1) / (kRowBlock / kWave)));
+#define HIPQ_PANEL_LN_E(RC, PAIR, E)                                                                                       \
+    hipLaunchKernelGGL((panel_layer_norm_kernel<RC, PAIR, E>), grid, dim3(kRowBlock), 0, ctx->stream, x, rows, nblocks, gamma, \
+                       beta, eps, out_packed, out_scales)
+#define HIPQ_PANEL_LN(RC, PAIR)              \
+    do {                                     \
+        if (mode & HIPQ_ROUND_HALF_EVEN)     \
+            HIPQ_PANEL_LN_E(RC, PAIR, true); \
+        else                                 \
+            HIPQ_PANEL_LN_E(RC, PAIR, false);\
+    } while (0)
+    if (fold.pair && wave_blocks <= 6) HIPQ_PANEL_LN(6, true);
+    else if (fold.pair) HIPQ_PANEL_LN(12, true);
+    else if (wave_blocks == 3) HIPQ_PANEL_LN(3, false);
+    else if (wave_blocks == 6) HIPQ_PANEL_LN(6, false);
+    else if (wave_blocks == 9) HIPQ_PANEL_LN(9, false);
+    else if (wave_blocks == 12) HIPQ_PANEL_LN(12, false);
+    else return fail(HIPQ_SHAPE_ERROR, "%s: no form of %d column blocks per wave", fn, wave_blocks);
+#undef HIPQ_PANEL_LN
+#undef HIPQ_PANEL_LN_E
+    return check_launch(fn);
 }
 
 int32_t gelu_quantize_packed(hipq_ctx *ctx, const float *x, size_t rows, size_t cols, int32_t mode, int8_t *out_packed,

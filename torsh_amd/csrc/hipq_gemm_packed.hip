@@ -70,6 +70,12 @@ bool pairs_share_an_xcd(hipq_ctx *ctx) {
     return known[ctx->device] > 0;
 }
 
+PanelFold panel_fold(const hipq_ctx *ctx, bool from_f32, size_t m, size_t n, size_t k) {
+    const int N = static_cast<int>(n);
+    return PanelFold{rows_wave_blocks(N),
+                     !from_f32 && rows_pair_applies<RP_RESID_LN_Q>(ctx, static_cast<int>(m), N, static_cast<int>(k))};
+}
+
 int32_t linear_packed_rows_f32(hipq_ctx *ctx, const int8_t *a_packed, const float *a_scales, const int8_t *w_packed,
                                const float *w_scales, const float *bias, const float *residual, size_t m, size_t n, size_t k,
                                float *out) {

@@ -858,16 +858,24 @@ __global__ __launch_bounds__(kRowsThreads) void gemm_i8_rows_pair_kernel(RowPane
 // costs ~9 us, more than the halved weight stream saves (~5 us at K = 3072).
 // Test hook 15 keeps the single-workgroup panels, 16 takes pairs wherever the shape allows them.  Returns false
 // when the caller should launch the single panels.
+static inline int rows_pair_grid(int M) { return ((M + 63) / 64 + 7) / 8 * 16; }
+template <int EPI>
+static bool rows_pair_applies(const hipq_ctx *ctx, int M, int N, int K) {
+    const int share = ctx->resident_share > 0 ? ctx->resident_share : 1;
+    if (!ctx->pair_ok || ctx->gemm_variant == 15 || N % 64 != 0 || M <= 32 || rows_pair_grid(M) > ctx->num_cus / share)
+        return false;
+    if (ctx->gemm_variant != 16) {
+        if ((EPI == RP_GELU_Q || EPI == RP_RESID_LN_Q) && N < 1536) return false;
+        if (EPI == RP_RESID_F32 && N > 1536) return false;
+        if (EPI == RP_RESID_LN_Q && size_t(N) * K < (size_t(2) << 20)) return false;
+    }
+    return true;
+}
+
 template <int EPI>
 static bool launch_rows_pair(hipq_ctx *ctx, const RowPanel &p, bool even, int32_t *rc) {
-    const int share = ctx->resident_share > 0 ? ctx->resident_share : 1;
-    const int pairs = (p.M + 63) / 64, grid = (pairs + 7) / 8 * 16;
-    if (!ctx->pair_ok || ctx->gemm_variant == 15 || p.N % 64 != 0 || p.M <= 32 || grid > ctx->num_cus / share) return false;
-    if (ctx->gemm_variant != 16) {
-        if ((EPI == RP_GELU_Q || EPI == RP_RESID_LN_Q) && p.N < 1536) return false;
-        if (EPI == RP_RESID_F32 && p.N > 1536) return false;
-        if (EPI == RP_RESID_LN_Q && size_t(p.N) * p.K < (size_t(2) << 20)) return false;
-    }
+    if (!rows_pair_applies<EPI>(ctx, p.M, p.N, p.K)) return false;
+    const int grid = rows_pair_grid(p.M);
     RowPairExchange px;
     int8_t *buf = nullptr;
     *rc = pair_area(ctx, size_t(grid) * 4 * sizeof(uint32_t), size_t(grid) * 3 * 64 * sizeof(float), &px.flags, &buf);
@@ -905,6 +913,9 @@ static bool launch_rows_pair(hipq_ctx *ctx, const RowPanel &p, bool even, int32_
     return true;
 }
 
+// Column blocks per wave of the single-panel instantiation that takes N columns.
+static inline int rows_wave_blocks(int N) { return ((N / 32 + kRowsWaves - 1) / kRowsWaves + 2) / 3 * 3; }
+
 // Launch of the row-panel kernel that quantizes its own fp32 activations (gemm_i8_rows_kernel<.., AF32>): single
 // panels, the whole panel of codes resident in LDS.
 template <int EPI>
@@ -919,7 +930,7 @@ static int32_t launch_rows_from_f32(hipq_ctx *ctx, const RowPanel &p, bool even)
                     "row-panel GEMM from fp32 rows: K = %d (at most 1536) and the row pitch %d must be multiples of 4, "
                     "the rows 16-byte aligned", p.K, p.lda);
     const dim3 grid((p.M + 31) / 32);
-    const int nbw = (p.N / 32 + kRowsWaves - 1) / kRowsWaves;
+    const int nbw = rows_wave_blocks(p.N);
 #define HIPQ_LAUNCH_ROWS_F32(NBW)                                                                                         \
     do {                                                                                                                  \
         if (even)                                                                                                         \
@@ -928,7 +939,7 @@ static int32_t launch_rows_from_f32(hipq_ctx *ctx, const RowPanel &p, bool even)
             hipLaunchKernelGGL((gemm_i8_rows_kernel<NBW, EPI, false, true>), grid, dim3(kRowsThreads), 0, ctx->stream,    \
                                p);                                                                                        \
     } while (0)
-    if (nbw <= 3)
+    if (nbw == 3)
         HIPQ_LAUNCH_ROWS_F32(3);
     else
         HIPQ_LAUNCH_ROWS_F32(6);
@@ -953,7 +964,7 @@ static int32_t launch_rows(hipq_ctx *ctx, const RowPanel &p, bool even) {
         if (launch_rows_pair<EPI>(ctx, p, even, &rc)) return rc;
     }
     const dim3 grid((p.M + 31) / 32);
-    const int nbw = (p.N / 32 + kRowsWaves - 1) / kRowsWaves;
+    const int nbw = rows_wave_blocks(p.N);
 #define HIPQ_LAUNCH_ROWS_NBW(NBW)                                                                                     \
     do {                                                                                                              \
         if (even)                                                                                                     \
@@ -961,11 +972,11 @@ static int32_t launch_rows(hipq_ctx *ctx, const RowPanel &p, bool even) {
         else                                                                                                          \
             hipLaunchKernelGGL((gemm_i8_rows_kernel<NBW, EPI, false>), grid, dim3(kRowsThreads), 0, ctx->stream, p); \
     } while (0)
-    if (nbw <= 3)
+    if (nbw == 3)
         HIPQ_LAUNCH_ROWS_NBW(3);
-    else if (nbw <= 6)
+    else if (nbw == 6)
         HIPQ_LAUNCH_ROWS_NBW(6);
-    else if (nbw <= 9)
+    else if (nbw == 9)
         HIPQ_LAUNCH_ROWS_NBW(9);
     else
         HIPQ_LAUNCH_ROWS_NBW(12);

@@ -119,10 +119,22 @@ int32_t quantize_activations_per_row(hipq_ctx *ctx, const float *x, size_t rows,
 // The same for rows that lie `ld` floats apart (a column slice of a wider matrix).
 int32_t quantize_activations_per_row_strided(hipq_ctx *ctx, const float *x, size_t rows, size_t cols, size_t ld,
                                              int32_t mode, int8_t *out, float *out_scales, bool packed);
+// How the row-panel GEMM that ends in LayerNorm folds a row's sums (hipq_gemm_rows.h): eight waves of `wave_blocks`
+// neighbouring column blocks of 32 each, or (pair) the two halves of the columns with the blocks of a half dealt round
+// eight waves.  panel_fold: the form that Linear + skip + LayerNorm on m rows takes, K = k, from packed codes or fp32 rows.
+struct PanelFold {
+    int wave_blocks;
+    bool pair;
+};
+PanelFold panel_fold(const hipq_ctx *ctx, bool from_f32, size_t m, size_t n, size_t k);
 // The row operations of the transformer stack with their codes in the packed operand layout (cols a multiple of 128; the
-// rows that pad the last row block are not written: products of them are discarded).  delta: x += delta first.
-int32_t layer_norm_quantize_packed(hipq_ctx *ctx, float *x, const float *delta, size_t rows, size_t cols, const float *gamma,
+// rows that pad the last row block are not written: products of them are discarded).  LayerNorm: in the order of the row
+// kernels, or (panel, cols at most 3072, gamma and beta at any alignment of a float) in the row-panel GEMM's.
+int32_t layer_norm_quantize_packed(hipq_ctx *ctx, const float *x, size_t rows, size_t cols, const float *gamma,
                                    const float *beta, float eps, int32_t mode, int8_t *out_packed, float *out_scales);
+int32_t panel_layer_norm_quantize_packed(hipq_ctx *ctx, const float *x, size_t rows, size_t cols, const float *gamma,
+                                         const float *beta, float eps, int32_t mode, PanelFold fold, int8_t *out_packed,
+                                         float *out_scales);
 int32_t gelu_quantize_packed(hipq_ctx *ctx, const float *x, size_t rows, size_t cols, int32_t mode, int8_t *out_packed,
                              float *out_scales);
 // hipq_linear_packed_i8_f32 on per-row scales and activations that the kernel just before wrote; residual (may be null,

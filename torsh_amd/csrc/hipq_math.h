@@ -288,6 +288,23 @@ __device__ __forceinline__ float wave_butterfly(float v, Op op) {
     return op(v, lane_move<0xB1>(v));  // quad_perm [1, 0, 3, 2]
 }
 
+// The sum over the 64 lanes folded in the order lane ^ 1, 2, 4, 8, 16, 32 (the mirrors of 8 and 16 lanes stand for ^ 4 and
+// ^ 8: the lanes they combine agree inside the smaller groups by then).
+__device__ __forceinline__ float wave_sum_ascending(float v) {
+    v = v + lane_move<0xB1>(v);   // quad_perm [1, 0, 3, 2]
+    v = v + lane_move<0x4E>(v);   // quad_perm [2, 3, 0, 1]
+    v = v + lane_move<0x141>(v);  // row_half_mirror
+    v = v + lane_move<0x140>(v);  // row_mirror
+    uint32_t b = __builtin_bit_cast(uint32_t, v);
+    const auto rows = __builtin_amdgcn_permlane16_swap(b, b, false, false);
+    const uint32_t r0 = rows[0], r1 = rows[1];
+    v = __builtin_bit_cast(float, r0) + __builtin_bit_cast(float, r1);
+    b = __builtin_bit_cast(uint32_t, v);
+    const auto halves = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+    const uint32_t h0 = halves[0], h1 = halves[1];
+    return __builtin_bit_cast(float, h0) + __builtin_bit_cast(float, h1);
+}
+
 __device__ __forceinline__ float wave_min(float v) {
     return wave_butterfly(v, [](float a, float b) { return fminf(a, b); });
 }

@@ -17,29 +17,43 @@ struct StackBuffers {
     int8_t *qa, *qb;  // packed int8 activations
     float *sa, *sb;   // their per-token scales
     float *qkv;
+    float *hidden;  // fc1 output of the tiled form; lies where qkv does, which is used up by then
 };
 
+// Whether the value slice's quantizer runs inside the out-projection (row panels: a workgroup holds its rows' codes).
+bool out_from_f32(const hipq_ctx *ctx, size_t d_model) { return d_model <= 1536 && ctx->gemm_variant != 6; }
+
+// The most tokens that may run tiled, on a device of 256 compute units (see the rule in the forward).
+constexpr size_t kTiledTokens = 256 * 20;
+
 // Few tokens: every product split over its columns (the packed tiled kernels), the row operations between them in
-// kernels of their own that write packed codes.  hidden: [tokens, d_ff] fp32.
+// kernels of their own that write packed codes.  The LayerNorms behind a Linear fold their sums as the row panels do that
+// would otherwise run, so the results are theirs, bit for bit.
 int32_t stack_tiled(hipq_ctx *ctx, const hipq_block_weights *blocks, size_t n_layers, size_t tokens, size_t d_model,
-                    size_t d_ff, float eps, int32_t mode, float *x, const StackBuffers &b, float *hidden) {
+                    size_t d_ff, float eps, int32_t mode, float *x, const StackBuffers &b) {
     using namespace hipq;
-    for (size_t l = 0; l < n_layers; ++l) {
+    const PanelFold after_out = panel_fold(ctx, out_from_f32(ctx, d_model), tokens, d_model, d_model);
+    const PanelFold after_fc2 = panel_fold(ctx, false, tokens, d_model, d_ff);
+    int32_t rc = layer_norm_quantize_packed(ctx, x, tokens, d_model, blocks[0].ln1_gamma, blocks[0].ln1_beta, eps, mode, b.qa,
+                                            b.sa);
+    for (size_t l = 0; l < n_layers && rc == HIPQ_SUCCESS; ++l) {
         const hipq_block_weights &w = blocks[l];
-        int32_t rc;
-        if ((rc = layer_norm_quantize_packed(ctx, x, nullptr, tokens, d_model, w.ln1_gamma, w.ln1_beta, eps, mode, b.qa, b.sa)) ||
+        if ((l != 0 && (rc = panel_layer_norm_quantize_packed(ctx, x, tokens, d_model, w.ln1_gamma, w.ln1_beta, eps, mode,
+                                                              after_fc2, b.qa, b.sa))) ||
             (rc = linear_packed_rows_f32(ctx, b.qa, b.sa, w.w_qkv, w.s_qkv, w.b_qkv, nullptr, tokens, 3 * d_model, d_model,
                                          b.qkv)) ||
             (rc = quantize_activations_per_row_strided(ctx, b.qkv + 2 * d_model, tokens, d_model, 3 * d_model, mode, b.qb, b.sb,
                                                        /*packed=*/true)) ||
             (rc = linear_packed_rows_f32(ctx, b.qb, b.sb, w.w_out, w.s_out, w.b_out, x, tokens, d_model, d_model, x)) ||
-            (rc = layer_norm_quantize_packed(ctx, x, nullptr, tokens, d_model, w.ln2_gamma, w.ln2_beta, eps, mode, b.qa, b.sa)) ||
-            (rc = linear_packed_rows_f32(ctx, b.qa, b.sa, w.w_fc1, w.s_fc1, w.b_fc1, nullptr, tokens, d_ff, d_model, hidden)) ||
-            (rc = gelu_quantize_packed(ctx, hidden, tokens, d_ff, mode, b.qb, b.sb)) ||
+            (rc = panel_layer_norm_quantize_packed(ctx, x, tokens, d_model, w.ln2_gamma, w.ln2_beta, eps, mode, after_out, b.qa,
+                                                   b.sa)) ||
+            (rc = linear_packed_rows_f32(ctx, b.qa, b.sa, w.w_fc1, w.s_fc1, w.b_fc1, nullptr, tokens, d_ff, d_model,
+                                         b.hidden)) ||
+            (rc = gelu_quantize_packed(ctx, b.hidden, tokens, d_ff, mode, b.qb, b.sb)) ||
             (rc = linear_packed_rows_f32(ctx, b.qb, b.sb, w.w_fc2, w.s_fc2, w.b_fc2, x, tokens, d_model, d_ff, x)))
             return rc;
     }
-    return HIPQ_SUCCESS;
+    return rc;
 }
 }  // namespace
 
@@ -126,9 +140,11 @@ size_t hipq_transformer_stack_prepared_workspace_bytes(size_t tokens, size_t d_m
     const size_t widest = d_model > d_ff ? d_model : d_ff;
     size_t a = 0, b = 0;
     if (hipq_packed_size(tokens, d_model, &a) || hipq_packed_size(tokens, widest, &b)) return 0;
-    return align256(a) + align256(b)                          // packed int8 activations (two in flight)
-           + 2 * align256(tokens * sizeof(float))             // their per-token scales
-           + align256(tokens * 3 * d_model * sizeof(float));  // qkv
+    // qkv; few tokens: or fc1's output, when that is the wider
+    const size_t row = tokens <= kTiledTokens && d_ff > 3 * d_model ? d_ff : 3 * d_model;
+    return align256(a) + align256(b)                // packed int8 activations (two in flight)
+           + 2 * align256(tokens * sizeof(float))   // their per-token scales
+           + align256(tokens * row * sizeof(float));
 }
 
 int32_t hipq_transformer_stack_forward_prepared_f32(hipq_ctx *ctx, const hipq_block_weights *blocks, size_t n_layers,
@@ -145,17 +161,18 @@ int32_t hipq_transformer_stack_forward_prepared_f32(hipq_ctx *ctx, const hipq_bl
                           "%s: d_model = %zu and d_ff = %zu must be multiples of 128 and at most 3072 (a workgroup "
                           "holds whole rows of each Linear's output); use hipq_transformer_stack_forward_f32",
                           __func__, d_model, d_ff);
-    const size_t need = hipq_transformer_stack_prepared_workspace_bytes(tokens, d_model, d_ff);
-    if (need == 0) return hipq::fail(HIPQ_SHAPE_ERROR, "%s: dimension too large", __func__);
+    const size_t widest = d_model > d_ff ? d_model : d_ff;
+    size_t bytes_a = 0, bytes_b = 0;
+    if (hipq_packed_size(tokens, d_model, &bytes_a) || hipq_packed_size(tokens, widest, &bytes_b))
+        return hipq::fail(HIPQ_SHAPE_ERROR, "%s: dimension too large", __func__);
+    // (what the row panels need; the size that is asked for may have room for the tiled form's fc1 output as well)
+    const size_t ahead = align256(bytes_a) + align256(bytes_b) + 2 * align256(tokens * sizeof(float));
+    const size_t need = ahead + align256(tokens * 3 * d_model * sizeof(float));
     if (workspace_bytes < need)
         return hipq::fail(HIPQ_INVALID_ARGUMENT, "%s: workspace of %zu bytes is smaller than the %zu needed", __func__,
                           workspace_bytes, need);
     if (reinterpret_cast<uintptr_t>(workspace) & 255u)
         return hipq::fail(HIPQ_INVALID_ARGUMENT, "%s: workspace must be 256-byte aligned", __func__);
-    const size_t widest = d_model > d_ff ? d_model : d_ff;
-    size_t bytes_a = 0, bytes_b = 0;
-    hipq_packed_size(tokens, d_model, &bytes_a);
-    hipq_packed_size(tokens, widest, &bytes_b);
     char *p = static_cast<char *>(workspace);
     int8_t *qa = reinterpret_cast<int8_t *>(p);  // LayerNorm outputs (the operand of qkv and fc1)
     p += align256(bytes_a);
@@ -168,24 +185,21 @@ int32_t hipq_transformer_stack_forward_prepared_f32(hipq_ctx *ctx, const hipq_bl
     float *qkv = reinterpret_cast<float *>(p);
     const int32_t round_bits = mode & HIPQ_ROUND_HALF_EVEN;
 
-    const StackBuffers buf{qa, qb, sa, sb, qkv};
     int32_t rc;
     // Row panels are 32 (or 64) rows of one workgroup (or pair), so a forward of few tokens leaves compute units idle and
     // every busy one streams the whole weight matrices: 1.5-1.65 ms for 12 layers at d 768, d_ff 3072 whatever the
     // number of tokens, up to 8192.  The separate tiled products and row kernels grow with it instead, us (panels / tiled):
-    //   d 768, d_ff 3072:  77 1510 / 530, 1000 1590 / 690, 4096 1660 / 1270, 8192 1835 / 2120
+    //   d 768, d_ff 3072:  77 1510 / 366, 1000 1590 / 640, 4096 1660 / 1270, 8192 1835 / 2120
     //   d 256, d_ff 1024:  77 635 / 480, 4096 660 / 630, 8192 705 / 860;   d 1024: 77 2425 / 590, 8192 2730 / 2700
-    // so the panels are taken when they fill five eighths of the device.  (Test hook 15: panels always.)
-    if (tokens <= size_t(ctx->num_cus) * 20 && ctx->gemm_variant != 15) {
-        void *s = nullptr;
-        if (hipq::scratch(ctx, hipq::kScratchHeader + tokens * d_ff * sizeof(float), &s) == HIPQ_SUCCESS)
-            return stack_tiled(ctx, blocks, n_layers, tokens, d_model, d_ff, eps, round_bits, x, buf,
-                               reinterpret_cast<float *>(static_cast<char *>(s) + hipq::kScratchHeader));
-        hipq::clear_error();  // (no memory, or a first call under stream capture: the panels need none)
-    }
+    // so the panels are taken when they fill five eighths of the device, and where a workspace sized for them alone has no
+    // room for fc1's output.  Both give the same bits.  (Test hook 15: panels always.)
+    const bool room = workspace_bytes - ahead >= tokens * d_ff * sizeof(float);
+    if (room && tokens <= kTiledTokens && tokens <= size_t(ctx->num_cus) * 20 && ctx->gemm_variant != 15)
+        return stack_tiled(ctx, blocks, n_layers, tokens, d_model, d_ff, eps, round_bits, x,
+                           StackBuffers{qa, qb, sa, sb, qkv, qkv});
     // quant(LN1(x)) of the first layer: the row kernel, then the packing pass (row-major codes parked in qb)
     rc = hipq_layer_norm_quantize_f32_i8(ctx, x, tokens, d_model, blocks[0].ln1_gamma, blocks[0].ln1_beta, eps,
-                                                 round_bits, qb, sa);
+                                         round_bits, qb, sa);
     if (rc) return rc;
     if ((rc = hipq_pack_rows_i8(ctx, qb, tokens, d_model, qa))) return rc;
     for (size_t l = 0; l < n_layers; ++l) {
@@ -202,7 +216,7 @@ int32_t hipq_transformer_stack_forward_prepared_f32(hipq_ctx *ctx, const hipq_bl
         if (rc) return rc;
         // Stand-in for the attention mixing, which is outside this path: the value slice passes through.  Its
         // per-token quantizer runs inside the out-projection where a workgroup can hold its rows' codes on chip.
-        if (d_model <= 1536 && ctx->gemm_variant != 6) {
+        if (out_from_f32(ctx, d_model)) {
             rc = hipq_linear_from_f32_residual_layer_norm_quantize_packed_i8(
                 ctx, qkv + 2 * d_model, 3 * d_model, b.w_out, b.s_out, b.b_out, tokens, d_model, d_model, x, b.ln2_gamma,
                 b.ln2_beta, eps, round_bits, qa, sa);
