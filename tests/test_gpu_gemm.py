@@ -400,3 +400,32 @@ def test_gemm_any_k_and_alignment(ctx, oracle, m, n, k, shift):
     bias = rng.standard_normal(n).astype(np.float32)
     got = host(ctx.linear_i8_f32(placed(a), dev(sa), placed(w), dev(sw), dev(bias)))
     np.testing.assert_array_equal(got, acc.astype(np.float32) * (sa[:, None] * sw[None, :]) + bias[None, :])
+
+
+@pytest.mark.parametrize("m,n", [(1, 8), (9, 40), (20, 24), (300, 1000), (4096, 1024), (4100, 1001)])
+def test_empty_reduction(hipq, oracle, m, n):
+    """K = 0 (operands without storage, so null): accumulators 0, and every epilogue of them, whatever the number of tiles
+    and the kernel form that is asked for."""
+    c = hipq.Context(0)
+    try:
+        rng = np.random.default_rng(m + n)
+        a, w = torch.empty((m, 0), dtype=torch.int8, device="cuda"), torch.empty((n, 0), dtype=torch.int8, device="cuda")
+        acc = np.zeros((m, n), np.int32)
+        sa = (rng.random(m) * 0.05 + 0.001).astype(np.float32)
+        sw = (rng.random(n) * 0.002 + 0.0001).astype(np.float32)
+        bias = rng.standard_normal(n).astype(np.float32)
+        res = rng.standard_normal((m, n)).astype(np.float32)
+        want = oracle.linear_dequant_epilogue(acc, sa, sw, bias)
+        wantq = oracle.requantize_epilogue(acc, sa, sw, bias, 0.021, -5)
+        for variant in (0, 2, 7, 10):
+            c.set_gemm_kernel_variant(variant)
+            np.testing.assert_array_equal(host(c.gemm_i8_i32(a, w)), acc)
+            np.testing.assert_array_equal(host(c.linear_i8_f32(a, dev(sa), w, dev(sw), dev(bias))), want)
+            np.testing.assert_array_equal(host(c.linear_i8_f32(a, dev(sa), w, dev(sw), None)), np.zeros_like(want))
+            np.testing.assert_array_equal(host(c.linear_i8_f32_residual(a, dev(sa), w, dev(sw), dev(bias), dev(res))),
+                                          want + res)
+            np.testing.assert_array_equal(host(c.linear_i8_i8(a, dev(sa), w, dev(sw), dev(bias), 0.021, -5)), wantq)
+        c.synchronize()
+    finally:
+        torch.cuda.synchronize()
+        c.close()

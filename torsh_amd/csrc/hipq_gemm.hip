@@ -254,7 +254,8 @@ static int32_t launch_gemv(hipq_ctx *ctx, const int8_t *a, const int8_t *w, int 
     return check_launch("gemv_i8 (LDS staged)");
 }
 
-// Any shape: one thread per output, plain integer dot product.  Used when K is below 16.
+// Any shape: one thread per output, plain integer dot product.  Used when K is below 16 (0: the sums are 0 and no operand
+// is touched, which may then be null).
 template <int EPI, bool EVEN>
 __global__ __launch_bounds__(kGemmThreads) void gemm_i8_generic_kernel(const int8_t *__restrict__ A,
                                                                         const int8_t *__restrict__ W, int M, int N,
@@ -305,7 +306,7 @@ static int32_t launch_gemm(hipq_ctx *ctx, const int8_t *a, const int8_t *w, size
     const int M = static_cast<int>(m), N = static_cast<int>(n), K = static_cast<int>(k);
     const bool fast = (K % 16 == 0) && ((reinterpret_cast<uintptr_t>(a) & 15u) == 0) &&
                       ((reinterpret_cast<uintptr_t>(w) & 15u) == 0);
-    if (!fast && K < 16) {
+    if (K < 16) {
         size_t blocks = (m * n + kGemmThreads - 1) / kGemmThreads;
         const size_t cap = size_t(ctx->num_cus) * 8;
         if (blocks > cap) blocks = cap;

@@ -822,6 +822,7 @@ static int32_t launch_pipe(hipq_ctx *ctx, const int8_t *a, const int8_t *w, int 
             return fail(HIPQ_DEVICE_ERROR, "gemm_i8: cannot reserve %d bytes of LDS: %s", kLds, hipGetErrorString(e));
         configured[ctx->device] = true;
     }
+    if (K % 16 != 0 || K < 16) return fail(HIPQ_INVALID_ARGUMENT, "gemm_i8 (pipelined): K must be a positive multiple of 16");
     const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
     GemmEpilogue placed = ep;
     pick_xcd_rectangle(tiles_m, tiles_n, BM, BN, &placed.xcd_gm, &placed.xcd_gn);

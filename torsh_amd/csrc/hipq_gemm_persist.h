@@ -577,7 +577,8 @@ static int32_t launch_persist(hipq_ctx *ctx, const int8_t *a, const int8_t *w, i
             return fail(HIPQ_DEVICE_ERROR, "gemm_i8: cannot reserve %d bytes of LDS: %s", kLds, hipGetErrorString(e));
         configured[ctx->device][with_residual] = true;
     }
-    if (K % 16 != 0) return fail(HIPQ_INVALID_ARGUMENT, "gemm_i8 (persistent): K must be a multiple of 16");
+    // (K = 0 would leave the consumers waiting for fills that never come)
+    if (K % 16 != 0 || K < 16) return fail(HIPQ_INVALID_ARGUMENT, "gemm_i8 (persistent): K must be a positive multiple of 16");
     if (EPI != EPI_I32 && (!ep.sa || !ep.sw)) return fail(HIPQ_INVALID_ARGUMENT, "gemm_i8 (persistent): scales must be given");
     const int tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
     const int grid = tiles < ctx->num_cus ? tiles : ctx->num_cus;
