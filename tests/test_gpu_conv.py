@@ -302,3 +302,43 @@ def test_conv_any_stride_and_channel_count(ctx, hipq, oracle, nb, c, h, w, oc, k
         for b, q in zip((bd, None), codes):
             got = host(ctx.conv2d_i8(xd, zp, float(s_in), wd, swd, b, s_out, -2, stride, pad, mode))
             np.testing.assert_array_equal(got.reshape(acc2d.shape), q)
+
+
+@pytest.mark.parametrize("c,h,w,k,stride,pad", [(0, 6, 9, (3, 3), (1, 1), (1, 1)), (0, 5, 5, (2, 2), (2, 1), (0, 0)),
+                                                (3, 0, 8, (3, 3), (1, 1), (2, 1)), (32, 0, 5, (1, 3), (1, 2), (1, 1)),
+                                                (3, 7, 0, (3, 3), (2, 1), (1, 2))])
+def test_conv_of_nothing(ctx, hipq, oracle, c, h, w, k, stride, pad):
+    """No channels, or an image without rows or columns inside its border: empty sums, so accumulators of 0 and the bias
+    through every epilogue.  (Pointers of operands without elements are any address that is not null.)"""
+    nb, oc = 2, 40
+    ho, wo = (h + 2 * pad[0] - k[0]) // stride[0] + 1, (w + 2 * pad[1] - k[1]) // stride[1] + 1
+    rng = np.random.default_rng(c + h + w)
+    wq = dev(rng.integers(-128, 128, size=(oc, max(c, 1)) + k, dtype=np.int8))
+    sw, bias = rng.uniform(1e-4, 1e-3, oc).astype(np.float32), rng.standard_normal(oc).astype(np.float32)
+    swd, bd, somewhere = dev(sw), dev(bias), torch.zeros(64, dtype=torch.uint8, device="cuda")
+    geom = (nb, c, h, w, oc, *k, *stride, *pad)
+    acc = torch.full((nb, oc, ho, wo), 7, dtype=torch.int32, device="cuda")
+    ctx.call("hipq_conv2d_u8i8_i32", somewhere.data_ptr(), 77, wq.data_ptr(), *geom, acc.data_ptr())
+    f = torch.full((nb, oc, ho, wo), 7.0, device="cuda")
+    ctx.call("hipq_conv2d_u8i8_f32", somewhere.data_ptr(), 77, 0.02, wq.data_ptr(), swd.data_ptr(), bd.data_ptr(), *geom,
+             f.data_ptr())
+    q = torch.full((nb, oc, ho, wo), 7, dtype=torch.int8, device="cuda")
+    ctx.call("hipq_conv2d_u8i8_i8", somewhere.data_ptr(), 77, 0.02, wq.data_ptr(), swd.data_ptr(), bd.data_ptr(), *geom,
+             0.011, -3, 0, q.data_ptr())
+    assert not host(acc).any()
+    want = np.broadcast_to(bias[None, :, None, None], (nb, oc, ho, wo))
+    np.testing.assert_array_equal(host(f), want)
+    # (rows of the epilogue are outputs, its columns the filters)
+    wantq = oracle.requantize_epilogue(np.zeros((1, oc), np.int32), np.array([0.02], np.float32), sw, bias, 0.011, -3)
+    np.testing.assert_array_equal(host(q), np.broadcast_to(wantq.reshape(1, oc, 1, 1), (nb, oc, ho, wo)))
+
+
+def test_conv_without_channels_on_prepared_filters_is_refused(ctx, hipq):
+    some = torch.zeros(4096, dtype=torch.uint8, device="cuda")
+    p = some.data_ptr()
+    with pytest.raises(hipq.HipqError):
+        ctx.call("hipq_conv2d_u8i8_i8_packed", p, 0, 0.02, p, p, p, None, 1, 0, 4, 4, 8, 3, 3, 1, 1, 0.05, 0, 0, p)
+    with pytest.raises(hipq.HipqError):
+        ctx.call("hipq_conv2d_dynamic_f32_i8_packed", p, hipq.PARAMS_BACKEND_ASYMMETRIC, 0, p, p, p, None, 1, 0, 4, 4, 8, 3, 3,
+                 1, 1, 0.05, 0, 0, p, p)
+    torch.cuda.synchronize()

@@ -203,8 +203,10 @@ struct ConvDynamicInput {
     hipq_qparams *params = nullptr;
 };
 
-// Geometry of the image layout of hipq_conv_window.h; false where its 32-bit offsets do not reach.
+// Geometry of the image layout of hipq_conv_window.h; false where its 32-bit offsets do not reach, or without channels
+// (nothing to lay out: the outputs are those of empty sums).
 static bool window_geometry(const ConvGeom &g, ConvWindow *cw) {
+    if (g.c == 0) return false;
     const size_t cgs = (size_t(g.c) + 31) / 32, pitch = ((size_t(g.c) + cgs - 1) / cgs + 3) / 4 * 4;
     const size_t segs = (size_t(g.kw) * pitch + 31) / 32, kblocks = size_t(g.kh) * segs * cgs;
     const size_t hp = size_t(g.h) + 2 * g.ph, wp = size_t(g.w) + 2 * g.pw;
@@ -238,7 +240,8 @@ static int32_t launch_conv_window(hipq_ctx *ctx, const int8_t *filters, const in
 // Layout pass of a u8 input, and of the filters when `f` has any, in one launch.
 static int32_t launch_window_pack(const char *fn, hipq_ctx *ctx, const uint8_t *x, int zp, const int32_t *zp_dev,
                                   const ConvGeom &g, const ConvWindow &cw, int8_t *image, const ConvWindowFilters &f) {
-    const int v = g.w >= 4 ? 4 : 1, runs = (cw.wp + v - 1) / v;
+    // (four pixels per thread load a dword of the nearest image row, so there has to be one)
+    const int v = g.w >= 4 && g.h >= 1 ? 4 : 1, runs = (cw.wp + v - 1) / v;
     const size_t items = size_t(g.nb) * cw.hp * runs;
     const ConvPackWalk walk{f.w ? g.oc : 0, static_cast<int>((items + 255) / 256), static_cast<int>(items), FastDiv::by(runs), FastDiv::by(cw.hp)};
     const dim3 grid(walk.filters + cw.cgs * walk.groups_per_cg);
@@ -282,7 +285,7 @@ static int32_t conv_forward(const char *fn, hipq_ctx *ctx, const uint8_t *x, int
     ep.cv_corr_mul = 128 - zp_in;
     ConvWindow cw;
     if (!window_geometry(g, &cw)) {
-        if (dyn.x || !w) return fail(HIPQ_SHAPE_ERROR, "%s: image or filters too large", fn);
+        if (dyn.x || !w) return fail(HIPQ_SHAPE_ERROR, "%s: image or filters too large, or no channels", fn);
         const size_t total = size_t(g.nb) * g.oc * g.ho * g.wo;
         size_t blocks = (total + kConvThreads - 1) / kConvThreads;
         const size_t cap = size_t(ctx->num_cus) * 32;

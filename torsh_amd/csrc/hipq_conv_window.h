@@ -66,7 +66,8 @@ struct __attribute__((packed, aligned(1))) ConvWord {
 // channels each (consecutive lanes are consecutive pixels: consecutive bytes of every channel plane).  V = 4: a channel's
 // four pixels are one dword at any alignment, loaded from inside the image row and shifted where the run reaches over
 // its end, and 4 x 4 bytes are transposed by eight permutes: a quarter of the loads and of the address arithmetic, which
-// is what bounded the pass ([32,3,224,224] pad 3: 11.1 -> 5.5 us, filters included; 12 MB moved).  V = 1: rows of fewer than four pixels.
+// is what bounded the pass ([32,3,224,224] pad 3: 11.1 -> 5.5 us, filters included; 12 MB moved).  V = 1: rows of fewer than
+// four pixels, images without rows.
 // Further workgroups pack the filters: one output channel each, a thread per 16-byte piece.
 struct ConvWindowFilters {
     const int8_t *w;  // [OC, IC, KH, KW]
