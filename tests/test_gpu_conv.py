@@ -342,3 +342,15 @@ def test_conv_without_channels_on_prepared_filters_is_refused(ctx, hipq):
         ctx.call("hipq_conv2d_dynamic_f32_i8_packed", p, hipq.PARAMS_BACKEND_ASYMMETRIC, 0, p, p, p, None, 1, 0, 4, 4, 8, 3, 3,
                  1, 1, 0.05, 0, 0, p, p)
     torch.cuda.synchronize()
+
+
+def test_conv_of_an_empty_batch_leaves_a_cleared_record(ctx, hipq):
+    """A call without outputs launches nothing; the record that it returns is one of zeros, not memory as it was found."""
+    packed, sums = ctx.conv2d_pack_weights(torch.ones((8, 32, 3, 3), dtype=torch.int8, device="cuda"))
+    sw, size = torch.ones(8, device="cuda"), ctx.new_qparams().numel()
+    # blocks of the record's size that hold something, for the allocator to hand out again
+    used = [torch.full((size,), 0xa5, dtype=torch.uint8, device="cuda") for _ in range(8)]
+    del used
+    out, params = ctx.conv2d_dynamic_packed(torch.empty((0, 32, 6, 6), device="cuda"), packed, sums, (3, 3), sw, None, 0.05, 0,
+                                            (1, 1))
+    assert out.numel() == 0 and not host(params).any()

@@ -740,7 +740,8 @@ class Context:
         ho = h + 2 * padding[0] - kh + 1
         wo = wd + 2 * padding[1] - kw + 1
         out = out if out is not None else torch.empty((nb, oc, ho, wo), dtype=torch.int8, device=self._dev())
-        params = params if params is not None else self._unset_qparams()
+        if params is None:  # (an empty batch launches nothing, and nothing writes its record)
+            params = self._unset_qparams() if nb else self.new_qparams()
         self.call("hipq_conv2d_dynamic_f32_i8_packed", _ptr(x), flavor, quant_mode, _ptr(w_packed), _ptr(w_sums),
                   _ptr(w_scales), _ptr(bias), nb, c, h, wd, oc, kh, kw, padding[0], padding[1], float(s_out),
                   int(zp_out), mode, _ptr(out), _ptr(params))
