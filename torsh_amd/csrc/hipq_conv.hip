@@ -240,20 +240,27 @@ static int32_t launch_conv_window(hipq_ctx *ctx, const int8_t *filters, const in
 // Layout pass of a u8 input, and of the filters when `f` has any, in one launch.
 static int32_t launch_window_pack(const char *fn, hipq_ctx *ctx, const uint8_t *x, int zp, const int32_t *zp_dev,
                                   const ConvGeom &g, const ConvWindow &cw, int8_t *image, const ConvWindowFilters &f) {
-    // (four pixels per thread load a dword of the nearest image row, so there has to be one)
-    const int v = g.w >= 4 && g.h >= 1 ? 4 : 1, runs = (cw.wp + v - 1) / v;
+    // Four pixels per thread or one (us, one / four, 32 images of 224 x 224; of 56 x 56 in brackets).  3 channels 8.3 / 6.4,
+    // 4 7.4 / 6.2; where the last group lacks channels, whose loads are then guarded one by one: 5 11.2 / 10.2, 11 15.4 / 12.4,
+    // 33 54 / 46 (7.5 / 6.9); but with all there the four pixels' 16-byte stores, up to 128 bytes apart, cost more than the
+    // loads they save: 8 8.1 / 9.7, 16 11.0 / 15.0, 32 (4.7 / 5.8), [32,512,28,28] 8.5 / 12.7.  A dword comes from the nearest
+    // image row, so four pixels need one.
+    const bool full = g.c == cw.cgs * cw.pitch;
+    const int v = g.w >= 4 && g.h >= 1 && (!full || cw.pitch == 4) ? 4 : 1, runs = (cw.wp + v - 1) / v;
     const size_t items = size_t(g.nb) * cw.hp * runs;
     const ConvPackWalk walk{f.w ? g.oc : 0, static_cast<int>((items + 255) / 256), static_cast<int>(items), FastDiv::by(runs), FastDiv::by(cw.hp)};
     const dim3 grid(walk.filters + cw.cgs * walk.groups_per_cg);
-#define HIPQ_PACK_WINDOWS_V(DW, V)                                                                                         \
-    hipLaunchKernelGGL((conv_window_pack_kernel<DW, V>), grid, dim3(256), 0, ctx->stream, x, g.c, g.h, g.w, g.ph, g.pw, zp, \
+#define HIPQ_PACK_WINDOWS_V(DW, V, FULL)                                                                                       \
+    hipLaunchKernelGGL((conv_window_pack_kernel<DW, V, FULL>), grid, dim3(256), 0, ctx->stream, x, g.c, g.h, g.w, g.ph, g.pw, zp, \
                        zp_dev, walk, image, cw, f)
 #define HIPQ_PACK_WINDOWS(DW)           \
     case DW:                            \
-        if (v == 4)                     \
-            HIPQ_PACK_WINDOWS_V(DW, 4); \
-        else                            \
-            HIPQ_PACK_WINDOWS_V(DW, 1); \
+        if (v == 4)                            \
+            HIPQ_PACK_WINDOWS_V(DW, 4, false); \
+        else if (full)                         \
+            HIPQ_PACK_WINDOWS_V(DW, 1, true);  \
+        else                                   \
+            HIPQ_PACK_WINDOWS_V(DW, 1, false); \
         break
     switch (cw.pitch / 4) {
         HIPQ_PACK_WINDOWS(1);

@@ -66,8 +66,9 @@ struct __attribute__((packed, aligned(1))) ConvWord {
 // channels each (consecutive lanes are consecutive pixels: consecutive bytes of every channel plane).  V = 4: a channel's
 // four pixels are one dword at any alignment, loaded from inside the image row and shifted where the run reaches over
 // its end, and 4 x 4 bytes are transposed by eight permutes: a quarter of the loads and of the address arithmetic, which
-// is what bounded the pass ([32,3,224,224] pad 3: 11.1 -> 5.5 us, filters included; 12 MB moved).  V = 1: rows of fewer than
-// four pixels, images without rows.
+// is what bounded the pass ([32,3,224,224] pad 3: 11.1 -> 5.5 us, filters included; 12 MB moved).  V = 1: groups
+// of more than four channels that are all there (FULL: the loads of a pixel need no guard, and its bytes are one run of
+// stores), rows of fewer than four pixels, images without rows.
 // Further workgroups pack the filters: one output channel each, a thread per 16-byte piece.
 struct ConvWindowFilters {
     const int8_t *w;  // [OC, IC, KH, KW]
@@ -84,12 +85,12 @@ struct ConvPackWalk {
     FastDiv by_runs, by_hp;
 };
 
-template <int DW, int V>
+template <int DW, int V, bool FULL>
 __global__ __launch_bounds__(256) void conv_window_pack_kernel(const uint8_t *__restrict__ x, int C, int H, int W, int pad_h,
                                                                  int pad_w, int zp, const int32_t *__restrict__ zp_dev,
                                                                  ConvPackWalk walk, int8_t *__restrict__ image,
                                                                  ConvWindow cw, ConvWindowFilters f) {
-    static_assert(V == 1 || V == 4, "pixels per thread");
+    static_assert(V == 1 || (V == 4 && !FULL), "pixels per thread");
     // The filters' workgroups come first: their chain (16 gathered bytes, a sum over the workgroup) is the longer one.
     if (static_cast<int>(blockIdx.x) < walk.filters) {
         __shared__ int part[4];
@@ -152,7 +153,7 @@ __global__ __launch_bounds__(256) void conv_window_pack_kernel(const uint8_t *__
             const uint8_t *src = x + ((size_t(n) * C + c0) * H + h) * W + v;
             uint32_t b[4 * DW];
 #pragma unroll
-            for (int c = 0; c < 4 * DW; ++c) b[c] = c0 + c < C ? src[size_t(c) * plane] : 0u;
+            for (int c = 0; c < 4 * DW; ++c) b[c] = FULL || c0 + c < C ? src[size_t(c) * plane] : 0u;
 #pragma unroll
             for (int i = 0; i < DW; ++i)
                 d[0][i] = (b[4 * i] | (b[4 * i + 1] << 8) | (b[4 * i + 2] << 16) | (b[4 * i + 3] << 24)) ^ 0x80808080u;
