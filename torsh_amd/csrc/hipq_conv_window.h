@@ -213,7 +213,7 @@ __global__ __launch_bounds__(256, FM * FN < 8 ? 3 : (SPLIT ? 1 : 2)) void conv_i
                                                                GemmEpilogue ep) {
     constexpr int NBLK = FM * FN;
     constexpr int OWN = SPLIT ? NBLK / 4 : NBLK;  // accumulator blocks a wave finishes
-    static_assert(!SPLIT || (NBLK % 4 == 0 && FN % OWN == 0), "the K-split waves share the blocks of one channel block each");
+    static_assert(!SPLIT || (FM == 4 && FN == 2) || (FM == 2 && FN == 2) || (FM == 1 && FN == 4), "K-split tiles");
     constexpr int COLS = SPLIT ? 1 : FM;          // channel blocks among them
     extern __shared__ __attribute__((aligned(16))) int8_t lds[];
     const int lane = threadIdx.x % kWave, half = lane / 32;
@@ -229,13 +229,17 @@ __global__ __launch_bounds__(256, FM * FN < 8 ? 3 : (SPLIT ? 1 : 2)) void conv_i
     const int q0 = tile_n * kTileN + (SPLIT ? 0 : wave * FN * 32);  // first window of this wave
     const int rb0 = tile_m * FM;
 
+    // K-split: a wave numbers the tile's blocks by exclusive or with its own place, so that the blocks it will own after
+    // the sum are its first ones and block b goes to wave `wave ^ (b / OWN)`: every wave runs the same code on the same
+    // registers, no wave-dependent choice behind the main loop.
+    const int jx = !SPLIT ? 0 : FM == 4 ? wave : FM == 2 ? wave >> 1 : 0;
+    const int ix = !SPLIT ? 0 : FM == 4 ? 0 : FM == 2 ? wave & 1 : wave;
     // Operands of the epilogue, ahead of the main loop: one channel per lane and channel block.
-    const int own0 = SPLIT ? wave * OWN : 0;  // first block (channel block own0 / FN, window fragment own0 % FN)
     int corr[COLS];
     float sc[COLS], bias[COLS];
 #pragma unroll
     for (int j = 0; j < COLS; ++j) {
-        const int oc = (rb0 + own0 / FN + j) * 32 + lane % 32;
+        const int oc = (rb0 + (j ^ jx)) * 32 + lane % 32;
         const int occ = oc < cw.M ? oc : cw.M - 1;
         corr[j] = (ep.cv_zp_in ? 128 - *ep.cv_zp_in : ep.cv_corr_mul) * ep.cv_wsum[occ];
         sc[j] = 1.0f;
@@ -253,13 +257,14 @@ __global__ __launch_bounds__(256, FM * FN < 8 ? 3 : (SPLIT ? 1 : 2)) void conv_i
     int sof[FM];
 #pragma unroll
     for (int j = 0; j < FM; ++j) {
-        const int rb = rb0 + j < (cw.M + 31) / 32 ? rb0 + j : (cw.M + 31) / 32 - 1;  // (repeated: not stored)
+        int rb = rb0 + (j ^ jx);
+        rb = rb < (cw.M + 31) / 32 ? rb : (cw.M + 31) / 32 - 1;  // (repeated: not stored)
         sof[j] = rb * cw.KB * 1024;
     }
     int voi[FN];
 #pragma unroll
     for (int i = 0; i < FN; ++i) {
-        int q = q0 + i * 32 + lane % 32;
+        int q = q0 + (i ^ ix) * 32 + lane % 32;
         q = q < cw.N ? q : cw.N - 1;
         uint32_t rem, ow;
         const uint32_t n = cw.by_plane.quotient(q, &rem), oh = cw.by_wo.quotient(rem, &ow);
@@ -425,37 +430,38 @@ __global__ __launch_bounds__(256, FM * FN < 8 ? 3 : (SPLIT ? 1 : 2)) void conv_i
                         emit_block(acc[j][i], j, (rb0 + j) * 32 + lane % 32, q0 + i * 32, plain);
         });
     } else {
-        // Block b = j * FN + i belongs to wave b / OWN; the other three park their partial sums of it in LDS.
+        // Blocks OWN .. NBLK - 1 are other waves': parked in LDS as [owner][slot][register quad][lane].
         v4i *red = reinterpret_cast<v4i *>(lds);
 #pragma unroll
-        for (int b = 0; b < NBLK; ++b) {
-            const int owner = b / OWN;
-            if (owner == wave) continue;
-            v4i *dst = red + (((wave - owner + 3) % 4) * NBLK + b) * 4 * kWave + lane;
+        for (int b = OWN; b < NBLK; ++b) {
+            const int owner = wave ^ (b / OWN);
+            v4i *dst = red + (owner * (NBLK - OWN) + b - OWN) * 4 * kWave + lane;
 #pragma unroll
             for (int g = 0; g < 4; ++g)
                 dst[g * kWave] = v4i{acc[b / FN][b % FN][4 * g], acc[b / FN][b % FN][4 * g + 1],
                                      acc[b / FN][b % FN][4 * g + 2], acc[b / FN][b % FN][4 * g + 3]};
         }
+        __syncthreads();
+        // All reads first, then the adds.
+        v4i part[3][OWN][4];
+        const v4i *src = red + wave * (NBLK - OWN) * 4 * kWave + lane;
+#pragma unroll
+        for (int s = 0; s < 3; ++s)
+#pragma unroll
+            for (int k = 0; k < OWN; ++k)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) part[s][k][g] = src[((s * OWN + k) * 4 + g) * kWave];
+        __builtin_amdgcn_sched_barrier(0);
         v16i own[OWN];
 #pragma unroll
-        for (int b = 0; b < NBLK; ++b)
-            if (b / OWN == wave) own[b % OWN] = acc[b / FN][b % FN];
-        __syncthreads();
+        for (int k = 0; k < OWN; ++k)
 #pragma unroll
-        for (int k = 0; k < OWN; ++k) {
-            v4i part[3][4];
-#pragma unroll
-            for (int s = 0; s < 3; ++s)
-#pragma unroll
-                for (int g = 0; g < 4; ++g) part[s][g] = red[((s * NBLK + own0 + k) * 4 + g) * kWave + lane];
-#pragma unroll
-            for (int r = 0; r < 16; ++r) own[k][r] += corr[0] + part[0][r / 4][r % 4] + part[1][r / 4][r % 4] + part[2][r / 4][r % 4];
-        }
+            for (int r = 0; r < 16; ++r)
+                own[k][r] = acc[0][k][r] + corr[0] + part[0][k][r / 4][r % 4] + part[1][k][r / 4][r % 4] + part[2][k][r / 4][r % 4];
         with_division([&](auto plain) {
 #pragma unroll
             for (int k = 0; k < OWN; ++k)
-                emit_block(own[k], 0, (rb0 + own0 / FN) * 32 + lane % 32, q0 + ((own0 + k) % FN) * 32, plain);
+                emit_block(own[k], 0, (rb0 + jx) * 32 + lane % 32, q0 + (k ^ ix) * 32, plain);
         });
     }
 }
