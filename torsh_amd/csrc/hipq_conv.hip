@@ -320,7 +320,8 @@ static int32_t conv_forward(const char *fn, hipq_ctx *ctx, const uint8_t *x, int
         return conv_gemm_patch(ctx, wpacked, x, elems, zp_in, g.h, g.w, g.ph, g.pw, g.kh, g.oc, g.nb * cw.hp * cw.wp,
                                static_cast<int>(k), ep, EPI, EVEN);
     }
-    const size_t img_bytes = align256(size_t(cw.image_bytes));
+    // (the last window's slice of a row of taps may end up to 31 bytes behind the image)
+    const size_t img_bytes = align256(size_t(cw.image_bytes) + 31);
     const size_t f_bytes = wpacked ? 0 : align256((size_t(cw.M) + 31) / 32 * cw.KB * 1024);
     const size_t w_bytes = wpacked ? 0 : f_bytes + align256(size_t(cw.M) * 4);
     // Dynamic input: in one launch with the image pack when its grid can be resident at once (the kernel holds 32

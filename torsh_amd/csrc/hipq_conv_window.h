@@ -287,14 +287,15 @@ __global__ __launch_bounds__(256, FM * FN < 8 ? 3 : (SPLIT ? 1 : 2)) void conv_i
     if constexpr (SPLIT) advance(wave);
     v4i ff[D][FM], fi[D][FN];
     auto issue = [&](int s) {
-        // k blocks past the last lie beyond both buffers: zeros, no memory access
+        // A k block past the last: the filters' load lies beyond its buffer (zeros, no memory access), so what the windows
+        // bring does not count: the first k block's.
         const bool real = kb < cw.kblocks;
-        const int kof = real ? kb * 1024 : 0x7fffff00;
-        const int koi = real ? cg * cw.plane_bytes + ty * cw.row_bytes + seg * 32 : 0x7fffff00;
+        const int vof = real ? lane * 16 : 0x7fffffff;
+        const int kof = real ? kb * 1024 : 0;
+        const int koi = real ? cg * cw.plane_bytes + ty * cw.row_bytes + seg * 32 : 0;
 #pragma unroll
         for (int j = 0; j < FM; ++j)
-            ff[s][j] = __builtin_bit_cast(
-                v4i, __builtin_amdgcn_raw_buffer_load_b128(rf, lane * 16, real ? sof[j] + kof : kof, 0));
+            ff[s][j] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rf, vof, real ? sof[j] + kof : 0, 0));
 #pragma unroll
         for (int i = 0; i < FN; ++i)
             fi[s][i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(ri, voi[i], koi, 0));
