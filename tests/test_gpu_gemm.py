@@ -429,3 +429,42 @@ def test_empty_reduction(hipq, oracle, m, n):
     finally:
         torch.cuda.synchronize()
         c.close()
+
+
+def _check_every_epilogue(c, oracle, m, n, k):
+    """Accumulators, dequantize with and without a residual, requantize of one row-major product against the oracle."""
+    rng = np.random.default_rng(m + n + k)
+    a, w = rand_i8(rng, (m, k)), rand_i8(rng, (n, k))
+    acc = oracle.gemm_i8_nk(a, w)
+    sa = (rng.random(m) * 0.05 + 0.001).astype(np.float32)
+    sw = (rng.random(n) * 0.002 + 0.0001).astype(np.float32)
+    bias = (rng.standard_normal(n) * 0.01).astype(np.float32)
+    res = rng.standard_normal((m, n)).astype(np.float32)
+    want = oracle.linear_dequant_epilogue(acc, sa, sw, bias)
+    s_out, _ = oracle.calculate_symmetric_params(*oracle.find_min_max(want), 0)
+    wantq = oracle.requantize_epilogue(acc, sa, sw, bias, s_out, -5)
+    ad, wd, sad, swd, bd = dev(a), dev(w), dev(sa), dev(sw), dev(bias)
+    np.testing.assert_array_equal(host(c.gemm_i8_i32(ad, wd)), acc)
+    np.testing.assert_array_equal(host(c.linear_i8_f32(ad, sad, wd, swd, bd)), want)
+    np.testing.assert_array_equal(host(c.linear_i8_f32_residual(ad, sad, wd, swd, bd, dev(res))), want + res)
+    np.testing.assert_array_equal(host(c.linear_i8_i8(ad, sad, wd, swd, bd, s_out, -5)), wantq)
+
+
+@pytest.mark.parametrize("k", [16, 64, 112, 128, 144, 320])
+@pytest.mark.parametrize("m,n", [(4100, 1100), (8200, 520)])
+def test_many_tiles_short_k_and_last_k_tile_over_the_end(ctx, oracle, m, n, k):
+    """Enough tiles for the persistent kernel, with one K-tile per output tile (every tile then starts on the other set of
+    fragments) and with a last K-tile that runs over the end of the rows."""
+    _check_every_epilogue(ctx, oracle, m, n, k)
+
+
+@pytest.mark.parametrize("variant", [1, 2, 3, 5, 6, 7, 8])
+def test_every_gemm_kernel_form_on_short_k_and_tails(ctx, oracle, variant):
+    """The same for each form forced on few tiles, ragged and whole ones: K of part of a K-tile, of one and of several."""
+    try:
+        ctx.set_gemm_kernel_variant(variant)
+        for k in (16, 128, 144, 272):
+            for m, n in ((300, 200), (512, 384)):
+                _check_every_epilogue(ctx, oracle, m, n, k)
+    finally:
+        ctx.set_gemm_kernel_variant(0)

@@ -620,7 +620,9 @@ __device__ __forceinline__ void store_block_interior(v16i (&own)[1][TNB], const 
 // wave while the texture path is busy, so mixing fills and MFMAs in one wave
 // serialises the two pipes; with the roles split, MFMA issue never waits behind a
 // memory instruction.  All waves meet at one barrier per K-tile.
-template <int BM, int BN, int STAGES, int PW, int WM, int WN, int WK, int EPI, bool EVEN>
+// TAIL: the last K-tile runs over the end of the rows (K % 128 != 0).  A form of its own, since the choice of address per
+// fill and its lane masks cost every K-tile: 512 x 4096 x 4096 16.4 us with it, 15.4 without.
+template <int BM, int BN, int STAGES, int PW, int WM, int WN, int WK, int EPI, bool EVEN, bool TAIL>
 __global__ __launch_bounds__((PW + WM * WN * WK) * kWave) void gemm_i8_pipe_kernel(const int8_t *__restrict__ A,
                                                                                     const int8_t *__restrict__ W,
                                                                                     int M, int N, int K,
@@ -654,13 +656,16 @@ __global__ __launch_bounds__((PW + WM * WN * WK) * kWave) void gemm_i8_pipe_kern
     if (wave < PW) {
         // ---------------- producer ----------------
         const int8_t *src[IPW];
-        bool past_end[IPW];  // the piece lies past the end of the rows in the last K-tile
+        // TAIL: the piece lies past the end of the rows in the last K-tile; a piece's column depends on whether its
+        // instruction is an even or an odd one only.
+        bool past_end[2] = {};
+        static_assert(IPW % 2 == 0, "even and odd instructions are the same ones in every wave");
 #pragma unroll
         for (int j = 0; j < IPW; ++j) {
             const int q = wave * IPW + j;
             const int trow = q * RPI + lane / CPR;  // row in the stacked [A rows | W rows] tile
             const int col = (lane % CPR) ^ ((trow >> 1) & 7);
-            past_end[j] = (nk - 1) * BK + col * 16 >= K;
+            if constexpr (TAIL) past_end[j % 2] = (nk - 1) * BK + col * 16 >= K;
             if (trow < BM) {
                 int gm = m0 + trow;
                 gm = gm < M ? gm : M - 1;  // rows past the edge are computed and discarded
@@ -674,11 +679,10 @@ __global__ __launch_bounds__((PW + WM * WN * WK) * kWave) void gemm_i8_pipe_kern
         auto issue_stage = [&](int kt, int buf) {
             int8_t *base = lds + buf * STAGE + wave * (IPW * 1024);
             const size_t koff_row = size_t(kt) * BK;
-            const bool last = kt == nk - 1;
 #pragma unroll
             for (int j = 0; j < IPW; ++j) {
                 const int8_t *from = src[j] + koff_row;
-                if (last && past_end[j]) from = reinterpret_cast<const int8_t *>(&kZeroPiece);
+                if (TAIL && kt == nk - 1 && past_end[j % 2]) from = reinterpret_cast<const int8_t *>(&kZeroPiece);
                 __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)from,
                                                  (__attribute__((address_space(3))) void *)(base + j * 1024), 16, 0, 0);
             }
@@ -808,12 +812,12 @@ __global__ __launch_bounds__((PW + WM * WN * WK) * kWave) void gemm_i8_pipe_kern
     store_tile<FM, FN, WK, EPI, EVEN>(acc, ep, M, N, m0 + wm * TM, wk, lane, nn, swv, bv, sa0);
 }
 
-template <int BM, int BN, int STAGES, int PW, int WM, int WN, int WK, int EPI, bool EVEN>
-static int32_t launch_pipe(hipq_ctx *ctx, const int8_t *a, const int8_t *w, int M, int N, int K,
+template <int BM, int BN, int STAGES, int PW, int WM, int WN, int WK, int EPI, bool EVEN, bool TAIL>
+static int32_t launch_pipe_form(hipq_ctx *ctx, const int8_t *a, const int8_t *w, int M, int N, int K,
                            const GemmEpilogue &ep) {
     constexpr int kLds = STAGES * (BM + BN) * 128;
     constexpr int kThreads = (PW + WM * WN * WK) * kWave;
-    auto kernel = gemm_i8_pipe_kernel<BM, BN, STAGES, PW, WM, WN, WK, EPI, EVEN>;
+    auto kernel = gemm_i8_pipe_kernel<BM, BN, STAGES, PW, WM, WN, WK, EPI, EVEN, TAIL>;
     static bool configured[16] = {false};  // per device: raise the dynamic LDS limit once
     if (ctx->device < 16 && !configured[ctx->device]) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
@@ -822,12 +826,19 @@ static int32_t launch_pipe(hipq_ctx *ctx, const int8_t *a, const int8_t *w, int 
             return fail(HIPQ_DEVICE_ERROR, "gemm_i8: cannot reserve %d bytes of LDS: %s", kLds, hipGetErrorString(e));
         configured[ctx->device] = true;
     }
-    if (K % 16 != 0 || K < 16) return fail(HIPQ_INVALID_ARGUMENT, "gemm_i8 (pipelined): K must be a positive multiple of 16");
     const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
     GemmEpilogue placed = ep;
     pick_xcd_rectangle(tiles_m, tiles_n, BM, BN, &placed.xcd_gm, &placed.xcd_gn);
     hipLaunchKernelGGL(kernel, dim3(tiles_m * tiles_n), dim3(kThreads), kLds, ctx->stream, a, w, M, N, K, placed);
     return check_launch("gemm_i8 (pipelined)");
+}
+
+template <int BM, int BN, int STAGES, int PW, int WM, int WN, int WK, int EPI, bool EVEN>
+static int32_t launch_pipe(hipq_ctx *ctx, const int8_t *a, const int8_t *w, int M, int N, int K,
+                           const GemmEpilogue &ep) {
+    if (K % 16 != 0 || K < 16) return fail(HIPQ_INVALID_ARGUMENT, "gemm_i8 (pipelined): K must be a positive multiple of 16");
+    if (K % 128 != 0) return launch_pipe_form<BM, BN, STAGES, PW, WM, WN, WK, EPI, EVEN, true>(ctx, a, w, M, N, K, ep);
+    return launch_pipe_form<BM, BN, STAGES, PW, WM, WN, WK, EPI, EVEN, false>(ctx, a, w, M, N, K, ep);
 }
 
 }  // namespace hipq
