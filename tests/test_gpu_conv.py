@@ -354,3 +354,31 @@ def test_conv_of_an_empty_batch_leaves_a_cleared_record(ctx, hipq):
     out, params = ctx.conv2d_dynamic_packed(torch.empty((0, 32, 6, 6), device="cuda"), packed, sums, (3, 3), sw, None, 0.05, 0,
                                             (1, 1))
     assert out.numel() == 0 and not host(params).any()
+
+
+def test_conv_with_a_stride_captured_by_a_new_context(hipq, oracle):
+    """A geometry that prepared filters do not take runs without memory of the context when the image does not fit what it
+    holds and none can be allocated (a first call under stream capture): the same bits, in every replay."""
+    rng = np.random.default_rng(3)
+    x = rng.integers(0, 256, size=(8, 4, 512, 512), dtype=np.uint8)  # an image of 8.45 MB, a new context holds 8 MiB
+    wq = rng.integers(-128, 128, size=(8, 4, 3, 3), dtype=np.int8)
+    want = oracle.backend_conv2d_i32(x, 9, wq, (2, 2), (1, 1))
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        dx, dw = dev(x), dev(wq)
+        c = hipq.Context(0)
+        try:
+            side.synchronize()
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph, stream=side):
+                out = c.conv2d_i32(dx, 9, dw, (2, 2), (1, 1))
+            for _ in range(3):
+                out.zero_()
+                side.synchronize()
+                graph.replay()
+                torch.cuda.synchronize()
+                np.testing.assert_array_equal(host(out), want)
+                np.testing.assert_array_equal(host(c.conv2d_i32(dx, 9, dw, (2, 2), (1, 1))), want)
+        finally:
+            torch.cuda.synchronize()
+            c.close()

@@ -291,8 +291,9 @@ static int32_t conv_forward(const char *fn, hipq_ctx *ctx, const uint8_t *x, int
     ep.sa_scalar = s_in;
     ep.cv_corr_mul = 128 - zp_in;
     ConvWindow cw;
-    if (!window_geometry(g, &cw)) {
-        if (dyn.x || !w) return fail(HIPQ_SHAPE_ERROR, "%s: image or filters too large, or no channels", fn);
+    // Needs no memory of the context: where the window kernel's offsets do not reach, and for a geometry that prepared
+    // filters do not take when the context cannot hold its image (a first call under stream capture, or no memory left).
+    auto direct = [&]() -> int32_t {
         const size_t total = size_t(g.nb) * g.oc * g.ho * g.wo;
         size_t blocks = (total + kConvThreads - 1) / kConvThreads;
         const size_t cap = size_t(ctx->num_cus) * 32;
@@ -300,6 +301,10 @@ static int32_t conv_forward(const char *fn, hipq_ctx *ctx, const uint8_t *x, int
         hipLaunchKernelGGL((conv_direct_kernel<EPI, EVEN>), dim3(static_cast<int>(blocks)), dim3(kConvThreads), 0,
                            ctx->stream, x, zp_in, w, g, s_in, sw, bias, s_out, zp_out, out);
         return check_launch(fn);
+    };
+    if (!window_geometry(g, &cw)) {
+        if (dyn.x || !w) return fail(HIPQ_SHAPE_ERROR, "%s: image or filters too large, or no channels", fn);
+        return direct();
     }
     // One launch, the image gathered by the convolution kernel itself (hipq_conv_patch.h): built, bit-exact, and
     // measured no faster than the two launches below on the shape it was built for (13.3 against 13.4 us at
@@ -332,6 +337,11 @@ static int32_t conv_forward(const char *fn, hipq_ctx *ctx, const uint8_t *x, int
     const size_t u8_bytes = (dyn.x && !fused_input) ? align256(elems) : 0;
     void *s = nullptr;
     int32_t rc = scratch(ctx, kScratchHeader + img_bytes + w_bytes + u8_bytes, &s);
+    if (rc == HIPQ_ALLOCATION_ERROR && w && !prepared_ok(g)) {
+        clear_error();
+        (void)hipGetLastError();  // (of the allocation: the launch's own check would report it)
+        return direct();
+    }
     if (rc) return rc;
     int8_t *image = reinterpret_cast<int8_t *>(static_cast<char *>(s) + kScratchHeader);
     ConvWindowFilters f{nullptr, nullptr, nullptr, g.c, g.kh, g.kw};
