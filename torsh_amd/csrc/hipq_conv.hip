@@ -225,9 +225,14 @@ static bool window_geometry(const ConvGeom &g, ConvWindow *cw) {
 template <int EPI, bool EVEN>
 static int32_t launch_conv_window(hipq_ctx *ctx, const int8_t *filters, const int8_t *image, const ConvWindow &cw,
                                   const GemmEpilogue &ep) {
-    // Waves on different windows while there are enough of them for two per SIMD, else K split between four.
-    const size_t waves = (size_t(cw.N) + 63) / 64 * ((size_t(cw.M) + 127) / 128);
-    if (waves >= size_t(ctx->num_cus) * 8 || cw.kblocks < 8) {
+    // Waves on different windows while there are enough of them for two per SIMD, else K split between four.  Fewer than
+    // eight k blocks are split only up to a tile of 128 channels x 64 windows per compute unit: there is little K to
+    // share, but a wave that finishes two blocks instead of eight has the shorter epilogue.  1 x 1 on prepared filters, us
+    // from own windows / K split (tiles): [3,128,5,5] x 128 13.9 / 8.5 (2), [2,160,14,14] x 512 11.8 / 7.8 (28),
+    // [4,224,38,38] x 192 13.1 / 8.7 (182), [49,96,9,9] x 512 12.5 / 9.7 (252), but [32,32,14,14] x 512 12.1 / 12.4 (392),
+    // [4,32,46,46] x 512 12.5 / 15.5 (532), [30,128,28,28] x 256 12.2 / 16.6 (736), [25,128,40,40] x 512 21 / 43 (2500).
+    const size_t tiles = (size_t(cw.N) + 63) / 64 * ((size_t(cw.M) + 127) / 128), cus = size_t(ctx->num_cus);
+    if (tiles >= cus * 8 || (cw.kblocks < 8 && tiles > cus)) {
         if (cw.M <= 32) return launch_conv_window_form<1, 4, 3, false, EPI, EVEN>(ctx, filters, image, cw, ep);
         if (cw.M <= 64) return launch_conv_window_form<2, 2, 4, false, EPI, EVEN>(ctx, filters, image, cw, ep);
         return launch_conv_window_form<4, 2, 2, false, EPI, EVEN>(ctx, filters, image, cw, ep);
