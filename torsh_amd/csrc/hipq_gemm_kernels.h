@@ -263,7 +263,7 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_i8_mfma_kernel(const int8_t
         }
     };
     auto load_global = [&](int k0) {
-        if (k0 + BK > K)
+        if (k0 + BK > K && K % 16 != 0)  // (else a piece lies inside the row or past it)
             load_pieces(k0, std::true_type{});
         else
             load_pieces(k0, std::false_type{});
@@ -651,7 +651,7 @@ __global__ __launch_bounds__((PW + WM * WN * WK) * kWave) void gemm_i8_pipe_kern
     tile_of_block((M + BM - 1) / BM, (N + BN - 1) / BN, ep.xcd_gm, ep.xcd_gn, &tile_m, &tile_n);
     const int m0 = tile_m * BM, n0 = tile_n * BN;
     const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
-    const int nk = (K + BK - 1) / BK;
+    const int nk = K / BK + (TAIL ? 1 : 0);
 
     if (wave < PW) {
         // ---------------- producer ----------------

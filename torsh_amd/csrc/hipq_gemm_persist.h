@@ -111,7 +111,7 @@ __global__ __launch_bounds__((PW + WM * WN) * kWave) void gemm_i8_persist_kernel
 
     const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
     const int ntiles = tiles_m * tiles_n;
-    const int nk = (K + BK - 1) / BK;  // >= 1
+    const int nk = K / BK + (TAIL ? 1 : 0);  // >= 1
     const int my_tiles = (ntiles - static_cast<int>(blockIdx.x) + static_cast<int>(gridDim.x) - 1) /
                          static_cast<int>(gridDim.x);
     const int T = my_tiles * nk;  // K-tiles this workgroup streams, in consumption order
