@@ -862,6 +862,10 @@ static int32_t launch_split_packed(hipq_ctx *ctx, const int8_t *pa, const int8_t
         hipLaunchKernelGGL((split_i8_packed_kernel<4, 4, EPI>), grid, dim3(256), 0, ctx->stream, pa, pw, M, N, K, ep);
     else if (KB <= 32)
         hipLaunchKernelGGL((split_i8_packed_kernel<8, 4, EPI>), grid, dim3(512), 0, ctx->stream, pa, pw, M, N, K, ep);
+    else if (((KB + 15) / 16 + 7) % 8 < 4)
+        // Four stages where eight would multiply zeros in half of a round or more (5 to 8 steps fill it), us, eight / four:
+        // 8 x 3392 x 1344 5.0 / 4.0, 16 x 2496 x 1792 5.1 / 4.1, 2 x 680 x 1664 4.1 / 3.6.
+        hipLaunchKernelGGL((split_i8_packed_kernel<16, 4, EPI>), grid, dim3(1024), 0, ctx->stream, pa, pw, M, N, K, ep);
     else
         hipLaunchKernelGGL((split_i8_packed_kernel<16, 8, EPI>), grid, dim3(1024), 0, ctx->stream, pa, pw, M, N, K, ep);
     return check_launch("gemm_i8 (packed, split)");
