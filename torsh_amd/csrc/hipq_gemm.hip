@@ -322,6 +322,22 @@ static int32_t launch_gemm(hipq_ctx *ctx, const int8_t *a, const int8_t *w, size
     // of a thread per output, us: M = 300, N = 1000, K = 1001 1206 -> 11; 1 x 11008 x 4001 19, 64 x 4096 x 4097 26,
     // 512 x 4096 x 4097 43.
     if (!fast) variant = M <= 16 ? 0 : 10;
+    // Short K (on whole, aligned pieces), where a product is little more than its launch and its stores.  Int32 results leave the register-staged tile
+    // straight from the accumulators; us, K-split or pipelined kernel / register-staged: 8 x 4870 x 16 3.0 / 2.6, 5 x 2119 x
+    // 80 2.9 / 2.6, but 4 x 2142 x 144 2.9 / 3.1; 32 x 960 x 80 4.0 / 2.7, 64 x 1408 x 176 4.3 / 3.5, 152 x 576 x 304 5.1 /
+    // 4.7, 1122 x 99 x 576 6.4 / 6.2, 57 x 2114 x 544 6.1 / 6.4, 2267 x 1268 x 16 8.7 / 6.2, 616 x 6464 x 352 10.7 / 10.0;
+    // with rows that are no whole number of 16 bytes it is the number of tiles that decides (50 of them 4.7 / 3.8, 110 5.0 /
+    // 5.3, 190 5.6 / 7.5), and many tiles are better not persistent: 1625 x 3159 x 48 14.8 / 13.4, 8108 x 1562 x 128 35 / 26,
+    // 7350 x 4037 x 48 93 / 71 (persistent / pipelined).  Int8 results of a few tiles of such rows: 95 x 310 x 16 7.4 / 7.0,
+    // 5073 x 37 x 80 8.0 / 6.8, 1040 x 330 x 160 9.1 / 8.2, but 21 x 961 x 16 6.3 / 6.6, 57 x 2114 x 544 8.9 / 10.0; of whole
+    // dwords 104 x 932 x 96 5.6 / 6.4.  Fp32 results: never.
+    if (variant == 0 && EPI == EPI_I32 && K <= (M <= 16 ? 128 : 512)) {
+        if (M <= 16 || (tiles(128, 64) < 2 * cus && (N % 4 == 0 || tiles(128, 64) <= cus / 4)))
+            variant = 10;
+        else if (N % 4 != 0)
+            variant = 2;
+    }
+    if (variant == 0 && EPI == EPI_I8 && K <= 256 && M > 32 && N % 4 != 0 && tiles(128, 64) <= cus / 4) variant = 10;
     if (variant == 0 && M <= 16) {
         if (fast && K % 256 == 0) return launch_gemv<EPI, EVEN>(ctx, a, w, M, N, K, ep);
         hipLaunchKernelGGL((gemv_i8_kernel<1, EPI, EVEN, true>), dim3((N + 15) / 16), dim3(kGemmThreads), 0, ctx->stream, a, w,
@@ -348,7 +364,8 @@ static int32_t launch_gemm(hipq_ctx *ctx, const int8_t *a, const int8_t *w, size
             };
             const bool with_residual = EPI == EPI_F32 && ep.residual;
             const double c5 = cost(128, 64, 900.0, 2700.0), c6 = cost(128, 128, 1350.0, 4700.0);
-            const double c7 = with_residual ? 1e30 : cost(256, 128, 1950.0, 9600.0);
+            // (Int8 results of a short K: 6008 x 1024 x 320 19.9 against 17.0 in tiles of 128 x 64, 8108 x 1562 x 128 34 / 28.)
+            const double c7 = with_residual || (EPI == EPI_I8 && K < 512) ? 1e30 : cost(256, 128, 1950.0, 9600.0);
             // 128x192: between the two in LDS bytes per MAC; divides N = 768 and 2304 into whole rounds.
             const double c8 = with_residual ? 1e30 : cost(128, 192, 1600.0, 7200.0);
             variant = (c7 <= c6 && c7 <= c5 && c7 <= c8) ? 7 : (c8 <= c6 && c8 <= c5 ? 8 : (c6 <= c5 ? 6 : 5));
