@@ -291,8 +291,8 @@ static void launch_tile(hipq_ctx *ctx, const int8_t *a, const int8_t *w, int M, 
     const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
     GemmEpilogue placed = ep;
     pick_xcd_rectangle(tiles_m, tiles_n, BM, BN, &placed.xcd_gm, &placed.xcd_gn);
-    hipLaunchKernelGGL((gemm_i8_mfma_kernel<BM, BN, WM, WN, EPI, EVEN>), dim3(tiles_m * tiles_n), dim3(kGemmThreads), 0,
-                       ctx->stream, a, w, M, N, K, placed);
+    auto kernel = K % 16 ? gemm_i8_mfma_kernel<BM, BN, WM, WN, EPI, EVEN, true> : gemm_i8_mfma_kernel<BM, BN, WM, WN, EPI, EVEN, false>;
+    hipLaunchKernelGGL(kernel, dim3(tiles_m * tiles_n), dim3(kGemmThreads), 0, ctx->stream, a, w, M, N, K, placed);
 }
 
 // Tuning and test hook, per context: HIPQ_GEMM_VARIANT=<n> in the environment (read when the context is

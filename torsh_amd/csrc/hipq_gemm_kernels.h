@@ -212,8 +212,9 @@ __device__ __forceinline__ v4i load_row_piece(const int8_t *row, int k, int K) {
 }
 
 // BM x BN output tile per workgroup, BK = 128 bytes of K per stage, WM x WN
-// waves each owning a (BM/WM) x (BN/WN) sub-tile.  Operands of any alignment and any K >= 16.
-template <int BM, int BN, int WM, int WN, int EPI, bool EVEN>
+// waves each owning a (BM/WM) x (BN/WN) sub-tile.  Operands of any alignment and any K >= 16; RAGGED: K is no multiple of
+// 16, so that a piece may cross the end of a row.
+template <int BM, int BN, int WM, int WN, int EPI, bool EVEN, bool RAGGED>
 __global__ __launch_bounds__(kGemmThreads) void gemm_i8_mfma_kernel(const int8_t *__restrict__ A,
                                                                      const int8_t *__restrict__ W, int M, int N,
                                                                      int K, GemmEpilogue ep) {
@@ -263,10 +264,10 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_i8_mfma_kernel(const int8_t
         }
     };
     auto load_global = [&](int k0) {
-        if (k0 + BK > K && K % 16 != 0)  // (else a piece lies inside the row or past it)
-            load_pieces(k0, std::true_type{});
-        else
-            load_pieces(k0, std::false_type{});
+        if constexpr (RAGGED) {
+            if (k0 + BK > K) return load_pieces(k0, std::true_type{});
+        }
+        load_pieces(k0, std::false_type{});
     };
     auto store_lds = [&](int stage) {
         int8_t *sa = lds + stage * STAGE;
