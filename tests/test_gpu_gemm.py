@@ -468,3 +468,11 @@ def test_every_gemm_kernel_form_on_short_k_and_tails(ctx, oracle, variant):
                 _check_every_epilogue(ctx, oracle, m, n, k)
     finally:
         ctx.set_gemm_kernel_variant(0)
+
+
+@pytest.mark.parametrize("m,n,k", [(16, 24, 128), (16, 24, 144), (9, 33, 16), (17, 40, 512), (17, 40, 528), (40, 45, 256), (40, 45, 272),
+                                   (33, 7000, 64), (129, 8190, 48), (8200, 518, 112), (600, 7100, 2048)])
+def test_shapes_beside_the_dispatch_lines(ctx, oracle, m, n, k):
+    """Both sides of the lines between the K-split, the register-staged, the pipelined and the persistent kernel at short K
+    and rows of odd length, and long K with a residual on many tiles."""
+    _check_every_epilogue(ctx, oracle, m, n, k)

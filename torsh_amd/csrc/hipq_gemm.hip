@@ -369,6 +369,11 @@ static int32_t launch_gemm(hipq_ctx *ctx, const int8_t *a, const int8_t *w, size
             // 128x192: between the two in LDS bytes per MAC; divides N = 768 and 2304 into whole rounds.
             const double c8 = with_residual ? 1e30 : cost(128, 192, 1600.0, 7200.0);
             variant = (c7 <= c6 && c7 <= c5 && c7 <= c8) ? 7 : (c8 <= c6 && c8 <= c5 ? 8 : (c6 <= c5 ? 6 : 5));
+            // Long K with a residual, where the 128 x 64 tiles fill their rounds best: a workgroup per tile, us, persistent /
+            // pipelined: 922 x 4136 x 6992 132 / 98, 726 x 5760 x 4864 85 / 62, 4467 x 939 x 3392 68 / 58, 1281 x 3904 x
+            // 2176 37.4 / 34.3, 4110 x 1280 x 2048 40.3 / 39.7, but 2228 x 2048 x 1664 29.3 / 29.3, 1370 x 4416 x 1280
+            // 28.6 / 28.9, 3475 x 1664 x 640 15.4 / 20.6.
+            if (with_residual && variant == 5 && K >= 2048) variant = 2;
         }
     }
     switch (variant) {
