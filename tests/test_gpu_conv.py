@@ -386,3 +386,38 @@ def test_conv_with_a_stride_captured_by_a_new_context(hipq, oracle):
         finally:
             torch.cuda.synchronize()
             c.close()
+
+
+@pytest.mark.parametrize("s_w,s_out,zp_out", [
+    (1e-3, 0.005, 0), (1e-3, 0.005, -128), (1e-3, 0.05, 127),                      # most outputs saturate, on either side
+    (0.5, 1.0, 3), (0.25, 1.0, -7), (0.5, 32.0, 0), (1.0, 2.0, 1),                 # quotients on ties
+    (1e-3, 0.5, 32000), (1e-3, 0.5, -32000), (1e-3, 0.5, 32001), (1e-3, 0.5, -32001), (1e-3, 0.5, 100000),
+    (0.015625, 1.0, 32050), (0.25, 1.0, -31950),                                   # zero points that the quotient cancels
+    (1e25, 1e-6, 0), (1e30, 1e-8, 5), (float("inf"), 1.0, 9),                      # quotients that overflow; NaN where acc is 0
+    (1e-3, 1e-39, 0), (1e-3, 3e38, 2), (0.0, 1.0, -1),                             # no usable reciprocal; all quotients 0
+])
+def test_conv_requantize_at_its_limits(ctx, hipq, oracle, s_w, s_out, zp_out):
+    """The requantize of the window kernel where its one multiply-add is not enough: saturation, ties, zero points past the
+    range of the packed clamp, scales without a finite quotient; few windows (K split) and many, both roundings."""
+    rng = np.random.default_rng(4)
+    for nb, c, h, w, oc, k in ((2, 3, 9, 11, 40, 3), (2, 32, 6, 5, 70, 3), (3, 4, 90, 80, 20, 2), (6, 2, 60, 58, 130, 1)):
+        x = rng.integers(0, 256, size=(nb, c, h, w), dtype=np.uint8)
+        wq = rng.integers(-3, 4, size=(oc, c, k, k), dtype=np.int8)
+        sw = np.full(oc, s_w, np.float32)
+        sw[oc // 2:] *= np.float32(0.5)
+        acc = oracle.backend_conv2d_i32(x, 128, wq, (1, 1), (0, 0)).reshape(nb * oc, -1)
+        xd, wd, swd = dev(x), dev(wq), dev(sw)
+        for mode, rm in ((hipq.ROUND_HALF_AWAY, 0), (hipq.ROUND_HALF_EVEN, 1)):
+            for bias in (None, np.where(np.arange(oc) % 3, np.float32(0.5), np.float32(-2.25)).astype(np.float32)):
+                oracle.set_round_mode(rm)
+                try:
+                    want = oracle.requantize_epilogue(acc, 1.0, sw, bias, s_out, zp_out, channel_axis_is_row=True, inner=oc)
+                finally:
+                    oracle.set_round_mode(0)
+                bd = None if bias is None else dev(bias)
+                got = host(ctx.conv2d_i8(xd, 128, 1.0, wd, swd, bd, s_out, zp_out, (1, 1), (0, 0), mode))
+                np.testing.assert_array_equal(got.reshape(acc.shape), want)
+                if c % 32 == 0:
+                    packed, sums = ctx.conv2d_pack_weights(wd)
+                    got = host(ctx.conv2d_i8_packed(xd, 128, 1.0, packed, sums, (k, k), swd, bd, s_out, zp_out, (0, 0), mode))
+                    np.testing.assert_array_equal(got.reshape(acc.shape), want)

@@ -76,7 +76,7 @@ __device__ __forceinline__ void conv_store_block(v16i (&own)[1][TNB], const Gemm
                     const float q0 = v * ep.s_out_inv;  // div_rn with a usable reciprocal
                     const float rem = fmaf(-q0, ep.s_out, v);
                     const float q1 = fmaf(rem, ep.s_out_inv, q0);
-                    q = (rem == rem) ? q1 : q0;
+                    q = (q1 == q1) ? q1 : q0;
                 } else {
                     q = v / ep.s_out;
                 }

@@ -74,8 +74,8 @@ __device__ __forceinline__ int f32_as_i32(float v) {
 // exponents x 3007 denominators (5.5e11 quotients) found no difference from a / b.  A division by
 // one scale for a whole row or tensor then costs 3-4 instructions per element instead of the
 // ~12 of the IEEE sequence.  y == 0 selects the plain division (recip_for_div returns 0 when
-// 1/b is not normal); a NaN remainder (a or q0 infinite, or NaN input) means q0 already is the
-// quotient.
+// 1/b is not normal); a NaN correction (a infinite, a quotient that overflows, NaN input) means q0
+// already is the quotient.
 __device__ __forceinline__ float recip_for_div(float b) {
     const float y = 1.0f / b;
     return (fabsf(y) >= FLT_MIN && fabsf(y) <= FLT_MAX) ? y : 0.0f;
@@ -85,7 +85,7 @@ __device__ __forceinline__ float div_rn(float a, float b, float y) {
     const float q0 = a * y;
     const float r = fmaf(-q0, b, a);
     const float q1 = fmaf(r, y, q0);
-    return (r == r) ? q1 : q0;
+    return (q1 == q1) ? q1 : q0;
 }
 
 // The reference's "quantize one value" formulas differ in where the zero point enters:
