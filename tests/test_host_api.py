@@ -104,6 +104,18 @@ def test_three_instruction_round_half_away_equals_roundf():
     assert "0 mismatches" in proc.stdout
 
 
+def test_one_multiply_add_requantize_equals_the_exact_chain():
+    """The convolution kernels' requantize in one fused multiply-add, and their division by multiply-high: no value that
+    they accept may differ from the exact chain (hipq_math.h), compared on the CPU."""
+    _binary()
+    exe = os.path.join(ROOT, "tests", "host", "bin", "requant_fast_check")
+    if not os.path.exists(exe):
+        subprocess.run(["make", "-C", os.path.join(ROOT, "tests", "host"), "bin/requant_fast_check"], check=True,
+                       capture_output=True)
+    proc = subprocess.run([exe], capture_output=True, text=True, timeout=600)
+    assert proc.returncode == 0, proc.stdout + proc.stderr
+
+
 def _run(args):
     proc = subprocess.run([_binary(), *args], capture_output=True, text=True, timeout=300)
     results = {}
