@@ -233,7 +233,7 @@ static int32_t launch_conv_window(hipq_ctx *ctx, const int8_t *filters, const in
     // [4,32,46,46] x 512 12.5 / 15.5 (532), [30,128,28,28] x 256 12.2 / 16.6 (736), [25,128,40,40] x 512 21 / 43 (2500).
     const size_t tiles = (size_t(cw.N) + 63) / 64 * ((size_t(cw.M) + 127) / 128), cus = size_t(ctx->num_cus);
     if (tiles >= cus * 8 || (cw.kblocks < 8 && tiles > cus)) {
-        if (cw.M <= 32) return launch_conv_window_form<1, 4, 3, false, EPI, EVEN>(ctx, filters, image, cw, ep);
+        if (cw.M <= 32) return launch_conv_window_form<1, 4, 2, false, EPI, EVEN>(ctx, filters, image, cw, ep);
         if (cw.M <= 64) return launch_conv_window_form<2, 2, 4, false, EPI, EVEN>(ctx, filters, image, cw, ep);
         return launch_conv_window_form<4, 2, 2, false, EPI, EVEN>(ctx, filters, image, cw, ep);
     }
