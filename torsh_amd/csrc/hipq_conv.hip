@@ -315,8 +315,19 @@ static int32_t conv_forward(const char *fn, hipq_ctx *ctx, const uint8_t *x, int
     // measured no faster than the two launches below on the shape it was built for (13.3 against 13.4 us at
     // [32, 256, 14, 14] x [256, 256, 3, 3]: the gather costs what the layout launch did, and the window fragments
     // leave LDS no faster than they leave the L2), so it runs only under test hook 14.
-    if (wpacked && !dyn.x && ctx->gemm_variant == 14 && elems < (size_t(1) << 31) && !(reinterpret_cast<uintptr_t>(x) & 3u) &&
-        conv_patch_applicable(g.nb, g.c, g.h, g.w, cw.hp, cw.wp, g.kh, g.kw)) {
+    if (!dyn.x && ctx->gemm_variant == 14 && g.sh == 1 && g.sw == 1 && elems < (size_t(1) << 31) &&
+        !(reinterpret_cast<uintptr_t>(x) & 3u) && conv_patch_applicable(g.nb, g.c, g.h, g.w, cw.hp, cw.wp, g.kh, g.kw)) {
+        if (!wpacked) {
+            const size_t bytes = packed_operand_bytes(g.oc, k), rows = align256(size_t(g.oc) * k);
+            void *s = nullptr;
+            int32_t rc = scratch(ctx, kScratchHeader + rows + align256(bytes) + align256(size_t(g.oc) * 4), &s);
+            if (rc) return rc;
+            int8_t *staging = reinterpret_cast<int8_t *>(static_cast<char *>(s) + kScratchHeader), *packed = staging + rows;
+            int32_t *sums = reinterpret_cast<int32_t *>(packed + align256(bytes));
+            if ((rc = pack_filters(ctx, w, g.oc, g.c, taps, staging, packed, sums))) return rc;
+            wpacked = packed;
+            wsum = sums;
+        }
         ep.cv_kw = g.kw;
         ep.cv_wp = cw.wp;
         ep.cv_hp = cw.hp;
