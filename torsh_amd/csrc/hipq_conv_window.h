@@ -17,13 +17,13 @@
 // sum (x - zp) w = sum (x - 128) w + (128 - zp) sum w is undone per output channel in the epilogue.
 //
 // Measured against what it replaced, u8 in, filters as rows (us per forward): [32,3,224,224] x [64,3,7,7] stride 2
-// 2288 -> 27 (a thread per output); [32,64,56,56] x [64,64,3,3] 63 -> 24, [32,128,28,28] x [128,128,3,3] 26.4 -> 20.4,
-// [32,256,14,14] x [256,256,3,3] 20.9 -> 17.5, [32,512,7,7] x [512,512,3,3] 28.0 -> 25.9, [32,256,56,56] x [64,256,1,1] 50 -> 33
+// 2288 -> 25.5 (a thread per output); [32,64,56,56] x [64,64,3,3] 63 -> 20, [32,128,28,28] x [128,128,3,3] 26.4 -> 17.6,
+// [32,256,14,14] x [256,256,3,3] 20.9 -> 16.2, [32,512,7,7] x [512,512,3,3] 28.0 -> 23.5, [32,256,56,56] x [64,256,1,1] 50 -> 22
 // (the packed GEMM over the padded grid, which always split K: its 128 x 64 tiles spend more on the sum of the partial
 // products than on short K, compute the windows of the border, and store single bytes).  What bounds it now: at long K
-// the vector-memory path, 6 KiB per 8 MFMAs; at short K (the first layer) instruction issue, ~1100 vector instructions
-// per wave of which 700 are the requantize of its 64 x 64 outputs, and the misaligned 16-byte pieces (34 L1 accesses
-// per load of overlapping windows, 16 where they are a contiguous KiB).
+// the vector-memory path, 6 KiB per 8 MFMAs; at short K (the first layer) instruction issue, 815 vector instructions per wave
+// of which most are the requantize of its 64 x 64 outputs, and the misaligned 16-byte pieces (21.7 L1 accesses per load on
+// average, 16 where they are a contiguous KiB).
 //
 // Waves.  A workgroup's four waves either take different windows (SPLIT = false: FM x FN accumulator blocks each, the
 // filters' fragments coming out of L1 for three of the four) or split K and sum through LDS (SPLIT = true), which keeps

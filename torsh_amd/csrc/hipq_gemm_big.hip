@@ -12,7 +12,7 @@
 // LDS, 256 registers a wave), so one converts and stores while the other multiplies.
 // Measured, fp32 out, us against the 128 x 64 tiles: 4096 x 11008 x 4096 270 -> 174 (2.1 POP/s), 8192^3 755 -> 450 (2.44),
 // 8192 x 3072 x 768 37 -> 31, 2048 x 4096 x 4096 43 -> 38, 256 x 32000 x 4096 49 -> 41.  What bounds it: power.  The matrix
-// pipes are busy 73 % of the cycles at 1.49 GHz; 256 x 256 tiles (256 accumulator registers a wave, one wave per SIMD: 58 %
+// pipes are busy 71 % of the cycles at 1.62 GHz; 256 x 256 tiles (256 accumulator registers a wave, one wave per SIMD: 58 %
 // of the cycles at 1.82 GHz; eight waves of 128 x 64 outputs) deliver the same 2.35-2.5 POP/s at 8192^3, and no more than
 // these at 4096 x 11008 x 4096, where their 688 tiles leave the last of three rounds two thirds full.
 //
