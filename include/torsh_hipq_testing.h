@@ -16,13 +16,14 @@ extern "C" {
 #endif
 
 /* Forces one of the GEMM kernel forms for every later call on this context wherever the shape
- * allows it (0 = automatic choice, the default; 1-3 one-tile-per-workgroup forms, 5-8 persistent
- * forms, 10 register-staged form); 6 also makes the dynamic per-tensor activation quantizer of the
+ * allows it (0 = automatic choice, the default; 1-3 one-tile-per-workgroup forms, 4 K split
+ * between the waves of small tiles, 5-8 persistent forms, 10 register-staged form); 6 also makes the dynamic per-tensor activation quantizer of the
  * Linear forwards run as two launches (range partials, then a quantizer that folds them) where it
  * would run as one, and the per-token forward of one or two rows as a quantizer and a product where
- * it would be one kernel; 9 and 11 leave the choice automatic and switch off, on prepared operands,
- * the forms of the GEMM that are picked by occupancy - two workgroups per compute unit, K split between the waves of few blocks, the
- * weight-streaming kernel for 33..128 rows - (9) and the touching of weight / filter lines by the
+ * it would be one kernel; 9 and 11 leave the choice automatic and switch off
+ * the forms of the GEMM that are picked by occupancy - on prepared operands two workgroups per compute unit, K split between
+ * the waves of few blocks, the weight-streaming kernel for 33..128 rows, on row-major operands of more than 16 rows K split
+ * between the waves of few tiles - (9) and the touching of weight / filter lines by the
  * one-launch activation quantizers of the dynamic Linear and Conv2d forwards while their grids wait
  * for the range (11); on prepared operands 7 and 8 force the tiles of 256 x 128 and 128 x 256 that are
  * staged through LDS; 12 runs shapes of whole 128 x 128 tiles that fill the device once as one tile

@@ -476,3 +476,39 @@ def test_shapes_beside_the_dispatch_lines(ctx, oracle, m, n, k):
     """Both sides of the lines between the K-split, the register-staged, the pipelined and the persistent kernel at short K
     and rows of odd length, and long K with a residual on many tiles."""
     _check_every_epilogue(ctx, oracle, m, n, k)
+
+
+def _at(a, shift):
+    """A device copy of `a` whose first byte lies `shift` bytes behind a 16-byte boundary."""
+    buf = torch.empty(a.size + 32, dtype=torch.int8, device="cuda")
+    start = -buf.data_ptr() % 16 + shift
+    out = buf[start:start + a.size].view(a.shape)
+    out.copy_(torch.from_numpy(a))
+    return out
+
+
+# one shape for each tile of the K-split form, rows and columns that no tile divides; K below, at and beside a step of 128
+# bytes and a round of all waves (1024 / 512 bytes), and of no step at all
+@pytest.mark.parametrize("m,n", [(7, 33), (41, 1702), (99, 1301), (201, 1503), (497, 1500)])
+@pytest.mark.parametrize("k,shift_a,shift_w", [(16, 0, 0), (17, 1, 3), (64, 4, 0), (79, 0, 2), (128, 0, 0), (131, 2, 1), (512, 0, 4),
+                                               (513, 3, 0), (1001, 0, 0), (1024, 1, 1), (1100, 0, 0)])
+def test_few_tiles_with_k_split_between_the_waves(ctx, oracle, m, n, k, shift_a, shift_w):
+    rng = np.random.default_rng(m + n + k)
+    a, w = rand_i8(rng, (m, k)), rand_i8(rng, (n, k))
+    acc = oracle.gemm_i8_nk(a, w)
+    sa = (rng.random(m) * 0.05 + 0.001).astype(np.float32)
+    sw = (rng.random(n) * 0.002 + 0.0001).astype(np.float32)
+    bias = (rng.standard_normal(n) * 0.01).astype(np.float32)
+    res = rng.standard_normal((m, n)).astype(np.float32)
+    want = oracle.linear_dequant_epilogue(acc, sa, sw, bias)
+    s_out, _ = oracle.calculate_symmetric_params(*oracle.find_min_max(want), 0)
+    wantq = oracle.requantize_epilogue(acc, sa, sw, bias, s_out, -5)
+    ad, wd, sad, swd, bd = _at(a, shift_a), _at(w, shift_w), dev(sa), dev(sw), dev(bias)
+    try:
+        ctx.set_gemm_kernel_variant(4)
+        np.testing.assert_array_equal(host(ctx.gemm_i8_i32(ad, wd)), acc)
+        np.testing.assert_array_equal(host(ctx.linear_i8_f32(ad, sad, wd, swd, bd)), want)
+        np.testing.assert_array_equal(host(ctx.linear_i8_f32_residual(ad, sad, wd, swd, bd, dev(res))), want + res)
+        np.testing.assert_array_equal(host(ctx.linear_i8_i8(ad, sad, wd, swd, bd, s_out, -5)), wantq)
+    finally:
+        ctx.set_gemm_kernel_variant(0)

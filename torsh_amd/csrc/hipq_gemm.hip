@@ -12,6 +12,7 @@
 
 #include "hipq_gemm_kernels.h"
 #include "hipq_gemm_persist.h"
+#include "hipq_gemm_split.h"
 
 namespace hipq {
 
@@ -79,8 +80,8 @@ __device__ __forceinline__ void gemv_store(const GemmEpilogue &ep, v4i sum, int 
 // MFMAs then run off registers while the next batch is already in flight.  The
 // four partial 16x16 accumulators are summed through LDS (integer adds: order
 // independent).
-// ANYK: operands of any alignment and any K >= 16, the steps dealt to the waves in four runs.
-template <int G, int EPI, bool EVEN, bool ANYK = false>
+// K % 256 == 0.
+template <int G, int EPI, bool EVEN>
 __global__ __launch_bounds__(kGemmThreads) void gemv_i8_kernel(const int8_t *__restrict__ A,
                                                                const int8_t *__restrict__ W, int M, int N, int K,
                                                                GemmEpilogue ep) {
@@ -90,9 +91,8 @@ __global__ __launch_bounds__(kGemmThreads) void gemv_i8_kernel(const int8_t *__r
     const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
     const int n0 = blockIdx.x * (16 * G);
     const int frow = lane % 16, g = lane / 16;
-    const int per = ANYK ? ((K + 63) / 64 + NW - 1) / NW * 64 : K / NW;  // bytes of K per wave, a multiple of 64
-    const int kbeg = wave * per;
-    const int kw = ANYK ? (K - kbeg < per ? K - kbeg : per) : per;  // (ANYK: the last waves' runs may be short or empty)
+    const int kw = K / NW;  // bytes of K per wave, a multiple of 64
+    const int kbeg = wave * kw;
     const int mrow = frow < M ? frow : M - 1;
     const int8_t *ap = A + size_t(mrow) * K + kbeg + g * 16;
     const int8_t *wp[G];
@@ -119,23 +119,17 @@ __global__ __launch_bounds__(kGemmThreads) void gemv_i8_kernel(const int8_t *__r
     v4i acc[G];
 #pragma unroll
     for (int r = 0; r < G; ++r) acc[r] = v4i{0, 0, 0, 0};
-    auto piece = [&](const int8_t *row, int k) {  // k: bytes from kbeg + g * 16
-        if constexpr (ANYK) {
-            if (kbeg + k + 64 > K) return load_row_piece<true>(row, kbeg + k + g * 16, K);
-        }
-        return load_row_piece<false>(row, kbeg + k + g * 16, K);
-    };
     for (int k0 = 0; k0 < kw; k0 += BATCH * 64) {
         v4i fa[BATCH];
 #pragma unroll
         for (int u = 0; u < BATCH; ++u)
-            if (k0 + u * 64 < kw) fa[u] = piece(ap - kbeg - g * 16, k0 + u * 64);
+            if (k0 + u * 64 < kw) fa[u] = *reinterpret_cast<const v4i *>(ap + k0 + u * 64);
 #pragma unroll
         for (int r = 0; r < G; ++r) {
             v4i fw[BATCH];
 #pragma unroll
             for (int u = 0; u < BATCH; ++u)
-                if (k0 + u * 64 < kw) fw[u] = piece(wp[r] - kbeg - g * 16, k0 + u * 64);
+                if (k0 + u * 64 < kw) fw[u] = *reinterpret_cast<const v4i *>(wp[r] + k0 + u * 64);
 #pragma unroll
             for (int u = 0; u < BATCH; ++u)
                 if (k0 + u * 64 < kw) acc[r] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fw[u], fa[u], acc[r], 0, 0, 0);
@@ -300,6 +294,23 @@ static void launch_tile(hipq_ctx *ctx, const int8_t *a, const int8_t *w, int M, 
 // allows it (0 = automatic).
 static int gemm_variant_override(hipq_ctx *ctx) { return ctx->gemm_variant; }
 
+// The tile of the K-split form (hipq_gemm_split.h).  Its time is the operand bytes a compute unit asks for: 16 (FM + FN)
+// per byte of K and workgroup (`blocks` = FM + FN), times the workgroups a compute unit gets (`cost`).
+struct SplitForm {
+    int blocks;
+    size_t cost;
+};
+template <class Tiles>
+static SplitForm pick_split_form(const Tiles &tiles, size_t cus) {
+    const SplitForm forms[] = {{2, tiles(16, 16)}, {3, tiles(16, 32)}, {4, tiles(32, 32)}, {6, tiles(64, 32)}, {8, tiles(64, 64)}};
+    SplitForm best{0, 0};
+    for (const SplitForm &f : forms) {
+        const size_t cost = size_t(f.blocks) * ((f.cost + cus - 1) / cus);
+        if (best.blocks == 0 || cost < best.cost) best = SplitForm{f.blocks, cost};
+    }
+    return best;
+}
+
 template <int EPI, bool EVEN>
 static int32_t launch_gemm(hipq_ctx *ctx, const int8_t *a, const int8_t *w, size_t m, size_t n, size_t k,
                            const GemmEpilogue &ep) {
@@ -318,32 +329,44 @@ static int32_t launch_gemm(hipq_ctx *ctx, const int8_t *a, const int8_t *w, size
     auto tiles = [&](size_t bm, size_t bn) { return ((m + bm - 1) / bm) * ((n + bn - 1) / bn); };
     int variant = gemm_variant_override(ctx);
     if (variant == 9 || variant == 11) variant = 0;  // switches of the packed forms only
-    // Rows at any alignment (load_row_piece): up to 16 of them the K-split kernel, else the register-staged tile.  Instead
-    // of a thread per output, us: M = 300, N = 1000, K = 1001 1206 -> 11; 1 x 11008 x 4001 19, 64 x 4096 x 4097 26,
-    // 512 x 4096 x 4097 43.
-    if (!fast) variant = M <= 16 ? 0 : 10;
-    // Short K (on whole, aligned pieces), where a product is little more than its launch and its stores.  Int32 results leave the register-staged tile
-    // straight from the accumulators; us, K-split or pipelined kernel / register-staged: 8 x 4870 x 16 3.0 / 2.6, 5 x 2119 x
-    // 80 2.9 / 2.6, but 4 x 2142 x 144 2.9 / 3.1; 32 x 960 x 80 4.0 / 2.7, 64 x 1408 x 176 4.3 / 3.5, 152 x 576 x 304 5.1 /
-    // 4.7, 1122 x 99 x 576 6.4 / 6.2, 57 x 2114 x 544 6.1 / 6.4, 2267 x 1268 x 16 8.7 / 6.2, 616 x 6464 x 352 10.7 / 10.0;
-    // with rows that are no whole number of 16 bytes it is the number of tiles that decides (50 of them 4.7 / 3.8, 110 5.0 /
-    // 5.3, 190 5.6 / 7.5), and many tiles are better not persistent: 1625 x 3159 x 48 14.8 / 13.4, 8108 x 1562 x 128 35 / 26,
-    // 7350 x 4037 x 48 93 / 71 (persistent / pipelined).  Int8 results of a few tiles of such rows: 95 x 310 x 16 7.4 / 7.0,
-    // 5073 x 37 x 80 8.0 / 6.8, 1040 x 330 x 160 9.1 / 8.2, but 21 x 961 x 16 6.3 / 6.6, 57 x 2114 x 544 8.9 / 10.0; of whole
-    // dwords 104 x 932 x 96 5.6 / 6.4.  Fp32 results: never.
-    if (variant == 0 && EPI == EPI_I32 && K <= (M <= 16 ? 128 : 512)) {
-        if (M <= 16 || (tiles(128, 64) < 2 * cus && (N % 4 == 0 || tiles(128, 64) <= cus / 4)))
+    // Rows at any alignment: the K-split form while its tiles are few, else the register-staged tile (load_row_piece).
+    if (!fast) variant = variant == 4 || M <= 16 ? 4 : 10;
+    // Few tiles: the K-split form, whose time grows with `cost` (pick_split_form) and K where the tiled kernels walk a chain
+    // of K-tiles.  us, register-staged / split, rows of any length: 300 x 1000 x 1001 11.7 / 6.6, 64 x 4096 x 4097 26.0 /
+    // 12.7, 19 x 101 x 245 6.9 / 3.4, 1129 x 128 x 3388 18.6 / 7.5, 2000 x 300 x 3001 20.7 / 16.6, at a cost of 16 512 x 4096 x
+    // 4097 44.6 / 44.1.  Whole, aligned pieces, pipelined / split: 128 x 1024 x 1024 7.1 / 4.3, 32 x 4096 x 4096 13.2 / 8.4,
+    // 422 x 158 x 688 7.3 / 3.8; cost 6: 512 x 1024 x 512 6.3 / 5.0, 256 x 2048 x 2048 9.4 / 9.1, 128 x 4096 x 4096 13.1 / 14.8;
+    // cost 8: 1165 x 704 x 208 6.3 / 6.7, 1020 x 899 x 16 6.1 / 7.7, int8 results of odd rows 249 x 3906 x 288 9.8 / 7.7.
+    // Int32 results of one K-tile, which the register-staged tile stores as they are: 439 x 543 x 63 5.2 / 4.1, cost 8: 226 x
+    // 2801 x 68 5.6 / 6.3; whole pieces 59 x 4480 x 112 3.8 / 4.5, 18 x 433 x 16 3.7 / 4.0.
+    if (variant == 0 && M <= 16 && K % 256 == 0) return launch_gemv<EPI, EVEN>(ctx, a, w, M, N, K, ep);
+    // Up to 16 rows always, where they are no multiple of 256 bytes (the sixteen-row kernel without a shift, which it
+    // replaced / split): 1 x 11008 x 4001 20.1 / 10.6, 16 x 4096 x 4032 5.7 / 5.5, 1 x 32000 x 1008 11.9 / 6.9, 8 x 300 x 300
+    // 3.8 / 3.2.
+    if (variant == 0 && M <= 16) variant = 4;
+    if (ctx->gemm_variant == 0 && M > 16) {
+        const size_t cost = pick_split_form(tiles, cus).cost;
+        const bool few_steps = EPI == EPI_I32 && K <= 128;
+        const size_t most = !fast                                       ? (few_steps ? 6 : 10)
+                            : few_steps                                 ? 0
+                            : EPI == EPI_I8 && N % 4 != 0 && K <= 768   ? 8
+                            : K <= 2048                                 ? 6
+                                                                        : 4;
+        if (cost <= most) variant = 4;
+    }
+    // Short K (on whole, aligned pieces) of the tiles that are left, where a product is little more than its launch and its
+    // stores.  Int32 results leave the register-staged tile straight from the accumulators; us, pipelined kernel /
+    // register-staged: 2267 x 1268 x 16 8.7 / 6.2, 616 x 6464 x 352 10.7 / 10.0; with rows that are no whole number of 16
+    // bytes it is the number of tiles that decides (50 of them 4.7 / 3.8, 110 5.0 / 5.3, 190 5.6 / 7.5), and many tiles are
+    // better not persistent: 1625 x 3159 x 48 14.8 / 13.4, 8108 x 1562 x 128 35 / 26, 7350 x 4037 x 48 93 / 71 (persistent /
+    // pipelined).  Int8 results of a few tiles of such rows: 1040 x 330 x 160 9.1 / 8.2.  Fp32 results: never.
+    if (variant == 0 && EPI == EPI_I32 && K <= 512) {
+        if (tiles(128, 64) < 2 * cus && (N % 4 == 0 || tiles(128, 64) <= cus / 4))
             variant = 10;
         else if (N % 4 != 0)
             variant = 2;
     }
     if (variant == 0 && EPI == EPI_I8 && K <= 256 && M > 32 && N % 4 != 0 && tiles(128, 64) <= cus / 4) variant = 10;
-    if (variant == 0 && M <= 16) {
-        if (fast && K % 256 == 0) return launch_gemv<EPI, EVEN>(ctx, a, w, M, N, K, ep);
-        hipLaunchKernelGGL((gemv_i8_kernel<1, EPI, EVEN, true>), dim3((N + 15) / 16), dim3(kGemmThreads), 0, ctx->stream, a, w,
-                           M, N, K, ep);
-        return check_launch("gemv_i8 (any K)");
-    }
     // The LDS-pipelined kernels for every K that is a multiple of 16 (a last K-tile that runs over the rows is filled
     // with zeros).  Against the register-staged tile, us: 512 x 4096 x 4112 37 / 20, 300 x 1000 x 1008 14.6 / 7.6,
     // 8192 x 3072 x 320 73 / 29, x 64 66 / 25, 100 x 1408 x 192 10.5 / 6.1, 50 x 300 x 64 6.0 / 5.7.
@@ -388,6 +411,15 @@ static int32_t launch_gemm(hipq_ctx *ctx, const int8_t *a, const int8_t *w, size
     case 8:
         if (!(EPI == EPI_F32 && ep.residual)) return launch_persist<128, 192, 3, 4, 2, 2, 1, EPI, EVEN>(ctx, a, w, M, N, K, ep);
         return launch_persist<128, 128, 4, 4, 2, 2, 2, EPI, EVEN>(ctx, a, w, M, N, K, ep);
+    case 4:
+        if (M > 16 * 65535) break;  // (row tiles are the grid's y)
+        switch (pick_split_form(tiles, cus).blocks) {
+        case 2: return launch_split_rows<1, 1, 8, 1, 2, EPI, EVEN>(ctx, a, w, M, N, K, ep);
+        case 3: return launch_split_rows<1, 2, 8, 1, 2, EPI, EVEN>(ctx, a, w, M, N, K, ep);
+        case 4: return launch_split_rows<2, 2, 4, 1, 2, EPI, EVEN>(ctx, a, w, M, N, K, ep);
+        case 6: return launch_split_rows<4, 2, 4, 1, 2, EPI, EVEN>(ctx, a, w, M, N, K, ep);
+        default: return launch_split_rows<4, 4, 4, 1, 2, EPI, EVEN>(ctx, a, w, M, N, K, ep);
+        }
     default: break;
     }
     // Register-staged kernel: any K from 16 on, any alignment.
