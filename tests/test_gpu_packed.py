@@ -200,6 +200,30 @@ def test_quantize_per_row_packed_matches_row_major(ctx, hipq, rows, cols):
         assert torch.equal(ps, s)
 
 
+@pytest.mark.parametrize("rows,cols", [(1, 1), (35, 1023), (550, 1024), (70, 1025), (513, 2048), (33, 2049), (530, 4096),
+                                       (2300, 4001), (33, 4097), (1100, 8190), (31, 8193), (1, 16384), (600, 16130), (2, 16385)])
+def test_quantize_per_row_packed_forms(ctx, hipq, rows, cols):
+    """Every form of the packed per-row quantizer (by row length, and by whether the device holds the matrix at once) on
+    rows that start at an odd float, with NaN elements and a row with an infinity: the codes and scales of the row-major
+    quantizer on an aligned copy; the row without a range has a NaN scale and zero codes; the padding is zeros."""
+    g = torch.Generator(device="cuda").manual_seed(rows * 17 + cols)
+    x = torch.randn(rows * cols + 1, generator=g, device="cuda")[1:].view(rows, cols)
+    x[rows // 2, cols // 2] = 30.0
+    if rows > 1:
+        x[rows // 3, :: max(2, cols // 5)] = float("nan")
+        x[rows // 3, 0] = 3.0
+        x[rows - 1, cols - 1] = float("inf")
+    for mode in (0, hipq.ROUND_HALF_EVEN):
+        q, s, _, _ = ctx.quantize_per_row(x.clone(), mode=mode)
+        if rows > 1:
+            q[rows - 1], s[rows - 1] = 0, float("nan")
+        dirty = torch.full((ctx.packed_size(rows, cols),), 77, dtype=torch.int8, device="cuda")
+        pq, ps = ctx.quantize_per_row_packed(x, mode=mode, out=dirty)
+        torch.cuda.synchronize()
+        assert torch.equal(pq, ctx.pack_rows(q))
+        assert torch.equal(torch.nan_to_num(ps, nan=-1.0), torch.nan_to_num(s, nan=-1.0))
+
+
 @pytest.mark.parametrize("m,n,k", [(8192, 768, 768), (4100, 1100, 272)])
 def test_linear_packed_many_tiles_matches_row_major(ctx, hipq, m, n, k):
     """More tiles than compute units (the packed kernel then runs two workgroups per compute unit and sums its K

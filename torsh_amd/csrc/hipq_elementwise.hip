@@ -8,6 +8,7 @@
 #include <type_traits>
 
 #include "hipq_meeting.h"
+#include "hipq_quantize_rows.h"
 
 namespace hipq {
 
@@ -670,8 +671,8 @@ __global__ __launch_bounds__(kBlock) void dequantize_kernel(const InT *__restric
 // across the row with wave shuffles, derive the row's parameters and quantize
 // with the division form.
 //
-// PACKED: the codes go straight into the fragment-packed operand layout of the packed GEMM
-// ([row block of 32][k block of 32 bytes][1 KiB]; lane l of a fragment = row l % 32, bytes 16 * (l / 32) .. +15)
+// PACKED (rows longer than quantize_rows_packed_kernel holds): the codes go straight into the fragment-packed operand layout
+// of the packed GEMM ([row block of 32][k block of 32 bytes][1 KiB]; lane l of a fragment = row l % 32, bytes 16 * (l / 32) .. +15)
 // instead of a dense [rows, cols] matrix, so that a per-token Linear forward needs no packing pass.  The grid
 // then covers the rows up to a multiple of 32, and the padding - rows past the matrix, k past cols up to a
 // multiple of 128 - is written as zeros.
@@ -1693,15 +1694,22 @@ static int32_t quantize_rows(const char *fn, hipq_ctx *ctx, const float *x, size
     HIPQ_REQUIRE_PTR(out);
     const bool even = (mode & HIPQ_ROUND_HALF_EVEN) != 0;
     if (rows >> 31) return fail(HIPQ_INVALID_ARGUMENT, "%s: too many rows", fn);
+    if (packed && cols <= kRowsPackedMaxCols) {
+        if (even)
+            launch_quantize_rows_packed<true>(ctx, x, rows, cols, ld, out, out_scales);
+        else
+            launch_quantize_rows_packed<false>(ctx, x, rows, cols, ld, out, out_scales);
+        return check_launch(fn);
+    }
     // Packed output: the grid also covers the padding rows of the last row block (they are written as zeros).
     const size_t grid_rows = packed ? (rows + 31) / 32 * 32 : rows;
     // A large dense tensor is read and written once: past the caches, as the per-tensor quantizer does it
     // (4096 x 4096: 19.9 -> 17.3 us).  Packed output is an operand of the GEMM that follows: it stays cached.
     const bool stream = !packed && rows * cols >= (size_t(1) << 22);
-#define HIPQ_LAUNCH_ROWS(TPR, E, P, G)                                                                               \
-    hipLaunchKernelGGL((quantize_per_row_kernel<TPR, E, P>), dim3(G), dim3(kBlock), 0, ctx->stream, x, rows, cols, ld, \
+#define HIPQ_LAUNCH_ROWS(TPR, E, G)                                                                                  \
+    hipLaunchKernelGGL((quantize_per_row_kernel<TPR, E>), dim3(G), dim3(kBlock), 0, ctx->stream, x, rows, cols, ld, \
                        flavor, qmin, qmax, out, out_scales, out_zero_points, out_status, poison)
-    if (cols > 4096 && ld % 4 == 0) {
+    if (packed || (cols > 4096 && ld % 4 == 0)) {
         // long rows: four times the registers, so that up to 16384 floats are read once and all requested up front
         const int grid = static_cast<int>(grid_rows);
 #define HIPQ_LAUNCH_LONG_ROWS(E, P)                                                                                   \
@@ -1736,16 +1744,10 @@ static int32_t quantize_rows(const char *fn, hipq_ctx *ctx, const float *x, size
                                out_status, poison);
     } else if (cols > 1024) {
         const int grid = static_cast<int>(grid_rows);
-        if (packed) {
-            if (even)
-                HIPQ_LAUNCH_ROWS(kBlock, true, true, grid);
-            else
-                HIPQ_LAUNCH_ROWS(kBlock, false, true, grid);
-        } else if (even) {
-            HIPQ_LAUNCH_ROWS(kBlock, true, false, grid);
-        } else {
-            HIPQ_LAUNCH_ROWS(kBlock, false, false, grid);
-        }
+        if (even)
+            HIPQ_LAUNCH_ROWS(kBlock, true, grid);
+        else
+            HIPQ_LAUNCH_ROWS(kBlock, false, grid);
     } else if (stream) {
         const int grid = static_cast<int>((grid_rows + 3) / 4);
         if (even)
@@ -1758,16 +1760,10 @@ static int32_t quantize_rows(const char *fn, hipq_ctx *ctx, const float *x, size
                                out_status, poison);
     } else {
         const int grid = static_cast<int>((grid_rows + 3) / 4);
-        if (packed) {
-            if (even)
-                HIPQ_LAUNCH_ROWS(kWave, true, true, grid);
-            else
-                HIPQ_LAUNCH_ROWS(kWave, false, true, grid);
-        } else if (even) {
-            HIPQ_LAUNCH_ROWS(kWave, true, false, grid);
-        } else {
-            HIPQ_LAUNCH_ROWS(kWave, false, false, grid);
-        }
+        if (even)
+            HIPQ_LAUNCH_ROWS(kWave, true, grid);
+        else
+            HIPQ_LAUNCH_ROWS(kWave, false, grid);
     }
 #undef HIPQ_LAUNCH_ROWS
     return check_launch(fn);
