@@ -572,6 +572,33 @@ def test_prepared_stack_few_tokens(hipq, tokens, d, dff, layers):
         c.close()
 
 
+# One and two column blocks per workgroup, the last token count of either and the first past it; a row block's edges.
+@pytest.mark.parametrize("tokens,d,dff", [(15, 768, 768), (17, 640, 3072), (42, 768, 3072), (77, 768, 3072), (81, 768, 3072),
+                                          (84, 384, 1536), (640, 128, 384), (673, 128, 256)])
+def test_prepared_stack_row_operations_in_front_of_the_products(hipq, tokens, d, dff):
+    """Very few tokens on rows of up to 768 floats: the products' workgroups run LayerNorm and the per-token quantizer
+    themselves.  The bits of the row panels, with a token that is not finite beside finite ones."""
+    c = hipq.Context(0)
+    try:
+        g = torch.Generator(device="cuda").manual_seed(tokens + d)
+        prepared = c.stack_prepare(_random_blocks(c, g, d, dff, 2))
+        x0 = torch.randn(tokens, d, generator=g, device="cuda")
+        x0[tokens // 2, d // 3] = float("inf")
+        x0[tokens - 1] *= 1e-30
+        ws = c.stack_workspace_prepared(tokens, d, dff)
+        for mode in (0, hipq.ROUND_HALF_EVEN):
+            got = c.stack_forward(prepared, x0.clone(), dff, ws, mode=mode, prepared=True)
+            c.set_gemm_kernel_variant(15)
+            want = c.stack_forward(prepared, x0.clone(), dff, ws, mode=mode, prepared=True)
+            c.set_gemm_kernel_variant(0)
+            torch.cuda.synchronize()
+            assert not torch.isfinite(got).all()
+            assert torch.equal(torch.nan_to_num(got, nan=-77.0), torch.nan_to_num(want, nan=-77.0)), mode
+    finally:
+        torch.cuda.synchronize()
+        c.close()
+
+
 def test_prepared_stack_few_tokens_layer_norm_vectors_at_any_float(hipq):
     """Gain and offset of every LayerNorm behind a Linear are taken at the alignment of a float, as the row panels take
     them (the first layer's ln1 is the row kernel's: 16 bytes)."""

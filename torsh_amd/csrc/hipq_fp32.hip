@@ -5,6 +5,7 @@
 // a single HBM read per element, wave shuffles for the row statistics.
 #include "hipq_internal.h"
 #include "hipq_math.h"
+#include "hipq_panel_norm.h"
 
 namespace hipq {
 
@@ -348,90 +349,29 @@ static int32_t launch_row_op(const char *fn, hipq_ctx *ctx, const float *x, size
     return check_launch(fn);
 }
 
-// Four floats at an address that is a multiple of four bytes only.
-struct __attribute__((packed, aligned(4))) AnyFloat4 {
-    float x, y, z, w;
-};
-
-// LayerNorm + per-token int8 of whole rows with the bits of the row-panel GEMM's epilogue (hipq_gemm_rows.h): its sums run
-// over a lane's column blocks first, then over the 32 columns of a block (neighbours first), then over the eight waves in
-// pairs, and in the pair form over the two halves of the columns last.  Eight lanes stand for a panel wave here, four
-// neighbouring columns each, so the panel's fold is this wave's butterfly in ascending order and a load is 16 bytes a lane.
-// One wave per row, RC float4 a lane; PAIR: the first RC / 2 of them belong to the first half of the columns.
+// LayerNorm + per-token int8 of whole rows in the row panels' order (hipq_panel_norm.h), packed: one wave per row.
 template <int RC, bool PAIR, bool EVEN>
 __global__ __launch_bounds__(kRowBlock) void panel_layer_norm_kernel(const float *__restrict__ x, size_t rows, int nblocks,
                                                                       const float *__restrict__ gamma,
                                                                       const float *__restrict__ beta, float eps,
                                                                       int8_t *__restrict__ out_q,
                                                                       float *__restrict__ out_scales) {
-    constexpr int H = PAIR ? 2 : 1, PER = RC / H;
     const size_t row = size_t(blockIdx.x) * (kRowBlock / kWave) + threadIdx.x / kWave;
     if (row >= rows) return;
-    const int lane = threadIdx.x % kWave, wave = lane / 8, part = lane % 8;  // panel wave, columns 4 part .. of its blocks
-    const int cols = nblocks * 32, half_blocks = nblocks / H;
-    int block[RC];
-    bool real[RC];
+    const int lane = threadIdx.x % kWave;
+    const PanelColumns<RC, PAIR> c(lane, nblocks);
+    const float *xr = x + row * c.cols;
+    float4 v[RC];
 #pragma unroll
-    for (int i = 0; i < RC; ++i) {
-        const int b = PAIR ? wave + 8 * (i % PER) : wave * RC + i;
-        real[i] = b < half_blocks;
-        block[i] = b + (i / PER) * half_blocks;
-    }
-    const float *xr = x + row * cols;
-    float4 v[RC], g[RC], b[RC];
-#pragma unroll
-    for (int i = 0; i < RC; ++i) v[i] = real[i] ? *reinterpret_cast<const float4 *>(xr + block[i] * 32 + part * 4) : float4{};
-    auto affine = [&](const float *p, int i, float missing) {
-        if (!p || !real[i]) return make_float4(missing, missing, missing, missing);
-        const AnyFloat4 t = *reinterpret_cast<const AnyFloat4 *>(p + block[i] * 32 + part * 4);
-        return make_float4(t.x, t.y, t.z, t.w);
-    };
-#pragma unroll
-    for (int i = 0; i < RC; ++i) {  // (y * 1.0f and y + -0.0f are y, bit for bit)
-        g[i] = affine(gamma, i, 1.0f);
-        b[i] = affine(beta, i, -0.0f);
-    }
-    auto total = [&](auto term) {
-        float half[H];
-#pragma unroll
-        for (int h = 0; h < H; ++h) {
-            float4 s = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-#pragma unroll
-            for (int i = h * PER; i < (h + 1) * PER; ++i)
-                if (real[i]) {
-                    const float4 t = term(v[i]);
-                    s = make_float4(s.x + t.x, s.y + t.y, s.z + t.z, s.w + t.w);
-                }
-            half[h] = wave_sum_ascending((s.x + s.y) + (s.z + s.w));
-        }
-        return PAIR ? half[0] + half[H - 1] : half[0];
-    };
-    const float cols_f = static_cast<float>(cols);
-    const float mean = total([](const float4 &t) { return t; }) / cols_f;
-    const float var = total([&](const float4 &t) {
-        const float p = t.x - mean, q = t.y - mean, r = t.z - mean, s = t.w - mean;
-        return make_float4(p * p, q * q, r * r, s * s);
-    }) / cols_f;
-    const float rstd = 1.0f / sqrtf(var + eps);
-    float am = 0.0f;
-#pragma unroll
-    for (int i = 0; i < RC; ++i) {
-        if (!real[i]) continue;
-        v[i] = make_float4((v[i].x - mean) * rstd * g[i].x + b[i].x, (v[i].y - mean) * rstd * g[i].y + b[i].y,
-                           (v[i].z - mean) * rstd * g[i].z + b[i].z, (v[i].w - mean) * rstd * g[i].w + b[i].w);
-        am = fmaxf(fmaxf(am, fmaxf(fabsf(v[i].x), fabsf(v[i].y))), fmaxf(fabsf(v[i].z), fabsf(v[i].w)));
-    }
-    am = wave_max(am);
-    float scale = am < FLT_EPSILON ? 1.0f : am / 127.0f;
-    if (!(fabsf(am) <= FLT_MAX)) scale = NAN;
+    for (int i = 0; i < RC; ++i) v[i] = c.real[i] ? *reinterpret_cast<const float4 *>(xr + c.at(i)) : float4{};
+    const PanelAffine<RC> affine(c, gamma, beta);
+    uint32_t q[RC];
+    const float scale = panel_norm_quantize<EVEN>(v, c, affine, eps, q);
     if (lane == 0) out_scales[row] = scale;
-    const float inv = recip_for_div(scale);
-    uint32_t *q4 = reinterpret_cast<uint32_t *>(out_q + (row / 32) * cols * 32 + (row % 32) * 16) + (part / 4) * 128 + part % 4;
+    uint32_t *q4 = reinterpret_cast<uint32_t *>(out_q + (row / 32) * c.cols * 32 + (row % 32) * 16) + (c.part / 4) * 128 + c.part % 4;
 #pragma unroll
     for (int i = 0; i < RC; ++i)
-        if (real[i])
-            q4[block[i] * 256] = pack4(quantize_int_sym<EVEN>(v[i].x, scale, inv), quantize_int_sym<EVEN>(v[i].y, scale, inv),
-                                       quantize_int_sym<EVEN>(v[i].z, scale, inv), quantize_int_sym<EVEN>(v[i].w, scale, inv));
+        if (c.real[i]) q4[c.block[i] * 256] = q[i];
 }
 
 int32_t layer_norm_quantize_packed(hipq_ctx *ctx, const float *x, size_t rows, size_t cols, const float *gamma,

@@ -135,6 +135,22 @@ int32_t layer_norm_quantize_packed(hipq_ctx *ctx, const float *x, size_t rows, s
 int32_t panel_layer_norm_quantize_packed(hipq_ctx *ctx, const float *x, size_t rows, size_t cols, const float *gamma,
                                          const float *beta, float eps, int32_t mode, PanelFold fold, int8_t *out_packed,
                                          float *out_scales);
+// A Linear of few tokens whose workgroups run the row operation on their fp32 rows (`ld` floats apart, 16-byte aligned)
+// themselves: LayerNorm in the panels' order and per-token int8 (norm), or per-token int8 alone; the bits of the two kernels.
+// residual (may be null, may be out) is added after the bias.  Where row_op_linear_fits says so.
+struct RowOpLinear {
+    const float *x;
+    size_t ld;
+    bool norm;
+    const float *gamma, *beta;
+    float eps;
+    const int8_t *w;
+    const float *w_scales, *bias, *residual;
+    size_t rows, n, k;
+    float *out;
+};
+bool row_op_linear_fits(const hipq_ctx *ctx, const float *x, size_t rows, size_t n, size_t k, PanelFold fold);
+int32_t row_op_linear(hipq_ctx *ctx, const RowOpLinear &p, int32_t mode);
 int32_t gelu_quantize_packed(hipq_ctx *ctx, const float *x, size_t rows, size_t cols, int32_t mode, int8_t *out_packed,
                              float *out_scales);
 // hipq_linear_packed_i8_f32 on per-row scales and activations that the kernel just before wrote; residual (may be null,

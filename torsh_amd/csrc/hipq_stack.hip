@@ -27,28 +27,43 @@ bool out_from_f32(const hipq_ctx *ctx, size_t d_model) { return d_model <= 1536 
 constexpr size_t kTiledTokens = 256 * 20;
 
 // Few tokens: every product split over its columns (the packed tiled kernels), the row operations between them in
-// kernels of their own that write packed codes.  The LayerNorms behind a Linear fold their sums as the row panels do that
+// kernels of their own that write packed codes, or (very few tokens) in front of the product itself.  The LayerNorms behind a Linear fold their sums as the row panels do that
 // would otherwise run, so the results are theirs, bit for bit.
 int32_t stack_tiled(hipq_ctx *ctx, const hipq_block_weights *blocks, size_t n_layers, size_t tokens, size_t d_model,
                     size_t d_ff, float eps, int32_t mode, float *x, const StackBuffers &b) {
     using namespace hipq;
     const PanelFold after_out = panel_fold(ctx, out_from_f32(ctx, d_model), tokens, d_model, d_model);
     const PanelFold after_fc2 = panel_fold(ctx, false, tokens, d_model, d_ff);
-    int32_t rc = layer_norm_quantize_packed(ctx, x, tokens, d_model, blocks[0].ln1_gamma, blocks[0].ln1_beta, eps, mode, b.qa,
-                                            b.sa);
+    auto norm_linear = [&](const float *gamma, const float *beta, PanelFold fold, const int8_t *weights, const float *scales,
+                           const float *bias, size_t n, float *out) -> int32_t {
+        if (row_op_linear_fits(ctx, x, tokens, n, d_model, fold))
+            return row_op_linear(ctx, RowOpLinear{x, d_model, true, gamma, beta, eps, weights, scales, bias, nullptr, tokens, n,
+                                                  d_model, out}, mode);
+        const int32_t rc = panel_layer_norm_quantize_packed(ctx, x, tokens, d_model, gamma, beta, eps, mode, fold, b.qa, b.sa);
+        return rc ? rc : linear_packed_rows_f32(ctx, b.qa, b.sa, weights, scales, bias, nullptr, tokens, n, d_model, out);
+    };
+    auto value_linear = [&](const hipq_block_weights &w) -> int32_t {  // x += W_out * quant(V)
+        const float *value = b.qkv + 2 * d_model;
+        if (row_op_linear_fits(ctx, value, tokens, d_model, d_model, after_out))
+            return row_op_linear(ctx, RowOpLinear{value, 3 * d_model, false, nullptr, nullptr, 0.0f, w.w_out, w.s_out, w.b_out, x,
+                                                  tokens, d_model, d_model, x}, mode);
+        const int32_t rc = quantize_activations_per_row_strided(ctx, value, tokens, d_model, 3 * d_model, mode, b.qb, b.sb,
+                                                                /*packed=*/true);
+        return rc ? rc : linear_packed_rows_f32(ctx, b.qb, b.sb, w.w_out, w.s_out, w.b_out, x, tokens, d_model, d_model, x);
+    };
+    int32_t rc = HIPQ_SUCCESS;
     for (size_t l = 0; l < n_layers && rc == HIPQ_SUCCESS; ++l) {
         const hipq_block_weights &w = blocks[l];
-        if ((l != 0 && (rc = panel_layer_norm_quantize_packed(ctx, x, tokens, d_model, w.ln1_gamma, w.ln1_beta, eps, mode,
-                                                              after_fc2, b.qa, b.sa))) ||
-            (rc = linear_packed_rows_f32(ctx, b.qa, b.sa, w.w_qkv, w.s_qkv, w.b_qkv, nullptr, tokens, 3 * d_model, d_model,
-                                         b.qkv)) ||
-            (rc = quantize_activations_per_row_strided(ctx, b.qkv + 2 * d_model, tokens, d_model, 3 * d_model, mode, b.qb, b.sb,
-                                                       /*packed=*/true)) ||
-            (rc = linear_packed_rows_f32(ctx, b.qb, b.sb, w.w_out, w.s_out, w.b_out, x, tokens, d_model, d_model, x)) ||
-            (rc = panel_layer_norm_quantize_packed(ctx, x, tokens, d_model, w.ln2_gamma, w.ln2_beta, eps, mode, after_out, b.qa,
-                                                   b.sa)) ||
-            (rc = linear_packed_rows_f32(ctx, b.qa, b.sa, w.w_fc1, w.s_fc1, w.b_fc1, nullptr, tokens, d_ff, d_model,
-                                         b.hidden)) ||
+        if (l == 0) {  // (the one LayerNorm that folds as the row kernels do)
+            if ((rc = layer_norm_quantize_packed(ctx, x, tokens, d_model, w.ln1_gamma, w.ln1_beta, eps, mode, b.qa, b.sa)) ||
+                (rc = linear_packed_rows_f32(ctx, b.qa, b.sa, w.w_qkv, w.s_qkv, w.b_qkv, nullptr, tokens, 3 * d_model, d_model,
+                                             b.qkv)))
+                return rc;
+        } else if ((rc = norm_linear(w.ln1_gamma, w.ln1_beta, after_fc2, w.w_qkv, w.s_qkv, w.b_qkv, 3 * d_model, b.qkv))) {
+            return rc;
+        }
+        if ((rc = value_linear(w)) ||
+            (rc = norm_linear(w.ln2_gamma, w.ln2_beta, after_out, w.w_fc1, w.s_fc1, w.b_fc1, d_ff, b.hidden)) ||
             (rc = gelu_quantize_packed(ctx, b.hidden, tokens, d_ff, mode, b.qb, b.sb)) ||
             (rc = linear_packed_rows_f32(ctx, b.qb, b.sb, w.w_fc2, w.s_fc2, w.b_fc2, x, tokens, d_model, d_ff, x)))
             return rc;
