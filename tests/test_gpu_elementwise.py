@@ -414,6 +414,79 @@ def test_per_channel_auto_spread_over_columns(ctx, hipq, oracle, shape, axis, gr
             np.testing.assert_array_equal(host(q), want_q.astype(np.int8))
 
 
+# One part of a group that fills a workgroup's registers or less of them; two parts, many; runs below and above a
+# workgroup's width; more items than resident workgroups (the last two).
+@pytest.mark.parametrize("outer,channels,inner", [(3, 40, 2500), (128, 20, 128), (130, 5, 516), (9, 33, 1000), (64, 6, 3136),
+                                                  (2, 9, 32772), (2, 2, 1 << 20), (3, 1100, 4100), (2, 2050, 8192)])
+def test_per_channel_auto_input_read_once(ctx, hipq, outer, channels, inner):
+    """The form that keeps a group in the registers of a few workgroups: codes, scales and zero points of the per-row quantizer
+    (held to the oracle above) on the channels as rows, for both roundings, with NaN elements, a channel with an infinity
+    (its codes stay untouched, the status says so), a constant one and one far from zero."""
+    g = torch.Generator(device="cuda").manual_seed(outer * channels + inner)
+    x = torch.randn(outer, channels, inner, generator=g, device="cuda")
+    x[:, channels // 2] = x[:, channels // 2] * 1e-3 + 1e4
+    x[0, 0, :: max(2, inner // 7)] = float("nan")
+    x[:, channels - 1] = 2.5
+    rows = x.transpose(0, 1).reshape(channels, outer * inner).contiguous()
+    for flavor in (hipq.PARAMS_SYMMETRIC, hipq.PARAMS_AFFINE):
+        for mode in (0, hipq.ROUND_HALF_EVEN):
+            want_q, want_s, want_z, _ = ctx.quantize_per_row(rows, flavor, mode)
+            q, s, z, status = ctx.quantize_per_channel_auto(x, 1, flavor, mode)
+            assert torch.equal(q, want_q.view(channels, outer, inner).transpose(0, 1)), (flavor, mode)
+            assert torch.equal(s, want_s) and torch.equal(z, want_z) and int(status) == 0
+    for flavor, qmin, qmax in ((hipq.PARAMS_AFFINE, 3, 90), (hipq.PARAMS_NN_SYMMETRIC, -128, 127), (hipq.PARAMS_SYMMETRIC, -8, 7)):
+        want = ctx.quantize_per_group_auto(rows, 1, channels, outer * inner, 1, flavor, qmin, qmax)
+        got = ctx.quantize_per_group_auto(x, outer, channels, inner, 1, flavor, qmin, qmax)
+        if qmin > 0:  # (a NaN is code 0 over channels, the nearest code in rows)
+            want[0][torch.isnan(rows)] = 0
+        assert torch.equal(got[0], want[0].view(channels, outer, inner).transpose(0, 1)), flavor
+        assert torch.equal(got[1], want[1]) and torch.equal(got[2], want[2])
+    x[outer - 1, channels - 1, inner - 1] = float("inf")
+    out = torch.full(x.shape, 77, dtype=torch.int8, device="cuda")
+    scales, zps = torch.empty(channels, device="cuda"), torch.empty(channels, dtype=torch.int32, device="cuda")
+    status = torch.empty(1, dtype=torch.int32, device="cuda")
+    ctx.call("hipq_quantize_per_channel_auto_f32_i8", x.data_ptr(), outer, channels, inner, hipq.PARAMS_SYMMETRIC, 0,
+             out.data_ptr(), scales.data_ptr(), zps.data_ptr(), status.data_ptr())
+    want_q = ctx.quantize_per_row(rows)[0].view(channels, outer, inner).transpose(0, 1)
+    assert int(status) != 0 and (out[:, channels - 1] == 77).all()
+    assert torch.equal(out[:, :channels - 1], want_q[:, :channels - 1])
+
+
+def test_per_channel_auto_input_read_once_gives_up_cleanly_and_replays(hipq):
+    """Parts that stop waiting mark the context and the status word, and the next call is whole again; a captured call gives
+    the eager call's bits on every replay."""
+    c = hipq.Context(0, own_stream=True)
+    stream = torch.cuda.ExternalStream(c.stream_handle)
+    try:
+        with torch.cuda.stream(stream):
+            x = torch.randn(64, 64, 3136, device="cuda")
+            want = c.quantize_per_channel_auto(x, 1)
+            c.synchronize()
+            c.set_wait_spin_limit(0)
+            lost = c.quantize_per_channel_auto(x, 1)
+            with pytest.raises(hipq.HipqError):
+                c.synchronize()
+            assert int(lost[3]) == hipq.DEVICE_ERROR
+            c.set_wait_spin_limit(-1)
+            again = c.quantize_per_channel_auto(x, 1)
+            c.synchronize()
+            assert all(torch.equal(a, b) for a, b in zip(want, again))
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph, stream=stream):
+                captured = c.quantize_per_channel_auto(x, 1)
+            for k in range(3):
+                x.mul_(1.5)
+                for t in captured:
+                    t.zero_()
+                graph.replay()
+                eager = c.quantize_per_channel_auto(x, 1)
+                c.synchronize()
+                assert all(torch.equal(a, b) for a, b in zip(eager, captured)), k
+    finally:
+        torch.cuda.synchronize()
+        c.close()
+
+
 def test_per_channel_auto_spread_half_even_and_bad_groups(ctx, hipq, oracle):
     """Round-half-even over columns equals the per-row kernel on the transposed matrix; a channel holding an infinity
     sets the status word and keeps its codes untouched while the other channels get theirs; NaNs are left out of a

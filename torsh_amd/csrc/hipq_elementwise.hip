@@ -981,6 +981,44 @@ __global__ __launch_bounds__(kBlock) void channel_range_kernel(const float *__re
     if (head) add_to_keys(g, m.mn, m.mx);
 }
 
+// Codes of a group's elements, round(x / scale) + zp clamped, NaN -> 0: without the guards of the division and with the clamp
+// on integers where the group's own range rules their cases out (`plain`; the same for all threads of a group).
+template <bool EVEN>
+struct ChannelCodes {
+    float scale, inv, zpf;
+    int zp, qmin, qmax;
+    bool int_cast, plain;
+    __device__ __forceinline__ ChannelCodes(float scale_, int zp_, float mn, float mx, int flavor, int qmin_, int qmax_)
+        : scale(scale_), inv(recip_for_div(scale_)), zpf(static_cast<float>(zp_)), zp(zp_), qmin(qmin_), qmax(qmax_),
+          // torsh-nn's per-channel weights pass each value through `as i32` before the zero point is added
+          // (crates/torsh-nn/src/quantization/ops.rs:153-162): a NaN becomes the code clamp(zero point).
+          int_cast(flavor >= HIPQ_PARAMS_NN_SYMMETRIC),
+          // (no quotient overflows, 0 is a code)
+          plain(!int_cast && inv != 0.0f && fmaxf(fabsf(mn), fabsf(mx)) * fabsf(inv) < 1e30f && qmin <= 0 && qmax >= 0) {}
+    __device__ __forceinline__ int fast(float x) const {
+        const float q0 = x * inv, t = fmaf(fmaf(-q0, scale, x), inv, q0);  // div_rn
+        return min(max(cvt_i32_sat(round_mode<EVEN>(t) + zpf), qmin), qmax);
+    }
+    __device__ __forceinline__ int fast_zp0(float x) const {  // (the conversion truncates, as the rounding ends)
+        const float q0 = x * inv, t = fmaf(fmaf(-q0, scale, x), inv, q0);
+        return min(max(cvt_i32_sat(EVEN ? rintf(t) : t + copysignf(0x1.fffffep-2f, t)), qmin), qmax);
+    }
+    __device__ __forceinline__ int general(float x) const {
+        return int_cast ? quantize_int_cast<EVEN>(x, scale, inv, zp, qmin, qmax)
+                        : to_int_nan0(quantize_value<true, EVEN>(x, scale, inv, zpf, static_cast<float>(qmin), static_cast<float>(qmax)));
+    }
+    // body(one), one(x) -> code
+    template <typename Body>
+    __device__ __forceinline__ void with(Body body) const {
+        if (plain && zp == 0)
+            body([this](float x) { return fast_zp0(x); });
+        else if (plain)
+            body([this](float x) { return fast(x); });
+        else
+            body([this](float x) { return general(x); });
+    }
+};
+
 // Parameters of the thread's group from the group's keys, then the codes of the thread's column.  The thread that
 // owns a group's first column on the first row writes the group's parameters and, for a range that gives none, the
 // status; such a group keeps what `out` held, as with a workgroup per group.
@@ -1005,15 +1043,7 @@ __global__ __launch_bounds__(kBlock) void channel_quantize_kernel(const float *_
         if (st != HIPQ_SUCCESS && out_status) *out_status = st;
     }
     if (st != HIPQ_SUCCESS) return;
-    const float inv = recip_for_div(scale), zpf = static_cast<float>(zp);
-    const float lo = static_cast<float>(qmin), hi = static_cast<float>(qmax);
-    // torsh-nn's per-channel weights pass each value through `as i32` before the zero point is added
-    // (crates/torsh-nn/src/quantization/ops.rs:153-162): a NaN becomes the code clamp(zero point).
-    const bool int_cast = flavor >= HIPQ_PARAMS_NN_SYMMETRIC;
-    auto one = [&](float v) {
-        return int_cast ? quantize_int_cast<EVEN>(v, scale, inv, zp, qmin, qmax)
-                        : to_int_nan0(quantize_value<true, EVEN>(v, scale, inv, zpf, lo, hi));
-    };
+    ChannelCodes<EVEN>(scale, zp, mn, mx, flavor, qmin, qmax).with([&](auto one) {
     using Vec = typename std::conditional<V == 4, float4, float>::type;
     auto load = [&](size_t row) {
         const Vec *p = reinterpret_cast<const Vec *>(x + row * cc.period + w.unit * V);
@@ -1039,9 +1069,112 @@ __global__ __launch_bounds__(kBlock) void channel_quantize_kernel(const float *_
         store(row + 3 * w.row_step, d);
     }
     for (; row < cc.outer; row += w.row_step) store(row, load(row));
+    });
 }
 
 // Explicit per-channel parameters over a dense [outer, channels, inner] view.
+// ---- the same with the input read once: a group's elements stay in the registers of the `parts` workgroups that share it
+// while those agree on its range.  Item g * parts + p is part p of group g; a workgroup takes every gridDim-th item.  Each
+// part publishes its range as two tagged words of its own and waits for the words of its group's other parts, so groups do
+// not wait for each other.  No circle of waits: the items before a part's group are taken, by every workgroup, before it, so
+// the first unfinished group always has all its parts at work - given that the grid is resident at once and no smaller than
+// a group.  Bound by memory and by vector instructions, some twelve per element, which the workgroups of a compute unit
+// overlap as they drift apart: 64 x 256 x 3136 81.7 -> 58.4 us (75.5 in two passes with the same codes arithmetic), 4.4 TB/s.
+// Half the registers a lane and twice the workgroups: 67.1.
+struct ChannelParts {
+    uint32_t items, parts, per_part;  // per_part: float4s of a part
+    uint32_t vecs, row_vecs, run;     // float4s of a group; of a row of all channels; of a group's run in it
+    uint32_t step_run, step_at;       // what kBlock float4s further on in the group is: run position (mod run) and address
+    FastDiv by_run, by_parts;
+};
+constexpr int kPartVec = 16;      // float4 a lane: what four workgroups per compute unit hold
+constexpr uint32_t kMostParts = 128;  // 64 x 32 x 12544 49 parts 40.4 -> 32.9 us, 256 x 16 x 6000 94 40.7 -> 34.8, 512 x 16 x 6000 188 72.5 -> 71.4
+constexpr uint32_t kPartTag = 1;
+
+__global__ void channel_parts_init_kernel(unsigned long long *words, uint32_t n, int *status) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) words[i] = 0;
+    if (i == 0 && status) *status = 0;
+}
+
+template <bool EVEN>
+__global__ __launch_bounds__(kBlock, 4) void channel_parts_kernel(const float *__restrict__ x, ChannelParts cp,
+                                                                  unsigned long long *words, int flavor, int qmin, int qmax,
+                                                                  int8_t *__restrict__ out, float *__restrict__ out_scales,
+                                                                  int32_t *__restrict__ out_zps, int32_t *__restrict__ out_status,
+                                                                  uint32_t *ctx_words, int spin_limit) {
+    __shared__ float lds[2 * kBlock / kWave];
+    const float4 *x4 = reinterpret_cast<const float4 *>(x);
+    uint32_t *out4 = reinterpret_cast<uint32_t *>(out);
+    for (uint32_t item = blockIdx.x; item < cp.items; item += gridDim.x) {
+        uint32_t p;
+        const uint32_t g = cp.by_parts.quotient(item, &p);
+        const uint32_t first = p * cp.per_part, end = min(first + cp.per_part, cp.vecs);
+        const uint32_t mine = first + threadIdx.x;
+        uint32_t r0;
+        const uint32_t row0 = cp.by_run.quotient(mine < end ? mine : first, &r0);
+        const uint32_t at0 = row0 * cp.row_vecs + g * cp.run + r0;
+        auto walk = [&](auto body) {  // body(i, address); past the part's end: its first float4 once more
+            uint32_t r = r0, at = at0;
+#pragma unroll
+            for (int i = 0; i < kPartVec; ++i) {
+                body(i, mine + uint32_t(i) * kBlock < end ? at : at0);
+                r += cp.step_run;
+                at += cp.step_at;
+                if (r >= cp.run) {
+                    r -= cp.run;
+                    at += cp.row_vecs - cp.run;
+                }
+            }
+        };
+        float4 v[kPartVec];
+        walk([&](int i, uint32_t at) { v[i] = load_stream(x4 + at); });
+        MinMax m{INFINITY, -INFINITY};
+#pragma unroll
+        for (int i = 0; i < kPartVec; ++i) {
+            m.mn = fminf(m.mn, fminf(fminf(v[i].x, v[i].y), fminf(v[i].z, v[i].w)));
+            m.mx = fmaxf(m.mx, fmaxf(fmaxf(v[i].x, v[i].y), fmaxf(v[i].z, v[i].w)));
+        }
+        m = block_minmax(m, lds);
+        bool lost = false;
+        if (cp.parts > 1) {
+            unsigned long long *group = words + 2 * size_t(g) * cp.parts;
+            if (threadIdx.x == 0) {
+                publish_tagged(group + 2 * p, kPartTag, __builtin_bit_cast(uint32_t, m.mn));
+                publish_tagged(group + 2 * p + 1, kPartTag, __builtin_bit_cast(uint32_t, m.mx));
+            }
+            MinMax t{INFINITY, -INFINITY};
+            if (threadIdx.x < cp.parts) {  // (at most kMostParts)
+                uint32_t lo = 0, hi = 0;
+                lost = !(poll_tagged(group + 2 * threadIdx.x, kPartTag, spin_limit, &lo) &&
+                         poll_tagged(group + 2 * threadIdx.x + 1, kPartTag, spin_limit, &hi));
+                if (!lost) t = MinMax{__builtin_bit_cast(float, lo), __builtin_bit_cast(float, hi)};
+            }
+            lost = __syncthreads_or(lost) != 0;
+            m = block_minmax(t, lds);
+        }
+        float scale;
+        int zp;
+        int st = params_from_minmax(m.mn, m.mx, flavor, qmin, qmax, &scale, &zp);
+        if (lost) st = HIPQ_DEVICE_ERROR;
+        if (threadIdx.x == 0) {
+            if (lost) record_give_up(ctx_words);
+            if (p == 0) {
+                if (out_scales) out_scales[g] = scale;
+                if (out_zps) out_zps[g] = zp;
+            }
+            if ((p == 0 || lost) && st != HIPQ_SUCCESS && out_status) *out_status = st;
+        }
+        if (st != HIPQ_SUCCESS) continue;
+        ChannelCodes<EVEN>(scale, zp, m.mn, m.mx, flavor, qmin, qmax).with([&](auto one) {
+            walk([&](int i, uint32_t at) {
+                if (mine + uint32_t(i) * kBlock < end)
+                    store_stream(out4 + at, pack4(one(v[i].x), one(v[i].y), one(v[i].z), one(v[i].w)));
+            });
+        });
+    }
+}
+
 template <bool DIV, bool EVEN>
 __global__ __launch_bounds__(kBlock) void quantize_per_channel_kernel(const float *__restrict__ x, size_t total,
                                                                        size_t channels, size_t inner,
@@ -1802,6 +1935,41 @@ static int32_t quantize_channels(const char *fn, hipq_ctx *ctx, const float *x, 
     if (spread) {
         const bool vec = inner % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15u) == 0 &&
                          (reinterpret_cast<uintptr_t>(out) & 3u) == 0;
+        // The input read once, where the device's registers hold it at once, or where runs are long enough that parts share
+        // few lines and the parts fill a third of the registers.  us, two passes / once: [500,30,300] 31.0 / 14.2, [64,40,1000]
+        // 21.6 / 14.2, [100,1000,128] 21.5 / 16.6; several rounds: [2,4096,4096] 58.9 / 37.8, [32,2048,768] 75.8 / 60.0,
+        // [2,8000,3000] (0.37 of the registers) 84 / 70, [4,8192,1024] (0.25) 54.4 / 55.2, [2,8192,1024] (0.12) 34.8 / 44.0,
+        // [128,1024,196] 39.4 / 40.8, [8,8192,400] 42 / 61.  No more context scratch than the smallest block of it.
+        constexpr size_t kPartVecs = size_t(kPartVec) * kBlock;
+        const size_t run = group * inner, vecs = outer * run / 4, parts = (vecs + kPartVecs - 1) / kPartVecs, items = parts * groups;
+        const size_t resident = resident_workgroups(ctx, true), words_at = kScratchHeader;
+        const size_t words_end = words_at + (parts > 1 ? 2 * items * sizeof(unsigned long long) : 0);
+        if (vec && channels % group == 0 && run >= 128 && parts <= kMostParts && parts <= resident &&
+            outer * period / 4 < (size_t(1) << 31) && (items <= resident || (run >= 512 && vecs >= parts * (kPartVecs * 5 / 16))) &&
+            (words_end <= (size_t(1) << 20) || words_end <= ctx->scratch_bytes) && four_wide_workgroups_fit(ctx)) {
+            ChannelParts cp;
+            cp.items = static_cast<uint32_t>(items);
+            cp.parts = static_cast<uint32_t>(parts);
+            cp.per_part = static_cast<uint32_t>((vecs + parts - 1) / parts);
+            cp.vecs = static_cast<uint32_t>(vecs);
+            cp.row_vecs = static_cast<uint32_t>(period / 4);
+            cp.run = static_cast<uint32_t>(run / 4);
+            cp.step_run = kBlock % cp.run;
+            cp.step_at = kBlock / cp.run * cp.row_vecs + cp.step_run;
+            cp.by_run = FastDiv::by(cp.run);
+            cp.by_parts = FastDiv::by(cp.parts);
+            void *s = nullptr;
+            if ((rc = scratch(ctx, words_end, &s))) return rc;
+            unsigned long long *words = reinterpret_cast<unsigned long long *>(static_cast<char *>(s) + words_at);
+            const uint32_t nwords = static_cast<uint32_t>((words_end - words_at) / sizeof(unsigned long long));
+            hipLaunchKernelGGL(channel_parts_init_kernel, dim3(nwords / kBlock + 1), dim3(kBlock), 0, ctx->stream, words, nwords,
+                               out_status);
+            const dim3 grid(static_cast<unsigned>(items < resident ? items : resident));
+            auto kernel = even ? channel_parts_kernel<true> : channel_parts_kernel<false>;
+            hipLaunchKernelGGL(kernel, grid, dim3(kBlock), 0, ctx->stream, x, cp, words, flavor, qmin, qmax, out, out_scales,
+                               out_zero_points, out_status, ctx->wait_error, ctx->wait_spin_limit);
+            return check_launch(fn);
+        }
         ChannelColumns cc;
         cc.outer = outer;
         cc.period = period;
