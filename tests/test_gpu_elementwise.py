@@ -353,6 +353,42 @@ def test_per_row_quantize(ctx, hipq, oracle, shape, flavor_name):
     np.testing.assert_array_equal(host(q), want_q.astype(np.int8))
 
 
+# Rows of odd length start anywhere in a vector of four: shorter than a vector, a wave's rows, a workgroup's, long ones
+# (registers hold 16384 floats), and enough elements for the streaming forms; bases that are aligned and not.
+@pytest.mark.parametrize("rows,cols", [(9, 1), (6, 3), (70, 33), (13, 1023), (9, 1027), (7, 4099), (5, 16387), (4500, 947), (2100, 2001),
+                                       (700, 6361)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_per_row_quantize_rows_of_odd_length(ctx, hipq, oracle, rows, cols, shift):
+    x = normal(rows + cols, (rows, cols))
+    if cols > 1:
+        x[rows // 2, cols // 2] = np.nan
+    x[rows - 1, 0], x[rows - 1, cols - 1] = -9.0, 7.0
+    want_q, want_s, want_z = oracle.quantize_per_channel_auto(x, 0, 0, oracle.PER_CHANNEL_AFFINE)
+    flat = torch.empty(rows * cols + shift, device="cuda")
+    flat[shift:] = dev(x).view(-1)
+    q, s, z, status = ctx.quantize_per_row(flat[shift:].view(rows, cols), hipq.PARAMS_AFFINE)
+    assert host(status)[0] == 0
+    np.testing.assert_array_equal(host(s), want_s)
+    np.testing.assert_array_equal(host(z), want_z)
+    np.testing.assert_array_equal(host(q), np.nan_to_num(want_q).astype(np.int8))
+
+
+# Runs of no multiple of four: one that a vector straddles once, the shortest, one per tensor; a last vector that is not whole;
+# several tiles of a workgroup; codes that start at any byte take the element kernel.
+@pytest.mark.parametrize("outer,channels,inner", [(1, 1, 5), (3, 7, 6), (2, 3, 7), (1, 2, 4097), (11, 257, 43), (300, 31, 1390), (9, 1, 9)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_per_channel_dequantize_runs_of_any_length(ctx, oracle, outer, channels, inner, shift):
+    rng = np.random.default_rng(outer + channels + inner)
+    codes = rng.integers(-128, 128, size=(outer, channels, inner), dtype=np.int8)
+    scales = rng.uniform(0.01, 1.0, channels).astype(np.float32)
+    zps = rng.integers(-20, 20, channels, dtype=np.int32)
+    flat = torch.empty(codes.size + shift, dtype=torch.int8, device="cuda")
+    flat[shift:] = dev(codes).view(-1)
+    got = ctx.dequantize_per_channel(flat[shift:].view(codes.shape), dev(scales), dev(zps), 1)
+    want = oracle.dequantize_per_channel_affine(codes.astype(np.float32), scales, zps, 1)
+    np.testing.assert_array_equal(host(got), want)
+
+
 def test_per_row_status_on_non_finite_row(ctx, hipq):
     x = normal(3, (4, 128))
     x[1, 5] = np.inf

@@ -702,10 +702,16 @@ __global__ __launch_bounds__(kBlock) void quantize_per_row_kernel(const float *_
     const size_t kpad = ((cols + 31) / 32 + 3) / 4 * 4 * 32;
     int8_t *prow = out + (row / 32) * (kpad / 32) * 1024 + (row % 32) * 16;  // + packed_k(k)
     auto packed_k = [](size_t k) { return (k / 32) * 1024 + ((k % 32) / 16) * 512 + (k % 16); };
-    const bool aligned = ((reinterpret_cast<uintptr_t>(x) & 15u) == 0) && (cols % 4 == 0) && (ld % 4 == 0) &&
-                         ((reinterpret_cast<uintptr_t>(out) & 3u) == 0);
-    const size_t nvec = aligned ? cols / 4 : 0;
-    const float4 *x4 = reinterpret_cast<const float4 *>(xr);
+    // Vectors of four: the whole row, or (rows of odd length without gaps, ld == cols: input and codes lie alike) what is left of it
+    // behind the first `head` elements, up to the next multiple of four of the tensor.  The other elements one by one.
+    // (One by one altogether, and long rows read twice, 2473 x 6361 took 36.4 us with these codes; quantize + dequantize 63.1 -> 37.5.)
+    const bool bases = ((reinterpret_cast<uintptr_t>(x) & 15u) == 0) && ((reinterpret_cast<uintptr_t>(out) & 3u) == 0);
+    const size_t gap = PACKED || ld != cols ? 0 : (0 - row * cols) % 4;
+    const size_t head = gap < cols ? gap : cols;
+    const size_t nvec = bases && (head == gap) && (PACKED || ld != cols ? cols % 4 == 0 && ld % 4 == 0 : true) ? (cols - head) / 4 : 0;
+    const size_t rest = nvec ? cols - nvec * 4 : cols;  // elements outside the vectors: head of them in front
+    auto rest_at = [&](size_t i) { return nvec == 0 || i < head ? i : i + nvec * 4; };
+    const float4 *x4 = reinterpret_cast<const float4 *>(xr + head);
 
     MinMax m{INFINITY, -INFINITY};
     float4 cache[kCache];
@@ -732,7 +738,7 @@ __global__ __launch_bounds__(kBlock) void quantize_per_row_kernel(const float *_
             acc_minmax(m, t.z);
             acc_minmax(m, t.w);
         }
-        for (size_t c = nvec * 4 + lane; c < cols; c += TPR) acc_minmax(m, xr[c]);
+        for (size_t i = lane; i < rest; i += TPR) acc_minmax(m, xr[rest_at(i)]);
     }
     if constexpr (TPR == kWave) {
         m.mn = wave_min(m.mn);
@@ -768,7 +774,7 @@ __global__ __launch_bounds__(kBlock) void quantize_per_row_kernel(const float *_
     }
     const float zpf = static_cast<float>(zp);
     const float inv = recip_for_div(scale);  // once per row; each element then divides with two FMAs
-    uint32_t *q4 = reinterpret_cast<uint32_t *>(qr);
+    uint32_t *q4 = reinterpret_cast<uint32_t *>(qr + head);
     // torsh-nn's per-channel weights pass each value through `as i32` before the zero point is added
     const bool int_cast = flavor >= HIPQ_PARAMS_NN_SYMMETRIC;
     auto quant1 = [&](float v) {
@@ -796,7 +802,10 @@ __global__ __launch_bounds__(kBlock) void quantize_per_row_kernel(const float *_
         if (v < nvec) put4(v, quant4(cache[i]));
     }
     for (size_t v = size_t(lane) + size_t(kCache) * TPR; v < nvec; v += TPR) put4(v, quant4(x4[v]));
-    for (size_t c = nvec * 4 + lane; c < cols; c += TPR) put1(c, static_cast<int8_t>(quant1(xr[c])));
+    for (size_t i = lane; i < rest; i += TPR) {
+        const size_t c = rest_at(i);
+        put1(c, static_cast<int8_t>(quant1(xr[c])));
+    }
     if constexpr (PACKED)
         for (size_t c = cols + lane; c < kpad; c += TPR) put1(c, int8_t(0));  // k padding: zeros add nothing
 }
@@ -1198,6 +1207,63 @@ __global__ __launch_bounds__(kBlock) void dequantize_per_channel_kernel(const in
                                                                          float *__restrict__ out) {
     for (size_t i = size_t(blockIdx.x) * kBlock + threadIdx.x; i < total; i += size_t(gridDim.x) * kBlock) {
         const size_t c = (i / inner) % channels;
+        out[i] = scales[c] * (static_cast<float>(q[i]) - static_cast<float>(zps[c]));
+    }
+}
+
+// The same where runs are no multiple of four, on vectors of four at any place in the view: a vector holds elements of its
+// first element's channel and, from `left` on, of the next one.  inner >= 4, total < 2^31, out 16-byte aligned, q 4-byte.
+// Bound by memory: 2473 x 6361 27.5 -> 12.8 us (6.1 TB/s), 73 x 4692 x 43 26.5 -> 11.3; before, an element a thread with two
+// 64-bit divisions each, which is left for runs below four and for bases that are not aligned.
+struct ChannelRuns {
+    uint32_t total, channels, inner;
+    FastDiv by_inner, by_channels;
+};
+constexpr int kRunsVec = 4;  // vectors in flight a thread
+
+__global__ __launch_bounds__(kBlock) void dequantize_per_channel_runs_kernel(const int8_t *__restrict__ q, ChannelRuns cr,
+                                                                              const float *__restrict__ scales,
+                                                                              const int32_t *__restrict__ zps,
+                                                                              float *__restrict__ out) {
+    const uint32_t *q4 = reinterpret_cast<const uint32_t *>(q);
+    float4 *out4 = reinterpret_cast<float4 *>(out);
+    const uint32_t nvec = cr.total / 4;
+    auto channel_at = [&](uint32_t i, uint32_t *r) {
+        uint32_t c;
+        cr.by_channels.quotient(cr.by_inner.quotient(i, r), &c);
+        return c;
+    };
+    for (uint32_t base = blockIdx.x * (kBlock * kRunsVec) + threadIdx.x; base < nvec; base += gridDim.x * (kBlock * kRunsVec)) {
+        uint32_t w[kRunsVec];
+        float s[kRunsVec][2], z[kRunsVec][2];
+        uint32_t left[kRunsVec];
+#pragma unroll
+        for (int i = 0; i < kRunsVec; ++i) {  // (past the last vector: that one once more, not stored)
+            const uint32_t j = min(base + uint32_t(i) * kBlock, nvec - 1);
+            w[i] = q4[j];
+            uint32_t r;
+            const uint32_t c = channel_at(4 * j, &r), next = c + 1 == cr.channels ? 0 : c + 1;
+            left[i] = cr.inner - r;
+            s[i][0] = scales[c];
+            s[i][1] = scales[next];
+            z[i][0] = static_cast<float>(zps[c]);
+            z[i][1] = static_cast<float>(zps[next]);
+        }
+#pragma unroll
+        for (int i = 0; i < kRunsVec; ++i) {
+            const uint32_t j = base + uint32_t(i) * kBlock;
+            auto one = [&](uint32_t e) {
+                const bool first = e < left[i];
+                return (first ? s[i][0] : s[i][1]) *
+                       (static_cast<float>(static_cast<int8_t>(w[i] >> (8 * e))) - (first ? z[i][0] : z[i][1]));
+            };
+            if (j < nvec) store_stream(out4 + j, make_float4(one(0), one(1), one(2), one(3)));
+        }
+    }
+    const uint32_t i = nvec * 4 + threadIdx.x;
+    if (blockIdx.x == 0 && i < cr.total) {
+        uint32_t r;
+        const uint32_t c = channel_at(i, &r);
         out[i] = scales[c] * (static_cast<float>(q[i]) - static_cast<float>(zps[c]));
     }
 }
@@ -1842,7 +1908,7 @@ static int32_t quantize_rows(const char *fn, hipq_ctx *ctx, const float *x, size
 #define HIPQ_LAUNCH_ROWS(TPR, E, G)                                                                                  \
     hipLaunchKernelGGL((quantize_per_row_kernel<TPR, E>), dim3(G), dim3(kBlock), 0, ctx->stream, x, rows, cols, ld, \
                        flavor, qmin, qmax, out, out_scales, out_zero_points, out_status, poison)
-    if (packed || (cols > 4096 && ld % 4 == 0)) {
+    if (packed || (cols > 4096 && (ld % 4 == 0 || ld == cols))) {
         // long rows: four times the registers, so that up to 16384 floats are read once and all requested up front
         const int grid = static_cast<int>(grid_rows);
 #define HIPQ_LAUNCH_LONG_ROWS(E, P)                                                                                   \
@@ -2232,6 +2298,14 @@ int32_t hipq_dequantize_per_channel_i8_f32(hipq_ctx *ctx, const int8_t *q, size_
     if (inner % 4 == 0 && (reinterpret_cast<uintptr_t>(q) & 3u) == 0 && (reinterpret_cast<uintptr_t>(out) & 15u) == 0) {
         hipLaunchKernelGGL(dequantize_per_channel_vec_kernel, dim3(grid_for_tiles(ctx, total)), dim3(kBlock), 0,
                            ctx->stream, q, total / 4, channels, inner, scales, zero_points, out);
+        return check_launch(__func__);
+    }
+    if (inner >= 4 && total >= 4 && total < (size_t(1) << 31) - (size_t(1) << 28) && (reinterpret_cast<uintptr_t>(q) & 3u) == 0 &&
+        (reinterpret_cast<uintptr_t>(out) & 15u) == 0) {
+        ChannelRuns cr{static_cast<uint32_t>(total), static_cast<uint32_t>(channels), static_cast<uint32_t>(inner),
+                       FastDiv::by(static_cast<uint32_t>(inner)), FastDiv::by(static_cast<uint32_t>(channels))};
+        hipLaunchKernelGGL(dequantize_per_channel_runs_kernel, dim3(grid_for_tiles(ctx, total)), dim3(kBlock), 0, ctx->stream, q, cr,
+                           scales, zero_points, out);
         return check_launch(__func__);
     }
     const int grid = grid_for_elems(ctx, total);
