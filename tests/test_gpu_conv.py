@@ -308,6 +308,16 @@ def test_conv_any_stride_and_channel_count(ctx, hipq, oracle, nb, c, h, w, oc, k
             np.testing.assert_array_equal(got.reshape(acc2d.shape), q)
 
 
+# As many 32 x 32 blocks as a workgroup each is taken for (256; 512 above 64 channels), and one row of blocks more: the K-split
+# tiles of 32, 64 and 128 channels, whose last tiles are not whole.  K that eight waves share unevenly, or that some get none of.
+@pytest.mark.parametrize("nb,c,h,w,oc,k,stride,pad,zp", [
+    (8, 32, 32, 32, 30, (1, 1), (1, 1), (0, 0), 3), (8, 17, 32, 33, 30, (3, 3), (1, 1), (1, 1), 90),
+    (4, 64, 32, 32, 60, (1, 1), (1, 1), (0, 0), 128), (4, 288, 33, 32, 60, (1, 1), (1, 1), (0, 0), 128),
+    (4, 40, 32, 32, 128, (3, 3), (1, 1), (1, 1), 0), (4, 40, 33, 32, 128, (3, 3), (1, 1), (1, 1), 255)])
+def test_conv_at_the_limits_of_one_block_per_workgroup(ctx, hipq, oracle, nb, c, h, w, oc, k, stride, pad, zp):
+    test_conv_any_stride_and_channel_count(ctx, hipq, oracle, nb, c, h, w, oc, k, stride, pad, zp)
+
+
 @pytest.mark.parametrize("c,h,w,k,stride,pad", [(0, 6, 9, (3, 3), (1, 1), (1, 1)), (0, 5, 5, (2, 2), (2, 1), (0, 0)),
                                                 (3, 0, 8, (3, 3), (1, 1), (2, 1)), (32, 0, 5, (1, 3), (1, 2), (1, 1)),
                                                 (3, 7, 0, (3, 3), (2, 1), (1, 2))])

@@ -232,6 +232,14 @@ static int32_t launch_conv_window(hipq_ctx *ctx, const int8_t *filters, const in
     // [4,224,38,38] x 192 13.1 / 8.7 (182), [49,96,9,9] x 512 12.5 / 9.7 (252), but [32,32,14,14] x 512 12.1 / 12.4 (392),
     // [4,32,46,46] x 512 12.5 / 15.5 (532), [30,128,28,28] x 256 12.2 / 16.6 (736), [25,128,40,40] x 512 21 / 43 (2500).
     const size_t tiles = (size_t(cw.N) + 63) / 64 * ((size_t(cw.M) + 127) / 128), cus = size_t(ctx->num_cus);
+    // Few windows: a workgroup per 32 channels x 32 windows, K split between eight waves.  The larger tiles then leave most of
+    // the device idle and each of their waves walks a quarter of K, two to four k blocks in flight.  us from fp32, larger
+    // tiles / this (blocks of 32 x 32): [1,128,14,17] x [128,128,5,5] 17.4 / 13.1 (32), [4,512,14,14] x [128,512,3,3] 19.3 / 13.4
+    // (100), [4,224,24,25] x [85,224,3,3] 15.5 / 12.2 (225), x [512,512,3,3] 19.9 / 16.7 (400), 8 images 20.6 / 22.1 (784); up to
+    // 64 channels, whose larger tile has four blocks, not eight: [11,192,10,11] x [49,192,5,5] 16.2 / 13.3 (76),
+    // [1,352,67,70] x [64,352,3,3] 15.1 / 15.3 (294), [1,32,71,74] x [37,32,7,7] 14.3 / 16.7 (330).
+    const size_t blocks = (size_t(cw.N) + 31) / 32 * ((size_t(cw.M) + 31) / 32);
+    if (blocks <= (cw.M > 64 ? cus * 2 : cus)) return launch_conv_window_form<1, 1, 4, true, EPI, EVEN>(ctx, filters, image, cw, ep);
     if (tiles >= cus * 8 || (cw.kblocks < 8 && tiles > cus)) {
         if (cw.M <= 32) return launch_conv_window_form<1, 4, 2, false, EPI, EVEN>(ctx, filters, image, cw, ep);
         if (cw.M <= 64) return launch_conv_window_form<2, 2, 4, false, EPI, EVEN>(ctx, filters, image, cw, ep);

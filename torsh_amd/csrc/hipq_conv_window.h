@@ -27,7 +27,8 @@
 //
 // Waves.  A workgroup's four waves either take different windows (SPLIT = false: FM x FN accumulator blocks each, the
 // filters' fragments coming out of L1 for three of the four) or split K and sum through LDS (SPLIT = true), which keeps
-// all SIMDs busy when there are fewer tiles than that.  A lane of the accumulators holds ONE output channel and 16
+// all SIMDs busy when there are fewer tiles than that; or eight waves split the K of one block, for few windows, where
+// latency is what counts.  A lane of the accumulators holds ONE output channel and 16
 // windows: its scale, bias and zero-point correction are one register each, and after one exchange between the halves
 // of the wave it owns 16 consecutive outputs of a channel's plane: one 16-byte store.
 #pragma once
@@ -207,13 +208,20 @@ __global__ __launch_bounds__(256) void conv_window_pack_kernel(const uint8_t *__
     }
 }
 
+// Waves of a workgroup: four, or eight where they share the K of one accumulator block.
+template <int FM, int FN, bool SPLIT>
+constexpr int conv_window_waves = SPLIT && FM * FN == 1 ? 8 : 4;
+
 template <int FM, int FN, int D, bool SPLIT, int EPI, bool EVEN>
-__global__ __launch_bounds__(256, FM * FN < 8 ? 3 : (SPLIT ? 1 : 2)) void conv_i8_window_kernel(const int8_t *__restrict__ filters,
+__global__ __launch_bounds__((64 * conv_window_waves<FM, FN, SPLIT>),
+                             FM * FN == 1 ? 2 : FM * FN < 8 ? 3 : (SPLIT ? 1 : 2)) void conv_i8_window_kernel(const int8_t *__restrict__ filters,
                                                                const int8_t *__restrict__ image, ConvWindow cw,
                                                                GemmEpilogue ep) {
     constexpr int NBLK = FM * FN;
-    constexpr int OWN = SPLIT ? NBLK / 4 : NBLK;  // accumulator blocks a wave finishes
-    static_assert(!SPLIT || (FM == 4 && FN == 2) || (FM == 2 && FN == 2) || (FM == 1 && FN == 4), "K-split tiles");
+    constexpr int WAVES = conv_window_waves<FM, FN, SPLIT>;
+    constexpr bool ONE = WAVES == 8;  // (wave 0 finishes the block)
+    constexpr int OWN = SPLIT && !ONE ? NBLK / 4 : NBLK;  // accumulator blocks a wave finishes
+    static_assert(!SPLIT || ONE || (FM == 4 && FN == 2) || (FM == 2 && FN == 2) || (FM == 1 && FN == 4), "K-split tiles");
     constexpr int COLS = SPLIT ? 1 : FM;          // channel blocks among them
     extern __shared__ __attribute__((aligned(16))) int8_t lds[];
     const int lane = threadIdx.x % kWave, half = lane / 32;
@@ -232,8 +240,8 @@ __global__ __launch_bounds__(256, FM * FN < 8 ? 3 : (SPLIT ? 1 : 2)) void conv_i
     // K-split: a wave numbers the tile's blocks by exclusive or with its own place, so that the blocks it will own after
     // the sum are its first ones and block b goes to wave `wave ^ (b / OWN)`: every wave runs the same code on the same
     // registers, no wave-dependent choice behind the main loop.
-    const int jx = !SPLIT ? 0 : FM == 4 ? wave : FM == 2 ? wave >> 1 : 0;
-    const int ix = !SPLIT ? 0 : FM == 4 ? 0 : FM == 2 ? wave & 1 : wave;
+    const int jx = !SPLIT || ONE ? 0 : FM == 4 ? wave : FM == 2 ? wave >> 1 : 0;
+    const int ix = !SPLIT || ONE ? 0 : FM == 4 ? 0 : FM == 2 ? wave & 1 : wave;
     // Operands of the epilogue, ahead of the main loop: one channel per lane and channel block.
     int corr[COLS];
     float sc[COLS], bias[COLS];
@@ -271,7 +279,7 @@ __global__ __launch_bounds__(256, FM * FN < 8 ? 3 : (SPLIT ? 1 : 2)) void conv_i
         voi[i] = ((n * cw.hp + oh * cw.sh) * cw.wp + ow * cw.sw) * cw.pitch + 16 * half;
     }
     // This wave's next k block as (tap row, piece, channel group) and its offset in the image.
-    constexpr int STEP = SPLIT ? 4 : 1;
+    constexpr int STEP = SPLIT ? WAVES : 1;
     int kb = 0, cg = 0, seg = 0, ty = 0;
     auto advance = [&](int by) {
         kb += by;
@@ -430,6 +438,28 @@ __global__ __launch_bounds__(256, FM * FN < 8 ? 3 : (SPLIT ? 1 : 2)) void conv_i
                     if ((rb0 + j) * 32 < cw.M)  // (a channel block past the last has no outputs)
                         emit_block(acc[j][i], j, (rb0 + j) * 32 + lane % 32, q0 + i * 32, plain);
         });
+    } else if constexpr (ONE) {
+        v4i *red = reinterpret_cast<v4i *>(lds);  // [wave - 1][register quad][lane]
+        if (wave > 0) {
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+                red[((wave - 1) * 4 + g) * kWave + lane] =
+                    v4i{acc[0][0][4 * g], acc[0][0][4 * g + 1], acc[0][0][4 * g + 2], acc[0][0][4 * g + 3]};
+        }
+        __syncthreads();
+        if (wave > 0) return;
+        v16i own;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) own[r] = acc[0][0][r] + corr[0];
+#pragma unroll
+        for (int s = 0; s < WAVES - 1; ++s)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const v4i part = red[(s * 4 + g) * kWave + lane];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) own[4 * g + i] += part[i];
+            }
+        with_division([&](auto plain) { emit_block(own, 0, rb0 * 32 + lane % 32, q0, plain); });
     } else {
         // Blocks OWN .. NBLK - 1 are other waves': parked in LDS as [owner][slot][register quad][lane].
         v4i *red = reinterpret_cast<v4i *>(lds);
@@ -470,7 +500,8 @@ __global__ __launch_bounds__(256, FM * FN < 8 ? 3 : (SPLIT ? 1 : 2)) void conv_i
 template <int FM, int FN, int D, bool SPLIT, int EPI, bool EVEN>
 static int32_t launch_conv_window_form(hipq_ctx *ctx, const int8_t *filters, const int8_t *image, const ConvWindow &cw,
                                        const GemmEpilogue &ep) {
-    constexpr int kLds = SPLIT ? FM * FN * 3 * 4096 : 0;
+    constexpr int kWaves = conv_window_waves<FM, FN, SPLIT>;
+    constexpr int kLds = SPLIT ? FM * FN * (kWaves - 1) * 4096 : 0;
     auto kernel = conv_i8_window_kernel<FM, FN, D, SPLIT, EPI, EVEN>;
     static bool configured[16] = {false};  // per device: raise the dynamic LDS limit once
     if (SPLIT && ctx->device < 16 && !configured[ctx->device]) {
@@ -482,7 +513,7 @@ static int32_t launch_conv_window_form(hipq_ctx *ctx, const int8_t *filters, con
     }
     constexpr int kTileN = (SPLIT ? 1 : 4) * FN * 32;
     const int tiles_m = ((cw.M + 31) / 32 + FM - 1) / FM, tiles_n = (cw.N + kTileN - 1) / kTileN;
-    hipLaunchKernelGGL(kernel, dim3((tiles_n + 7) / 8 * 8 * tiles_m), dim3(256), kLds, ctx->stream, filters, image, cw, ep);
+    hipLaunchKernelGGL(kernel, dim3((tiles_n + 7) / 8 * 8 * tiles_m), dim3(64 * kWaves), kLds, ctx->stream, filters, image, cw, ep);
     return check_launch("conv2d (windows)");
 }
 
