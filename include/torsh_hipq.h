@@ -228,7 +228,10 @@ HIPQ_API int32_t hipq_quantize_per_row_strided_f32_i8(hipq_ctx *ctx, const float
  * not finite sets *out_status and keeps what `out` held for it.  From 256 Ki
  * elements on, a channel axis that is not the leading one takes two range keys
  * per channel from the context's scratch memory (grown on first use), so calls
- * on one context must not overlap, as for every entry point that uses it. */
+ * on one context must not overlap, as for every entry point that uses it.
+ * Where the device's registers hold a channel (or the tensor) at once, x is read
+ * once: the workgroups of a channel wait for each other's ranges, a bounded time;
+ * one that waited in vain reads its channel's range itself (same result). */
 HIPQ_API int32_t hipq_quantize_per_channel_auto_f32_i8(hipq_ctx *ctx, const float *x, size_t outer,
                                                        size_t channels, size_t inner, int32_t flavor,
                                                        int32_t mode, int8_t *out, float *out_scales,

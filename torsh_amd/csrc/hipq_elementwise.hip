@@ -1087,7 +1087,8 @@ __global__ __launch_bounds__(kBlock) void channel_quantize_kernel(const float *_
 // part publishes its range as two tagged words of its own and waits for the words of its group's other parts, so groups do
 // not wait for each other.  No circle of waits: the items before a part's group are taken, by every workgroup, before it, so
 // the first unfinished group always has all its parts at work - given that the grid is resident at once and no smaller than
-// a group.  Bound by memory and by vector instructions, some twelve per element, which the workgroups of a compute unit
+// a group.  Where it is not (other work on the device), the wait ends after kPartLooks looks and the workgroup reads the whole
+// group's range itself: the same bits, later.  Bound by memory and by vector instructions, some twelve per element, which the workgroups of a compute unit
 // overlap as they drift apart: 64 x 256 x 3136 81.7 -> 58.4 us (75.5 in two passes with the same codes arithmetic), 4.4 TB/s.
 // Half the registers a lane and twice the workgroups: 67.1.
 struct ChannelParts {
@@ -1099,6 +1100,7 @@ struct ChannelParts {
 constexpr int kPartVec = 16;      // float4 a lane: what four workgroups per compute unit hold
 constexpr uint32_t kMostParts = 128;  // 64 x 32 x 12544 49 parts 40.4 -> 32.9 us, 256 x 16 x 6000 94 40.7 -> 34.8, 512 x 16 x 6000 188 72.5 -> 71.4
 constexpr uint32_t kPartTag = 1;
+constexpr int kPartLooks = 1 << 13;  // some milliseconds; a part is microseconds behind
 
 __global__ void channel_parts_init_kernel(unsigned long long *words, uint32_t n, int *status) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1111,7 +1113,7 @@ __global__ __launch_bounds__(kBlock, 4) void channel_parts_kernel(const float *_
                                                                   unsigned long long *words, int flavor, int qmin, int qmax,
                                                                   int8_t *__restrict__ out, float *__restrict__ out_scales,
                                                                   int32_t *__restrict__ out_zps, int32_t *__restrict__ out_status,
-                                                                  uint32_t *ctx_words, int spin_limit) {
+                                                                  int looks) {
     __shared__ float lds[2 * kBlock / kWave];
     const float4 *x4 = reinterpret_cast<const float4 *>(x);
     uint32_t *out4 = reinterpret_cast<uint32_t *>(out);
@@ -1145,7 +1147,6 @@ __global__ __launch_bounds__(kBlock, 4) void channel_parts_kernel(const float *_
             m.mx = fmaxf(m.mx, fmaxf(fmaxf(v[i].x, v[i].y), fmaxf(v[i].z, v[i].w)));
         }
         m = block_minmax(m, lds);
-        bool lost = false;
         if (cp.parts > 1) {
             unsigned long long *group = words + 2 * size_t(g) * cp.parts;
             if (threadIdx.x == 0) {
@@ -1153,26 +1154,31 @@ __global__ __launch_bounds__(kBlock, 4) void channel_parts_kernel(const float *_
                 publish_tagged(group + 2 * p + 1, kPartTag, __builtin_bit_cast(uint32_t, m.mx));
             }
             MinMax t{INFINITY, -INFINITY};
+            bool lost = false;
             if (threadIdx.x < cp.parts) {  // (at most kMostParts)
                 uint32_t lo = 0, hi = 0;
-                lost = !(poll_tagged(group + 2 * threadIdx.x, kPartTag, spin_limit, &lo) &&
-                         poll_tagged(group + 2 * threadIdx.x + 1, kPartTag, spin_limit, &hi));
+                lost = !(poll_tagged(group + 2 * threadIdx.x, kPartTag, looks, &lo) &&
+                         poll_tagged(group + 2 * threadIdx.x + 1, kPartTag, looks, &hi));
                 if (!lost) t = MinMax{__builtin_bit_cast(float, lo), __builtin_bit_cast(float, hi)};
             }
-            lost = __syncthreads_or(lost) != 0;
+            if (__syncthreads_or(lost)) {
+                for (uint32_t i = threadIdx.x; i < cp.vecs; i += kBlock) {
+                    uint32_t r;
+                    const uint32_t row = cp.by_run.quotient(i, &r);
+                    const float4 e = x4[row * cp.row_vecs + g * cp.run + r];
+                    t.mn = fminf(t.mn, fminf(fminf(e.x, e.y), fminf(e.z, e.w)));
+                    t.mx = fmaxf(t.mx, fmaxf(fmaxf(e.x, e.y), fmaxf(e.z, e.w)));
+                }
+            }
             m = block_minmax(t, lds);
         }
         float scale;
         int zp;
-        int st = params_from_minmax(m.mn, m.mx, flavor, qmin, qmax, &scale, &zp);
-        if (lost) st = HIPQ_DEVICE_ERROR;
-        if (threadIdx.x == 0) {
-            if (lost) record_give_up(ctx_words);
-            if (p == 0) {
-                if (out_scales) out_scales[g] = scale;
-                if (out_zps) out_zps[g] = zp;
-            }
-            if ((p == 0 || lost) && st != HIPQ_SUCCESS && out_status) *out_status = st;
+        const int st = params_from_minmax(m.mn, m.mx, flavor, qmin, qmax, &scale, &zp);
+        if (p == 0 && threadIdx.x == 0) {
+            if (out_scales) out_scales[g] = scale;
+            if (out_zps) out_zps[g] = zp;
+            if (st != HIPQ_SUCCESS && out_status) *out_status = st;
         }
         if (st != HIPQ_SUCCESS) continue;
         ChannelCodes<EVEN>(scale, zp, m.mn, m.mx, flavor, qmin, qmax).with([&](auto one) {
@@ -2033,7 +2039,8 @@ static int32_t quantize_channels(const char *fn, hipq_ctx *ctx, const float *x, 
             const dim3 grid(static_cast<unsigned>(items < resident ? items : resident));
             auto kernel = even ? channel_parts_kernel<true> : channel_parts_kernel<false>;
             hipLaunchKernelGGL(kernel, grid, dim3(kBlock), 0, ctx->stream, x, cp, words, flavor, qmin, qmax, out, out_scales,
-                               out_zero_points, out_status, ctx->wait_error, ctx->wait_spin_limit);
+                               out_zero_points, out_status,
+                               ctx->wait_spin_limit < kPartLooks ? ctx->wait_spin_limit : kPartLooks);
             return check_launch(fn);
         }
         ChannelColumns cc;
