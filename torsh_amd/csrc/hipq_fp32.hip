@@ -6,6 +6,7 @@
 #include "hipq_internal.h"
 #include "hipq_math.h"
 #include "hipq_panel_norm.h"
+#include "hipq_quantize_rows.h"
 
 namespace hipq {
 
@@ -48,24 +49,6 @@ __device__ __forceinline__ float row_max(float v, float *lds) {
         for (int w = 1; w < TPR / kWave; ++w) r = fmaxf(r, lds[w]);
         return r;
     }
-}
-
-// tanh-form GELU, crates/torsh-nn/src/layers/activation/modern.rs:124-136:
-//   0.5 * x * (1 + tanh(u)),  u = sqrt(2/pi) * (x + 0.044715 x^3).
-// Evaluated as x / (1 + exp(-2u)), which is the same function (1 + tanh(u) = 2 / (1 + exp(-2u)))
-// without the cancellation of 1 + tanh(u) for negative x, and costs one v_exp_f32 and one
-// v_rcp_f32 instead of a tanhf call: the fused GELU + quantize kernel was bound by tanhf, not by
-// HBM.  Against the reference's evaluation order in f32 the difference stays below 2e-6
-// relative + 1e-7 absolute (the reference form itself carries up to |x| * 3e-8 of cancellation
-// error).
-// -2u * log2(e) = x * (K + K*c*x^2) with K = -2*log2(e)*sqrt(2/pi): one multiply, one fused
-// multiply-add, one multiply (this function is compared at a tolerance, so the contraction is
-// allowed here).  No clamp of the exponent: exp2 saturates to inf / 0, and rcp(1 + inf) = 0,
-// rcp(1 + 0) = 1 give the right limits x * 0 and x.
-__device__ __forceinline__ float gelu_tanh(float x) {
-    constexpr float K = -2.8853900817779268f * 0.7978845608028654f;
-    const float arg = x * fmaf(x * x, K * 0.044715f, K);
-    return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(arg));
 }
 
 enum { ROW_LAYERNORM = 0, ROW_GELU = 1 };
@@ -412,6 +395,18 @@ int32_t panel_layer_norm_quantize_packed(hipq_ctx *ctx, const float *x, size_t r
 
 int32_t gelu_quantize_packed(hipq_ctx *ctx, const float *x, size_t rows, size_t cols, int32_t mode, int8_t *out_packed,
                              float *out_scales) {
+    // Rows of whole 128-byte k blocks, on which the two write the same operand.  Few long rows keep a workgroup per row: 12
+    // layers of the stack, us, row kernel / this: d_ff 3072 300 tokens 415 / 421, 640 537 / 526, 2048 848 / 826; 2048 16 tokens
+    // 279 / 287, 300 348 / 351, 1000 543 / 531; 1024 16 tokens 274 / 267, 300 310 / 302, 2048 485 / 471.
+    if (rows != 0 && rows >> 31 == 0 && cols != 0 && cols % 128 == 0 && cols <= size_t(kRowBlock) * kRowCacheMax * 4 &&
+        (cols <= 1024 || rows > size_t(ctx->num_cus) * 2) &&
+        ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(out_packed)) & 15u) == 0) {
+        if (mode & HIPQ_ROUND_HALF_EVEN)
+            launch_quantize_rows_packed<true, true>(ctx, x, rows, cols, cols, out_packed, out_scales);
+        else
+            launch_quantize_rows_packed<false, true>(ctx, x, rows, cols, cols, out_packed, out_scales);
+        return check_launch("gelu_quantize (packed)");
+    }
     return launch_row_op<ROW_GELU, true>("gelu_quantize (packed)", ctx, x, rows, cols, nullptr, nullptr, 0.0f, mode, nullptr,
                                          out_packed, out_scales, nullptr, nullptr, true);
 }

@@ -53,7 +53,7 @@ constexpr int kRowsWaves = 8;
 constexpr int kRowsThreads = kRowsWaves * kWave;
 constexpr int kRowsStage = 24;  // k blocks of the activation panel per LDS buffer (24 KiB)
 
-// tanh-form GELU as the row kernels evaluate it (gelu_tanh in hipq_fp32.hip: the same three lines).
+// tanh-form GELU as the row kernels evaluate it (gelu_tanh in hipq_quantize_rows.h: the same three lines).
 __device__ __forceinline__ float rp_gelu_tanh(float x) {
     constexpr float K = -2.8853900817779268f * 0.7978845608028654f;
     const float arg = x * fmaf(x * x, K * 0.044715f, K);

@@ -17,7 +17,26 @@ struct __attribute__((packed, aligned(4))) Floats4 {
     float v[4];
 };
 
-template <int LPR, int ROWS, int VPT, bool EVEN>
+// tanh-form GELU, crates/torsh-nn/src/layers/activation/modern.rs:124-136:
+//   0.5 * x * (1 + tanh(u)),  u = sqrt(2/pi) * (x + 0.044715 x^3).
+// Evaluated as x / (1 + exp(-2u)), which is the same function (1 + tanh(u) = 2 / (1 + exp(-2u)))
+// without the cancellation of 1 + tanh(u) for negative x, and costs one v_exp_f32 and one
+// v_rcp_f32 instead of a tanhf call: the fused GELU + quantize kernel was bound by tanhf, not by
+// HBM.  Against the reference's evaluation order in f32 the difference stays below 2e-6
+// relative + 1e-7 absolute (the reference form itself carries up to |x| * 3e-8 of cancellation
+// error).
+// -2u * log2(e) = x * (K + K*c*x^2) with K = -2*log2(e)*sqrt(2/pi): one multiply, one fused
+// multiply-add, one multiply (this function is compared at a tolerance, so the contraction is
+// allowed here).  No clamp of the exponent: exp2 saturates to inf / 0, and rcp(1 + inf) = 0,
+// rcp(1 + 0) = 1 give the right limits x * 0 and x.
+__device__ __forceinline__ float gelu_tanh(float x) {
+    constexpr float K = -2.8853900817779268f * 0.7978845608028654f;
+    const float arg = x * fmaf(x * x, K * 0.044715f, K);
+    return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(arg));
+}
+
+// GELU: of the activated row, with the scale of the row kernels (a row of NaN elements has the maximum 0).
+template <int LPR, int ROWS, int VPT, bool EVEN, bool GELU>
 __global__ __launch_bounds__(LPR *ROWS) void quantize_rows_packed_kernel(const float *__restrict__ x, unsigned rows, unsigned cols,
                                                                          size_t ld, int8_t *__restrict__ out,
                                                                          float *__restrict__ out_scales, unsigned dies) {
@@ -50,7 +69,13 @@ __global__ __launch_bounds__(LPR *ROWS) void quantize_rows_packed_kernel(const f
                 if (c + j < mine) v[i].v[j] = xr[c + j];
         }
     }
-    float mn = INFINITY, mx = -INFINITY;
+    if constexpr (GELU) {
+#pragma unroll
+        for (int i = 0; i < VPT; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[i].v[j] = gelu_tanh(v[i].v[j]);
+    }
+    float mn = GELU ? 0.0f : INFINITY, mx = GELU ? 0.0f : -INFINITY;
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
         mn = fminf(mn, fminf(fminf(v[i].v[0], v[i].v[1]), fminf(v[i].v[2], v[i].v[3])));
@@ -71,9 +96,16 @@ __global__ __launch_bounds__(LPR *ROWS) void quantize_rows_packed_kernel(const f
         }
     }
     float scale;
-    int zp;
+    [[maybe_unused]] int zp;
     // A row whose range is not finite gets a NaN scale and zero codes, so that every output of it is NaN.
-    const bool good = params_from_minmax(mn, mx, HIPQ_PARAMS_SYMMETRIC, -128, 127, &scale, &zp) == HIPQ_SUCCESS;
+    bool good;
+    if constexpr (GELU) {
+        const float am = fmaxf(fabsf(mn), fabsf(mx));
+        scale = am < FLT_EPSILON ? 1.0f : am / 127.0f;
+        good = am <= FLT_MAX;
+    } else {
+        good = params_from_minmax(mn, mx, HIPQ_PARAMS_SYMMETRIC, -128, 127, &scale, &zp) == HIPQ_SUCCESS;
+    }
     if (active && lane == 0) out_scales[row] = good ? scale : __builtin_nanf("");
     const float inv = recip_for_div(scale);
 #pragma unroll
@@ -101,20 +133,23 @@ constexpr size_t kRowsPackedMaxCols = 16384;
 // 15.3 / 13.6 (18.1).  Rows of up to 2048 floats: four, 8192 x 2048 16.0 / 17.9 (26.8).  Few rows want one each where a lane
 // holds four: 64 x 8000 4.7, two side by side 4.9 (6.5); 16 x 11008 5.0 (6.8).  Rows that start at an odd float lose nothing:
 // 4096 x 4095 16.8 (49.9).
-template <bool EVEN>
+// GELU is twice the vector work: a row per workgroup until there are four per compute unit (640 tokens at d_ff 3072).
+template <bool EVEN, bool GELU = false>
 static void launch_quantize_rows_packed(hipq_ctx *ctx, const float *x, size_t rows, size_t cols, size_t ld, int8_t *out,
                                         float *out_scales) {
     const size_t row_blocks = (rows + 31) / 32;
     const unsigned dies = row_blocks >= 16 ? 8 : 1;  // (fewer blocks: every die gets workgroups of each)
     const bool many = rows * cols > size_t(ctx->num_cus) * 2048 * 16;
 #define HIPQ_ROWS_PACKED(LPR, ROWS, VPT)                                                                                     \
-    hipLaunchKernelGGL((quantize_rows_packed_kernel<LPR, ROWS, VPT, EVEN>),                                                  \
+    hipLaunchKernelGGL((quantize_rows_packed_kernel<LPR, ROWS, VPT, EVEN, GELU>),                                            \
                        dim3(static_cast<unsigned>((row_blocks + dies - 1) / dies * dies * (32 / ROWS))), dim3(LPR * ROWS), 0, \
                        ctx->stream, x, static_cast<unsigned>(rows), static_cast<unsigned>(cols), ld, out, out_scales, dies)
     if (cols <= 1024)
         HIPQ_ROWS_PACKED(64, 4, 4);
     else if (cols <= 2048)
         HIPQ_ROWS_PACKED(128, 4, 4);
+    else if (GELU && cols <= 4096 && rows < size_t(ctx->num_cus) * 4)
+        HIPQ_ROWS_PACKED(256, 1, 4);
     else if (cols <= 4096 && !many)
         HIPQ_ROWS_PACKED(256, 4, 4);
     else if (cols <= 4096)
