@@ -46,7 +46,7 @@ HIPQ_API int32_t hipq_set_gemm_kernel_variant(hipq_ctx *ctx, int32_t variant);
  * silently (the quantizers also leave zero codes, a NaN scale and status HIPQ_DEVICE_ERROR in
  * out_params).  `limit` is the number of polls after the first look (negative = the default, 2^20);
  * 0 lets a test see the error path without hanging anything.  The per-channel quantizer over a middle axis waits
- * at most 2^13 polls and then reads its channel's range itself: no error there. */
+ * at most 2^13 polls, and a few once that was in vain, and then reads its channel's range itself: no error there. */
 HIPQ_API int32_t hipq_ctx_set_wait_spin_limit(hipq_ctx *ctx, int32_t limit);
 /* While a device buffer is set, hipq_linear_packed_i8_f32 (and the forwards built on it) run a
  * form of the packed GEMM kernel in which every wave records the shader clock at six points -

@@ -7,6 +7,7 @@
 #include "hipq_math.h"
 #include <type_traits>
 
+#include "hipq_channel_parts.h"
 #include "hipq_meeting.h"
 #include "hipq_quantize_rows.h"
 
@@ -1087,8 +1088,8 @@ __global__ __launch_bounds__(kBlock) void channel_quantize_kernel(const float *_
 // part publishes its range as two tagged words of its own and waits for the words of its group's other parts, so groups do
 // not wait for each other.  No circle of waits: the items before a part's group are taken, by every workgroup, before it, so
 // the first unfinished group always has all its parts at work - given that the grid is resident at once and no smaller than
-// a group.  Where it is not (other work on the device), the wait ends after kPartLooks looks and the workgroup reads the whole
-// group's range itself: the same bits, later.  Bound by memory and by vector instructions, some twelve per element, which the workgroups of a compute unit
+// a group.  Where it is not (other work on the device), the wait ends (PartPatience) and the workgroup reads the whole group's
+// range itself: the same bits, later.  Bound by memory and by vector instructions, some twelve per element, which the workgroups of a compute unit
 // overlap as they drift apart: 64 x 256 x 3136 81.7 -> 58.4 us (75.5 in two passes with the same codes arithmetic), 4.4 TB/s.
 // Half the registers a lane and twice the workgroups: 67.1.
 struct ChannelParts {
@@ -1097,10 +1098,8 @@ struct ChannelParts {
     uint32_t step_run, step_at;       // what kBlock float4s further on in the group is: run position (mod run) and address
     FastDiv by_run, by_parts;
 };
-constexpr int kPartVec = 16;      // float4 a lane: what four workgroups per compute unit hold
-constexpr uint32_t kMostParts = 128;  // 64 x 32 x 12544 49 parts 40.4 -> 32.9 us, 256 x 16 x 6000 94 40.7 -> 34.8, 512 x 16 x 6000 188 72.5 -> 71.4
+static_assert(kPartThreads == kBlock, "float4s of a part");
 constexpr uint32_t kPartTag = 1;
-constexpr int kPartLooks = 1 << 13;  // some milliseconds; a part is microseconds behind
 
 __global__ void channel_parts_init_kernel(unsigned long long *words, uint32_t n, int *status) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1113,10 +1112,11 @@ __global__ __launch_bounds__(kBlock, 4) void channel_parts_kernel(const float *_
                                                                   unsigned long long *words, int flavor, int qmin, int qmax,
                                                                   int8_t *__restrict__ out, float *__restrict__ out_scales,
                                                                   int32_t *__restrict__ out_zps, int32_t *__restrict__ out_status,
-                                                                  int looks) {
+                                                                  int most_looks) {
     __shared__ float lds[2 * kBlock / kWave];
     const float4 *x4 = reinterpret_cast<const float4 *>(x);
     uint32_t *out4 = reinterpret_cast<uint32_t *>(out);
+    PartPatience patience(most_looks);
     for (uint32_t item = blockIdx.x; item < cp.items; item += gridDim.x) {
         uint32_t p;
         const uint32_t g = cp.by_parts.quotient(item, &p);
@@ -1157,11 +1157,13 @@ __global__ __launch_bounds__(kBlock, 4) void channel_parts_kernel(const float *_
             bool lost = false;
             if (threadIdx.x < cp.parts) {  // (at most kMostParts)
                 uint32_t lo = 0, hi = 0;
+                const int looks = patience.looks(cp.parts);
                 lost = !(poll_tagged(group + 2 * threadIdx.x, kPartTag, looks, &lo) &&
                          poll_tagged(group + 2 * threadIdx.x + 1, kPartTag, looks, &hi));
                 if (!lost) t = MinMax{__builtin_bit_cast(float, lo), __builtin_bit_cast(float, hi)};
             }
             if (__syncthreads_or(lost)) {
+                patience.lost = true;
                 for (uint32_t i = threadIdx.x; i < cp.vecs; i += kBlock) {
                     uint32_t r;
                     const uint32_t row = cp.by_run.quotient(i, &r);
