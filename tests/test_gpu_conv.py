@@ -275,6 +275,8 @@ WINDOW_GEOMS = [
     # fewer k blocks than the four waves' register stages, K split (few windows) and not, 1 to 4 channel blocks per tile
     (2, 64, 7, 6, 130, (1, 1), (1, 1), (0, 0), 8), (1, 96, 8, 8, 40, (1, 1), (1, 1), (0, 0), 130), (3, 160, 5, 5, 96, (1, 1), (1, 1), (0, 0), 1),
     (1, 32, 9, 9, 20, (7, 1), (1, 1), (3, 0), 99), (1, 32, 2, 2, 33, (1, 1), (1, 1), (0, 0), 0),
+    # one block per workgroup: one channel group in several rounds of the eight waves, more groups than waves
+    (1, 32, 12, 11, 33, (7, 7), (1, 1), (3, 3), 17), (2, 300, 6, 7, 40, (3, 3), (2, 1), (1, 1), 40), (1, 3, 16, 16, 100, (11, 11), (4, 4), (2, 2), 6),
     (5, 32, 60, 58, 130, (1, 1), (1, 1), (0, 0), 8), (5, 96, 60, 58, 40, (1, 1), (1, 1), (0, 0), 7), (5, 20, 60, 58, 20, (1, 1), (1, 1), (0, 0), 255),
 ]
 

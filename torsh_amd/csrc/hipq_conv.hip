@@ -218,7 +218,8 @@ static bool window_geometry(const ConvGeom &g, ConvWindow *cw) {
     *cw = ConvWindow{g.oc, static_cast<int>(windows), static_cast<int>(KB), static_cast<int>(kblocks), static_cast<int>(cgs),
                      static_cast<int>(segs), static_cast<int>(pitch), static_cast<int>(wp * pitch), static_cast<int>(plane),
                      static_cast<int>(cgs * plane), static_cast<int>(hp), static_cast<int>(wp), g.sh, g.sw, g.ho, g.wo,
-                     FastDiv::by(static_cast<uint32_t>(g.ho) * g.wo), FastDiv::by(g.wo)};
+                     FastDiv::by(static_cast<uint32_t>(g.ho) * g.wo), FastDiv::by(g.wo),
+                     FastDiv::by(static_cast<uint32_t>(cgs)), FastDiv::by(static_cast<uint32_t>(segs))};
     return true;
 }
 
@@ -237,7 +238,9 @@ static int32_t launch_conv_window(hipq_ctx *ctx, const int8_t *filters, const in
     // tiles / this (blocks of 32 x 32): [1,128,14,17] x [128,128,5,5] 17.4 / 13.1 (32), [4,512,14,14] x [128,512,3,3] 19.3 / 13.4
     // (100), [4,224,24,25] x [85,224,3,3] 15.5 / 12.2 (225), x [512,512,3,3] 19.9 / 16.7 (400), 8 images 20.6 / 22.1 (784); up to
     // 64 channels, whose larger tile has four blocks, not eight: [11,192,10,11] x [49,192,5,5] 16.2 / 13.3 (76),
-    // [1,352,67,70] x [64,352,3,3] 15.1 / 15.3 (294), [1,32,71,74] x [37,32,7,7] 14.3 / 16.7 (330).
+    // [1,352,67,70] x [64,352,3,3] 15.1 / 15.3 (294).  Fewer k blocks than waves are no exception, 1 x 1 from u8 (k blocks):
+    // [1,32,7,7] x 32 8.2 / 7.8 (1), [4,32,28,28] x 128 9.2 / 8.5 (1), [3,64,5,5] x 128 10.0 / 8.5 (2), [32,96,7,7] x 256 10.3 /
+    // 9.2 (3).
     const size_t blocks = (size_t(cw.N) + 31) / 32 * ((size_t(cw.M) + 31) / 32);
     if (blocks <= (cw.M > 64 ? cus * 2 : cus)) return launch_conv_window_form<1, 1, 4, true, EPI, EVEN>(ctx, filters, image, cw, ep);
     if (tiles >= cus * 8 || (cw.kblocks < 8 && tiles > cus)) {

@@ -49,6 +49,7 @@ struct ConvWindow {
     int image_bytes;      // cgs * plane_bytes
     int hp, wp, sh, sw, ho, wo;
     FastDiv by_plane, by_wo;  // window -> (image, position), position -> (row, column)
+    FastDiv by_cgs, by_segs;  // k block -> (piece of all tap rows, channel group), -> (tap row, piece)
 };
 
 // 16, 4 x 4 and 4 bytes at an address that need not be aligned (global memory takes it; the outputs of a channel's plane
@@ -278,11 +279,20 @@ __global__ __launch_bounds__((64 * conv_window_waves<FM, FN, SPLIT>),
         const uint32_t n = cw.by_plane.quotient(q, &rem), oh = cw.by_wo.quotient(rem, &ow);
         voi[i] = ((n * cw.hp + oh * cw.sh) * cw.wp + ow * cw.sw) * cw.pitch + 16 * half;
     }
-    // This wave's next k block as (tap row, piece, channel group) and its offset in the image.
+    // This wave's next k block as (tap row, piece, channel group) and its offset in the image.  Steps of eight are divided,
+    // not counted: with one channel group (images of up to 32 channels) counting is eight turns of the loop for every step
+    // ahead of the first loads, us from u8 [4,32,28,28] x [128,32,1,1] 10.7 -> 8.5, [1,32,56,56] x [64,32,3,3] 9.0 -> 8.1.
     constexpr int STEP = SPLIT ? WAVES : 1;
     int kb = 0, cg = 0, seg = 0, ty = 0;
     auto advance = [&](int by) {
         kb += by;
+        if constexpr (ONE) {
+            uint32_t g, t;
+            ty = cw.by_segs.quotient(cw.by_cgs.quotient(kb, &g), &t);
+            cg = g;
+            seg = t;
+            return;
+        }
         cg += by;
         while (cg >= cw.cgs) {
             cg -= cw.cgs;
