@@ -353,9 +353,10 @@ def test_per_row_quantize(ctx, hipq, oracle, shape, flavor_name):
     np.testing.assert_array_equal(host(q), want_q.astype(np.int8))
 
 
-# Rows of odd length start anywhere in a vector of four: shorter than a vector, a wave's rows, a workgroup's, long ones
+# Rows of odd length start anywhere in a vector of four: shorter than a vector, up to two elements a lane (none are vectors) and
+# more, a wave's rows, a workgroup's, long ones
 # (registers hold 16384 floats), and enough elements for the streaming forms; bases that are aligned and not.
-@pytest.mark.parametrize("rows,cols", [(9, 1), (6, 3), (70, 33), (13, 1023), (9, 1027), (7, 4099), (5, 16387), (4500, 947), (2100, 2001),
+@pytest.mark.parametrize("rows,cols", [(9, 1), (6, 3), (70, 33), (70, 65), (41, 127), (39, 129), (13, 1023), (9, 1027), (7, 4099), (5, 16387), (4500, 947), (2100, 2001),
                                        (700, 6361)])
 @pytest.mark.parametrize("shift", [0, 1])
 def test_per_row_quantize_rows_of_odd_length(ctx, hipq, oracle, rows, cols, shift):

@@ -694,7 +694,7 @@ __global__ __launch_bounds__(kBlock) void quantize_per_row_kernel(const float *_
     constexpr int kRowsPerBlock = kBlock / TPR;
     constexpr int kCache = KC;
     __shared__ float lds[2 * kBlock / kWave];
-    const int sub = threadIdx.x / TPR, lane = threadIdx.x % TPR;
+    const int sub = __builtin_amdgcn_readfirstlane(threadIdx.x / TPR), lane = threadIdx.x % TPR;  // (a wave has one row)
     const size_t row = size_t(blockIdx.x) * kRowsPerBlock + sub;
     const bool active = row < rows;
     const float *xr = x + (active ? row : 0) * ld;  // input rows are ld elements apart, output is dense
@@ -706,17 +706,24 @@ __global__ __launch_bounds__(kBlock) void quantize_per_row_kernel(const float *_
     // Vectors of four: the whole row, or (rows of odd length without gaps, ld == cols: input and codes lie alike) what is left of it
     // behind the first `head` elements, up to the next multiple of four of the tensor.  The other elements one by one.
     // (One by one altogether, and long rows read twice, 2473 x 6361 took 36.4 us with these codes; quantize + dequantize 63.1 -> 37.5.)
+    // Odd rows of one or two elements a lane stay with that: elements / vectors, us, 6852 x 13 6.8 / 7.5, 300 x 33 5.3 / 5.8,
+    // 6852 x 127 7.3 / 7.6, but 715 x 255 6.3 / 5.8.
     const bool bases = ((reinterpret_cast<uintptr_t>(x) & 15u) == 0) && ((reinterpret_cast<uintptr_t>(out) & 3u) == 0);
-    const size_t gap = PACKED || ld != cols ? 0 : (0 - row * cols) % 4;
+    const bool odd_rows = !PACKED && ld == cols && cols > size_t(TPR) * 2;
+    const size_t gap = odd_rows ? (0 - row * cols) % 4 : 0;
     const size_t head = gap < cols ? gap : cols;
-    const size_t nvec = bases && (head == gap) && (PACKED || ld != cols ? cols % 4 == 0 && ld % 4 == 0 : true) ? (cols - head) / 4 : 0;
+    const size_t nvec = bases && head == gap && (odd_rows || (cols % 4 == 0 && ld % 4 == 0)) ? (cols - head) / 4 : 0;
     const size_t rest = nvec ? cols - nvec * 4 : cols;  // elements outside the vectors: head of them in front
     auto rest_at = [&](size_t i) { return nvec == 0 || i < head ? i : i + nvec * 4; };
     const float4 *x4 = reinterpret_cast<const float4 *>(xr + head);
 
     MinMax m{INFINITY, -INFINITY};
     float4 cache[kCache];
+    // The lane's first element outside the vectors (all there are, where there are vectors) is requested with them and held:
+    // one trip instead of three.
+    float edge = __builtin_nanf("");
     if (active) {
+        if (size_t(lane) < rest) edge = xr[rest_at(lane)];
 #pragma unroll
         for (int i = 0; i < kCache; ++i) {
             const size_t v = size_t(lane) + size_t(i) * TPR;
@@ -739,7 +746,8 @@ __global__ __launch_bounds__(kBlock) void quantize_per_row_kernel(const float *_
             acc_minmax(m, t.z);
             acc_minmax(m, t.w);
         }
-        for (size_t i = lane; i < rest; i += TPR) acc_minmax(m, xr[rest_at(i)]);
+        acc_minmax(m, edge);
+        for (size_t i = size_t(lane) + TPR; i < rest; i += TPR) acc_minmax(m, xr[rest_at(i)]);
     }
     if constexpr (TPR == kWave) {
         m.mn = wave_min(m.mn);
@@ -803,7 +811,8 @@ __global__ __launch_bounds__(kBlock) void quantize_per_row_kernel(const float *_
         if (v < nvec) put4(v, quant4(cache[i]));
     }
     for (size_t v = size_t(lane) + size_t(kCache) * TPR; v < nvec; v += TPR) put4(v, quant4(x4[v]));
-    for (size_t i = lane; i < rest; i += TPR) {
+    if (size_t(lane) < rest) put1(rest_at(lane), static_cast<int8_t>(quant1(edge)));
+    for (size_t i = size_t(lane) + TPR; i < rest; i += TPR) {
         const size_t c = rest_at(i);
         put1(c, static_cast<int8_t>(quant1(xr[c])));
     }
