@@ -200,7 +200,8 @@ def test_quantize_per_row_packed_matches_row_major(ctx, hipq, rows, cols):
         assert torch.equal(ps, s)
 
 
-@pytest.mark.parametrize("rows,cols", [(1, 1), (35, 1023), (550, 1024), (70, 1025), (513, 2048), (33, 2049), (530, 4096),
+@pytest.mark.parametrize("rows,cols", [(1, 1), (33, 129), (900, 255), (5, 256), (70, 257), (255, 1025), (256, 1030), (5, 2048), (255, 2049),
+                                       (256, 4095), (17, 4096), (35, 1023), (550, 1024), (70, 1025), (513, 2048), (33, 2049), (530, 4096),
                                        (2300, 4001), (33, 4097), (1100, 8190), (31, 8193), (1, 16384), (600, 16130), (2, 16385)])
 def test_quantize_per_row_packed_forms(ctx, hipq, rows, cols):
     """Every form of the packed per-row quantizer (by row length, and by whether the device holds the matrix at once) on

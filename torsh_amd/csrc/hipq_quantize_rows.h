@@ -130,9 +130,11 @@ constexpr size_t kRowsPackedMaxCols = 16384;
 // Four float4 a lane while the device's lanes hold the whole matrix like that at once (2048 lanes a compute unit), else eight
 // on half the lanes.  us, four / eight, inputs from memory: 1024 x 4096 6.7 / 7.4, 2048 x 4096 9.8 / 10.7, 4096 x 4096 17.3 /
 // 16.4 (a row per workgroup of 256, its codes stored where they lie: 28.3), 4096 x 11008 42.3 / 35.3 (60.3), 1000 x 11008
-// 15.3 / 13.6 (18.1).  Rows of up to 2048 floats: four, 8192 x 2048 16.0 / 17.9 (26.8).  Few rows want one each where a lane
-// holds four: 64 x 8000 4.7, two side by side 4.9 (6.5); 16 x 11008 5.0 (6.8).  Rows that start at an odd float lose nothing:
-// 4096 x 4095 16.8 (49.9).
+// 15.3 / 13.6 (18.1).  Rows of up to 2048 floats: four, 8192 x 2048 16.0 / 17.9 (26.8).  Rows that start at an odd float lose
+// nothing: 4096 x 4095 16.8 (49.9).
+// Few rows want a workgroup each: 64 x 8000 4.7, two side by side 4.9 (6.5); 16 x 11008 5.0 (6.8); 16 x 3072 4.4, four side by side
+// 5.1 (4.6); 1 x 2048 4.1, 4.4 (4.2); as many as compute units they are even, 300 x 2100 5.3, 5.3 (5.3).  Short rows want one
+// float4 a lane, the others are work for nothing: 6852 x 128 5.4, four 6.6 (5.4); 2667 x 54 4.3, 4.9 (4.5).
 // GELU is twice the vector work: a row per workgroup until there are four per compute unit (640 tokens at d_ff 3072).
 template <bool EVEN, bool GELU = false>
 static void launch_quantize_rows_packed(hipq_ctx *ctx, const float *x, size_t rows, size_t cols, size_t ld, int8_t *out,
@@ -140,15 +142,20 @@ static void launch_quantize_rows_packed(hipq_ctx *ctx, const float *x, size_t ro
     const size_t row_blocks = (rows + 31) / 32;
     const unsigned dies = row_blocks >= 16 ? 8 : 1;  // (fewer blocks: every die gets workgroups of each)
     const bool many = rows * cols > size_t(ctx->num_cus) * 2048 * 16;
+    const bool few = rows < size_t(ctx->num_cus) * (GELU ? 4 : 1);
 #define HIPQ_ROWS_PACKED(LPR, ROWS, VPT)                                                                                     \
     hipLaunchKernelGGL((quantize_rows_packed_kernel<LPR, ROWS, VPT, EVEN, GELU>),                                            \
                        dim3(static_cast<unsigned>((row_blocks + dies - 1) / dies * dies * (32 / ROWS))), dim3(LPR * ROWS), 0, \
                        ctx->stream, x, static_cast<unsigned>(rows), static_cast<unsigned>(cols), ld, out, out_scales, dies)
-    if (cols <= 1024)
+    if (cols <= 256)
+        HIPQ_ROWS_PACKED(64, 4, 1);
+    else if (cols <= 1024)
         HIPQ_ROWS_PACKED(64, 4, 4);
+    else if (!GELU && cols <= 2048 && few)
+        HIPQ_ROWS_PACKED(256, 1, 2);
     else if (cols <= 2048)
         HIPQ_ROWS_PACKED(128, 4, 4);
-    else if (GELU && cols <= 4096 && rows < size_t(ctx->num_cus) * 4)
+    else if (cols <= 4096 && few)
         HIPQ_ROWS_PACKED(256, 1, 4);
     else if (cols <= 4096 && !many)
         HIPQ_ROWS_PACKED(256, 4, 4);
