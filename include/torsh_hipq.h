@@ -226,11 +226,14 @@ HIPQ_API int32_t hipq_quantize_per_row_strided_f32_i8(hipq_ctx *ctx, const float
 /* quantize_per_channel_auto for any axis of a dense tensor viewed as
  * [outer, channels, inner] (algorithms.rs:126-242).  A channel whose range is
  * not finite sets *out_status and keeps what `out` held for it.  From 256 Ki
- * elements on, a channel axis that is not the leading one takes two range keys
- * per channel from the context's scratch memory (grown on first use), so calls
- * on one context must not overlap, as for every entry point that uses it.
- * Where the device's registers hold a channel (or the tensor) at once, x is read
- * once: the workgroups of a channel wait for each other's ranges, a bounded time;
+ * elements on, a channel axis that is not the leading one uses the context's
+ * scratch memory, so calls on one context must not overlap, as for every entry
+ * point that uses it: two range keys per channel (the scratch grows on first use
+ * where it has no room for them), or, where the device's registers hold a channel
+ * (or the tensor) at once and x is read once, two 64-bit words per 64 KiB of a
+ * channel, never more than every context has.  Which of the two depends on the shape,
+ * the alignment and the context's share of the device alone.  In the second form
+ * the workgroups of a channel wait for each other's ranges, a bounded time;
  * one that waited in vain reads its channel's range itself (same result). */
 HIPQ_API int32_t hipq_quantize_per_channel_auto_f32_i8(hipq_ctx *ctx, const float *x, size_t outer,
                                                        size_t channels, size_t inner, int32_t flavor,

@@ -117,7 +117,7 @@ def test_one_multiply_add_requantize_equals_the_exact_chain():
 
 
 def test_rules_of_the_per_channel_quantizer_that_reads_once():
-    """How long a workgroup waits for the others of its channel, on the CPU."""
+    """Which views are read once and how long a workgroup waits for the others of its channel, on the CPU."""
     subprocess.run(["make", "-C", os.path.join(ROOT, "tests", "host"), "bin/channel_parts_check"], check=True, capture_output=True)
     proc = subprocess.run([os.path.join(ROOT, "tests", "host", "bin", "channel_parts_check")], capture_output=True, text=True,
                           timeout=60)

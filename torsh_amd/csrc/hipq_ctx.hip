@@ -163,7 +163,7 @@ static int32_t ctx_new(int32_t device, hipStream_t stream, bool own, hipq_ctx **
     }
     void *p = nullptr;
     int32_t rc = hipq::linear_noalloc_setup(device);
-    if (rc == HIPQ_SUCCESS) rc = hipq::scratch(ctx, size_t(8) << 20, &p);
+    if (rc == HIPQ_SUCCESS) rc = hipq::scratch(ctx, hipq::kScratchAtCreation, &p);
     if (rc == HIPQ_SUCCESS) {
         e = hipMalloc(reinterpret_cast<void **>(&ctx->wait_error), hipq::kCtxWordsBytes);
         if (e != hipSuccess)

@@ -1091,7 +1091,6 @@ __global__ __launch_bounds__(kBlock) void channel_quantize_kernel(const float *_
     });
 }
 
-// Explicit per-channel parameters over a dense [outer, channels, inner] view.
 // ---- the same with the input read once: a group's elements stay in the registers of the `parts` workgroups that share it
 // while those agree on its range.  Item g * parts + p is part p of group g; a workgroup takes every gridDim-th item.  Each
 // part publishes its range as two tagged words of its own and waits for the words of its group's other parts, so groups do
@@ -1201,6 +1200,7 @@ __global__ __launch_bounds__(kBlock, 4) void channel_parts_kernel(const float *_
     }
 }
 
+// Explicit per-channel parameters over a dense [outer, channels, inner] view.
 template <bool DIV, bool EVEN>
 __global__ __launch_bounds__(kBlock) void quantize_per_channel_kernel(const float *__restrict__ x, size_t total,
                                                                        size_t channels, size_t inner,
@@ -2018,36 +2018,28 @@ static int32_t quantize_channels(const char *fn, hipq_ctx *ctx, const float *x, 
     if (spread) {
         const bool vec = inner % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15u) == 0 &&
                          (reinterpret_cast<uintptr_t>(out) & 3u) == 0;
-        // The input read once, where the device's registers hold it at once, or where runs are long enough that parts share
-        // few lines and the parts fill a third of the registers.  us, two passes / once: [500,30,300] 31.0 / 14.2, [64,40,1000]
-        // 21.6 / 14.2, [100,1000,128] 21.5 / 16.6; several rounds: [2,4096,4096] 58.9 / 37.8, [32,2048,768] 75.8 / 60.0,
-        // [2,8000,3000] (0.37 of the registers) 84 / 70, [4,8192,1024] (0.25) 54.4 / 55.2, [2,8192,1024] (0.12) 34.8 / 44.0,
-        // [128,1024,196] 39.4 / 40.8, [8,8192,400] 42 / 61.  No more context scratch than the smallest block of it.
-        constexpr size_t kPartVecs = size_t(kPartVec) * kBlock;
-        const size_t run = group * inner, vecs = outer * run / 4, parts = (vecs + kPartVecs - 1) / kPartVecs, items = parts * groups;
-        const size_t resident = resident_workgroups(ctx, true), words_at = kScratchHeader;
-        const size_t words_end = words_at + (parts > 1 ? 2 * items * sizeof(unsigned long long) : 0);
-        if (vec && channels % group == 0 && run >= 128 && parts <= kMostParts && parts <= resident &&
-            outer * period / 4 < (size_t(1) << 31) && (items <= resident || (run >= 512 && vecs >= parts * (kPartVecs * 5 / 16))) &&
-            (words_end <= (size_t(1) << 20) || words_end <= ctx->scratch_bytes) && four_wide_workgroups_fit(ctx)) {
+        ChannelPartsPlan plan;
+        const size_t resident = resident_workgroups(ctx, true);
+        if (vec && plan_channel_parts(outer, channels, inner, group, resident, kScratchAtCreation - kScratchHeader, &plan) &&
+            four_wide_workgroups_fit(ctx)) {
             ChannelParts cp;
-            cp.items = static_cast<uint32_t>(items);
-            cp.parts = static_cast<uint32_t>(parts);
-            cp.per_part = static_cast<uint32_t>((vecs + parts - 1) / parts);
-            cp.vecs = static_cast<uint32_t>(vecs);
+            cp.items = static_cast<uint32_t>(plan.items);
+            cp.parts = static_cast<uint32_t>(plan.parts);
+            cp.per_part = static_cast<uint32_t>((plan.vecs + plan.parts - 1) / plan.parts);
+            cp.vecs = static_cast<uint32_t>(plan.vecs);
             cp.row_vecs = static_cast<uint32_t>(period / 4);
-            cp.run = static_cast<uint32_t>(run / 4);
+            cp.run = static_cast<uint32_t>(plan.run / 4);
             cp.step_run = kBlock % cp.run;
             cp.step_at = kBlock / cp.run * cp.row_vecs + cp.step_run;
             cp.by_run = FastDiv::by(cp.run);
             cp.by_parts = FastDiv::by(cp.parts);
             void *s = nullptr;
-            if ((rc = scratch(ctx, words_end, &s))) return rc;
-            unsigned long long *words = reinterpret_cast<unsigned long long *>(static_cast<char *>(s) + words_at);
-            const uint32_t nwords = static_cast<uint32_t>((words_end - words_at) / sizeof(unsigned long long));
+            if ((rc = scratch(ctx, kScratchHeader + plan.words * sizeof(unsigned long long), &s))) return rc;
+            unsigned long long *words = reinterpret_cast<unsigned long long *>(static_cast<char *>(s) + kScratchHeader);
+            const uint32_t nwords = static_cast<uint32_t>(plan.words);
             hipLaunchKernelGGL(channel_parts_init_kernel, dim3(nwords / kBlock + 1), dim3(kBlock), 0, ctx->stream, words, nwords,
                                out_status);
-            const dim3 grid(static_cast<unsigned>(items < resident ? items : resident));
+            const dim3 grid(static_cast<unsigned>(plan.items < resident ? plan.items : resident));
             auto kernel = even ? channel_parts_kernel<true> : channel_parts_kernel<false>;
             hipLaunchKernelGGL(kernel, grid, dim3(kBlock), 0, ctx->stream, x, cp, words, flavor, qmin, qmax, out, out_scales,
                                out_zero_points, out_status,

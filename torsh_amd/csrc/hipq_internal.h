@@ -168,6 +168,8 @@ bool four_wide_workgroups_fit(const hipq_ctx *ctx);
 // Bytes reserved at the head of the context scratch for small device records
 // (hipq_qparams, min/max pairs, status words); bulk scratch starts after it.
 constexpr size_t kScratchHeader = 4096;
+// Bytes of scratch that hipq_ctx_create gives a context.
+constexpr size_t kScratchAtCreation = size_t(8) << 20;
 
 }  // namespace hipq
 
