@@ -4,6 +4,7 @@ against the mirrored C++ API, and parity of the device results with the CPU orac
 The program is built ahead of time (``make -C tests/host``, also done by ``__graft_entry__.build()``); it is built
 here only when no binary exists.  It runs once per session; each case is reported as its own pytest test."""
 import os
+import re
 import subprocess
 
 import pytest
@@ -122,6 +123,17 @@ def test_rules_of_the_per_channel_quantizer_that_reads_once():
     proc = subprocess.run([os.path.join(ROOT, "tests", "host", "bin", "channel_parts_check")], capture_output=True, text=True,
                           timeout=60)
     assert proc.returncode == 0, proc.stdout + proc.stderr
+
+
+def test_every_kernel_that_must_be_resident_at_once_is_asked_about():
+    """The kernels of the quantizers that are built for four workgroups per compute unit, because their workgroups wait for each
+    other, are the ones whose occupancy decides whether they are taken."""
+    text = open(os.path.join(ROOT, "torsh_amd", "csrc", "hipq_elementwise.hip")).read()
+    kernels = set(re.findall(r"__launch_bounds__\(kBlock, 4\) void (\w+)\(", text))
+    assert len(kernels) >= 3
+    asked = text[text.index("bool four_wide_workgroups_fit("):]
+    asked = asked[:asked.index("\n}\n")]
+    assert kernels <= set(re.findall(r"\b(\w+)<", asked)), kernels
 
 
 def _run(args):

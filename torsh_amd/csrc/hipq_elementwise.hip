@@ -499,23 +499,6 @@ __global__ __launch_bounds__(kBlock, 4) void quantize_flat_one_launch_kernel(con
     }
 }
 
-// The one-launch quantizers that hold 64 floats a lane need four workgroups per compute unit resident: what the
-// runtime says about the widest flat form (the packed one has the same launch bound), asked once per device -
-// hipq_ctx_create does, so that no later call (one under stream capture, say) is the first to ask.
-bool four_wide_workgroups_fit(const hipq_ctx *ctx) {
-    static int resident[16] = {0};  // workgroups per compute unit; 0 = not asked yet, -1 = the query failed
-    if (ctx->device < 0 || ctx->device >= 16) return false;
-    if (resident[ctx->device] == 0) {
-        int a = 0, b = 0;
-        const hipError_t ea = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &a, reinterpret_cast<const void *>(quantize_flat_one_launch_kernel<int8_t, false, 0, 16>), kBlock, 0);
-        const hipError_t eb = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &b, reinterpret_cast<const void *>(quantize_packed_one_launch_kernel<false, 0, 4>), kBlock, 0);
-        resident[ctx->device] = (ea == hipSuccess && eb == hipSuccess && a > 0 && b > 0) ? (a < b ? a : b) : -1;
-    }
-    return resident[ctx->device] >= 4;
-}
-
 // Launches the kernel above when the call qualifies (returns true), else leaves the two-launch path to the caller.
 // The grid must be resident at once: at most four workgroups per compute unit, which the kernel's launch bound
 // makes room for; checked against the runtime's own occupancy figure the first time.
@@ -1198,6 +1181,28 @@ __global__ __launch_bounds__(kBlock, 4) void channel_parts_kernel(const float *_
             });
         });
     }
+}
+
+// The quantizers that hold 64 floats a lane and whose workgroups wait for each other need four workgroups per compute unit
+// resident: the least that the runtime says about the widest forms, asked once per device - hipq_ctx_create does, so that no
+// later call (one under stream capture, say) is the first to ask.
+bool four_wide_workgroups_fit(const hipq_ctx *ctx) {
+    static int resident[16] = {0};  // workgroups per compute unit; 0 = not asked yet, -1 = a query failed
+    if (ctx->device < 0 || ctx->device >= 16) return false;
+    if (resident[ctx->device] == 0) {
+        const void *wide[] = {reinterpret_cast<const void *>(quantize_flat_one_launch_kernel<int8_t, false, 0, 16>),
+                              reinterpret_cast<const void *>(quantize_packed_one_launch_kernel<false, 0, 4>),
+                              reinterpret_cast<const void *>(channel_parts_kernel<false>),
+                              reinterpret_cast<const void *>(channel_parts_kernel<true>)};
+        int least = 1 << 30;
+        for (const void *kernel : wide) {
+            int n = 0;
+            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, kBlock, 0) != hipSuccess || n <= 0) n = -1;
+            if (n < least) least = n;
+        }
+        resident[ctx->device] = least;
+    }
+    return resident[ctx->device] >= 4;
 }
 
 // Explicit per-channel parameters over a dense [outer, channels, inner] view.
