@@ -512,3 +512,22 @@ def test_few_tiles_with_k_split_between_the_waves(ctx, oracle, m, n, k, shift_a,
         np.testing.assert_array_equal(host(ctx.linear_i8_i8(ad, sad, wd, swd, bd, s_out, -5)), wantq)
     finally:
         ctx.set_gemm_kernel_variant(0)
+
+
+@pytest.mark.parametrize("m,n,k", [(300, 1000, 1001), (128, 1024, 1024)])
+def test_hook_of_the_operand_lines_leaves_the_product_alone(stream_ctx, launched_kernels, m, n, k):
+    """Hook 11 switches off the touching of operand lines and nothing else: a row-major product keeps its kernel.  Hook 9 takes the
+    K-split form away."""
+    a, w = (torch.zeros((r, k), dtype=torch.int8, device="cuda") for r in (m, n))
+    out = torch.empty((m, n), dtype=torch.int32, device="cuda")
+    torch.cuda.synchronize()
+    kernels = {}
+    try:
+        for hook in (0, 9, 11):
+            stream_ctx.set_gemm_kernel_variant(hook)
+            kernels[hook] = launched_kernels(stream_ctx, lambda: stream_ctx.gemm_i8_i32(a, w, out=out))
+    finally:
+        stream_ctx.set_gemm_kernel_variant(0)
+    assert len(kernels[0]) == 1 and "split_i8_rows_kernel" in kernels[0][0]
+    assert kernels[11] == kernels[0]
+    assert "split_i8_rows_kernel" not in kernels[9][0]

@@ -289,11 +289,6 @@ static void launch_tile(hipq_ctx *ctx, const int8_t *a, const int8_t *w, int M, 
     hipLaunchKernelGGL(kernel, dim3(tiles_m * tiles_n), dim3(kGemmThreads), 0, ctx->stream, a, w, M, N, K, placed);
 }
 
-// Tuning and test hook, per context: HIPQ_GEMM_VARIANT=<n> in the environment (read when the context is
-// created), or hipq_set_gemm_kernel_variant(ctx, n), forces one kernel configuration wherever the shape
-// allows it (0 = automatic).
-static int gemm_variant_override(hipq_ctx *ctx) { return ctx->gemm_variant; }
-
 // The tile of the K-split form (hipq_gemm_split.h).  Its time is the operand bytes a compute unit asks for: 16 (FM + FN)
 // per byte of K and workgroup (`blocks` = FM + FN), times the workgroups a compute unit gets (`cost`).
 struct SplitForm {
@@ -327,8 +322,10 @@ static int32_t launch_gemm(hipq_ctx *ctx, const int8_t *a, const int8_t *w, size
     }
     const size_t cus = static_cast<size_t>(ctx->num_cus);
     auto tiles = [&](size_t bm, size_t bn) { return ((m + bm - 1) / bm) * ((n + bn - 1) / bn); };
-    int variant = gemm_variant_override(ctx);
-    if (variant == 9 || variant == 11) variant = 0;  // switches of the packed forms only
+    // Test and tuning hook (torsh_hipq_testing.h): one kernel form wherever the shape allows it; 9 and 11 leave the choice
+    // automatic, 9 without the K-split form above 16 rows.
+    const bool automatic = ctx->gemm_variant == 0 || ctx->gemm_variant == 9 || ctx->gemm_variant == 11;
+    int variant = automatic ? 0 : ctx->gemm_variant;
     // Rows at any alignment: the K-split form while its tiles are few, else the register-staged tile (load_row_piece).
     if (!fast) variant = variant == 4 || M <= 16 ? 4 : 10;
     // Few tiles: the K-split form, whose time grows with `cost` (pick_split_form) and K where the tiled kernels walk a chain
@@ -344,7 +341,7 @@ static int32_t launch_gemm(hipq_ctx *ctx, const int8_t *a, const int8_t *w, size
     // replaced / split): 1 x 11008 x 4001 20.1 / 10.6, 16 x 4096 x 4032 5.7 / 5.5, 1 x 32000 x 1008 11.9 / 6.9, 8 x 300 x 300
     // 3.8 / 3.2.
     if (variant == 0 && M <= 16) variant = 4;
-    if (ctx->gemm_variant == 0 && M > 16) {
+    if (automatic && ctx->gemm_variant != 9 && M > 16) {
         const size_t cost = pick_split_form(tiles, cus).cost;
         const bool few_steps = EPI == EPI_I32 && K <= 128;
         const size_t most = !fast                                       ? (few_steps ? 6 : 10)
