@@ -489,6 +489,48 @@ def test_per_channel_auto_input_read_once(ctx, hipq, outer, channels, inner):
     assert torch.equal(out[:, :channels - 1], want_q[:, :channels - 1])
 
 
+# Several parts per group AND more items than the 1024 resident workgroups: a workgroup waits at every item it takes, for words of
+# later groups, and goes on past a group without a range.  Groups of several channels, in one round and in more.
+@pytest.mark.parametrize("outer,channels,inner,group", [(64, 100, 3136, 1), (32, 1040, 768, 1), (4, 900, 8196, 3), (90, 60, 200, 5),
+                                                        (160, 24, 132, 4)])
+@pytest.mark.parametrize("limit", [-1, 0])
+def test_per_channel_auto_input_read_once_in_rounds(hipq, stream_ctx, launched_kernels, outer, channels, inner, group, limit):
+    """The per-row quantizer's codes and parameters on the groups as rows, whether the parts of a group wait for each other or read its
+    range themselves; a group in the middle holds an infinity."""
+    groups, c = channels // group, stream_ctx
+    torch.cuda.synchronize()
+    with torch.cuda.stream(torch.cuda.ExternalStream(c.stream_handle)):
+        g = torch.Generator(device="cuda").manual_seed(outer + channels + inner)
+        x = torch.randn(outer, groups, group * inner, generator=g, device="cuda") * torch.linspace(0.2, 3.0, groups, device="cuda")[:, None]
+        x[outer - 1, :, group * inner - 1] = torch.linspace(-30.0, 40.0, groups, device="cuda")  # in every group's last part
+        x[outer // 2, groups // 2, 5] = float("inf")
+        rows = x.transpose(0, 1).reshape(groups, outer * group * inner).contiguous()
+        out = torch.full(x.shape, 77, dtype=torch.int8, device="cuda")
+        scales, zps = torch.empty(groups, device="cuda"), torch.empty(groups, dtype=torch.int32, device="cuda")
+        status = torch.empty(1, dtype=torch.int32, device="cuda")
+
+        def call():
+            c.call("hipq_quantize_per_group_auto_f32_i8", x.data_ptr(), outer, channels, inner, group, hipq.PARAMS_AFFINE, -128, 127, 0,
+                   out.data_ptr(), scales.data_ptr(), zps.data_ptr(), status.data_ptr())
+
+        want_q, want_s, want_z, _ = c.quantize_per_row(rows, hipq.PARAMS_AFFINE)
+        good = torch.arange(groups, device="cuda") != groups // 2
+        try:
+            c.set_wait_spin_limit(limit)
+            for _ in range(2):
+                out.fill_(77)
+                call()
+                assert int(status) == hipq.INVALID_ARGUMENT
+                assert (out[:, ~good] == 77).all()
+                assert torch.equal(out[:, good], want_q.view(groups, outer, group * inner).transpose(0, 1)[:, good])
+                assert torch.equal(scales[good], want_s[good]) and torch.equal(zps[good], want_z[good])
+            c.synchronize()  # no wait is reported
+        finally:
+            c.set_wait_spin_limit(-1)
+        torch.cuda.synchronize()
+        assert "channel_parts_kernel" in launched_kernels(c, call)[-1]
+
+
 def test_per_channel_auto_input_read_once_without_waiting_and_replays(hipq):
     """Parts that stop waiting read their group's range themselves: the same bits and no error; a captured call gives the eager
     call's bits on every replay."""

@@ -11,6 +11,7 @@ import torch
 pytestmark = pytest.mark.gpu
 
 RTOL = 1e-5
+ROUND_HALF_EVEN = 1  # hipq.ROUND_HALF_EVEN
 
 
 def dev(a):
@@ -118,10 +119,11 @@ def test_quantized_linear_forward(ctx, hipq, oracle, m, n, k, per_token):
     np.testing.assert_array_equal(got, oracle.linear_dequant_epilogue(acc, sa, sw, None))
 
 
-# K % 128 == 0 reaches the pipelined kernel, whose int8 epilogue stores dwords when N % 4 == 0 (ragged M and N tiles
-# included) and bytes otherwise; the other shapes reach the register-staged and the generic kernels.
+# Few tiles: the K-split form.  The last three have too many: the pipelined kernel, whose int8 epilogue stores dwords when
+# N % 4 == 0 (ragged M and N tiles included) and bytes otherwise, and the register-staged one.
 @pytest.mark.parametrize("m,n,k", [(7, 24, 64), (128, 96, 512), (50, 130, 272), (50, 100, 256), (130, 132, 384),
-                                   (67, 130, 256), (300, 260, 128), (512, 1024, 1024)])
+                                   (67, 130, 256), (300, 260, 128), (512, 1024, 1024), (1030, 1100, 384), (1030, 1101, 400),
+                                   (1030, 1101, 393)])
 def test_quantized_linear_requant_epilogue(ctx, hipq, oracle, m, n, k):
     x, wf, bias, wq, sw, aq, sa, acc, out = _quantized_linear_case(oracle, m, n, k, False, 5 * m + k)
     s_out, _ = oracle.calculate_symmetric_params(*oracle.find_min_max(out), 0)
@@ -308,7 +310,7 @@ def test_every_gemm_kernel_form_gives_the_same_bits(ctx, hipq, oracle, variant):
     the oracle's accumulators and epilogue outputs bit for bit (interior and ragged tiles, all four epilogues)."""
     try:
         ctx.set_gemm_kernel_variant(variant)
-        for (m, n, k) in ((300, 200, 256), (1024, 768, 512), (130, 2304, 256)):
+        for (m, n, k) in ((300, 200, 256), (1024, 768, 512), (130, 2304, 256), (300, 203, 256)):
             rng = np.random.default_rng(variant * 1000 + m)
             a, w = rand_i8(rng, (m, k)), rand_i8(rng, (n, k))
             acc = oracle.gemm_i8_nk(a, w)
@@ -322,8 +324,9 @@ def test_every_gemm_kernel_form_gives_the_same_bits(ctx, hipq, oracle, variant):
             got = host(ctx.linear_i8_f32_residual(dev(a), dev(sa), dev(w), dev(sw), dev(bias), dev(res)))
             np.testing.assert_array_equal(got, want + res)
             s_out, _ = oracle.calculate_symmetric_params(*oracle.find_min_max(want), 0)
-            wantq = oracle.requantize_epilogue(acc, sa, sw, bias, s_out, -5)
-            np.testing.assert_array_equal(host(ctx.linear_i8_i8(dev(a), dev(sa), dev(w), dev(sw), dev(bias), s_out, -5)), wantq)
+            for mode, wantq in _both_roundings(oracle, acc, sa, sw, bias, s_out, -5):
+                got = host(ctx.linear_i8_i8(dev(a), dev(sa), dev(w), dev(sw), dev(bias), s_out, -5, mode))
+                np.testing.assert_array_equal(got, wantq)
     finally:
         ctx.set_gemm_kernel_variant(0)
     with pytest.raises(hipq.HipqError):
@@ -431,8 +434,30 @@ def test_empty_reduction(hipq, oracle, m, n):
         c.close()
 
 
-def _check_every_epilogue(c, oracle, m, n, k):
-    """Accumulators, dequantize with and without a residual, requantize of one row-major product against the oracle."""
+def _at(a, shift):
+    """A device copy of `a` whose first byte lies `shift` bytes behind a 16-byte boundary, other values behind its end."""
+    buf = torch.full((a.size + 96,), 77, dtype=torch.int8, device="cuda")
+    start = -buf.data_ptr() % 16 + shift
+    out = buf[start:start + a.size].view(a.shape)
+    out.copy_(torch.from_numpy(a))
+    return out
+
+
+def _both_roundings(oracle, acc, sa, sw, bias, s_out, zp):
+    """[(mode, codes)] of the requantize epilogue: ties away from zero, ties to even."""
+    codes = []
+    for mode in (0, ROUND_HALF_EVEN):
+        oracle.set_round_mode(1 if mode else 0)
+        try:
+            codes.append((mode, oracle.requantize_epilogue(acc, sa, sw, bias, s_out, zp)))
+        finally:
+            oracle.set_round_mode(0)
+    return codes
+
+
+def _check_every_epilogue(c, oracle, m, n, k, shift_a=0, shift_w=0):
+    """Accumulators, dequantize with and without a residual, requantize with both roundings of one row-major product against
+    the oracle."""
     rng = np.random.default_rng(m + n + k)
     a, w = rand_i8(rng, (m, k)), rand_i8(rng, (n, k))
     acc = oracle.gemm_i8_nk(a, w)
@@ -442,12 +467,12 @@ def _check_every_epilogue(c, oracle, m, n, k):
     res = rng.standard_normal((m, n)).astype(np.float32)
     want = oracle.linear_dequant_epilogue(acc, sa, sw, bias)
     s_out, _ = oracle.calculate_symmetric_params(*oracle.find_min_max(want), 0)
-    wantq = oracle.requantize_epilogue(acc, sa, sw, bias, s_out, -5)
-    ad, wd, sad, swd, bd = dev(a), dev(w), dev(sa), dev(sw), dev(bias)
+    ad, wd, sad, swd, bd = _at(a, shift_a), _at(w, shift_w), dev(sa), dev(sw), dev(bias)
     np.testing.assert_array_equal(host(c.gemm_i8_i32(ad, wd)), acc)
     np.testing.assert_array_equal(host(c.linear_i8_f32(ad, sad, wd, swd, bd)), want)
     np.testing.assert_array_equal(host(c.linear_i8_f32_residual(ad, sad, wd, swd, bd, dev(res))), want + res)
-    np.testing.assert_array_equal(host(c.linear_i8_i8(ad, sad, wd, swd, bd, s_out, -5)), wantq)
+    for mode, wantq in _both_roundings(oracle, acc, sa, sw, bias, s_out, -5):
+        np.testing.assert_array_equal(host(c.linear_i8_i8(ad, sad, wd, swd, bd, s_out, -5, mode)), wantq)
 
 
 @pytest.mark.parametrize("k", [16, 64, 112, 128, 144, 320])
@@ -478,40 +503,42 @@ def test_shapes_beside_the_dispatch_lines(ctx, oracle, m, n, k):
     _check_every_epilogue(ctx, oracle, m, n, k)
 
 
-def _at(a, shift):
-    """A device copy of `a` whose first byte lies `shift` bytes behind a 16-byte boundary."""
-    buf = torch.empty(a.size + 32, dtype=torch.int8, device="cuda")
-    start = -buf.data_ptr() % 16 + shift
-    out = buf[start:start + a.size].view(a.shape)
-    out.copy_(torch.from_numpy(a))
-    return out
-
-
 # one shape for each tile of the K-split form, rows and columns that no tile divides; K below, at and beside a step of 128
 # bytes and a round of all waves (1024 / 512 bytes), and of no step at all
 @pytest.mark.parametrize("m,n", [(7, 33), (41, 1702), (99, 1301), (201, 1503), (497, 1500)])
 @pytest.mark.parametrize("k,shift_a,shift_w", [(16, 0, 0), (17, 1, 3), (64, 4, 0), (79, 0, 2), (128, 0, 0), (131, 2, 1), (512, 0, 4),
                                                (513, 3, 0), (1001, 0, 0), (1024, 1, 1), (1100, 0, 0)])
 def test_few_tiles_with_k_split_between_the_waves(ctx, oracle, m, n, k, shift_a, shift_w):
-    rng = np.random.default_rng(m + n + k)
-    a, w = rand_i8(rng, (m, k)), rand_i8(rng, (n, k))
-    acc = oracle.gemm_i8_nk(a, w)
-    sa = (rng.random(m) * 0.05 + 0.001).astype(np.float32)
-    sw = (rng.random(n) * 0.002 + 0.0001).astype(np.float32)
-    bias = (rng.standard_normal(n) * 0.01).astype(np.float32)
-    res = rng.standard_normal((m, n)).astype(np.float32)
-    want = oracle.linear_dequant_epilogue(acc, sa, sw, bias)
-    s_out, _ = oracle.calculate_symmetric_params(*oracle.find_min_max(want), 0)
-    wantq = oracle.requantize_epilogue(acc, sa, sw, bias, s_out, -5)
-    ad, wd, sad, swd, bd = _at(a, shift_a), _at(w, shift_w), dev(sa), dev(sw), dev(bias)
     try:
         ctx.set_gemm_kernel_variant(4)
-        np.testing.assert_array_equal(host(ctx.gemm_i8_i32(ad, wd)), acc)
-        np.testing.assert_array_equal(host(ctx.linear_i8_f32(ad, sad, wd, swd, bd)), want)
-        np.testing.assert_array_equal(host(ctx.linear_i8_f32_residual(ad, sad, wd, swd, bd, dev(res))), want + res)
-        np.testing.assert_array_equal(host(ctx.linear_i8_i8(ad, sad, wd, swd, bd, s_out, -5)), wantq)
+        _check_every_epilogue(ctx, oracle, m, n, k, shift_a, shift_w)
     finally:
         ctx.set_gemm_kernel_variant(0)
+
+
+# (the lists of the tests of rows at any alignment, above the rows of the K-split form)
+@pytest.mark.parametrize("m,n,k", [(17, 64, 31), (64, 65, 127), (65, 130, 129), (130, 4200, 143), (33, 90, 257), (300, 200, 1023), (70, 33, 16),
+                                   (65, 66, 17)])
+@pytest.mark.parametrize("shift_a,shift_w", [(0, 0), (1, 1), (4, 3), (0, 2)])
+def test_register_staged_tile_any_k_and_alignment(ctx, oracle, m, n, k, shift_a, shift_w):
+    """The register-staged tile, which few tiles no longer reach by themselves: pieces of rows at any alignment, the piece over a
+    row's end shifted down."""
+    try:
+        ctx.set_gemm_kernel_variant(10)
+        _check_every_epilogue(ctx, oracle, m, n, k, shift_a, shift_w)
+    finally:
+        ctx.set_gemm_kernel_variant(0)
+
+
+# Too many tiles for the K-split form: one shape for each tile of the register-staged form, its last tiles not whole.
+@pytest.mark.parametrize("m,n,tile", [(500, 2100, 64), (2000, 1100, 12864), (2900, 2901, 128)])
+@pytest.mark.parametrize("k,shift_a,shift_w", [(65, 0, 0), (143, 1, 3), (144, 4, 0)])
+def test_many_tiles_of_rows_at_any_alignment(stream_ctx, ctx, oracle, launched_kernels, m, n, tile, k, shift_a, shift_w):
+    bm, bn = {64: (64, 64), 128: (128, 128), 12864: (128, 64)}[tile]
+    a, w = (_at(np.zeros((r, k), np.int8), s) for r, s in ((m, shift_a), (n, shift_w)))
+    kernel = launched_kernels(stream_ctx, lambda: stream_ctx.gemm_i8_i32(a, w))[0]
+    assert f"gemm_i8_mfma_kernelILi{bm}ELi{bn}E" in kernel and (f"Lb{int(k % 16 != 0)}EEEv" in kernel), kernel
+    _check_every_epilogue(ctx, oracle, m, n, k, shift_a, shift_w)
 
 
 @pytest.mark.parametrize("m,n,k", [(300, 1000, 1001), (128, 1024, 1024)])
