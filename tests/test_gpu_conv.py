@@ -315,7 +315,10 @@ def test_conv_any_stride_and_channel_count(ctx, hipq, oracle, nb, c, h, w, oc, k
 @pytest.mark.parametrize("nb,c,h,w,oc,k,stride,pad,zp", [
     (8, 32, 32, 32, 30, (1, 1), (1, 1), (0, 0), 3), (8, 17, 32, 33, 30, (3, 3), (1, 1), (1, 1), 90),
     (4, 64, 32, 32, 60, (1, 1), (1, 1), (0, 0), 128), (4, 288, 33, 32, 60, (1, 1), (1, 1), (0, 0), 128),
-    (4, 40, 32, 32, 128, (3, 3), (1, 1), (1, 1), 0), (4, 40, 33, 32, 128, (3, 3), (1, 1), (1, 1), 255)])
+    (4, 40, 32, 32, 128, (3, 3), (1, 1), (1, 1), 0), (4, 40, 33, 32, 128, (3, 3), (1, 1), (1, 1), 255),
+    # the larger K-split tiles with fewer k blocks than waves and with many, which fewer windows no longer give them
+    (8, 32, 32, 33, 30, (1, 1), (1, 1), (0, 0), 4), (4, 64, 33, 32, 60, (1, 1), (1, 1), (0, 0), 129), (4, 96, 33, 32, 130, (1, 1), (1, 1), (0, 0), 31),
+    (8, 100, 33, 32, 20, (3, 3), (1, 1), (1, 1), 66), (4, 64, 33, 32, 60, (7, 7), (1, 1), (3, 3), 2), (4, 200, 33, 32, 129, (3, 3), (1, 1), (1, 1), 8)])
 def test_conv_at_the_limits_of_one_block_per_workgroup(ctx, hipq, oracle, nb, c, h, w, oc, k, stride, pad, zp):
     test_conv_any_stride_and_channel_count(ctx, hipq, oracle, nb, c, h, w, oc, k, stride, pad, zp)
 
