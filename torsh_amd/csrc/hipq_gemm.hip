@@ -356,14 +356,13 @@ static int32_t launch_gemm(hipq_ctx *ctx, const int8_t *a, const int8_t *w, size
     // register-staged: 2267 x 1268 x 16 8.7 / 6.2, 616 x 6464 x 352 10.7 / 10.0; with rows that are no whole number of 16
     // bytes it is the number of tiles that decides (50 of them 4.7 / 3.8, 110 5.0 / 5.3, 190 5.6 / 7.5), and many tiles are
     // better not persistent: 1625 x 3159 x 48 14.8 / 13.4, 8108 x 1562 x 128 35 / 26, 7350 x 4037 x 48 93 / 71 (persistent /
-    // pipelined).  Int8 results of a few tiles of such rows: 1040 x 330 x 160 9.1 / 8.2.  Fp32 results: never.
+    // pipelined).  Int8 and fp32 results: never.
     if (variant == 0 && EPI == EPI_I32 && K <= 512) {
         if (tiles(128, 64) < 2 * cus && (N % 4 == 0 || tiles(128, 64) <= cus / 4))
             variant = 10;
         else if (N % 4 != 0)
             variant = 2;
     }
-    if (variant == 0 && EPI == EPI_I8 && K <= 256 && M > 32 && N % 4 != 0 && tiles(128, 64) <= cus / 4) variant = 10;
     // The LDS-pipelined kernels for every K that is a multiple of 16 (a last K-tile that runs over the rows is filled
     // with zeros).  Against the register-staged tile, us: 512 x 4096 x 4112 37 / 20, 300 x 1000 x 1008 14.6 / 7.6,
     // 8192 x 3072 x 320 73 / 29, x 64 66 / 25, 100 x 1408 x 192 10.5 / 6.1, 50 x 300 x 64 6.0 / 5.7.
@@ -411,11 +410,11 @@ static int32_t launch_gemm(hipq_ctx *ctx, const int8_t *a, const int8_t *w, size
     case 4:
         if (M > 16 * 65535) break;  // (row tiles are the grid's y)
         switch (pick_split_form(tiles, cus).blocks) {
-        case 2: return launch_split_rows<1, 1, 8, 1, 2, EPI, EVEN>(ctx, a, w, M, N, K, ep);
-        case 3: return launch_split_rows<1, 2, 8, 1, 2, EPI, EVEN>(ctx, a, w, M, N, K, ep);
-        case 4: return launch_split_rows<2, 2, 4, 1, 2, EPI, EVEN>(ctx, a, w, M, N, K, ep);
-        case 6: return launch_split_rows<4, 2, 4, 1, 2, EPI, EVEN>(ctx, a, w, M, N, K, ep);
-        default: return launch_split_rows<4, 4, 4, 1, 2, EPI, EVEN>(ctx, a, w, M, N, K, ep);
+        case 2: return launch_split_rows<1, 1, 8, 2, EPI, EVEN>(ctx, a, w, M, N, K, ep);
+        case 3: return launch_split_rows<1, 2, 8, 2, EPI, EVEN>(ctx, a, w, M, N, K, ep);
+        case 4: return launch_split_rows<2, 2, 4, 2, EPI, EVEN>(ctx, a, w, M, N, K, ep);
+        case 6: return launch_split_rows<4, 2, 4, 2, EPI, EVEN>(ctx, a, w, M, N, K, ep);
+        default: return launch_split_rows<4, 4, 4, 2, EPI, EVEN>(ctx, a, w, M, N, K, ep);
         }
     default: break;
     }

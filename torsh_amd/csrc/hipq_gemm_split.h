@@ -3,7 +3,7 @@
 // A product of few tiles is latency: a tiled kernel walks K with one or two K-tiles in flight and leaves compute units
 // idle.  Here a workgroup of WK waves owns a tile of 16 FM x 16 FN outputs, wave w takes the steps w, w + WK, ... of
 // 64 P bytes of K and loads its rows' pieces straight into the operand registers of v_mfma_i32_16x16x64_i8 (no LDS:
-// nothing is shared between waves that split K), D steps requested at once, and the partial sums meet in LDS once.  A lane
+// nothing is shared between waves that split K), a step in flight per wave, and the partial sums meet in LDS once.  A lane
 // takes 16 P consecutive bytes of its row per step (the sums do not care which bytes of K share an MFMA, as long as both
 // operands agree), which is what makes odd rows affordable: they need one dword more per P pieces.
 //
@@ -155,7 +155,7 @@ constexpr int split_rows_lds_bytes() {
 }
 
 // SHIFT: rows that are not all dword aligned.
-template <int FM, int FN, int WK, int D, int EPI, bool EVEN, bool SHIFT, int P>
+template <int FM, int FN, int WK, int EPI, bool EVEN, bool SHIFT, int P>
 __global__ __launch_bounds__(64 * WK) void split_i8_rows_kernel(const int8_t *__restrict__ A, const int8_t *__restrict__ W,
                                                                 int M, int N, int K, GemmEpilogue ep) {
     constexpr int BLOCKS = FM * FN, PER_WAVE = (BLOCKS + WK - 1) / WK;
@@ -175,25 +175,24 @@ __global__ __launch_bounds__(64 * WK) void split_i8_rows_kernel(const int8_t *__
         const int n = n0 + 16 * j + frow;
         wp[j] = RowStart(W + size_t(n < N ? n : N - 1) * K);
     }
-    ShiftedPieces<P> fa[D][FM], fw[D][FN];
+    ShiftedPieces<P> fa[FM], fw[FN];
     const int whole = K / (64 * P);  // steps of 64 bytes; what is left is one more, taken by the wave whose turn it is
-    auto issue = [&](int s, int slot) {  // step wave + WK * s; past the last: nothing is read, zeros
+    auto issue = [&](int s) {  // step wave + WK * s; past the last: nothing is read, zeros
         const int step = wave + WK * s;
         if (step < whole) {
             const int k = (step * 64 + 16 * g) * P;
 #pragma unroll
-            for (int i = 0; i < FM; ++i) fa[slot][i] = ap[i].template load<SHIFT, P>(k);
+            for (int i = 0; i < FM; ++i) fa[i] = ap[i].template load<SHIFT, P>(k);
 #pragma unroll
-            for (int j = 0; j < FN; ++j) fw[slot][j] = wp[j].template load<SHIFT, P>(k);
+            for (int j = 0; j < FN; ++j) fw[j] = wp[j].template load<SHIFT, P>(k);
         } else {
 #pragma unroll
-            for (int i = 0; i < FM; ++i) fa[slot][i] = ShiftedPieces<P>{};
+            for (int i = 0; i < FM; ++i) fa[i] = ShiftedPieces<P>{};
 #pragma unroll
-            for (int j = 0; j < FN; ++j) fw[slot][j] = ShiftedPieces<P>{};
+            for (int j = 0; j < FN; ++j) fw[j] = ShiftedPieces<P>{};
         }
     };
-#pragma unroll
-    for (int u = 0; u < D; ++u) issue(u, u);
+    issue(0);
     // Block b = (b / FN, b % FN) of the tile is finished by wave b % WK; a lane holds row lane % 16, channels 4 g .. 4 g + 3.
     EpilogueOperands eo[PER_WAVE];
     if constexpr (EPI != EPI_I32) {
@@ -215,14 +214,14 @@ __global__ __launch_bounds__(64 * WK) void split_i8_rows_kernel(const int8_t *__
 #pragma unroll
             for (int j = 0; j < FN; ++j) acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w[j], a[i], acc[i][j], 0, 0, 0);
     };
-    auto multiply_slot = [&](int u) {
+    auto multiply_step = [&]() {
 #pragma unroll
         for (int p = 0; p < P; ++p) {
             v4i a[FM], w[FN];
 #pragma unroll
-            for (int i = 0; i < FM; ++i) a[i] = SHIFT ? fa[u][i].get(p, ap[i].shift) : fa[u][i].v[p];
+            for (int i = 0; i < FM; ++i) a[i] = SHIFT ? fa[i].get(p, ap[i].shift) : fa[i].v[p];
 #pragma unroll
-            for (int j = 0; j < FN; ++j) w[j] = SHIFT ? fw[u][j].get(p, wp[j].shift) : fw[u][j].v[p];
+            for (int j = 0; j < FN; ++j) w[j] = SHIFT ? fw[j].get(p, wp[j].shift) : fw[j].v[p];
             multiply(a, w);
         }
     };
@@ -243,16 +242,12 @@ __global__ __launch_bounds__(64 * WK) void split_i8_rows_kernel(const int8_t *__
         for (int j = 0; j < FN; ++j) w[j] = tw[j].get();
         multiply(a, w);
     }
-    const int steps = (whole + WK - 1) / WK, rounds_end = (steps + D - 1) / D * D;
-    for (int s0 = D; s0 < rounds_end; s0 += D) {
-#pragma unroll
-        for (int u = 0; u < D; ++u) {
-            multiply_slot(u);
-            issue(s0 + u, u);
-        }
+    const int steps = (whole + WK - 1) / WK;
+    for (int s = 1; s < steps; ++s) {
+        multiply_step();
+        issue(s);
     }
-#pragma unroll
-    for (int u = 0; u < D; ++u) multiply_slot(u);
+    multiply_step();
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
@@ -269,12 +264,12 @@ __global__ __launch_bounds__(64 * WK) void split_i8_rows_kernel(const int8_t *__
     }
 }
 
-template <int FM, int FN, int WK, int D, int P, int EPI, bool EVEN>
+template <int FM, int FN, int WK, int P, int EPI, bool EVEN>
 static int32_t launch_split_rows(hipq_ctx *ctx, const int8_t *a, const int8_t *w, int M, int N, int K, const GemmEpilogue &ep) {
     constexpr int kLds = split_rows_lds_bytes<FM, FN, WK>();
     static_assert(kLds <= 65536, "no more LDS than a kernel may have without asking");
     const bool dwords = K % 4 == 0 && ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(w)) & 3u) == 0;
-    auto kernel = dwords ? split_i8_rows_kernel<FM, FN, WK, D, EPI, EVEN, false, P> : split_i8_rows_kernel<FM, FN, WK, D, EPI, EVEN, true, P>;
+    auto kernel = dwords ? split_i8_rows_kernel<FM, FN, WK, EPI, EVEN, false, P> : split_i8_rows_kernel<FM, FN, WK, EPI, EVEN, true, P>;
     const dim3 grid((N + 16 * FN - 1) / (16 * FN), (M + 16 * FM - 1) / (16 * FM));
     hipLaunchKernelGGL(kernel, grid, dim3(64 * WK), kLds, ctx->stream, a, w, M, N, K, ep);
     return check_launch("gemm_i8 (split)");
