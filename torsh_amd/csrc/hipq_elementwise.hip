@@ -697,7 +697,7 @@ __global__ __launch_bounds__(kBlock) void quantize_per_row_kernel(const float *_
     const size_t head = gap < cols ? gap : cols;
     const size_t nvec = bases && head == gap && (odd_rows || (cols % 4 == 0 && ld % 4 == 0)) ? (cols - head) / 4 : 0;
     const size_t rest = nvec ? cols - nvec * 4 : cols;  // elements outside the vectors: head of them in front
-    auto rest_at = [&](size_t i) { return nvec == 0 || i < head ? i : i + nvec * 4; };
+    auto rest_at = [&](size_t i) { return i < head ? i : i + nvec * 4; };
     const float4 *x4 = reinterpret_cast<const float4 *>(xr + head);
 
     MinMax m{INFINITY, -INFINITY};
@@ -705,8 +705,9 @@ __global__ __launch_bounds__(kBlock) void quantize_per_row_kernel(const float *_
     // The lane's first element outside the vectors (all there are, where there are vectors) is requested with them and held:
     // one trip instead of three.
     float edge = __builtin_nanf("");
+    const int edges = static_cast<int>(rest < size_t(TPR) ? rest : size_t(TPR));
     if (active) {
-        if (size_t(lane) < rest) edge = xr[rest_at(lane)];
+        if (lane < edges) edge = xr[rest_at(lane)];
 #pragma unroll
         for (int i = 0; i < kCache; ++i) {
             const size_t v = size_t(lane) + size_t(i) * TPR;
@@ -730,7 +731,8 @@ __global__ __launch_bounds__(kBlock) void quantize_per_row_kernel(const float *_
             acc_minmax(m, t.w);
         }
         acc_minmax(m, edge);
-        for (size_t i = size_t(lane) + TPR; i < rest; i += TPR) acc_minmax(m, xr[rest_at(i)]);
+        if (nvec == 0)
+            for (size_t i = size_t(lane) + TPR; i < cols; i += TPR) acc_minmax(m, xr[i]);
     }
     if constexpr (TPR == kWave) {
         m.mn = wave_min(m.mn);
@@ -794,11 +796,9 @@ __global__ __launch_bounds__(kBlock) void quantize_per_row_kernel(const float *_
         if (v < nvec) put4(v, quant4(cache[i]));
     }
     for (size_t v = size_t(lane) + size_t(kCache) * TPR; v < nvec; v += TPR) put4(v, quant4(x4[v]));
-    if (size_t(lane) < rest) put1(rest_at(lane), static_cast<int8_t>(quant1(edge)));
-    for (size_t i = size_t(lane) + TPR; i < rest; i += TPR) {
-        const size_t c = rest_at(i);
-        put1(c, static_cast<int8_t>(quant1(xr[c])));
-    }
+    if (lane < edges) put1(rest_at(lane), static_cast<int8_t>(quant1(edge)));
+    if (nvec == 0)
+        for (size_t c = size_t(lane) + TPR; c < cols; c += TPR) put1(c, static_cast<int8_t>(quant1(xr[c])));
     if constexpr (PACKED)
         for (size_t c = cols + lane; c < kpad; c += TPR) put1(c, int8_t(0));  // k padding: zeros add nothing
 }
