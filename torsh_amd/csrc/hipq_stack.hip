@@ -202,10 +202,12 @@ int32_t hipq_transformer_stack_forward_prepared_f32(hipq_ctx *ctx, const hipq_bl
 
     int32_t rc;
     // Row panels are 32 (or 64) rows of one workgroup (or pair), so a forward of few tokens leaves compute units idle and
-    // every busy one streams the whole weight matrices: 1.5-1.65 ms for 12 layers at d 768, d_ff 3072 whatever the
+    // every busy one streams the whole weight matrices: 1.6-1.9 ms for 12 layers at d 768, d_ff 3072 whatever the
     // number of tokens, up to 8192.  The separate tiled products and row kernels grow with it instead, us (panels / tiled):
-    //   d 768, d_ff 3072:  77 1510 / 366, 1000 1590 / 640, 4096 1660 / 1270, 8192 1835 / 2120
-    //   d 256, d_ff 1024:  77 635 / 480, 4096 660 / 630, 8192 705 / 860;   d 1024: 77 2425 / 590, 8192 2730 / 2700
+    //   d 768, d_ff 3072:  77 1665 / 333, 1000 1638 / 631, 4096 1646 / 1253, 5120 1678 / 1490, 6144 1733 / 1844, 8192 1920 / 2329
+    //   d 256, d_ff 1024:  77 624 / 285, 4096 647 / 604, 5120 652 / 724, 8192 693 / 900
+    //   d 512, d_ff 2048:  4096 1072 / 911, 5120 1092 / 1044, 6144 1124 / 1190;   d 1024, d_ff 3072: 77 2405 / 411, 5120 2390 / 1861,
+    //                      6144 2451 / 2267, 8192 2721 / 2874
     // so the panels are taken when they fill five eighths of the device, and where a workspace sized for them alone has no
     // room for fc1's output.  Both give the same bits.  (Test hook 15: panels always.)
     const bool room = workspace_bytes - ahead >= tokens * d_ff * sizeof(float);
