@@ -272,7 +272,7 @@ WINDOW_GEOMS = [
     (2, 3, 6, 4, 20, (3, 3), (1, 1), (5, 5), 31),        # rows of one run of four pixels, runs wholly inside the border
     (3, 70, 4, 3, 8, (3, 1), (1, 1), (1, 2), 12),        # rows shorter than a run: a pixel per thread
     (2, 32, 5, 9, 32, (1, 3), (1, 2), (0, 1), 250),      # a whole group of 32 channels, rows of 2 1/4 runs
-    # fewer k blocks than the four waves' register stages, K split (few windows) and not, 1 to 4 channel blocks per tile
+    # fewer k blocks than the waves and their register stages: one block per workgroup (few windows) and a wave on its own windows
     (2, 64, 7, 6, 130, (1, 1), (1, 1), (0, 0), 8), (1, 96, 8, 8, 40, (1, 1), (1, 1), (0, 0), 130), (3, 160, 5, 5, 96, (1, 1), (1, 1), (0, 0), 1),
     (1, 32, 9, 9, 20, (7, 1), (1, 1), (3, 0), 99), (1, 32, 2, 2, 33, (1, 1), (1, 1), (0, 0), 0),
     # one block per workgroup: one channel group in several rounds of the eight waves, more groups than waves

@@ -531,6 +531,40 @@ def test_per_channel_auto_input_read_once_in_rounds(hipq, stream_ctx, launched_k
         assert "channel_parts_kernel" in launched_kernels(c, call)[-1]
 
 
+def test_per_channel_auto_input_read_once_by_two_contexts_at_once(hipq):
+    """Two contexts that launch together without having been told of each other: each grid may find part of the device taken, and a
+    workgroup whose partners do not come reads its group's range itself.  The results are those of an idle device, and neither
+    context reports anything."""
+    contexts = [hipq.Context(0, own_stream=True) for _ in range(2)]
+    try:
+        xs = [torch.randn(64, 100, 3136, device="cuda") * (i + 1) for i in range(2)]
+        outs = [[(torch.empty(x.shape, dtype=torch.int8, device="cuda"), torch.empty(100, device="cuda"),
+                  torch.empty(100, dtype=torch.int32, device="cuda"), torch.empty(1, dtype=torch.int32, device="cuda")) for _ in range(4)]
+                for x in xs]
+        torch.cuda.synchronize()
+
+        def call(i, k):
+            contexts[i].call("hipq_quantize_per_channel_auto_f32_i8", xs[i].data_ptr(), 64, 100, 3136, hipq.PARAMS_SYMMETRIC, 0,
+                             *(t.data_ptr() for t in outs[i][k]))
+
+        for i, c in enumerate(contexts):  # alone
+            call(i, 0)
+            c.synchronize()
+        for k in (1, 2, 3):
+            for i in range(2):
+                call(i, k)
+        for c in contexts:
+            c.synchronize()
+        for i in range(2):
+            for k in (1, 2, 3):
+                assert all(torch.equal(a, b) for a, b in zip(outs[i][0], outs[i][k])), (i, k)
+            assert int(outs[i][0][3]) == 0
+    finally:
+        torch.cuda.synchronize()
+        for c in contexts:
+            c.close()
+
+
 def test_per_channel_auto_input_read_once_without_waiting_and_replays(hipq):
     """Parts that stop waiting read their group's range themselves: the same bits and no error; a captured call gives the eager
     call's bits on every replay."""

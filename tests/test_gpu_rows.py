@@ -599,8 +599,8 @@ def test_prepared_stack_row_operations_in_front_of_the_products(hipq, tokens, d,
         c.close()
 
 
-# Each form of the GELU quantizer: rows of up to 1024 floats, few long rows (a row kernel), a row per workgroup, four, eight float4 a lane.
-@pytest.mark.parametrize("tokens,dff", [(9, 1024), (512, 1152), (513, 1152), (513, 2176), (1030, 3072), (2800, 3072)])
+# Each form of the GELU quantizer: rows of up to 256 and of up to 1024 floats, few long rows (a row kernel), a row per workgroup, four, eight float4 a lane.
+@pytest.mark.parametrize("tokens,dff", [(33, 128), (70, 256), (70, 384), (9, 1024), (512, 1152), (513, 1152), (513, 2176), (1030, 3072), (2800, 3072)])
 def test_prepared_stack_forms_of_the_gelu_quantizer(hipq, tokens, dff):
     test_prepared_stack_row_operations_in_front_of_the_products(hipq, tokens, 128, dff)
 
