@@ -183,6 +183,27 @@ def test_quantize_per_tensor_packed_matches_row_major(ctx, hipq, rows, cols):
         assert ctx.read_qparams(sp).scale == np.float32(0.037)
 
 
+# One, two and four fragments a wave and more than the grid holds at once; rows at every alignment of a float, last pieces of
+# 1 to 16 floats.
+@pytest.mark.parametrize("rows,cols", [(5, 1), (31, 17), (260, 1023), (300, 1011), (257, 4063), (1100, 4061), (2100, 8190)])
+def test_quantize_per_tensor_packed_rows_at_any_float(ctx, hipq, rows, cols):
+    g = torch.Generator(device="cuda").manual_seed(rows * 7 + cols)
+    flat = torch.randn(rows * cols + 1, generator=g, device="cuda")
+    for start in (0, 1):
+        x = flat[start:start + rows * cols].view(rows, cols)
+        x[-1, -1] = 2.5 * flat.abs().max()  # (the range ends in the last element)
+        x[0, cols // 2] = float("nan")
+        for mode in (hipq.FORM_MUL_INV, hipq.FORM_DIV | hipq.ROUND_HALF_EVEN):
+            q, params = ctx.quantize_dynamic_per_tensor(x.clone(), mode=mode)
+            pq, pparams = ctx.quantize_per_tensor_packed(x, dynamic=True, mode=mode)
+            qs = ctx.quantize_per_tensor_i8(x.clone(), 0.037, 0, mode)
+            pqs, _ = ctx.quantize_per_tensor_packed(x, dynamic=False, scale=0.037, mode=mode)
+            torch.cuda.synchronize()
+            assert torch.equal(pq, ctx.pack_rows(q)) and torch.equal(pqs, ctx.pack_rows(qs))
+            a, b = ctx.read_qparams(params), ctx.read_qparams(pparams)
+            assert (a.scale, a.zero_point, a.min_val, a.max_val, a.status) == (b.scale, b.zero_point, b.min_val, b.max_val, b.status)
+
+
 @pytest.mark.parametrize("rows,cols", [(1, 8), (3, 70), (64, 256), (100, 304), (33, 1001), (40, 1500), (512, 4096)])
 def test_quantize_per_row_packed_matches_row_major(ctx, hipq, rows, cols):
     """Codes and scales of the packed per-row quantizer = those of the row-major one (bit-exact with the oracle,

@@ -32,6 +32,11 @@ __device__ __forceinline__ void store_stream(float4 *p, float4 v) {
 }
 __device__ __forceinline__ void store_stream(uint32_t *p, uint32_t v) { __builtin_nontemporal_store(v, p); }
 
+// Four floats at an address that is a multiple of four bytes only.
+struct __attribute__((packed, aligned(4))) AnyFloat4 {
+    float x, y, z, w;
+};
+
 // RND 0: f32::round (half away from zero); 1: IEEE nearest-even; 2: floor(v + 0.5), the
 // "faster rounding" of quantize_mobile_optimized (crates/torsh-quantization/src/simd_ops.rs:426-428),
 // with the f32 sum rounded before the floor as there.  Callers that know two modes pass a bool.

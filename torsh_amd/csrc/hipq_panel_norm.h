@@ -10,11 +10,6 @@
 
 namespace hipq {
 
-// Four floats at an address that is a multiple of four bytes only.
-struct __attribute__((packed, aligned(4))) AnyFloat4 {
-    float x, y, z, w;
-};
-
 template <int RC, bool PAIR>
 struct PanelColumns {  // the lane's columns: part * 4 .. + 3 of the blocks of 32 that are real
     int block[RC], part, cols;
