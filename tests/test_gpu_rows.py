@@ -657,6 +657,71 @@ def test_prepared_stack_first_call_in_a_graph(hipq):
             maker.close()
 
 
+# One row per team and the most, rows in a wave's second round, teams without rows, a last team with fewer; column blocks of one
+# workgroup in 1 .. 3, k blocks past the last wave's; one launch's layers, one more and two.
+@pytest.mark.parametrize("tokens,d,dff,layers", [(1, 768, 3072, 2), (8, 128, 128, 3), (9, 128, 512, 2), (80, 768, 3072, 2),
+                                                 (81, 640, 2560, 2), (127, 384, 1408, 2), (128, 768, 1152, 2), (129, 256, 1024, 2),
+                                                 (5, 128, 256, 24), (21, 128, 384, 25), (66, 256, 128, 26)])
+def test_prepared_stack_by_teams(hipq, tokens, d, dff, layers):
+    """Up to 128 tokens, rows of up to 768 floats: the workgroups of an XCD take an eighth of the rows through all layers.  The
+    bits of the row panels (hook 15), also where no team assembles (a spin limit of 0: one workgroup a team instead) and where
+    the context has a share of the device only; a row that is not finite stays alone."""
+    c = hipq.Context(0)
+    try:
+        g = torch.Generator(device="cuda").manual_seed(tokens + d + layers)
+        prepared = c.stack_prepare(_random_blocks(c, g, d, dff, layers))
+        x0 = torch.randn(tokens, d, generator=g, device="cuda")
+        x0[tokens // 2, d // 3] = float("nan")
+        x0[tokens - 1] *= 1e-30
+        ws = c.stack_workspace_prepared(tokens, d, dff)
+        for mode in (0, hipq.ROUND_HALF_EVEN):
+            run = lambda: c.stack_forward(prepared, x0.clone(), dff, ws, mode=mode, prepared=True)
+            c.set_gemm_kernel_variant(15)
+            want = run()
+            c.set_gemm_kernel_variant(0)
+            same = lambda y: torch.equal(torch.nan_to_num(y, nan=-77.0), torch.nan_to_num(want, nan=-77.0))
+            assert same(run()) and same(run()), mode
+            c.set_wait_spin_limit(0)
+            assert same(run()) and same(run()), mode
+            c.set_wait_spin_limit(-1)
+            assert same(run()), mode
+            c.set_resident_share(2)
+            assert same(run()), mode
+            c.set_resident_share(1)
+            c.synchronize()  # nothing gave up
+    finally:
+        torch.cuda.synchronize()
+        c.close()
+
+
+def test_prepared_stacks_of_two_streams_at_once(hipq):
+    """Two contexts on streams of their own, each with stacks of few tokens queued, and nobody has said that they share the
+    device: teams that cannot assemble leave their rows to one workgroup each, so every call gives the bits of a call alone."""
+    d, dff, layers = 256, 1024, 4
+    contexts = [hipq.Context(0, own_stream=True) for _ in range(2)]
+    maker = hipq.Context(0)
+    try:
+        g = torch.Generator(device="cuda").manual_seed(31)
+        prepared = maker.stack_prepare(_random_blocks(maker, g, d, dff, layers))
+        x0 = [torch.randn(40 + 30 * i, d, generator=g, device="cuda") for i in range(2)]
+        ws = [maker.stack_workspace_prepared(x.shape[0], d, dff) for x in x0]
+        want = [maker.stack_forward(prepared, x.clone(), dff, w, prepared=True) for x, w in zip(x0, ws)]
+        xs = [[x.clone() for _ in range(12)] for x in x0]
+        torch.cuda.synchronize()
+        for rep in range(12):
+            for i, c in enumerate(contexts):
+                c.stack_forward(prepared, xs[i][rep], dff, ws[i], prepared=True)
+        for c in contexts:
+            c.synchronize()
+        for i in range(2):
+            for rep in range(12):
+                assert torch.equal(xs[i][rep], want[i]), (i, rep)
+    finally:
+        torch.cuda.synchronize()
+        for c in contexts + [maker]:
+            c.close()
+
+
 def test_prepared_stack_full_size_equals_its_parts(ctx, hipq):
     """Config 5 at its real size (8192 tokens, d = 768, d_ff = 3072; 3 layers keep the test short): the one call is
     bit-identical to the same layers composed from the entry points tested above, and stays within the drift bound

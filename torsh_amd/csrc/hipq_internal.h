@@ -69,7 +69,11 @@ constexpr size_t kCtxEpochWord = 16;
 constexpr size_t kCtxReadyWord = 32;
 constexpr size_t kCtxRangeWord = 64;
 constexpr size_t kCtxSlots = 2048;  // workgroups that can meet
-constexpr size_t kCtxWordsBytes = (kCtxRangeWord + kCtxSlots * 4) * 4;
+// Per team of the stack of few tokens (hipq_stack_team.hip): how many of its workgroups have arrived and the verdict on its last
+// launch; on a line of their own, the phase that each workgroup has finished.
+constexpr size_t kCtxTeamWord = kCtxRangeWord + kCtxSlots * 4;
+constexpr size_t kCtxTeams = 8, kCtxTeamWords = 64, kCtxTeamFlags = 32;
+constexpr size_t kCtxWordsBytes = (kCtxTeamWord + kCtxTeams * kCtxTeamWords) * 4;
 // Number the first meeting of a context gets, a few launches before the counter wraps, so that the wrap (which
 // wipes the slots) is a path every context takes early, not once in 2^32 launches.
 constexpr uint32_t kCtxFirstEpoch = 0xfffffff0u;
@@ -149,6 +153,19 @@ struct RowOpLinear {
     size_t rows, n, k;
     float *out;
 };
+// The layers of the prepared stack on few tokens in one launch (hipq_stack_team.hip), behind the first layer's qkv product
+// (q, k, v rows of 3 d floats in `qkv`).  maxima: room for tokens rounded up to a multiple of 8, times d_ff / 16 floats; codes:
+// as many rows of d_ff bytes.
+struct TeamStackCall {
+    const hipq_block_weights *blocks;
+    size_t layers, tokens, d, d_ff;
+    float eps;
+    float *x, *qkv, *maxima;
+    int8_t *codes;
+};
+bool team_stack_fits(const hipq_ctx *ctx, const float *x, size_t tokens, size_t d, size_t d_ff, PanelFold after_out,
+                     PanelFold after_fc2);
+int32_t team_stack(hipq_ctx *ctx, const TeamStackCall &call, int32_t mode);
 bool row_op_linear_fits(const hipq_ctx *ctx, const float *x, size_t rows, size_t n, size_t k, PanelFold fold);
 int32_t row_op_linear(hipq_ctx *ctx, const RowOpLinear &p, int32_t mode);
 int32_t gelu_quantize_packed(hipq_ctx *ctx, const float *x, size_t rows, size_t cols, int32_t mode, int8_t *out_packed,

@@ -31,6 +31,7 @@ struct PanelColumns {  // the lane's columns: part * 4 .. + 3 of the blocks of 3
 template <int RC>
 struct PanelAffine {
     float4 g[RC], b[RC];
+    __device__ __forceinline__ PanelAffine() {}
     template <bool PAIR>
     __device__ __forceinline__ PanelAffine(const PanelColumns<RC, PAIR> &c, const float *gamma, const float *beta) {
         auto affine = [&](const float *p, int i, float missing) {
@@ -91,6 +92,30 @@ __device__ __forceinline__ float panel_norm_quantize(float4 (&v)[RC], const Pane
             q[i] = pack4(quantize_int_sym<EVEN>(v[i].x, scale, inv), quantize_int_sym<EVEN>(v[i].y, scale, inv),
                          quantize_int_sym<EVEN>(v[i].z, scale, inv), quantize_int_sym<EVEN>(v[i].w, scale, inv));
     return scale;
+}
+
+// Per-token int8 of the row: its codes in q, its scale returned (NaN, with zero codes, for a row whose range is not finite, so
+// that every output of the row is NaN).
+template <bool EVEN, int RC>
+__device__ __forceinline__ float row_range_quantize(const float4 (&v)[RC], const PanelColumns<RC, false> &c, uint32_t (&q)[RC]) {
+    float mn = INFINITY, mx = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < RC; ++i)
+        if (c.real[i]) {
+            mn = fminf(mn, fminf(fminf(v[i].x, v[i].y), fminf(v[i].z, v[i].w)));
+            mx = fmaxf(mx, fmaxf(fmaxf(v[i].x, v[i].y), fmaxf(v[i].z, v[i].w)));
+        }
+    float scale;
+    int zp;
+    const bool good =
+        params_from_minmax(wave_min(mn), wave_max(mx), HIPQ_PARAMS_SYMMETRIC, -128, 127, &scale, &zp) == HIPQ_SUCCESS;
+    const float inv = recip_for_div(scale);
+#pragma unroll
+    for (int i = 0; i < RC; ++i)
+        q[i] = good ? pack4(quantize_int_sym<EVEN>(v[i].x, scale, inv), quantize_int_sym<EVEN>(v[i].y, scale, inv),
+                            quantize_int_sym<EVEN>(v[i].z, scale, inv), quantize_int_sym<EVEN>(v[i].w, scale, inv))
+                    : 0u;
+    return good ? scale : NAN;
 }
 
 }  // namespace hipq

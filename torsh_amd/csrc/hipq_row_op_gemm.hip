@@ -61,24 +61,7 @@ __global__ __launch_bounds__(1024) void row_op_split_kernel(RowOpLinear p) {
     if constexpr (NORM) {
         scale = panel_norm_quantize<EVEN>(v, c, affine, p.eps, q);
     } else {
-        float mn = INFINITY, mx = -INFINITY;
-#pragma unroll
-        for (int i = 0; i < RC; ++i)
-            if (c.real[i]) {
-                mn = fminf(mn, fminf(fminf(v[i].x, v[i].y), fminf(v[i].z, v[i].w)));
-                mx = fmaxf(mx, fmaxf(fmaxf(v[i].x, v[i].y), fmaxf(v[i].z, v[i].w)));
-            }
-        int zp;
-        // a range that is not finite: NaN scale and zero codes, so that every output of the row is NaN
-        const bool good =
-            params_from_minmax(wave_min(mn), wave_max(mx), HIPQ_PARAMS_SYMMETRIC, -128, 127, &scale, &zp) == HIPQ_SUCCESS;
-        const float inv = recip_for_div(scale);
-#pragma unroll
-        for (int i = 0; i < RC; ++i)
-            q[i] = good ? pack4(quantize_int_sym<EVEN>(v[i].x, scale, inv), quantize_int_sym<EVEN>(v[i].y, scale, inv),
-                                quantize_int_sym<EVEN>(v[i].z, scale, inv), quantize_int_sym<EVEN>(v[i].w, scale, inv))
-                        : 0u;
-        if (!good) scale = NAN;
+        scale = row_range_quantize<EVEN>(v, c, q);
     }
     if (lane == 0) row_scale[wave] = scale;
     uint32_t *dword = reinterpret_cast<uint32_t *>(codes);

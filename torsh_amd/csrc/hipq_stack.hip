@@ -52,6 +52,7 @@ int32_t stack_tiled(hipq_ctx *ctx, const hipq_block_weights *blocks, size_t n_la
         return rc ? rc : linear_packed_rows_f32(ctx, b.qb, b.sb, w.w_out, w.s_out, w.b_out, x, tokens, d_model, d_model, x);
     };
     int32_t rc = HIPQ_SUCCESS;
+    const bool teams = team_stack_fits(ctx, x, tokens, d_model, d_ff, after_out, after_fc2);
     for (size_t l = 0; l < n_layers && rc == HIPQ_SUCCESS; ++l) {
         const hipq_block_weights &w = blocks[l];
         if (l == 0) {  // (the one LayerNorm that folds as the row kernels do)
@@ -59,6 +60,9 @@ int32_t stack_tiled(hipq_ctx *ctx, const hipq_block_weights *blocks, size_t n_la
                 (rc = linear_packed_rows_f32(ctx, b.qa, b.sa, w.w_qkv, w.s_qkv, w.b_qkv, nullptr, tokens, 3 * d_model, d_model,
                                              b.qkv)))
                 return rc;
+            if (teams)
+                return team_stack(ctx, TeamStackCall{blocks, n_layers, tokens, d_model, d_ff, eps, x, b.qkv,
+                                                     reinterpret_cast<float *>(b.qa), b.qb}, mode);
         } else if ((rc = norm_linear(w.ln1_gamma, w.ln1_beta, after_fc2, w.w_qkv, w.s_qkv, w.b_qkv, 3 * d_model, b.qkv))) {
             return rc;
         }

@@ -1,0 +1,678 @@
+// The prepared transformer stack on few tokens, all layers in one launch: eight teams, the workgroups of one XCD each, take an
+// eighth of the rows through every layer.
+//
+// As separate launches a layer of few tokens is five kernels of 4 to 7 us, each a launch, a cold start on weights that nobody
+// has asked for yet, and a trip through memory to the next one's compute units on the other XCDs.  Rows do not meet in this
+// stack, so nothing has to leave an XCD: a team's 32 workgroups split the columns of every product, hand their results on through
+// the L2 they share and meet there (a flag per workgroup, one line per team, read past the L1).  While it waits, a workgroup's
+// share of the next product's weights is already on its way into registers.  The price is that every XCD streams all
+// the weights; they come from the memory-side cache for all but the first.
+//
+// Per layer: LayerNorm + quantize + qkv | quantize V + out-projection + skip | LayerNorm + quantize + fc1 + GELU and row maxima |
+// GELU codes | fc2 + skip.  The row operations in front of a product are repeated by every workgroup, a row per wave, as in
+// row_op_split_kernel, whose arithmetic and orders these are: the bits of the separate kernels.
+//
+// A team needs all its workgroups on the device at once, which other work may prevent (another stream's team is enough).
+// So it first counts itself: either the last workgroup to arrive finds that nobody has stopped waiting, and all 32 go on and
+// wait for nothing but each other from there on; or somebody stops waiting first, all of them leave without having touched
+// anything, and the kernel behind this one takes the team's rows through the layers with one workgroup that waits for nobody.
+#include "hipq_gemm_kernels.h"
+#include "hipq_internal.h"
+#include "hipq_panel_norm.h"
+#include "hipq_quantize_rows.h"
+
+namespace hipq {
+namespace {
+
+constexpr int kTeams = static_cast<int>(kCtxTeams);
+constexpr int kTeamSize = 32;     // workgroups of a team
+constexpr int kTeamWaves = 16;    // waves of a workgroup: the first multiply, the others take the rows
+constexpr int kTeamProducts = 6;  // waves that multiply
+constexpr int kTeamRowWaves = kTeamWaves - kTeamProducts;
+constexpr int kTeamRows = 16;     // rows of a team at most
+constexpr int kTeamLayers = 24;   // layers of one launch (their pointers are kernel arguments)
+constexpr int kTeamFloats = 3;    // float4 a lane per row: d_model <= 768
+constexpr int kTeamColumns = 3;   // column blocks of 32 a workgroup: N <= 3072
+constexpr int kTeamSteps = 8;     // pairs of k blocks a wave: K <= 3072
+constexpr int kTeamRowSteps = 2;  // the same where K is d_model
+constexpr uint32_t kTeamPhases = 256;  // numbers a launch may use: five meetings a layer
+static_assert(kTeamLayers * 5 < int(kTeamPhases), "phase numbers");
+constexpr int kPastL1 = /*sc1*/ 16;
+
+// Looks at the verdict before a workgroup stops waiting for its team, some 0.4 us each: a team that other work keeps from
+// assembling for longer than a millisecond or two is better off with the one workgroup.
+constexpr int kAssemblyLimit = 4096;
+
+struct StackTeam {
+    hipq_block_weights blocks[kTeamLayers];
+    float *x, *qkv, *maxima;
+    int8_t *codes;
+    uint32_t *words, *wait_error;
+    int layers, qkv_done, tokens, rows, d, d_ff, spin_limit, assembly_limit;
+    float eps;
+};
+static_assert(sizeof(StackTeam) <= 4096, "kernel arguments");
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t team_buffer(const void *base, int bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, bytes, 0x00020000);
+}
+
+// Words of a team: how many workgroups have ever arrived (32 a launch) and what was decided about the last launch: its number
+// and whether the team goes on.
+constexpr int kTeamArrivals = 0, kTeamVerdict = 1, kTeamGo = 1, kTeamAlone = 2;
+
+// One lane of a workgroup: arrives and waits for the verdict on this launch, whose number is left in `launch`.
+__device__ __forceinline__ bool team_assembles(uint32_t *words, int spin_limit, uint32_t *launch) {
+    const uint32_t before = __hip_atomic_fetch_add(words + kTeamArrivals, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const uint32_t n = before / kTeamSize;
+    *launch = n;
+    uint32_t *verdict = words + kTeamVerdict, seen = 0;
+    auto decided = [&] { return seen != 0 && (seen >> 2) == n; };
+    auto decide = [&](uint32_t v) {  // unless it has been decided already
+        seen = __hip_atomic_load(verdict, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        while (!decided())
+            if (__hip_atomic_compare_exchange_strong(verdict, &seen, n << 2 | v, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                     __HIP_MEMORY_SCOPE_AGENT))
+                seen = n << 2 | v;
+    };
+    if (before % kTeamSize == kTeamSize - 1) {
+        decide(kTeamGo);
+    } else {
+        for (int spin = 0; spin < spin_limit && !decided(); ++spin) {
+            __builtin_amdgcn_s_sleep(1);
+            seen = __hip_atomic_load(verdict, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        if (!decided()) decide(kTeamAlone);
+    }
+    return (seen & 3u) == kTeamGo;
+}
+
+__device__ __forceinline__ uint32_t team_xcc_id() {
+    uint32_t v;
+    asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID, 0, 4)" : "=s"(v));
+    return v;
+}
+
+// Maximum over a row of 16 lanes, in every lane.
+__device__ __forceinline__ float lane_row_max(float v) {
+    v = fmaxf(v, lane_move<0xB1>(v));   // quad_perm [1, 0, 3, 2]
+    v = fmaxf(v, lane_move<0x4E>(v));   // quad_perm [2, 3, 0, 1]
+    v = fmaxf(v, lane_move<0x141>(v));  // row_half_mirror
+    return fmaxf(v, lane_move<0x140>(v));  // row_mirror
+}
+
+// Waves have roles, because a wave's loads return in the order of their requests: the six that multiply ask for the next
+// product's weights as soon as they have parked their partial sums (and touch those of the one after it, so that they are in the
+// L2 by then), the ten others poll, run the row operations, and finish and store results, and never wait for a weight.
+template <bool EVEN>
+__global__ __launch_bounds__(1024) void stack_team_kernel(StackTeam p) {
+    constexpr int RC = kTeamFloats, kPiece = kTeamRows + 1;  // (a piece of padding: the lanes of a store hit all banks)
+    __shared__ __attribute__((aligned(16))) v4i codes[kTeamColumns * kTeamSize * 2 * kPiece];  // [k block][half][row]
+    __shared__ __attribute__((aligned(16))) v4i part[kTeamProducts][2 * kTeamColumns][kWave];
+    __shared__ __attribute__((aligned(16))) float4 gain[RC * 64], offset[RC * 64];  // of the LayerNorm ahead
+    __shared__ float col_scale[2][kTeamColumns * 32], col_bias[2][kTeamColumns * 32];  // of this product and the next
+    __shared__ float row_scale[kTeamRows], row_inv[kTeamRows];
+    __shared__ int together;
+    int lane = threadIdx.x % kWave;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const bool multiplies = wave < kTeamProducts;
+    const int rw = wave - kTeamProducts;  // of the waves that take rows
+    const int team = static_cast<int>(blockIdx.x) % kTeams, me = static_cast<int>(blockIdx.x) / kTeams;
+    const int T = p.rows, row0 = team * T;
+    if (row0 >= p.tokens) return;
+    const int R = T < p.tokens - row0 ? T : p.tokens - row0;
+    const int d = p.d, dblocks = d / 32, fblocks = p.d_ff / 32;
+    uint32_t *words = p.words + team * kCtxTeamWords;
+    const __amdgpu_buffer_rsrc_t rflags = team_buffer(words + kCtxTeamFlags, kTeamSize * 4);
+    const __amdgpu_buffer_rsrc_t rx = team_buffer(p.x + size_t(row0) * d, R * d * 4);
+    const __amdgpu_buffer_rsrc_t rqkv = team_buffer(p.qkv + size_t(row0) * 3 * d, R * 3 * d * 4);
+    const __amdgpu_buffer_rsrc_t rmaxima = team_buffer(p.maxima + size_t(team) * T * fblocks * 2, T * fblocks * 8);  // [16 columns][row]
+    const __amdgpu_buffer_rsrc_t rcodes = team_buffer(p.codes + size_t(team) * T * p.d_ff, T * p.d_ff);  // [k block][half][row][16]
+
+    // A product is v_mfma_i32_16x16x64_i8, as the rows are 16 at most.  Operands: a lane's 16 bytes are of row or column lane % 16
+    // and of quarter lane / 16 of two consecutive k blocks.  Results: column lane % 16, rows `mine` + 0 .. 3.
+    int mine = 4 * (lane / 16), fragment = lane / 16 * 512 + lane % 16 * 16;
+    // Columns: this workgroup has blocks me, me + 32, ... of a product's 32-column blocks.
+    auto column_block = [&](int j) { return me + kTeamSize * j; };
+    const std::integral_constant<int, 1> narrow;
+    const std::integral_constant<int, kTeamColumns> wide;
+    const std::integral_constant<int, kTeamRowSteps> shallow;
+    const std::integral_constant<int, kTeamSteps> deep;
+
+
+    if (multiplies) {
+        v4i fw[2 * kTeamSteps];
+        uint32_t touched[kTeamColumns] = {0, 0, 0};
+#pragma unroll
+        for (int i = 0; i < 2 * kTeamSteps; ++i) fw[i] = v4i{0, 0, 0, 0};
+        // This wave's fragments of a product's weights.
+        auto request = [&](auto steps, auto columns, const int8_t *w, int nblocks, int kblocks) {
+            constexpr int STEPS = decltype(steps)::value, CB = decltype(columns)::value;
+            static_assert(STEPS * CB <= kTeamSteps, "registers for the fragments");
+            const __amdgpu_buffer_rsrc_t rw_ = team_buffer(w, nblocks * kblocks * 1024);
+#pragma unroll
+            for (int s = 0; s < STEPS; ++s) {
+                const int kb = 2 * (wave + kTeamProducts * s);
+#pragma unroll
+                for (int jc = 0; jc < 2 * CB; ++jc)
+                    if (kb < kblocks && column_block(jc / 2) < nblocks)  // (the others are not multiplied or not looked at)
+                        fw[s * 2 * CB + jc] = __builtin_bit_cast(
+                            v4i, __builtin_amdgcn_raw_buffer_load_b128(rw_, fragment, (column_block(jc / 2) * kblocks + kb) * 1024 + jc % 2 * 256, 0));
+            }
+        };
+        // One dword of every line of the workgroup's share of a product's weights.
+        auto touch = [&](auto columns, const int8_t *w, int nblocks, int kblocks) {
+            constexpr int CB = decltype(columns)::value;
+            const __amdgpu_buffer_rsrc_t rw_ = team_buffer(w, nblocks * kblocks * 1024);
+#pragma unroll
+            for (int u = 0; u < kTeamColumns; ++u) {
+                const int line = CB == 1 ? wave * kWave + lane + u * (kTeamProducts * kWave) : wave * kWave + lane;
+                const int j = CB == 1 ? 0 : u;
+                if (line < kblocks * 8 && column_block(j) < nblocks)
+                    touched[u] = __builtin_amdgcn_raw_buffer_load_b32(rw_, line * 128, column_block(j) * kblocks * 1024, 0);
+            }
+        };
+        auto settle = [&] {
+#pragma unroll
+            for (int u = 0; u < kTeamColumns; ++u) {
+                const uint32_t t = touched[u];
+                asm volatile("" ::"v"(t));
+            }
+        };
+        // Multiplies this wave's k blocks and parks the partial blocks.  (Rows past the team's hold whatever is there; their results
+        // are not looked at.)
+        auto multiply = [&](auto steps, auto columns, int nblocks, int kblocks, auto touch_next) {
+            constexpr int STEPS = decltype(steps)::value, CB = decltype(columns)::value;
+            __syncthreads();  // the rows are there
+            touch_next();
+            __syncthreads();  // and their codes
+            v4i acc[2 * CB];
+#pragma unroll
+            for (int jc = 0; jc < 2 * CB; ++jc) acc[jc] = v4i{0, 0, 0, 0};
+#pragma unroll
+            for (int s = 0; s < STEPS; ++s) {
+                const int kb = 2 * (wave + kTeamProducts * s);
+                if (kb >= kblocks) break;
+                const v4i fa = codes[(kb * 2 + lane / 16) * kPiece + lane % kTeamRows];
+#pragma unroll
+                for (int jc = 0; jc < 2 * CB; ++jc)
+                    acc[jc] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa, fw[s * 2 * CB + jc], acc[jc], 0, 0, 0);
+            }
+#pragma unroll
+            for (int jc = 0; jc < 2 * CB; ++jc)
+                if (column_block(jc / 2) < nblocks) part[wave][jc][lane] = acc[jc];
+            __syncthreads();
+            settle();
+        };
+        auto others = [&](int barriers) {  // the row waves' further ones of a phase
+            for (int i = 0; i < barriers; ++i) __syncthreads();
+            // (addresses are made again in every phase: kept from layer to layer, they would take more registers than there are)
+            asm volatile("" : "+v"(lane), "+v"(fragment)::"memory");
+        };
+        if (p.qkv_done)
+            request(shallow, narrow, p.blocks[0].w_out, dblocks, dblocks);
+        else
+            request(shallow, wide, p.blocks[0].w_qkv, 3 * dblocks, dblocks);
+        __syncthreads();
+        if (!together) return;
+#pragma unroll 1
+        for (int l = 0; l < p.layers; ++l) {
+            const hipq_block_weights &b = p.blocks[l];
+            const bool last = l + 1 == p.layers;
+            if (l > 0 || !p.qkv_done) {
+                multiply(shallow, wide, 3 * dblocks, dblocks, [&] { touch(narrow, b.w_out, dblocks, dblocks); });
+                request(shallow, narrow, b.w_out, dblocks, dblocks);
+                others(2);
+            }
+            multiply(shallow, narrow, dblocks, dblocks, [&] { touch(wide, b.w_fc1, fblocks, dblocks); });
+            request(shallow, wide, b.w_fc1, fblocks, dblocks);
+            others(2);
+            multiply(shallow, wide, fblocks, dblocks, [&] { touch(narrow, b.w_fc2, dblocks, fblocks); });
+            request(deep, narrow, b.w_fc2, dblocks, fblocks);
+            others(5);  // (the scales of GELU's rows, and another meeting)
+            multiply(deep, narrow, dblocks, fblocks, [&] {
+                if (!last) touch(wide, p.blocks[l + 1].w_qkv, 3 * dblocks, dblocks);
+            });
+            if (last) break;
+            request(shallow, wide, p.blocks[l + 1].w_qkv, 3 * dblocks, dblocks);
+            others(2);
+        }
+        return;
+    }
+
+    // Phases are numbered through the launches of the team; the low four bits of a flag name the XCD.
+    const uint32_t xcc = team_xcc_id();
+    uint32_t phase = 0;
+    if (wave == kTeamWaves - 1) {
+        uint32_t launch = 0;
+        const bool go = lane == 0 && team_assembles(words, p.assembly_limit, &launch);
+        if (lane == 0) together = go;
+        phase = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(launch))) * (kTeamPhases * 16);
+    }
+    bool lost = false;  // (of the wave that polls)
+    auto acknowledged = [] {  // this wave's stores have reached the L2
+        asm volatile("" ::: "memory");
+        wait_vmcnt<0>();
+        asm volatile("" ::: "memory");
+    };
+    auto meet = [&] {
+        phase += 16;
+        __syncthreads();
+        if (wave == kTeamWaves - 1 && !lost) {
+            if (lane == 0) __builtin_amdgcn_raw_buffer_store_b32(static_cast<int>(phase | xcc), rflags, me * 4, 0, 0);
+            bool all = false;
+            uint32_t seen = 0;
+            for (int spin = 0; spin <= p.spin_limit && !all; ++spin) {
+                asm volatile("" ::: "memory");
+                seen = static_cast<uint32_t>(__builtin_amdgcn_raw_buffer_load_b32(rflags, lane % kTeamSize * 4, 0, kPastL1));
+                all = __all(static_cast<int32_t>(seen - phase) >= 0);
+            }
+            lost = !all || !__all((seen & 15u) == xcc);
+        }
+        __syncthreads();
+        // (addresses are made again in every phase: kept from layer to layer, they would take more registers than there are)
+        asm volatile("" : "+v"(lane), "+v"(mine), "+v"(fragment)::"memory");
+    };
+
+    // Scales and biases of a product's columns and, for a LayerNorm in front of it, its vectors: three of the waves that take rows
+    // ask for them while the product before it runs, and leave them in LDS behind it.
+    const bool fetches = rw >= 6 && rw < 9;
+    AnyFloat4 next_gain, next_offset;
+    float next_scale = 0.0f, next_bias = 0.0f;
+    int product = 0;  // parity of the product whose scales are in use
+    auto ask_vectors = [&](const float *scales, const float *biases, int nblocks, bool norm, const float *gamma, const float *beta) {
+        if (!fetches) return;
+        const int at = (rw - 6) * kWave + lane, block = column_block(at / 32);
+        if (at < kTeamColumns * 32 && block < nblocks) {
+            next_scale = scales[block * 32 + at % 32];
+            next_bias = biases ? biases[block * 32 + at % 32] : 0.0f;
+        }
+        if (norm && at < d / 4) {  // (y * 1.0f and y + -0.0f are y, bit for bit)
+            next_gain = gamma ? reinterpret_cast<const AnyFloat4 *>(gamma)[at] : AnyFloat4{1.0f, 1.0f, 1.0f, 1.0f};
+            next_offset = beta ? reinterpret_cast<const AnyFloat4 *>(beta)[at] : AnyFloat4{-0.0f, -0.0f, -0.0f, -0.0f};
+        }
+    };
+    auto leave_vectors = [&](bool norm) {
+        product ^= 1;
+        if (!fetches) return;
+        const int at = (rw - 6) * kWave + lane;
+        if (at < kTeamColumns * 32) {
+            col_scale[product][at] = next_scale;
+            col_bias[product][at] = next_bias;
+        }
+        if (norm && at < d / 4) {
+            gain[at] = make_float4(next_gain.x, next_gain.y, next_gain.z, next_gain.w);
+            offset[at] = make_float4(next_offset.x, next_offset.y, next_offset.z, next_offset.w);
+        }
+    };
+    // The codes of the team's rows into LDS, in fragment order, a row per wave.
+    auto row_codes = [&](auto norm, const __amdgpu_buffer_rsrc_t &rows, int ld, int first) {
+        constexpr int kRounds = (kTeamRows + kTeamRowWaves - 1) / kTeamRowWaves;
+        const PanelColumns<RC, false> c(lane, dblocks);
+        v4i raw[kRounds][RC];
+#pragma unroll
+        for (int u = 0; u < kRounds; ++u) {
+            const int row = rw + u * kTeamRowWaves;
+            if (row < R) {
+#pragma unroll
+                for (int i = 0; i < RC; ++i)
+                    raw[u][i] = __builtin_bit_cast(
+                        v4i, __builtin_amdgcn_raw_buffer_load_b128(rows, c.real[i] ? c.at(i) * 4 : 0x7fffffff,
+                                                                   (row * ld + first) * 4, kPastL1));
+            }
+        }
+        acknowledged();
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < kRounds; ++u) {
+            const int row = rw + u * kTeamRowWaves;
+            if (row >= R) break;
+            float4 v[RC];
+#pragma unroll
+            for (int i = 0; i < RC; ++i) {  // (a bit cast of a vector's element takes its first one)
+                const int t0 = raw[u][i][0], t1 = raw[u][i][1], t2 = raw[u][i][2], t3 = raw[u][i][3];
+                v[i] = make_float4(__builtin_bit_cast(float, t0), __builtin_bit_cast(float, t1), __builtin_bit_cast(float, t2),
+                                   __builtin_bit_cast(float, t3));
+            }
+            uint32_t q[RC];
+            float scale;
+            if constexpr (decltype(norm)::value) {
+                PanelAffine<RC> affine;
+#pragma unroll
+                for (int i = 0; i < RC; ++i)
+                    if (c.real[i]) {
+                        affine.g[i] = gain[c.at(i) / 4];
+                        affine.b[i] = offset[c.at(i) / 4];
+                    }
+                scale = panel_norm_quantize<EVEN>(v, c, affine, p.eps, q);
+            } else {
+                scale = row_range_quantize<EVEN>(v, c, q);
+            }
+            if (lane == 0) row_scale[row] = scale;
+            uint32_t *dword = reinterpret_cast<uint32_t *>(codes);
+#pragma unroll
+            for (int i = 0; i < RC; ++i)
+                if (c.real[i]) dword[((c.block[i] * 2 + c.part / 4) * kPiece + row) * 4 + c.part % 4] = q[i];
+        }
+        __syncthreads();
+    };
+    // Row wave 2 j + c finishes column half c of block j: its four results of every lane.
+    auto finishes = [&](int nblocks) { return rw >= 0 && rw < 2 * kTeamColumns && column_block(rw / 2) < nblocks; };
+    constexpr int kPieces = (kTeamColumns * kTeamSize * 2 * kTeamRows + kTeamRowWaves * kWave - 1) / (kTeamRowWaves * kWave);
+    auto column = [&] { return column_block(rw / 2) * 32 + rw % 2 * 16 + lane % 16; };
+    auto results = [&](float(&o)[4]) {
+        v4i sum = part[0][rw][lane];
+#pragma unroll
+        for (int w = 1; w < kTeamProducts; ++w) sum += part[w][rw][lane];
+        const float sw = col_scale[product][rw * 16 + lane % 16], bias = col_bias[product][rw * 16 + lane % 16];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            o[i] = static_cast<float>(sum[i]) * (row_scale[mine + i] * sw);
+            o[i] = o[i] + bias;
+        }
+    };
+    // Result i of this lane, if its row is one of the team's.
+    auto store = [&](float v, const __amdgpu_buffer_rsrc_t &to, int at, int i) {
+        if (mine + i < R) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, v), to, at * 4, 0, 0);
+    };
+    // The stream's values that this lane finishes: the same in out-projection and fc2, so they stay in registers.
+    const bool stream = rw < 2 && finishes(dblocks);
+    float res[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (stream) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (mine + i < R)
+                res[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rx, ((mine + i) * d + column()) * 4, 0, 0));
+    }
+    auto add_to_stream = [&] {
+        if (!stream) return;
+        float o[4];
+        results(o);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            res[i] = o[i] + res[i];
+            store(res[i], rx, (mine + i) * d + column(), i);
+        }
+        acknowledged();
+    };
+    auto ask_qkv = [&](const hipq_block_weights &b) { ask_vectors(b.s_qkv, b.b_qkv, 3 * dblocks, true, b.ln1_gamma, b.ln1_beta); };
+    auto ask_out = [&](const hipq_block_weights &b) { ask_vectors(b.s_out, b.b_out, dblocks, false, nullptr, nullptr); };
+    if (p.qkv_done)
+        ask_out(p.blocks[0]);
+    else
+        ask_qkv(p.blocks[0]);
+    leave_vectors(!p.qkv_done);
+    __syncthreads();
+    if (!together) return;
+#pragma unroll 1
+    for (int l = 0; l < p.layers; ++l) {
+        const hipq_block_weights &b = p.blocks[l];
+        if (l > 0 || !p.qkv_done) {
+            row_codes(std::true_type{}, rx, d, 0);
+            ask_out(b);
+            __syncthreads();
+            if (finishes(3 * dblocks)) {
+                float o[4];
+                results(o);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) store(o[i], rqkv, (mine + i) * (3 * d) + column(), i);
+                acknowledged();
+            }
+            leave_vectors(false);
+            meet();
+        }
+        // Stand-in for the attention mixing, which is outside this path: the value slice passes through.
+        row_codes(std::false_type{}, rqkv, 3 * d, 2 * d);
+        ask_vectors(b.s_fc1, b.b_fc1, fblocks, true, b.ln2_gamma, b.ln2_beta);
+        __syncthreads();
+        add_to_stream();
+        leave_vectors(true);
+        meet();
+        row_codes(std::true_type{}, rx, d, 0);
+        ask_vectors(b.s_fc2, b.b_fc2, dblocks, false, nullptr, nullptr);
+        __syncthreads();
+        const bool hidden = finishes(fblocks);
+        const int hblock = column_block(rw / 2) * 2 + rw % 2;  // of 16 columns
+        float h[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (hidden) {
+            results(h);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                h[i] = gelu_tanh(h[i]);
+                const float m = lane_row_max(fmaxf(fabsf(h[i]), 0.0f));  // (a NaN is no maximum)
+                if (lane % 16 == 0) store(m, rmaxima, hblock * T + mine + i, i);
+            }
+            acknowledged();
+        }
+        leave_vectors(false);
+        meet();
+        {
+#pragma unroll 1
+            for (int row = rw; row < R; row += kTeamRowWaves) {
+                float am = 0.0f;
+#pragma unroll
+                for (int i = 0; i < (2 * kTeamColumns * kTeamSize + kWave - 1) / kWave; ++i) {  // (past the last block: zeros)
+                    const int at = lane + kWave * i;
+                    am = fmaxf(am, __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                                                 rmaxima, at < 2 * fblocks ? (at * T + row) * 4 : 0x7fffffff, 0, kPastL1)));
+                }
+                am = wave_max(am);
+                const float scale = am < FLT_EPSILON ? 1.0f : am / 127.0f;
+                if (lane == 0) {
+                    row_scale[row] = am <= FLT_MAX ? scale : NAN;
+                    row_inv[row] = recip_for_div(scale);
+                }
+            }
+        }
+        __syncthreads();
+        if (hidden) {
+            int q[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float scale = row_scale[mine + i];
+                q[i] = scale == scale ? quantize_int_sym<EVEN>(h[i], scale, row_inv[mine + i]) : 0;
+            }
+            const int qd = lane % 4;
+            const uint32_t word = quad_byte_transpose(pack4(q[0], q[1], q[2], q[3]), (qd & 1) ? 0x03070105u : 0x06020400u,
+                                                      (qd & 2) ? 0x03020706u : 0x05040100u);
+            if (mine + qd < R)
+                __builtin_amdgcn_raw_buffer_store_b32(static_cast<int>(word), rcodes,
+                                                      (hblock * T + mine + qd) * 16 + lane % 16 / 4 * 4, 0, 0);
+            acknowledged();
+        }
+        meet();
+        const bool last = l + 1 == p.layers;
+        {
+            v4i piece[kPieces];
+#pragma unroll
+            for (int u = 0; u < kPieces; ++u)
+                piece[u] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(
+                                                       rcodes, ((u * kTeamRowWaves + rw) * kWave + lane) * 16, 0, kPastL1));
+            acknowledged();
+            __syncthreads();
+            const unsigned by_rows = (65536u + T - 1) / T;  // (i / T for i < 3072 and T <= 16: off by less than 1 / T)
+#pragma unroll
+            for (int u = 0; u < kPieces; ++u) {
+                const unsigned i = (u * kTeamRowWaves + rw) * kWave + lane, at = i * by_rows >> 16;
+                if (i < unsigned(fblocks * 2 * T)) codes[at * kPiece + (i - at * T)] = piece[u];
+            }
+        }
+        __syncthreads();
+        if (!last) ask_qkv(p.blocks[l + 1]);
+        __syncthreads();  // the partial blocks are there
+        add_to_stream();
+        if (!last) {
+            leave_vectors(true);
+            meet();
+        }
+    }
+    if (wave == kTeamWaves - 1 && lane == 0 && lost)
+        __hip_atomic_store(p.wait_error, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// The same layers of a team's rows by one workgroup that waits for nobody, where the team did not assemble: 16 columns at a time
+// per wave, fc1 once for the rows' maxima and once more for the codes (its results have no room here).
+template <bool EVEN>
+__global__ __launch_bounds__(1024) void stack_alone_kernel(StackTeam p) {
+    constexpr int RC = kTeamFloats, kPiece = kTeamRows + 1;
+    __shared__ __attribute__((aligned(16))) v4i codes[RC * 8 * 2 * kPiece], hidden[kTeamColumns * kTeamSize * 2 * kPiece];
+    __shared__ float row_scale[kTeamRows], hidden_scale[kTeamRows], hidden_inv[kTeamRows];
+    __shared__ uint32_t row_max[kTeamRows];
+    const int team = static_cast<int>(blockIdx.x), T = p.rows, row0 = team * T;
+    if (row0 >= p.tokens) return;
+    if ((p.words[team * kCtxTeamWords + kTeamVerdict] & 3u) != kTeamAlone) return;
+    const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int R = T < p.tokens - row0 ? T : p.tokens - row0;
+    const int d = p.d, dblocks = d / 32, fblocks = p.d_ff / 32, mine = 4 * (lane / 16);
+    const __amdgpu_buffer_rsrc_t rx = team_buffer(p.x + size_t(row0) * d, R * d * 4);
+    const __amdgpu_buffer_rsrc_t rqkv = team_buffer(p.qkv + size_t(row0) * 3 * d, R * 3 * d * 4);
+    auto row_codes = [&](auto norm, const __amdgpu_buffer_rsrc_t &rows, int ld, int first, const float *gamma, const float *beta) {
+        __syncthreads();
+        if (wave < R) {
+            const PanelColumns<RC, false> c(lane, dblocks);
+            float4 v[RC];
+#pragma unroll
+            for (int i = 0; i < RC; ++i)
+                v[i] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                      rows, c.real[i] ? c.at(i) * 4 : 0x7fffffff, (wave * ld + first) * 4, kPastL1));
+            uint32_t q[RC];
+            float scale;
+            if constexpr (decltype(norm)::value)
+                scale = panel_norm_quantize<EVEN>(v, c, PanelAffine<RC>(c, gamma, beta), p.eps, q);
+            else
+                scale = row_range_quantize<EVEN>(v, c, q);
+            if (lane == 0) row_scale[wave] = scale;
+            uint32_t *dword = reinterpret_cast<uint32_t *>(codes);
+#pragma unroll
+            for (int i = 0; i < RC; ++i)
+                if (c.real[i]) dword[((c.block[i] * 2 + c.part / 4) * kPiece + wave) * 4 + c.part % 4] = q[i];
+        }
+        __syncthreads();
+    };
+    auto product = [&](const v4i *operand, const float *row_scales, const int8_t *w, const float *scales, const float *biases,
+                       int nblocks, int kblocks, auto use) {
+        const __amdgpu_buffer_rsrc_t rw = team_buffer(w, nblocks * kblocks * 1024);
+#pragma unroll 1
+        for (int half = wave; half < 2 * nblocks; half += kTeamWaves) {
+            v4i acc{0, 0, 0, 0};
+            for (int kb = 0; kb < kblocks; kb += 2)
+                acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(
+                    operand[(kb * 2 + lane / 16) * kPiece + lane % kTeamRows],
+                    __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(
+                                                rw, lane / 16 * 512 + lane % 16 * 16, (half / 2 * kblocks + kb) * 1024 + half % 2 * 256, 0)),
+                    acc, 0, 0, 0);
+            const int n = half * 16 + lane % 16;
+            const float sw = scales[n], bias = biases ? biases[n] : 0.0f;
+            float o[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                o[i] = static_cast<float>(acc[i]) * (row_scales[mine + i] * sw);
+                o[i] = o[i] + bias;
+            }
+            use(half, n, o);
+        }
+        asm volatile("" ::: "memory");
+        wait_vmcnt<0>();
+        asm volatile("" ::: "memory");
+    };
+    auto add_to_stream = [&](int, int n, float(&o)[4]) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (mine + i < R) {
+                const int at = ((mine + i) * d + n) * 4;
+                const float x = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rx, at, 0, kPastL1));
+                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, o[i] + x), rx, at, 0, 0);
+            }
+    };
+#pragma unroll 1
+    for (int l = 0; l < p.layers; ++l) {
+        const hipq_block_weights &b = p.blocks[l];
+        if (l > 0 || !p.qkv_done) {
+            row_codes(std::true_type{}, rx, d, 0, b.ln1_gamma, b.ln1_beta);
+            product(codes, row_scale, b.w_qkv, b.s_qkv, b.b_qkv, 3 * dblocks, dblocks, [&](int, int n, float(&o)[4]) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (mine + i < R)
+                        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, o[i]), rqkv, ((mine + i) * 3 * d + n) * 4, 0, 0);
+            });
+        }
+        row_codes(std::false_type{}, rqkv, 3 * d, 2 * d, nullptr, nullptr);
+        product(codes, row_scale, b.w_out, b.s_out, b.b_out, dblocks, dblocks, add_to_stream);
+        if (threadIdx.x < kTeamRows) row_max[threadIdx.x] = 0;
+        row_codes(std::true_type{}, rx, d, 0, b.ln2_gamma, b.ln2_beta);
+        product(codes, row_scale, b.w_fc1, b.s_fc1, b.b_fc1, fblocks, dblocks, [&](int, int, float(&o)[4]) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {  // (not negative, so ordered as the bits are; a NaN is no maximum)
+                const float m = lane_row_max(fmaxf(fabsf(gelu_tanh(o[i])), 0.0f));
+                if (lane % 16 == 0) atomicMax(&row_max[mine + i], __builtin_bit_cast(uint32_t, m));
+            }
+        });
+        __syncthreads();
+        if (threadIdx.x < kTeamRows) {
+            const float am = __builtin_bit_cast(float, row_max[threadIdx.x]);
+            const float scale = am < FLT_EPSILON ? 1.0f : am / 127.0f;
+            hidden_scale[threadIdx.x] = am <= FLT_MAX ? scale : NAN;
+            hidden_inv[threadIdx.x] = recip_for_div(scale);
+        }
+        __syncthreads();
+        product(codes, row_scale, b.w_fc1, b.s_fc1, b.b_fc1, fblocks, dblocks, [&](int half, int, float(&o)[4]) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float scale = hidden_scale[mine + i];
+                const int q = scale == scale ? quantize_int_sym<EVEN>(gelu_tanh(o[i]), scale, hidden_inv[mine + i]) : 0;
+                reinterpret_cast<int8_t *>(hidden)[(half * kPiece + mine + i) * 16 + lane % 16] = static_cast<int8_t>(q);
+            }
+        });
+        __syncthreads();
+        product(hidden, hidden_scale, b.w_fc2, b.s_fc2, b.b_fc2, dblocks, fblocks, add_to_stream);
+    }
+}
+
+}  // namespace
+
+// Up to 128 tokens of rows of up to 768 floats (16 rows a team, three float4 a lane).  Separate kernels / this, us: 12 layers of d 768,
+// d_ff 3072 1 token 303 / 191, 16 313 / 217, 77 334 / 240, 128 368 / 281; d 384, d_ff 1152, 10 layers, 3 tokens 231 / 118; d 256,
+// d_ff 1024, 6 layers, 40 tokens 140 / 82.  What is left is 2.3 us a phase (rows 0.5, LayerNorm and codes 1.1, product 0.3, results
+// and their acknowledgement 0.9, meeting 0.35) and, at d 768, 7 MB of weights a layer through each XCD's port, at some 0.7 TB/s.
+bool team_stack_fits(const hipq_ctx *ctx, const float *x, size_t tokens, size_t d, size_t d_ff, PanelFold after_out,
+                     PanelFold after_fc2) {
+    const int share = ctx->resident_share > 0 ? ctx->resident_share : 1;
+    auto folds = [](PanelFold f) { return !f.pair && f.wave_blocks == kTeamFloats; };
+    return ctx->pair_ok && share == 1 && ctx->num_cus >= kTeams * kTeamSize && folds(after_out) && folds(after_fc2) &&
+           tokens <= size_t(kTeams) * kTeamRows && d % 128 == 0 && d <= size_t(kTeamFloats) * 256 && d_ff % 128 == 0 &&
+           d_ff <= size_t(kTeamColumns) * kTeamSize * 32 && d_ff <= 4 * d && (reinterpret_cast<uintptr_t>(x) & 15u) == 0;
+}
+
+int32_t team_stack(hipq_ctx *ctx, const TeamStackCall &call, int32_t mode) {
+    StackTeam p;
+    p.x = call.x;
+    p.qkv = call.qkv;
+    p.maxima = call.maxima;
+    p.codes = call.codes;
+    p.words = ctx->wait_error + kCtxTeamWord;
+    p.wait_error = ctx->wait_error;
+    p.tokens = static_cast<int>(call.tokens);
+    p.rows = static_cast<int>((call.tokens + kTeams - 1) / kTeams);
+    p.d = static_cast<int>(call.d);
+    p.d_ff = static_cast<int>(call.d_ff);
+    p.spin_limit = ctx->wait_spin_limit < 1024 ? 1 << 20 : ctx->wait_spin_limit;  // (a small one, a test's, is for the assembly)
+    p.assembly_limit = ctx->wait_spin_limit < kAssemblyLimit ? ctx->wait_spin_limit : kAssemblyLimit;
+    p.eps = call.eps;
+    for (size_t l = 0; l < call.layers; l += kTeamLayers) {
+        p.layers = static_cast<int>(call.layers - l < size_t(kTeamLayers) ? call.layers - l : size_t(kTeamLayers));
+        p.qkv_done = l == 0;
+        for (int i = 0; i < p.layers; ++i) p.blocks[i] = call.blocks[l + i];
+        if (mode & HIPQ_ROUND_HALF_EVEN) {
+            hipLaunchKernelGGL(stack_team_kernel<true>, dim3(kTeams * kTeamSize), dim3(1024), 0, ctx->stream, p);
+            hipLaunchKernelGGL(stack_alone_kernel<true>, dim3(kTeams), dim3(1024), 0, ctx->stream, p);
+        } else {
+            hipLaunchKernelGGL(stack_team_kernel<false>, dim3(kTeams * kTeamSize), dim3(1024), 0, ctx->stream, p);
+            hipLaunchKernelGGL(stack_alone_kernel<false>, dim3(kTeams), dim3(1024), 0, ctx->stream, p);
+        }
+        const int32_t rc = check_launch("transformer stack (teams)");
+        if (rc) return rc;
+    }
+    return HIPQ_SUCCESS;
+}
+
+}  // namespace hipq
