@@ -1,4 +1,4 @@
-"""Builds libtorsh_hipq.so (the C-ABI library) for gfx950 with hipcc.
+"""Builds libtorsh_hipq.so (the C-ABI library) for gfx950 with hipcc, and the module that carries Python's calls into it.
 
 Run as ``python -m torsh_amd.build``.  hipcc cross-compiles, so no GPU is
 needed to build.  Objects are compiled in parallel and linked in-tree at
@@ -17,6 +17,7 @@ ROOT = os.path.dirname(PKG)
 CSRC = os.path.join(PKG, "csrc")
 OBJ_DIR = os.path.join(PKG, "lib", "obj")
 LIB_PATH = os.path.join(PKG, "lib", "libtorsh_hipq.so")
+PYTHON_PATH = os.path.join(PKG, "lib", "_hipq_python.so")
 
 ARCH = "gfx950"
 
@@ -72,6 +73,31 @@ def _compile(src: str, force: bool) -> str:
     return obj
 
 
+def _build_python(force: bool) -> None:
+    """The Python side of the library's calls (csrc/hipq_python.cpp), host code against torch's headers."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    src = os.path.join(CSRC, "hipq_python.cpp")
+    newest = max(os.path.getmtime(src), os.path.getmtime(os.path.join(ROOT, "include", "torsh_hipq.h")))
+    if not force and os.path.exists(PYTHON_PATH) and os.path.getmtime(PYTHON_PATH) >= newest:
+        return
+    cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-I", os.path.join(ROOT, "include"),
+           "-isystem", sysconfig.get_paths()["include"]]
+    for path in cpp_extension.include_paths():
+        cmd += ["-isystem", path]
+    cmd += [src, "-o", PYTHON_PATH, "-L", os.path.dirname(LIB_PATH), "-l:libtorsh_hipq.so", "-Wl,-rpath,$ORIGIN"]
+    for path in cpp_extension.library_paths():
+        cmd += ["-L", path]
+    cmd += ["-ltorch_python", "-ltorch_cpu", "-lc10"]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"building {src} failed:\n{proc.stdout}\n{proc.stderr}")
+
+
 def build(force: bool = True, jobs: int = 8) -> str:
     os.makedirs(OBJ_DIR, exist_ok=True)
     srcs = sources()
@@ -81,6 +107,7 @@ def build(force: bool = True, jobs: int = 8) -> str:
     proc = subprocess.run(cmd, capture_output=True, text=True)
     if proc.returncode != 0:
         raise RuntimeError(f"link failed:\n{proc.stdout}\n{proc.stderr}")
+    _build_python(force)
     return LIB_PATH
 
 

@@ -1,20 +1,25 @@
-"""ctypes binding of ``libtorsh_hipq.so`` for tests, the smoke check and the benchmark.
+"""Binding of ``libtorsh_hipq.so`` for tests, the smoke check and the benchmark.
 
 The binding is deliberately thin: every function forwards raw device pointers
 (``torch.Tensor.data_ptr()``) to the C-ABI entry point of the same name and turns
 a non-zero status into :class:`HipqError` carrying the library's last-error
-string.  torch is used for device memory and streams only.  There is no
-fallback: if the shared library is missing, loading raises.
+string.  The entry points of the forward paths are called through a small native
+module (``csrc/hipq_python.cpp``), the others through ctypes.  torch is used for
+device memory and streams only.  There is no fallback: if the shared library is
+missing, loading raises.
 """
 from __future__ import annotations
 
 import ctypes as C
+import importlib.machinery
+import importlib.util
 import os
 from typing import Optional
 
 import torch
 
 _LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib", "libtorsh_hipq.so")
+_NATIVE_PATH = os.path.join(os.path.dirname(_LIB_PATH), "_hipq_python.so")
 
 SUCCESS, INVALID_ARGUMENT, SHAPE_ERROR, DIMENSION_MISMATCH, DEVICE_ERROR, ALLOCATION_ERROR, SYNCHRONIZATION_ERROR, UNKNOWN_ERROR = range(8)
 ROUND_HALF_AWAY, ROUND_HALF_EVEN = 0, 1
@@ -42,6 +47,9 @@ class BlockWeights(C.Structure):
     _fields_ = [(n, C.c_void_p) for n in (
         "ln1_gamma", "ln1_beta", "ln2_gamma", "ln2_beta", "w_qkv", "s_qkv", "b_qkv", "w_out", "s_out", "b_out",
         "w_fc1", "s_fc1", "b_fc1", "w_fc2", "s_fc2", "b_fc2")]
+
+
+_BLOCK_TENSORS = tuple(name for name, _ in BlockWeights._fields_)
 
 
 class QParams(C.Structure):
@@ -199,8 +207,26 @@ def load() -> C.CDLL:
             fn = getattr(lib, name)
             fn.argtypes = argtypes
             fn.restype = restype
+        _load_native()
         _lib = lib
     return _lib
+
+
+_native = None
+
+
+def _load_native():
+    """Loads the native module that carries the forward paths' calls; raises if it has not been built."""
+    global _native
+    if _native is None:
+        if not os.path.exists(_NATIVE_PATH):
+            raise FileNotFoundError(f"{_NATIVE_PATH} is missing: build it with `python -m torsh_amd.build`")
+        loader = importlib.machinery.ExtensionFileLoader("_hipq_python", _NATIVE_PATH)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_hipq_python", loader))
+        loader.exec_module(module)
+        module.set_error_handler(_check)
+        _native = module
+    return _native
 
 
 def last_error() -> str:
@@ -227,6 +253,8 @@ class Context:
 
     def __init__(self, device: int = 0, stream: Optional[torch.cuda.Stream] = None, own_stream: bool = False):
         self._lib = load()
+        self._native = _native
+        self._address = 0  # the handle's value
         self.handle = _vp()
         self.device = device
         self._device = torch.device("cuda", device)
@@ -235,11 +263,12 @@ class Context:
         else:
             st = stream if stream is not None else torch.cuda.current_stream(device)
             _check(self._lib.hipq_ctx_create_on_stream(device, _vp(st.cuda_stream), C.byref(self.handle)))
+        self._address = self.handle.value
 
     def close(self) -> None:
         if self.handle:
             self._lib.hipq_ctx_destroy(self.handle)
-            self.handle = _vp()
+            self.handle, self._address = _vp(), 0
 
     def __del__(self):
         try:
@@ -283,23 +312,22 @@ class Context:
         return self._device
 
     def _empty(self, shape, dtype) -> torch.Tensor:
-        """An output of `shape`: its sizes handed over one by one cost 1.3 us where a torch.Size costs 2.1, and a small call is
-        its launches and its outputs (a quantize and a dequantize of 33333 floats: 15.2 -> 13.6 us)."""
-        return torch.empty(*shape, dtype=dtype, device=self._device) if shape else torch.empty((), dtype=dtype, device=self._device)
+        """An output of `shape` on the context's device."""
+        return self._native.empty(shape, dtype, self.device)
 
     def minmax(self, x: torch.Tensor) -> torch.Tensor:
-        out = torch.empty(2, dtype=torch.float32, device=self._dev())
+        out = self._empty((2,), torch.float32)
         self.call("hipq_minmax_f32", _ptr(x), x.numel(), _ptr(out))
         return out
 
     def absmax(self, x: torch.Tensor) -> torch.Tensor:
-        out = torch.empty(1, dtype=torch.float32, device=self._dev())
+        out = self._empty((1,), torch.float32)
         self.call("hipq_absmax_f32", _ptr(x), x.numel(), _ptr(out))
         return out
 
     def _unset_qparams(self) -> torch.Tensor:
         """A record for a call that writes every field of it (a zeroed one costs a launch of its own)."""
-        return torch.empty(_QPARAMS_BYTES, dtype=torch.uint8, device=self._device)
+        return self._empty((_QPARAMS_BYTES,), torch.uint8)
 
     def new_qparams(self) -> torch.Tensor:
         return torch.zeros(C.sizeof(QParams), dtype=torch.uint8, device=self._dev())
@@ -387,12 +415,12 @@ class Context:
 
     def quantize_per_tensor_i8(self, x, scale, zp, mode=0, out=None):
         out = out if out is not None else self._empty(x.shape, torch.int8)
-        self.call("hipq_quantize_per_tensor_f32_i8", _ptr(x), x.numel(), float(scale), int(zp), mode, _ptr(out))
+        self._native.hipq_quantize_per_tensor_f32_i8(self._address, x, x.numel(), float(scale), int(zp), mode, out)
         return out
 
     def quantize_per_tensor_u8(self, x, scale, zp, mode=FORM_DIV, out=None):
         out = out if out is not None else self._empty(x.shape, torch.uint8)
-        self.call("hipq_quantize_per_tensor_f32_u8", _ptr(x), x.numel(), float(scale), int(zp), mode, _ptr(out))
+        self._native.hipq_quantize_per_tensor_f32_u8(self._address, x, x.numel(), float(scale), int(zp), mode, out)
         return out
 
     def quantize_per_tensor_carrier(self, x, scale, zp, mode=0, qmin=-128, qmax=127):
@@ -405,8 +433,8 @@ class Context:
         tdt = torch.int8 if dtype == DTYPE_I8 else torch.uint8
         out = out if out is not None else self._empty(x.shape, tdt)
         params = params if params is not None else self._unset_qparams()
-        self.call("hipq_quantize_dynamic_per_tensor_f32", _ptr(x), x.numel(), flavor, dtype, mode, _ptr(out),
-                  _ptr(params))
+        self._native.hipq_quantize_dynamic_per_tensor_f32(self._address, x, x.numel(), flavor, dtype, mode, out,
+                                                          params)
         return out, params
 
     def dequantize(self, q, scale, zp, out=None):
@@ -418,26 +446,26 @@ class Context:
 
     def dequantize_with_params(self, q, params, out=None):
         out = out if out is not None else self._empty(q.shape, torch.float32)
-        self.call("hipq_dequantize_with_params_i8_f32", _ptr(q), q.numel(), _ptr(params), _ptr(out))
+        self._native.hipq_dequantize_with_params_i8_f32(self._address, q, q.numel(), params, out)
         return out
 
     def quantize_per_row(self, x, flavor=PARAMS_SYMMETRIC, mode=0):
         rows, cols = x.shape
-        out = torch.empty(rows, cols, dtype=torch.int8, device=self._device)
-        scales = torch.empty(rows, dtype=torch.float32, device=self._dev())
-        zps = torch.empty(rows, dtype=torch.int32, device=self._dev())
-        status = torch.empty(1, dtype=torch.int32, device=self._dev())
-        self.call("hipq_quantize_per_row_f32_i8", _ptr(x), rows, cols, flavor, mode, _ptr(out), _ptr(scales),
-                  _ptr(zps), _ptr(status))
+        out = self._empty((rows, cols), torch.int8)
+        scales = self._empty((rows,), torch.float32)
+        zps = self._empty((rows,), torch.int32)
+        status = self._empty((1,), torch.int32)
+        self._native.hipq_quantize_per_row_f32_i8(self._address, x, rows, cols, flavor, mode, out, scales, zps,
+                                                  status)
         return out, scales, zps, status
 
     def quantize_per_group_auto(self, x, outer, channels, inner, group_size, flavor, qmin, qmax, mode=0):
         """Group-wise quantize of the dense [outer, channels, inner] view of x into [qmin, qmax]; parameters per group."""
         groups = -(-channels // group_size) if group_size > 0 else 1
         out = self._empty(x.shape, torch.int8)
-        scales = torch.empty(groups, dtype=torch.float32, device=self._dev())
-        zps = torch.empty(groups, dtype=torch.int32, device=self._dev())
-        status = torch.empty(1, dtype=torch.int32, device=self._dev())
+        scales = self._empty((groups,), torch.float32)
+        zps = self._empty((groups,), torch.int32)
+        status = self._empty((1,), torch.int32)
         self.call("hipq_quantize_per_group_auto_f32_i8", _ptr(x), outer, channels, inner, group_size, flavor, qmin,
                   qmax, mode, _ptr(out), _ptr(scales), _ptr(zps), _ptr(status))
         return out, scales, zps, status
@@ -478,11 +506,11 @@ class Context:
             inner *= s
         ch = shape[axis]
         out = self._empty(x.shape, torch.int8)
-        scales = torch.empty(ch, dtype=torch.float32, device=self._dev())
-        zps = torch.empty(ch, dtype=torch.int32, device=self._dev())
-        status = torch.empty(1, dtype=torch.int32, device=self._dev())
-        self.call("hipq_quantize_per_channel_auto_f32_i8", _ptr(x), outer, ch, inner, flavor, mode, _ptr(out),
-                  _ptr(scales), _ptr(zps), _ptr(status))
+        scales = self._empty((ch,), torch.float32)
+        zps = self._empty((ch,), torch.int32)
+        status = self._empty((1,), torch.int32)
+        self._native.hipq_quantize_per_channel_auto_f32_i8(self._address, x, outer, ch, inner, flavor, mode, out,
+                                                           scales, zps, status)
         return out, scales, zps, status
 
     def quantize_per_channel(self, x, scales, zps, axis, mode=FORM_DIV):
@@ -494,8 +522,8 @@ class Context:
         for s in shape[axis + 1:]:
             inner *= s
         out = self._empty(x.shape, torch.int8)
-        self.call("hipq_quantize_per_channel_f32_i8", _ptr(x), outer, shape[axis], inner, _ptr(scales), _ptr(zps),
-                  mode, _ptr(out))
+        self._native.hipq_quantize_per_channel_f32_i8(self._address, x, outer, shape[axis], inner, scales, zps, mode,
+                                                      out)
         return out
 
     def dequantize_per_channel(self, q, scales, zps, axis):
@@ -507,8 +535,7 @@ class Context:
         for s in shape[axis + 1:]:
             inner *= s
         out = self._empty(q.shape, torch.float32)
-        self.call("hipq_dequantize_per_channel_i8_f32", _ptr(q), outer, shape[axis], inner, _ptr(scales), _ptr(zps),
-                  _ptr(out))
+        self._native.hipq_dequantize_per_channel_i8_f32(self._address, q, outer, shape[axis], inner, scales, zps, out)
         return out
 
     def gemm_i8_i32(self, a, w, out=None):
@@ -516,16 +543,16 @@ class Context:
         n, k2 = w.shape
         if k != k2:
             raise HipqError(DIMENSION_MISMATCH, f"gemm dimension mismatch: a has K={k} but w has K={k2}")
-        out = out if out is not None else torch.empty(m, n, dtype=torch.int32, device=self._device)
+        out = out if out is not None else self._empty((m, n), torch.int32)
         self.call("hipq_gemm_i8_i32", _ptr(a), _ptr(w), m, n, k, _ptr(out))
         return out
 
     def linear_i8_f32(self, a, a_scale, w, w_scales, bias=None, out=None):
         m, k = a.shape
         n, _ = w.shape
-        out = out if out is not None else torch.empty(m, n, dtype=torch.float32, device=self._device)
-        self.call("hipq_linear_i8_f32", _ptr(a), _ptr(a_scale), int(a_scale.numel() > 1), _ptr(w), _ptr(w_scales),
-                  _ptr(bias), m, n, k, _ptr(out))
+        out = out if out is not None else self._empty((m, n), torch.float32)
+        self._native.hipq_linear_i8_f32(self._address, a, a_scale, int(a_scale.numel() > 1), w, w_scales, bias, m, n,
+                                        k, out)
         return out
 
     def quantize_static_per_tensor(self, x, scale, zp=0, mode=0, out=None, params=None):
@@ -540,22 +567,21 @@ class Context:
         """Quantized Linear forward with a calibrated (static) per-tensor activation scale."""
         m, k = x.shape
         n, _ = w.shape
-        out = out if out is not None else torch.empty(m, n, dtype=torch.float32, device=self._device)
-        self.call("hipq_linear_static_f32", _ptr(x), float(a_scale), _ptr(w), _ptr(w_scales), _ptr(bias), m, n, k, mode,
-                  _ptr(out))
+        out = out if out is not None else self._empty((m, n), torch.float32)
+        self._native.hipq_linear_static_f32(self._address, x, float(a_scale), w, w_scales, bias, m, n, k, mode, out)
         return out
 
     def linear_i8_i8(self, a, a_scale, w, w_scales, bias, out_scale, out_zp, mode=0, out=None):
         m, k = a.shape
         n, _ = w.shape
-        out = out if out is not None else torch.empty(m, n, dtype=torch.int8, device=self._device)
+        out = out if out is not None else self._empty((m, n), torch.int8)
         self.call("hipq_linear_i8_i8", _ptr(a), _ptr(a_scale), int(a_scale.numel() > 1), _ptr(w), _ptr(w_scales),
                   _ptr(bias), m, n, k, float(out_scale), int(out_zp), mode, _ptr(out))
         return out
 
     def requantize(self, acc, a_scale, w_scales, bias, out_scale, out_zp, mode=0):
         rows, cols = acc.shape
-        out = torch.empty(rows, cols, dtype=torch.int8, device=self._device)
+        out = self._empty((rows, cols), torch.int8)
         self.call("hipq_requantize_i32_i8", _ptr(acc), rows, cols, _ptr(a_scale), int(a_scale.numel() > 1),
                   _ptr(w_scales), _ptr(bias), float(out_scale), int(out_zp), mode, _ptr(out))
         return out
@@ -563,9 +589,8 @@ class Context:
     def linear_dynamic(self, x, w, w_scales, bias=None, per_token=False, mode=0, out=None):
         m, k = x.shape
         n, _ = w.shape
-        out = out if out is not None else torch.empty(m, n, dtype=torch.float32, device=self._device)
-        self.call("hipq_linear_dynamic_f32", _ptr(x), int(per_token), _ptr(w), _ptr(w_scales), _ptr(bias), m, n, k,
-                  mode, _ptr(out))
+        out = out if out is not None else self._empty((m, n), torch.float32)
+        self._native.hipq_linear_dynamic_f32(self._address, x, int(per_token), w, w_scales, bias, m, n, k, mode, out)
         return out
 
     # ---- fragment-packed operands ------------------------------------------------------
@@ -578,22 +603,22 @@ class Context:
         """int8 [rows, k] -> the packed operand of the fast GEMM (a flat int8 buffer)."""
         rows, k = q.shape
         out = out if out is not None else torch.empty(self.packed_size(rows, k), dtype=torch.int8, device=self._dev())
-        self.call("hipq_pack_rows_i8", _ptr(q), rows, k, _ptr(out))
+        self._native.hipq_pack_rows_i8(self._address, q, rows, k, out)
         return out
 
     def gemm_packed_i8_i32(self, a_packed, w_packed, m, n, k, out=None):
-        out = out if out is not None else torch.empty(m, n, dtype=torch.int32, device=self._device)
+        out = out if out is not None else self._empty((m, n), torch.int32)
         self.call("hipq_gemm_packed_i8_i32", _ptr(a_packed), _ptr(w_packed), m, n, k, _ptr(out))
         return out
 
     def linear_packed_i8_f32(self, a_packed, a_scale, w_packed, w_scales, bias, m, n, k, out=None):
-        out = out if out is not None else torch.empty(m, n, dtype=torch.float32, device=self._device)
-        self.call("hipq_linear_packed_i8_f32", _ptr(a_packed), _ptr(a_scale), int(a_scale.numel() > 1), _ptr(w_packed),
-                  _ptr(w_scales), _ptr(bias), m, n, k, _ptr(out))
+        out = out if out is not None else self._empty((m, n), torch.float32)
+        self._native.hipq_linear_packed_i8_f32(self._address, a_packed, a_scale, int(a_scale.numel() > 1), w_packed,
+                                               w_scales, bias, m, n, k, out)
         return out
 
     def linear_packed_i8_i8(self, a_packed, a_scale, w_packed, w_scales, bias, m, n, k, out_scale, out_zp, mode=0):
-        out = torch.empty(m, n, dtype=torch.int8, device=self._device)
+        out = self._empty((m, n), torch.int8)
         self.call("hipq_linear_packed_i8_i8", _ptr(a_packed), _ptr(a_scale), int(a_scale.numel() > 1), _ptr(w_packed),
                   _ptr(w_scales), _ptr(bias), m, n, k, float(out_scale), int(out_zp), mode, _ptr(out))
         return out
@@ -613,29 +638,29 @@ class Context:
         rows, cols = x.shape
         out = out if out is not None else torch.empty(self.packed_size(rows, cols), dtype=torch.int8,
                                                       device=self._dev())
-        scales = scales if scales is not None else torch.empty(rows, dtype=torch.float32, device=self._dev())
+        scales = scales if scales is not None else self._empty((rows,), torch.float32)
         self.call("hipq_quantize_per_row_packed_f32_i8", _ptr(x), rows, cols, mode, _ptr(out), _ptr(scales))
         return out, scales
 
     def linear_dynamic_packed(self, x, w_packed, w_scales, bias=None, per_token=False, mode=0, out=None):
         m, k = x.shape
         n = w_scales.numel()
-        out = out if out is not None else torch.empty(m, n, dtype=torch.float32, device=self._device)
-        self.call("hipq_linear_dynamic_packed_f32", _ptr(x), int(per_token), _ptr(w_packed), _ptr(w_scales), _ptr(bias),
-                  m, n, k, mode, _ptr(out))
+        out = out if out is not None else self._empty((m, n), torch.float32)
+        self._native.hipq_linear_dynamic_packed_f32(self._address, x, int(per_token), w_packed, w_scales, bias, m, n,
+                                                    k, mode, out)
         return out
 
     def linear_static_packed(self, x, a_scale, w_packed, w_scales, bias=None, mode=0, out=None):
         m, k = x.shape
         n = w_scales.numel()
-        out = out if out is not None else torch.empty(m, n, dtype=torch.float32, device=self._device)
-        self.call("hipq_linear_static_packed_f32", _ptr(x), float(a_scale), _ptr(w_packed), _ptr(w_scales), _ptr(bias),
-                  m, n, k, mode, _ptr(out))
+        out = out if out is not None else self._empty((m, n), torch.float32)
+        self._native.hipq_linear_static_packed_f32(self._address, x, float(a_scale), w_packed, w_scales, bias, m, n,
+                                                   k, mode, out)
         return out
 
     # ---- a panel of whole rows per workgroup: the Linear and the row operation after it ----
     def linear_rows_packed_i8_f32(self, a_packed, a_scale, w_packed, w_scales, bias, m, n, k, out=None):
-        out = out if out is not None else torch.empty(m, n, dtype=torch.float32, device=self._device)
+        out = out if out is not None else self._empty((m, n), torch.float32)
         self.call("hipq_linear_rows_packed_i8_f32", _ptr(a_packed), _ptr(a_scale), int(a_scale.numel() > 1),
                   _ptr(w_packed), _ptr(w_scales), _ptr(bias), m, n, k, _ptr(out))
         return out
@@ -644,7 +669,7 @@ class Context:
                                     scales=None):
         """-> (packed int8 [m, n] of GELU(linear), row scales [m])"""
         out = out if out is not None else torch.empty(self.packed_size(m, n), dtype=torch.int8, device=self._dev())
-        scales = scales if scales is not None else torch.empty(m, dtype=torch.float32, device=self._dev())
+        scales = scales if scales is not None else self._empty((m,), torch.float32)
         self.call("hipq_linear_gelu_quantize_packed_i8", _ptr(a_packed), _ptr(a_scale), int(a_scale.numel() > 1),
                   _ptr(w_packed), _ptr(w_scales), _ptr(bias), m, n, k, mode, _ptr(out), _ptr(scales))
         return out, scales
@@ -656,7 +681,7 @@ class Context:
         if normalize:
             out = out if out is not None else torch.empty(self.packed_size(m, n), dtype=torch.int8,
                                                           device=self._dev())
-            scales = scales if scales is not None else torch.empty(m, dtype=torch.float32, device=self._dev())
+            scales = scales if scales is not None else self._empty((m,), torch.float32)
         else:
             out = scales = None
         self.call("hipq_linear_residual_layer_norm_quantize_packed_i8", _ptr(a_packed), _ptr(a_scale),
@@ -669,9 +694,9 @@ class Context:
         should be given by callers that must not allocate; it is created here only as a convenience."""
         m, k = x.shape
         n, _ = w.shape
-        out = out if out is not None else torch.empty(m, n, dtype=torch.float32, device=self._device)
-        self.call("hipq_linear_dynamic_f32_noalloc", _ptr(x), int(per_token), _ptr(w), _ptr(w_scales), _ptr(bias), m, n,
-                  k, mode, _ptr(out))
+        out = out if out is not None else self._empty((m, n), torch.float32)
+        self._native.hipq_linear_dynamic_f32_noalloc(self._address, x, int(per_token), w, w_scales, bias, m, n, k,
+                                                     mode, out)
         return out
 
     def conv2d_i32(self, x_u8, zp_in, w_i8, stride=(1, 1), padding=(0, 0)):
@@ -681,7 +706,7 @@ class Context:
             raise HipqError(DIMENSION_MISMATCH, f"qconv2d channel mismatch: input C_in={c} but weight C_in={c2}")
         ho = max((h + 2 * padding[0] - kh) // stride[0] + 1, 0)  # the library rejects impossible geometry
         wo = max((wd + 2 * padding[1] - kw) // stride[1] + 1, 0)
-        out = torch.empty(nb, oc, ho, wo, dtype=torch.int32, device=self._device)
+        out = self._empty((nb, oc, ho, wo), torch.int32)
         self.call("hipq_conv2d_u8i8_i32", _ptr(x_u8), int(zp_in), _ptr(w_i8), nb, c, h, wd, oc, kh, kw, stride[0],
                   stride[1], padding[0], padding[1], _ptr(out))
         return out
@@ -694,10 +719,10 @@ class Context:
             raise HipqError(DIMENSION_MISMATCH, f"qconv2d channel mismatch: input C_in={c} but weight C_in={c2}")
         ho = max((h + 2 * padding[0] - kh) // stride[0] + 1, 0)  # the library rejects impossible geometry
         wo = max((wd + 2 * padding[1] - kw) // stride[1] + 1, 0)
-        out = out if out is not None else torch.empty(nb, oc, ho, wo, dtype=torch.int8, device=self._device)
-        self.call("hipq_conv2d_u8i8_i8", _ptr(x_u8), int(zp_in), float(s_in), _ptr(w_i8), _ptr(w_scales), _ptr(bias), nb,
-                  c, h, wd, oc, kh, kw, stride[0], stride[1], padding[0], padding[1], float(s_out), int(zp_out), mode,
-                  _ptr(out))
+        out = out if out is not None else self._empty((nb, oc, ho, wo), torch.int8)
+        self._native.hipq_conv2d_u8i8_i8(self._address, x_u8, int(zp_in), float(s_in), w_i8, w_scales, bias, nb, c, h,
+                                         wd, oc, kh, kw, stride[0], stride[1], padding[0], padding[1], float(s_out),
+                                         int(zp_out), mode, out)
         return out
 
     def conv2d_f32(self, x_u8, zp_in, s_in, w_i8, w_scales, bias, stride=(1, 1), padding=(0, 0), out=None):
@@ -707,7 +732,7 @@ class Context:
             raise HipqError(DIMENSION_MISMATCH, f"qconv2d channel mismatch: input C_in={c} but weight C_in={c2}")
         ho = max((h + 2 * padding[0] - kh) // stride[0] + 1, 0)
         wo = max((wd + 2 * padding[1] - kw) // stride[1] + 1, 0)
-        out = out if out is not None else torch.empty(nb, oc, ho, wo, dtype=torch.float32, device=self._device)
+        out = out if out is not None else self._empty((nb, oc, ho, wo), torch.float32)
         self.call("hipq_conv2d_u8i8_f32", _ptr(x_u8), int(zp_in), float(s_in), _ptr(w_i8), _ptr(w_scales), _ptr(bias), nb,
                   c, h, wd, oc, kh, kw, stride[0], stride[1], padding[0], padding[1], _ptr(out))
         return out
@@ -718,7 +743,7 @@ class Context:
         n = C.c_size_t(0)
         _check(self._lib.hipq_conv2d_packed_weights_size(oc, ic, kh, kw, C.byref(n)))
         packed = torch.empty(int(n.value), dtype=torch.int8, device=self._dev())
-        sums = torch.empty(oc, dtype=torch.int32, device=self._dev())
+        sums = self._empty((oc,), torch.int32)
         self.call("hipq_conv2d_pack_weights_i8", _ptr(w_i8), oc, ic, kh, kw, _ptr(packed), _ptr(sums))
         return packed, sums
 
@@ -729,10 +754,10 @@ class Context:
         kh, kw = kernel
         ho = h + 2 * padding[0] - kh + 1
         wo = wd + 2 * padding[1] - kw + 1
-        out = out if out is not None else torch.empty(nb, oc, ho, wo, dtype=torch.int8, device=self._device)
-        self.call("hipq_conv2d_u8i8_i8_packed", _ptr(x_u8), int(zp_in), float(s_in), _ptr(w_packed), _ptr(w_sums),
-                  _ptr(w_scales), _ptr(bias), nb, c, h, wd, oc, kh, kw, padding[0], padding[1], float(s_out),
-                  int(zp_out), mode, _ptr(out))
+        out = out if out is not None else self._empty((nb, oc, ho, wo), torch.int8)
+        self._native.hipq_conv2d_u8i8_i8_packed(self._address, x_u8, int(zp_in), float(s_in), w_packed, w_sums,
+                                                w_scales, bias, nb, c, h, wd, oc, kh, kw, padding[0], padding[1],
+                                                float(s_out), int(zp_out), mode, out)
         return out
 
     def conv2d_dynamic_packed(self, x, w_packed, w_sums, kernel, w_scales, bias, s_out, zp_out, padding=(0, 0),
@@ -744,17 +769,17 @@ class Context:
         kh, kw = kernel
         ho = h + 2 * padding[0] - kh + 1
         wo = wd + 2 * padding[1] - kw + 1
-        out = out if out is not None else torch.empty(nb, oc, ho, wo, dtype=torch.int8, device=self._device)
+        out = out if out is not None else self._empty((nb, oc, ho, wo), torch.int8)
         if params is None:  # (an empty batch launches nothing, and nothing writes its record)
             params = self._unset_qparams() if nb else self.new_qparams()
-        self.call("hipq_conv2d_dynamic_f32_i8_packed", _ptr(x), flavor, quant_mode, _ptr(w_packed), _ptr(w_sums),
-                  _ptr(w_scales), _ptr(bias), nb, c, h, wd, oc, kh, kw, padding[0], padding[1], float(s_out),
-                  int(zp_out), mode, _ptr(out), _ptr(params))
+        self._native.hipq_conv2d_dynamic_f32_i8_packed(self._address, x, flavor, quant_mode, w_packed, w_sums,
+                                                       w_scales, bias, nb, c, h, wd, oc, kh, kw, padding[0],
+                                                       padding[1], float(s_out), int(zp_out), mode, out, params)
         return out, params
 
     def quantize_per_row_strided(self, x_base, rows, cols, ld, elem_offset=0, flavor=PARAMS_SYMMETRIC, mode=0):
-        out = torch.empty(rows, cols, dtype=torch.int8, device=self._device)
-        scales = torch.empty(rows, dtype=torch.float32, device=self._dev())
+        out = self._empty((rows, cols), torch.int8)
+        scales = self._empty((rows,), torch.float32)
         self.call("hipq_quantize_per_row_strided_f32_i8", x_base.data_ptr() + 4 * elem_offset, rows, cols, ld, flavor,
                   mode, _ptr(out), _ptr(scales), None, None)
         return out, scales
@@ -762,7 +787,7 @@ class Context:
     def linear_i8_f32_residual(self, a, a_scale, w, w_scales, bias, residual, out=None):
         m, k = a.shape
         n, _ = w.shape
-        out = out if out is not None else torch.empty(m, n, dtype=torch.float32, device=self._device)
+        out = out if out is not None else self._empty((m, n), torch.float32)
         self.call("hipq_linear_i8_f32_residual", _ptr(a), _ptr(a_scale), int(a_scale.numel() > 1), _ptr(w),
                   _ptr(w_scales), _ptr(bias), _ptr(residual), m, n, k, _ptr(out))
         return out
@@ -775,8 +800,8 @@ class Context:
 
     def layer_norm_quantize(self, x, gamma=None, beta=None, eps=1e-5, mode=0):
         rows, cols = x.shape
-        out = torch.empty(rows, cols, dtype=torch.int8, device=self._device)
-        scales = torch.empty(rows, dtype=torch.float32, device=self._dev())
+        out = self._empty((rows, cols), torch.int8)
+        scales = self._empty((rows,), torch.float32)
         self.call("hipq_layer_norm_quantize_f32_i8", _ptr(x), rows, cols, _ptr(gamma), _ptr(beta), float(eps), mode,
                   _ptr(out), _ptr(scales))
         return out, scales
@@ -791,7 +816,7 @@ class Context:
         if normalize:
             out = out if out is not None else torch.empty(self.packed_size(m, n), dtype=torch.int8,
                                                           device=self._dev())
-            scales = scales if scales is not None else torch.empty(m, dtype=torch.float32, device=self._dev())
+            scales = scales if scales is not None else self._empty((m,), torch.float32)
         else:
             out = scales = None
         self.call("hipq_linear_from_f32_residual_layer_norm_quantize_packed_i8", a.data_ptr(), a.stride(0),
@@ -802,8 +827,8 @@ class Context:
     def add_layer_norm_quantize(self, x, delta, gamma=None, beta=None, eps=1e-5, mode=0):
         """x += delta in place, then LayerNorm + per-token int8 of the new x."""
         rows, cols = x.shape
-        out = torch.empty(rows, cols, dtype=torch.int8, device=self._device)
-        scales = torch.empty(rows, dtype=torch.float32, device=self._dev())
+        out = self._empty((rows, cols), torch.int8)
+        scales = self._empty((rows,), torch.float32)
         self.call("hipq_add_layer_norm_quantize_f32_i8", _ptr(x), _ptr(delta), rows, cols, _ptr(gamma), _ptr(beta),
                   float(eps), mode, _ptr(out), _ptr(scales))
         return out, scales
@@ -815,8 +840,8 @@ class Context:
 
     def gelu_tanh_quantize(self, x, mode=0):
         rows, cols = x.shape
-        out = torch.empty(rows, cols, dtype=torch.int8, device=self._device)
-        scales = torch.empty(rows, dtype=torch.float32, device=self._dev())
+        out = self._empty((rows, cols), torch.int8)
+        scales = self._empty((rows,), torch.float32)
         self.call("hipq_gelu_tanh_quantize_f32_i8", _ptr(x), rows, cols, mode, _ptr(out), _ptr(scales))
         return out, scales
 
@@ -827,7 +852,7 @@ class Context:
 
     def stack_workspace(self, tokens, d_model, d_ff):
         nbytes = self._lib.hipq_transformer_stack_workspace_bytes(tokens, d_model, d_ff)
-        return torch.empty(nbytes, dtype=torch.uint8, device=self._dev())
+        return self._empty((nbytes,), torch.uint8)
 
     def stack_prepare(self, blocks):
         """The blocks with every int8 weight matrix in packed order (done once per model)."""
@@ -835,18 +860,14 @@ class Context:
 
     def stack_workspace_prepared(self, tokens, d_model, d_ff):
         nbytes = self._lib.hipq_transformer_stack_prepared_workspace_bytes(tokens, d_model, d_ff)
-        return torch.empty(nbytes, dtype=torch.uint8, device=self._dev())
+        return self._empty((nbytes,), torch.uint8)
 
     def stack_forward(self, blocks, x, d_ff, workspace, eps=1e-5, mode=0, prepared=False):
         """blocks: list of dicts of device tensors keyed like BlockWeights; x [tokens, d_model] is updated in place.
         prepared: the blocks come from stack_prepare and the workspace from stack_workspace_prepared."""
-        arr = (BlockWeights * len(blocks))()
-        for rec, blk in zip(arr, blocks):
-            for name, _ in BlockWeights._fields_:
-                t = blk.get(name)
-                setattr(rec, name, None if t is None else t.data_ptr())
+        records = self._native.pointers(blocks, _BLOCK_TENSORS)  # one BlockWeights per block
         tokens, d_model = x.shape
         self.call("hipq_transformer_stack_forward_prepared_f32" if prepared else "hipq_transformer_stack_forward_f32",
-                  C.cast(arr, C.c_void_p), len(blocks), tokens, d_model, d_ff, float(eps), mode, _ptr(x),
+                  records, len(blocks), tokens, d_model, d_ff, float(eps), mode, _ptr(x),
                   _ptr(workspace), workspace.numel())
         return x
