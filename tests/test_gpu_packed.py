@@ -892,3 +892,72 @@ def test_products_of_few_blocks(hipq, m, n, k):
                 assert torch.equal(got[0], got[1])
     finally:
         c.close()
+
+
+# Rows and columns around a tile, K around one 64-byte quad, a wave's second quad, both register forms and their ends, rows of
+# weights at odd bytes; per tensor up to the last size that is read by every workgroup.
+@pytest.mark.parametrize("m,n,k", [(1, 1, 16), (3, 33, 17), (16, 32, 64), (17, 31, 63), (40, 70, 65), (5, 100, 127), (15, 8192, 24), (4095, 30, 16),
+                                   (33, 65, 1023), (64, 96, 1024), (31, 40, 1025), (32, 64, 2048), (20, 33, 2047), (9, 5, 1), (9, 5, 15)])
+def test_linear_of_small_sizes_in_one_launch(hipq, m, n, k):
+    """Quantizer and product in one launch: the bits of the two (hook 11 leaves the kernels as they are but keeps the two), for
+    every range, both forms and roundings, with and without a bias, weights packed and as rows, x and the weights at any
+    alignment; values that saturate, a row of zeros, and ranges that are not finite."""
+    c = hipq.Context(0)
+    try:
+        g = torch.Generator(device="cuda").manual_seed(m * 7 + n + k)
+        x = torch.randn(m * k + 1, generator=g, device="cuda")[1:].view(m, k)
+        x[m // 2] = 0.0
+        x[-1, -1] = 9.0
+        x[0, k // 2] = float("nan")
+        w = torch.randint(-128, 128, (n * k + 3,), generator=g, device="cuda", dtype=torch.int8)[3:].view(n, k)
+        sw = torch.rand(n, generator=g, device="cuda") * 1e-3 + 1e-4
+        bias = torch.randn(n, generator=g, device="cuda")
+        pw, aligned = c.pack_rows(w), w.clone()
+        infinite = x.clone()
+        infinite[m - 1, 0] = float("-inf")
+        same = lambda a, b: torch.equal(torch.nan_to_num(a, nan=-77.0), torch.nan_to_num(b, nan=-77.0))
+        for mode in (0, hipq.FORM_DIV, hipq.ROUND_HALF_EVEN, hipq.FORM_DIV | hipq.ROUND_HALF_EVEN):
+            for xs in (x, infinite):
+                for b in (bias, None):
+                    calls = [lambda w_=w_, t=t: c.linear_dynamic(xs, w_, sw, b, per_token=t, mode=mode) for t in (False, True) for w_ in (w, aligned)]
+                    calls += [lambda t=t: c.linear_dynamic_packed(xs, pw, sw, b, per_token=t, mode=mode) for t in (False, True)]
+                    calls += [lambda w_=w_, s=s: c.linear_static(xs, s, w_, sw, b, mode=mode) for s in (4.0 / 127, 1e-39) for w_ in (w, aligned)]
+                    calls += [lambda s=s: c.linear_static_packed(xs, s, pw, sw, b, mode=mode) for s in (4.0 / 127, 1e-39)]
+                    for i, call in enumerate(calls):
+                        got = call()
+                        c.set_gemm_kernel_variant(11)
+                        want = call()
+                        c.set_gemm_kernel_variant(0)
+                        assert same(got, want), (mode, i, b is None, xs is x)
+        c.synchronize()
+    finally:
+        torch.cuda.synchronize()
+        c.close()
+
+
+def test_linear_of_small_sizes_keeps_its_errors(hipq):
+    c = hipq.Context(0)
+    try:
+        x, sw = torch.randn(4, 64, device="cuda"), torch.ones(8, device="cuda")
+        w = torch.ones(8, 64, dtype=torch.int8, device="cuda")
+        pw = c.pack_rows(w)
+        for bad in (0.0, -1.0, float("nan")):
+            for call in (lambda: c.linear_static(x, bad, w, sw), lambda: c.linear_static_packed(x, bad, pw, sw)):
+                c.set_gemm_kernel_variant(11)
+                try:
+                    call()
+                    refused = None
+                except hipq.HipqError as e:
+                    refused = (e.code, e.message)
+                c.set_gemm_kernel_variant(0)
+                try:
+                    call()
+                    assert refused is None
+                except hipq.HipqError as e:
+                    assert (e.code, e.message) == refused
+        for call in (lambda: c.linear_dynamic(x, w, sw, mode=1 << 20), lambda: c.linear_static_packed(x, 0.1, pw, sw, mode=1 << 20)):
+            with pytest.raises(hipq.HipqError):
+                call()
+    finally:
+        torch.cuda.synchronize()
+        c.close()

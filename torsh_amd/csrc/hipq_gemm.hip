@@ -464,6 +464,9 @@ static int32_t linear_dynamic_on(hipq_ctx *ctx, char *base, const float *x, int3
     float *row_scales = reinterpret_cast<float *>(base + kScratchHeader + partial_bytes);
     int8_t *qa = reinterpret_cast<int8_t *>(base + kScratchHeader + partial_bytes + linear_dynamic_scales_bytes(m));
     int32_t rc;
+    if (linear_small(ctx, per_token ? LINEAR_PER_TOKEN : LINEAR_PER_TENSOR, x, 1.0f, w, /*w_rows=*/true, w_scales, bias, m, n, k, mode,
+                     out, &rc))
+        return rc;
     if (per_token) {
         rc = quantize_activations_per_row(ctx, x, m, k, mode & HIPQ_ROUND_HALF_EVEN, qa, row_scales);
         if (rc) return rc;
@@ -623,6 +626,7 @@ int32_t hipq_linear_static_f32(hipq_ctx *ctx, const float *x, float a_scale, con
     HIPQ_REQUIRE_PTR(w);
     HIPQ_REQUIRE_PTR(w_scales);
     HIPQ_REQUIRE_PTR(out);
+    if (linear_small(ctx, LINEAR_STATIC, x, a_scale, w, /*w_rows=*/true, w_scales, bias, m, n, k, mode, out, &rc)) return rc;
     void *s = nullptr;
     rc = scratch(ctx, kScratchHeader + m * k + 256, &s);
     if (rc) return rc;

@@ -290,11 +290,13 @@ int32_t hipq_linear_dynamic_packed_f32(hipq_ctx *ctx, const float *x, int32_t pe
                                    : launch_gemv_packed_from_f32<false, false>(ctx, x, w_packed, m, n, k, ep, 0, &rc);
             if (fused) return rc;
         }
+        if (linear_small(ctx, LINEAR_PER_TOKEN, x, 1.0f, w_packed, false, w_scales, bias, m, n, k, mode, out, &rc)) return rc;
         // one pass over the activations: the per-row quantizer writes the packed operand itself
         rc = quantize_activations_per_row(ctx, x, m, k, mode & HIPQ_ROUND_HALF_EVEN, pa, row_scales, /*packed=*/true);
         if (rc) return rc;
         return linear_packed_launch(ctx, pa, row_scales, 1, w_packed, w_scales, bias, m, n, k, out, true);
     }
+    if (linear_small(ctx, LINEAR_PER_TENSOR, x, 1.0f, w_packed, false, w_scales, bias, m, n, k, mode, out, &rc)) return rc;
     set_weight_warming(ctx, w_packed, m, n, k);
     rc = quantize_activations_per_tensor(ctx, x, m, k, true, 1.0f, mode, true, pa, params, base + L.partials,
                                          L.scales - L.partials);
@@ -326,6 +328,7 @@ int32_t hipq_linear_static_packed_f32(hipq_ctx *ctx, const float *x, float a_sca
                                : launch_gemv_packed_from_f32<false, true>(ctx, x, w_packed, m, n, k, ep, div, &rc);
         if (fused) return rc;
     }
+    if (linear_small(ctx, LINEAR_STATIC, x, a_scale, w_packed, /*w_rows=*/false, w_scales, bias, m, n, k, mode, out, &rc)) return rc;
     const PackedScratch L = packed_scratch_layout(ctx->num_cus, m, k);
     void *s = nullptr;
     rc = scratch(ctx, L.total, &s);

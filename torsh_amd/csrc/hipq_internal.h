@@ -175,6 +175,11 @@ int32_t gelu_quantize_packed(hipq_ctx *ctx, const float *x, size_t rows, size_t 
 int32_t linear_packed_rows_f32(hipq_ctx *ctx, const int8_t *a_packed, const float *a_scales, const int8_t *w_packed,
                                const float *w_scales, const float *bias, const float *residual, size_t m, size_t n, size_t k,
                                float *out);
+// A Linear of small sizes in one launch (hipq_linear_small.hip): x fp32 [m, k], weights packed or (w_rows) rows of k bytes; the codes
+// and results of the quantizer and the product it stands for.  Returns false, having done nothing, where those are to run.
+enum LinearRange { LINEAR_PER_TENSOR, LINEAR_PER_TOKEN, LINEAR_STATIC };
+bool linear_small(hipq_ctx *ctx, LinearRange range, const float *x, float scale, const int8_t *w, bool w_rows, const float *w_scales,
+                  const float *bias, size_t m, size_t n, size_t k, int32_t mode, float *out, int32_t *rc);
 // Looks up, once per device, the address of the static device array behind
 // hipq_linear_dynamic_f32_noalloc; called by hipq_ctx_create with the device current.
 int32_t linear_noalloc_setup(int device);
