@@ -299,12 +299,12 @@ struct FragmentWalk {
         kb_shift = __builtin_ffsll(static_cast<long long>(KB)) - 1;
     }
     __device__ size_t first() const { return size_t(blockIdx.x) * (kBlock / kWave) + threadIdx.x / kWave; }
-    // The lane's 16 floats of fragment `frag`.  Rows start at any float (a load of four floats needs the alignment of one), and
-    // elements past the matrix are NaN: neither the minimum nor the maximum changes, and the code is 0.  Returns false where
-    // the lane has no element.
-    // Element by element, rows that were not all 16-byte aligned took (Linear from fp32, us, before / now): 4140 x 576 x 4063
-    // 219 / 69, 1500 x 2048 x 1050 18.7 / 15.0, 77 x 1024 x 1001 13.5 / 9.7 (the last as they may also take the one-launch form).
-    __device__ bool load(size_t frag, AnyFloat4 (&v)[4]) const {
+    // Requests the lane's 16 floats of fragment `frag`; returns false where the lane has no element.  Rows start at any float (a
+    // load of four floats needs the alignment of one).  The last piece of a row is read where its last 16 floats lie and moved
+    // into place by settle, so that a request is four loads on one path and can stay in flight: where the end of a row had a path of
+    // its own, the loads were waited for at its end (6424 x 12992 with a static scale 80 -> 91 us).  SHORT: rows of less than 16 floats.
+    template <bool SHORT>
+    __device__ __forceinline__ bool request(size_t frag, AnyFloat4 (&v)[4], int *drop) const {
         size_t rb, kb;
         if (kb_pow2) {
             rb = frag >> kb_shift;
@@ -317,18 +317,41 @@ struct FragmentWalk {
             kb = frag % KB;
         }
         const size_t row = rb * 32 + lane % 32, k0 = kb * 32 + 16 * (lane / 32);
+        *drop = 0;
         if (frag >= nfrag || row >= rows || k0 >= cols) return false;
-        const float *p = x + row * cols + k0;
-        if (k0 + 16 <= cols) {
+        if constexpr (SHORT) {
+            const float *p = x + row * cols;
+            const int left = static_cast<int>(cols);
+            auto at = [&](int b) { return b < left ? p[b] : __builtin_nanf(""); };
 #pragma unroll
-            for (int i = 0; i < 4; ++i) v[i] = reinterpret_cast<const AnyFloat4 *>(p)[i];
-            return true;
+            for (int i = 0; i < 4; ++i) v[i] = AnyFloat4{at(4 * i), at(4 * i + 1), at(4 * i + 2), at(4 * i + 3)};
+        } else {
+            const size_t at = k0 + 16 <= cols ? k0 : cols - 16;
+            *drop = static_cast<int>(k0 - at);
+            const AnyFloat4 *p = reinterpret_cast<const AnyFloat4 *>(x + row * cols + at);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = p[i];
         }
-        const int left = static_cast<int>(cols - k0);
-        auto at = [&](int b) { return b < left ? p[b] : __builtin_nanf(""); };
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = AnyFloat4{at(4 * i), at(4 * i + 1), at(4 * i + 2), at(4 * i + 3)};
         return true;
+    }
+    // Drops the first `drop` floats of what was requested, for NaN behind the last: neither the minimum nor the maximum changes,
+    // and the code is 0.
+    static __device__ __forceinline__ void settle(AnyFloat4 (&v)[4], int drop) {
+        if (!__any(drop != 0)) return;
+        float e[16];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            e[4 * i] = v[i].x;
+            e[4 * i + 1] = v[i].y;
+            e[4 * i + 2] = v[i].z;
+            e[4 * i + 3] = v[i].w;
+        }
+#pragma unroll
+        for (int step = 8; step > 0; step /= 2)
+#pragma unroll
+            for (int b = 0; b < 16; ++b) e[b] = drop & step ? (b + step < 16 ? e[b + step < 16 ? b + step : b] : __builtin_nanf("")) : e[b];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = AnyFloat4{e[4 * i], e[4 * i + 1], e[4 * i + 2], e[4 * i + 3]};
     }
     static __device__ __forceinline__ void fold(MinMax &m, const AnyFloat4 (&v)[4]) {
 #pragma unroll
@@ -341,6 +364,7 @@ struct FragmentWalk {
 
 // Range pass over a matrix in the packed quantizer's order (see FragmentWalk): one (min, max) partial per
 // workgroup, the same numbers as minmax_partial_kernel's fold whatever the order (min and max are exact).
+template <bool SHORT>
 __global__ __launch_bounds__(kBlock) void minmax_fragments_kernel(const float *__restrict__ x, size_t rows, size_t cols,
                                                                    float2 *__restrict__ partials) {
     __shared__ float lds[2 * kBlock / kWave];
@@ -348,7 +372,10 @@ __global__ __launch_bounds__(kBlock) void minmax_fragments_kernel(const float *_
     MinMax m{INFINITY, -INFINITY};
     for (size_t f = fw.first(); f < fw.nfrag; f += fw.fstep) {
         AnyFloat4 v[4];
-        if (fw.load(f, v)) FragmentWalk::fold(m, v);
+        int drop;
+        const bool have = fw.request<SHORT>(f, v, &drop);
+        if constexpr (!SHORT) FragmentWalk::settle(v, drop);
+        if (have) FragmentWalk::fold(m, v);
     }
     const MinMax r = block_minmax(m, lds);
     if (threadIdx.x == 0) partials[blockIdx.x] = make_float2(r.mn, r.mx);
@@ -361,7 +388,7 @@ __global__ __launch_bounds__(kBlock) void minmax_fragments_kernel(const float *_
 // covers 16 Mi elements.  The launch bound keeps the kernel at 128 registers, so that four workgroups fit a
 // compute unit: the caller relies on the grid being resident at once.  Wave w of the grid takes fragments
 // w, w + waves, ...
-template <bool DIV, int RND, int FPW>
+template <bool DIV, int RND, int FPW, bool SHORT>
 __global__ __launch_bounds__(kBlock, 4) void quantize_packed_one_launch_kernel(const float *__restrict__ x, size_t rows,
                                                                                 size_t cols, hipq_qparams *out_params,
                                                                                 uint32_t *words, int spin_limit,
@@ -372,18 +399,21 @@ __global__ __launch_bounds__(kBlock, 4) void quantize_packed_one_launch_kernel(c
     size_t f[FPW];
     bool have[FPW];
     AnyFloat4 v[FPW][4];
+    int drop[FPW];
 #pragma unroll
     for (int u = 0; u < FPW; ++u) {
         f[u] = fw.first() + u * fw.fstep;
-        have[u] = fw.load(f[u], v[u]);
+        have[u] = fw.request<SHORT>(f[u], v[u], &drop[u]);
     }
     // Behind the fragments' loads in program order: memory operations return in order, and the number is not
     // needed before the fragments have been folded.
     const uint32_t gen = meeting_number(words);
     MinMax m{INFINITY, -INFINITY};
 #pragma unroll
-    for (int u = 0; u < FPW; ++u)
+    for (int u = 0; u < FPW; ++u) {
+        if constexpr (!SHORT) FragmentWalk::settle(v[u], drop[u]);
         if (have[u]) FragmentWalk::fold(m, v[u]);
+    }
     const MinMax r = block_minmax(m, lds);
     // While the grid agrees on the range the memory system is idle: touch the lines of the next kernel's operand
     // that the workgroups of this die (workgroups are dealt to the dies in turn) will read first thing, one load
@@ -539,7 +569,7 @@ static bool launch_flat_one_launch(hipq_ctx *ctx, const float *x, size_t n, int 
     return true;
 }
 
-template <bool DIV, int RND>
+template <bool DIV, int RND, bool SHORT>
 __global__ __launch_bounds__(kBlock) void quantize_packed_kernel(const float *__restrict__ x, size_t rows,
                                                                   size_t cols, float scale, int zp,
                                                                   const hipq_qparams *__restrict__ params,
@@ -552,13 +582,15 @@ __global__ __launch_bounds__(kBlock) void quantize_packed_kernel(const float *__
     // partials and two workgroup barriers in a dynamic call): the loads do not depend on the scale, and a
     // launch of this size is bound by latency, not by bandwidth.
     AnyFloat4 v[4];
-    bool have = fw.load(f, v);
+    int drop;
+    bool have = fw.request<SHORT>(f, v, &drop);
     __shared__ float range_lds[2 * kBlock / kWave];
     if (!resolve_quantize_params(dyn, params, range_lds, scale, zp)) return;
     const float inv = DIV ? recip_for_div(scale) : 1.0f / scale;
     const float zpf = static_cast<float>(zp);
     for (; f < nfrag; f += fstep) {
         uint32_t w[4] = {0u, 0u, 0u, 0u};
+        if constexpr (!SHORT) FragmentWalk::settle(v, drop);
         if (have) {
 #pragma unroll
             for (int i = 0; i < 4; ++i)
@@ -568,7 +600,7 @@ __global__ __launch_bounds__(kBlock) void quantize_packed_kernel(const float *__
                              quantize_int<DIV, RND>(v[i].w, scale, inv, zpf, -128, 127));
         }
         *reinterpret_cast<uint4 *>(out + f * 1024 + size_t(lane) * 16) = make_uint4(w[0], w[1], w[2], w[3]);
-        have = fw.load(f + fstep, v);
+        have = fw.request<SHORT>(f + fstep, v, &drop);
     }
 }
 
@@ -1172,7 +1204,8 @@ bool four_wide_workgroups_fit(const hipq_ctx *ctx) {
     if (ctx->device < 0 || ctx->device >= 16) return false;
     if (resident[ctx->device] == 0) {
         const void *wide[] = {reinterpret_cast<const void *>(quantize_flat_one_launch_kernel<int8_t, false, 0, 16>),
-                              reinterpret_cast<const void *>(quantize_packed_one_launch_kernel<false, 0, 4>),
+                              reinterpret_cast<const void *>(quantize_packed_one_launch_kernel<false, 0, 4, false>),
+                              reinterpret_cast<const void *>(quantize_packed_one_launch_kernel<false, 0, 4, true>),
                               reinterpret_cast<const void *>(channel_parts_kernel<false>),
                               reinterpret_cast<const void *>(channel_parts_kernel<true>)};
         int least = 1 << 30;
@@ -2115,10 +2148,16 @@ int32_t hipq::quantize_activations_per_tensor(hipq_ctx *ctx, const float *x, siz
     const size_t q1_blocks = (blocks + fpw - 1) / fpw;
     if (dynamic && packed && ctx->gemm_variant != 6 && q1_blocks <= resident_workgroups(ctx, fpw == 4) &&
         (fpw == 1 || four_wide_workgroups_fit(ctx))) {
-#define HIPQ_LAUNCH_Q1(D, E, F)                                                                                           \
-    hipLaunchKernelGGL((quantize_packed_one_launch_kernel<D, E, F>), dim3(static_cast<int>(q1_blocks)), dim3(kBlock), 0, \
-                       ctx->stream, x, rows, cols, out_params, ctx->wait_error, ctx->wait_spin_limit, out,              \
-                       ctx->warm)
+#define HIPQ_LAUNCH_Q1_ROWS(D, E, F, S)                                                                                      \
+    hipLaunchKernelGGL((quantize_packed_one_launch_kernel<D, E, F, S>), dim3(static_cast<int>(q1_blocks)), dim3(kBlock), 0, \
+                       ctx->stream, x, rows, cols, out_params, ctx->wait_error, ctx->wait_spin_limit, out, ctx->warm)
+#define HIPQ_LAUNCH_Q1(D, E, F)                  \
+    do {                                         \
+        if (cols < 16)                           \
+            HIPQ_LAUNCH_Q1_ROWS(D, E, F, true);  \
+        else                                     \
+            HIPQ_LAUNCH_Q1_ROWS(D, E, F, false); \
+    } while (0)
 #define HIPQ_LAUNCH_Q1_MODE(F)          \
     do {                                \
         if (div && even)                \
@@ -2138,6 +2177,7 @@ int32_t hipq::quantize_activations_per_tensor(hipq_ctx *ctx, const float *x, siz
             HIPQ_LAUNCH_Q1_MODE(4);
 #undef HIPQ_LAUNCH_Q1_MODE
 #undef HIPQ_LAUNCH_Q1
+#undef HIPQ_LAUNCH_Q1_ROWS
         return check_launch("quantize (packed, one launch)");
     }
     if (dynamic && packed) {
@@ -2151,7 +2191,7 @@ int32_t hipq::quantize_activations_per_tensor(hipq_ctx *ctx, const float *x, siz
             if ((rc = scratch(ctx, kScratchHeader + size_t(grid) * sizeof(float2), &s))) return rc;
             p = reinterpret_cast<float2 *>(static_cast<char *>(s) + kScratchHeader);
         }
-        hipLaunchKernelGGL(minmax_fragments_kernel, dim3(grid), dim3(kBlock), 0, ctx->stream, x, rows, cols, p);
+        hipLaunchKernelGGL(cols < 16 ? minmax_fragments_kernel<true> : minmax_fragments_kernel<false>, dim3(grid), dim3(kBlock), 0, ctx->stream, x, rows, cols, p);
         if ((rc = check_launch("minmax (fragments)"))) return rc;
         dyn.partials = p;
         dyn.nparts = grid;
@@ -2168,9 +2208,16 @@ int32_t hipq::quantize_activations_per_tensor(hipq_ctx *ctx, const float *x, siz
         scale = static_scale;
     }
     if (!packed) return launch_quantize<int8_t>(ctx, x, rows * cols, scale, 0, nullptr, mode, -128.0f, 127.0f, out, dyn);
-#define HIPQ_LAUNCH_QP(D, E)                                                                                       \
-    hipLaunchKernelGGL((quantize_packed_kernel<D, E>), dim3(grid), dim3(kBlock), 0, ctx->stream, x, rows, cols, scale, \
+#define HIPQ_LAUNCH_QP_ROWS(D, E, S)                                                                                     \
+    hipLaunchKernelGGL((quantize_packed_kernel<D, E, S>), dim3(grid), dim3(kBlock), 0, ctx->stream, x, rows, cols, scale, \
                        0, static_cast<const hipq_qparams *>(nullptr), dyn, out)
+#define HIPQ_LAUNCH_QP(D, E)                  \
+    do {                                      \
+        if (cols < 16)                        \
+            HIPQ_LAUNCH_QP_ROWS(D, E, true);  \
+        else                                  \
+            HIPQ_LAUNCH_QP_ROWS(D, E, false); \
+    } while (0)
     if (div && even)
         HIPQ_LAUNCH_QP(true, 1);
     else if (div)
@@ -2180,6 +2227,7 @@ int32_t hipq::quantize_activations_per_tensor(hipq_ctx *ctx, const float *x, siz
     else
         HIPQ_LAUNCH_QP(false, 0);
 #undef HIPQ_LAUNCH_QP
+#undef HIPQ_LAUNCH_QP_ROWS
     return check_launch("quantize (packed)");
 }
 
