@@ -961,3 +961,36 @@ def test_linear_of_small_sizes_keeps_its_errors(hipq):
     finally:
         torch.cuda.synchronize()
         c.close()
+
+
+# 3, 5, 7 and 33 steps of K a wave (two a round and one over), one and two (neither has a remainder); edges of 128 x 64 tiles.
+@pytest.mark.parametrize("m,n,k", [(130, 70, 352), (128, 64, 640), (257, 129, 896), (65, 200, 4224), (100, 100, 128), (100, 100, 256)])
+def test_gemm_tiles_with_an_odd_number_of_steps(hipq, m, n, k):
+    c = hipq.Context(0)
+    try:
+        g = torch.Generator(device="cuda").manual_seed(m + n + k)
+        a = torch.randint(-128, 128, (m, k), generator=g, device="cuda", dtype=torch.int8)
+        w = torch.randint(-128, 128, (n, k), generator=g, device="cuda", dtype=torch.int8)
+        c.set_gemm_kernel_variant(9)  # the 128 x 64 tiles
+        got = c.gemm_packed_i8_i32(c.pack_rows(a), c.pack_rows(w), m, n, k)
+        torch.cuda.synchronize()
+        assert torch.equal(got.cpu(), (a.cpu().double() @ w.cpu().double().t()).to(torch.int32))
+    finally:
+        torch.cuda.synchronize()
+        c.close()
+
+
+# Three rounds of 128 x 64 tiles on long rows: dealt evenly to eight dies (24 x 22), not (23 x 25; the tiles staged through LDS).
+@pytest.mark.parametrize("m,n", [(24 * 128, 22 * 64), (23 * 128 - 5, 25 * 64 - 3)])
+def test_gemm_three_rounds_of_tiles(hipq, m, n):
+    c, k = hipq.Context(0), 1100
+    try:
+        g = torch.Generator(device="cuda").manual_seed(m + n)
+        pa = c.pack_rows(torch.randint(-128, 128, (m, k), generator=g, device="cuda", dtype=torch.int8))
+        pw = c.pack_rows(torch.randint(-128, 128, (n, k), generator=g, device="cuda", dtype=torch.int8))
+        got = c.gemm_packed_i8_i32(pa, pw, m, n, k)
+        c.set_gemm_kernel_variant(9)
+        assert torch.equal(got, c.gemm_packed_i8_i32(pa, pw, m, n, k))
+    finally:
+        torch.cuda.synchronize()
+        c.close()

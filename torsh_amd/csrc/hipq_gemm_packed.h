@@ -40,7 +40,9 @@ namespace hipq {
 // Issuing the loads of a stage between the MFMAs of the stage being multiplied (a third register slot, one load
 // behind each of the first six MFMAs, the order pinned with sched_group_barrier) instead of behind all eight was
 // measured: K loop 19.6 k -> 18.4 k cycles under the stamps, 14.7 us from launch to launch either way.  Not kept.
-template <int TMB, int TNB, int D, int EPI, bool EVEN, bool TRACE = false, bool HALVES = false>
+//
+// ODD: a last step that two stages a round leave over, as a form of its own (the branches for it cost the other shapes 1 to 8 %).
+template <int TMB, int TNB, int D, int EPI, bool EVEN, bool TRACE = false, bool HALVES = false, bool ODD = false>
 __global__ __launch_bounds__(256) void gemm_i8_packed_kernel(const int8_t *__restrict__ PA,
                                                              const int8_t *__restrict__ PW, int M, int N, int K,
                                                              GemmEpilogue ep) {
@@ -132,22 +134,26 @@ __global__ __launch_bounds__(256) void gemm_i8_packed_kernel(const int8_t *__res
                 acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[slot][i], fb[slot][j], acc[i][j], 0, 0, 0);
     };
 
-    // steps is a positive multiple of D (the host picks D so).
+    // steps is a positive multiple of D, or (ODD) one more than that (the host picks the form so).
+    static_assert(!ODD || D == 2, "a remainder of one step");
 #pragma unroll
     for (int u = 0; u < D; ++u) issue(u, u);
     if constexpr (TRACE) {
         wait_vmcnt<(D - 1) * (TMB + TNB)>();  // the first stage has landed
         mark(1);
     }
-    for (int s0 = D; s0 < steps; s0 += D) {
+    for (int s0 = D; s0 < steps - ODD; s0 += D) {
 #pragma unroll
         for (int u = 0; u < D; ++u) {
             compute(u);
             issue(s0 + u, u);
         }
     }
+    compute(0);
+    if constexpr (ODD) issue(steps - 1, 0);
 #pragma unroll
-    for (int u = 0; u < D; ++u) compute(u);
+    for (int u = 1; u < D; ++u) compute(u);
+    if constexpr (ODD) compute(0);
     if constexpr (TRACE) {
         // the last MFMA has retired once its result can be read
         asm volatile("s_nop 15\n\ts_nop 15" ::"v"(acc[TMB - 1][TNB - 1][0]));
@@ -904,11 +910,11 @@ __global__ __launch_bounds__(256) void pack_rows_i8_kernel(const int8_t *__restr
 
 namespace hipq {
 
-template <int TMB, int TNB, int D, int EPI, bool EVEN, bool TRACE = false, bool HALVES = false>
+template <int TMB, int TNB, int D, int EPI, bool EVEN, bool TRACE = false, bool HALVES = false, bool ODD = false>
 static int32_t launch_packed(hipq_ctx *ctx, const int8_t *pa, const int8_t *pw, int M, int N, int K,
                              const GemmEpilogue &ep) {
     constexpr int kLds = TMB * (HALVES ? 1 : TNB) * 3 * 4096;
-    auto kernel = gemm_i8_packed_kernel<TMB, TNB, D, EPI, EVEN, TRACE, HALVES>;
+    auto kernel = gemm_i8_packed_kernel<TMB, TNB, D, EPI, EVEN, TRACE, HALVES, ODD>;
     static bool configured[16] = {false};  // per device: raise the dynamic LDS limit once
     if (ctx->device < 16 && !configured[ctx->device]) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
@@ -926,7 +932,7 @@ static int32_t launch_packed(hipq_ctx *ctx, const int8_t *pa, const int8_t *pw, 
     return check_launch("gemm_i8 (packed)");
 }
 
-// Register depth 2 where it divides the k blocks per wave (else 1): two stages of 6 KiB per wave in flight.  Depth
+// Register depth 2 (1 where a wave has one step of K): two stages of 6 KiB per wave in flight.  Depth
 // 4 is as fast when the kernel is launched back to back at sustained clocks (14.8 us at M = 512, N = K = 4096) but
 // slower from idle clocks (17.6 against 15.7 us) and inside the Linear step, where the kernel follows the small
 // quantize kernels (24.2 against 23.5 us per step); depth 1 is 2-3 us slower everywhere.
@@ -974,7 +980,13 @@ static int32_t launch_gemm_packed(hipq_ctx *ctx, const int8_t *pa, const int8_t 
         const size_t rbA = packed_row_blocks(m), rbW = packed_row_blocks(n), cus = size_t(ctx->num_cus);
         const size_t rounds = (((rbA + 3) / 4) * ((rbW + 1) / 2) + cus - 1) / cus;
         const bool forced = ctx->gemm_variant == 7 || ctx->gemm_variant == 8;
-        if (forced || (ctx->gemm_variant != 9 && !ctx->trace && (rounds >= 4 || (rounds == 3 && K <= 1024)))) {
+        // Three rounds on longer rows: the 128 x 64 tiles where they are dealt to the eight dies evenly, else these: 6424 x 704 x
+        // 12992 148 / 98, 3608 x 1344 x 14592 175 / 107, 5210 x 1088 x 3520 52 / 33, 803 x 6016 x 2624 31 / 26, 1128 x 3840 x 9216 79 /
+        // 73, 1113 x 3840 x 2752 27.0 / 26.3, 1230 x 4160 x 2816 25.9 / 27.1; evenly: 5050 x 832 x 7616 54 / 59, 1400 x 4096 x 4096 34 / 36.
+        const size_t tiles_m = (rbA + 3) / 4, tiles_n = (rbW + 1) / 2;
+        // (With a residual, which these tiles add in their checked epilogue: not measured to gain, left as it is.)
+        const bool third = rounds == 3 && (K <= 1024 || (tiles_m % 8 != 0 && tiles_n % 8 != 0 && !ep.residual));
+        if (forced || (ctx->gemm_variant != 9 && !ctx->trace && (rounds >= 4 || third))) {
             const bool tall = forced ? ctx->gemm_variant == 7
                                      : ((rbA + 7) / 8) * ((rbW + 3) / 4) < ((rbA + 3) / 4) * ((rbW + 7) / 8);
             return gemm_packed_lds(ctx, tall, pa, pw, M, N, K, ep, EPI, EVEN);
@@ -995,10 +1007,15 @@ static int32_t launch_gemm_packed(hipq_ctx *ctx, const int8_t *pa, const int8_t 
         const size_t tiles = ((packed_row_blocks(m) + 3) / 4) * ((packed_row_blocks(n) + 1) / 2);
         if (tiles > size_t(ctx->num_cus) && ctx->gemm_variant != 9) {
             if (steps % 2 == 0) return launch_packed<4, 2, 2, EPI, EVEN, false, true>(ctx, pa, pw, M, N, K, ep);
+            // (an odd number of steps: one stage in flight, as two workgroups share a compute unit: 400 x 5000 x 5504 29.9, with two
+            // and a remainder 33.1, 1000 x 3000 x 3200 22.9 / 24.7, 1500 x 1500 x 6528 39.3 / 41.0, 1200 x 2000 x 1408 15.2 / 14.8)
             return launch_packed<4, 2, 1, EPI, EVEN, false, true>(ctx, pa, pw, M, N, K, ep);
         }
     }
     if (steps % 2 == 0) return launch_packed<4, 2, 2, EPI, EVEN>(ctx, pa, pw, M, N, K, ep);
+    // (Linear from fp32, one stage / two and a remainder: 512 x 4096 x 4224 22.5 / 18.8, 600 x 2600 x 2944 19.6 / 17.2, 2000 x 1000 x
+    // 4480 27.4 / 23.8)
+    if (steps > 2) return launch_packed<4, 2, 2, EPI, EVEN, false, false, true>(ctx, pa, pw, M, N, K, ep);
     return launch_packed<4, 2, 1, EPI, EVEN>(ctx, pa, pw, M, N, K, ep);
 }
 
