@@ -951,3 +951,58 @@ def test_torsh_nn_flavour(ctx, hipq, oracle):
         np.testing.assert_array_equal(host(z), want_z)
         got = host(q).view(np.uint8).transpose(1, 0, 2).reshape(7, outer * inner).astype(np.float32)
         np.testing.assert_array_equal(got, want_carrier)
+
+
+# A row per wave and per workgroup, one workgroup and many, the last count of rows that the kernel's own status takes and the
+# first that a launch clears it for; groups along an inner axis.
+@pytest.mark.parametrize("rows,cols", [(1, 7), (4, 64), (5, 64), (1023, 20), (1025, 20), (4096, 20), (4097, 20), (3, 5000), (4096, 1100), (4097, 1100)])
+def test_status_word_of_the_row_quantizer(hipq, rows, cols):
+    """The status word holds whatever it held; the call leaves 0 or the refusal, whichever row it comes from, call after call and
+    in replays of a captured call."""
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        c = hipq.Context(0)
+        try:
+            g = torch.Generator(device="cuda").manual_seed(rows + cols)
+            good = torch.randn(rows, cols, generator=g, device="cuda")
+            x, q = good.clone(), torch.empty(rows, cols, dtype=torch.int8, device="cuda")
+            scales, status = torch.empty(rows, device="cuda"), torch.empty(1, dtype=torch.int32, device="cuda")
+
+            def call():
+                status.fill_(77)
+                c.call("hipq_quantize_per_row_f32_i8", x.data_ptr(), rows, cols, hipq.PARAMS_SYMMETRIC, 0, q.data_ptr(),
+                       scales.data_ptr(), None, status.data_ptr())
+                return status
+
+            def spoil(row):
+                x.copy_(good)
+                if row is not None:
+                    x[row, cols - 1] = float("inf")
+
+            call()
+            side.synchronize()
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph, stream=side):
+                call()
+            for row in (None, 0, None, rows - 1, rows // 2, None):
+                spoil(row)
+                want = 0 if row is None else hipq.INVALID_ARGUMENT
+                assert int(call().item()) == want, row
+                graph.replay()
+                assert int(status.item()) == want, row
+            c.synchronize()
+        finally:
+            side.synchronize()
+            c.close()
+
+
+@pytest.mark.parametrize("outer,channels,inner", [(3, 1, 5), (2, 4096, 7), (2, 4097, 7), (5, 40, 33)])
+def test_status_word_of_the_channel_quantizer(ctx, hipq, outer, channels, inner):
+    x = torch.randn(outer, channels, inner, device="cuda")
+    for channel in (None, 0, channels - 1, None):
+        y = x.clone()
+        if channel is not None:
+            y[outer - 1, channel, inner - 1] = float("-inf")
+        _, _, _, status = ctx.quantize_per_channel_auto(y, 1)
+        assert int(status.item()) == (0 if channel is None else hipq.INVALID_ARGUMENT)
+    ctx.synchronize()
