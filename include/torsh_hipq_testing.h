@@ -25,7 +25,7 @@ extern "C" {
  * the waves of few blocks, the weight-streaming kernel for 33..128 rows, on row-major operands of more than 16 rows K split
  * between the waves of few tiles - (9) and the touching of weight / filter lines by the
  * one-launch activation quantizers of the dynamic Linear and Conv2d forwards while their grids wait
- * for the range (11); on prepared operands 7 and 8 force the tiles of 256 x 128 and 128 x 256 that are
+ * for the range (11); any value keeps a Linear of small sizes as a quantizer and a product; on prepared operands 7 and 8 force the tiles of 256 x 128 and 128 x 256 that are
  * staged through LDS; 12 runs shapes of whole 128 x 128 tiles that fill the device once as one tile
  * per PAIR of compute units, K halved between the two, partial sums exchanged through their XCD's L2
  * (measured slower than the default forms; kept as a measured alternative); 14 runs a Conv2d
