@@ -935,6 +935,48 @@ def test_linear_of_small_sizes_in_one_launch(hipq, m, n, k):
         c.close()
 
 
+# One row tile and many, one column tile (nobody else reads the rows) and many; packed weights beyond the decode kernel's rows.
+@pytest.mark.parametrize("m,k", [(5, 32), (40, 64), (33, 100), (17, 1024), (700, 90)])
+def test_linear_of_small_sizes_over_its_input(hipq, m, k):
+    """out may be x, or lie over a part of it: every form has read x before it stores a result."""
+    c = hipq.Context(0)
+    try:
+        g = torch.Generator(device="cuda").manual_seed(m + k)
+        x0 = torch.randn(m * k, generator=g, device="cuda")
+        w = torch.randint(-128, 128, (k, k), generator=g, device="cuda", dtype=torch.int8)
+        sw, pw = torch.rand(k, generator=g, device="cuda") * 1e-3 + 1e-4, c.pack_rows(w)
+        calls = [lambda x, out, t=t: c.linear_dynamic(x, w, sw, per_token=t, out=out) for t in (False, True)]
+        calls += [lambda x, out, t=t: c.linear_dynamic_packed(x, pw, sw, per_token=t, out=out) for t in (False, True)]
+        calls += [lambda x, out, t=t: c.linear_dynamic_noalloc(x, w, sw, per_token=t, out=out) for t in (False, True)]
+        calls += [lambda x, out: c.linear_static(x, 0.02, w, sw, out=out), lambda x, out: c.linear_static_packed(x, 0.02, pw, sw, out=out)]
+        for i, call in enumerate(calls):
+            want = call(x0.view(m, k), torch.empty(m, k, device="cuda"))
+            for at in (0, 1, (m - 1) * k, -1, -(m - 1) * k):  # floats from x to out
+                flat = torch.empty(3 * m * k, device="cuda")
+                x, out = (flat[m * k + b:2 * m * k + b].view(m, k) for b in (0, at))
+                for _ in range(3):
+                    x.copy_(x0.view(m, k))
+                    call(x, out)
+                    assert torch.equal(out, want), (i, at)
+        c.synchronize()
+    finally:
+        torch.cuda.synchronize()
+        c.close()
+
+
+@pytest.mark.parametrize("at,small", [(0, False), (1, False), (40 * 64 - 1, False), (1 - 40 * 64, False), (40 * 64, True), (-40 * 64, True)])
+def test_linear_of_small_sizes_leaves_calls_over_their_input(stream_ctx, launched_kernels, at, small):
+    """The one launch, whose workgroups read rows while others store, up to the first float that input and output share."""
+    m, k, n = 40, 64, 64
+    flat = torch.zeros(3 * m * k, device="cuda")
+    x, out = (flat[m * k + b:2 * m * k + b].view(m, k) for b in (0, at))
+    w, sw = torch.ones(n, k, dtype=torch.int8, device="cuda"), torch.ones(n, device="cuda")
+    torch.cuda.synchronize()
+    for call in (lambda: stream_ctx.linear_dynamic(x, w, sw, out=out), lambda: stream_ctx.linear_dynamic_packed(x, w.view(-1), sw, per_token=True, out=out),
+                 lambda: stream_ctx.linear_static(x, 0.1, w, sw, out=out), lambda: stream_ctx.linear_static_packed(x, 0.1, w.view(-1), sw, out=out)):
+        assert any("linear_small_kernel" in name for name in launched_kernels(stream_ctx, call)) == small
+
+
 def test_linear_of_small_sizes_keeps_its_errors(hipq):
     c = hipq.Context(0)
     try:
