@@ -1006,3 +1006,78 @@ def test_status_word_of_the_channel_quantizer(ctx, hipq, outer, channels, inner)
         _, _, _, status = ctx.quantize_per_channel_auto(y, 1)
         assert int(status.item()) == (0 if channel is None else hipq.INVALID_ARGUMENT)
     ctx.synchronize()
+
+
+@pytest.mark.parametrize("rows,cols", [(4, 64), (4096, 20), (3000, 1100)])
+def test_status_word_of_a_quantizer_waits_for_nobody(hipq, rows, cols):
+    """A quantizer of rows or channels has no wait that could be in vain: with a limit of no polls its status is what it is."""
+    c = hipq.Context(0)
+    try:
+        c.set_wait_spin_limit(0)
+        x = torch.randn(rows, cols, device="cuda")
+        for row in (None, rows - 1, 0, None):
+            y = x.clone()
+            if row is not None:
+                y[row, 0] = float("inf")
+            want = 0 if row is None else hipq.INVALID_ARGUMENT
+            assert int(c.quantize_per_row(y)[3].item()) == want
+            assert int(c.quantize_per_channel_auto(y.view(rows, 1, cols).transpose(0, 1).contiguous(), 0)[3].item()) == want
+        for row in range(0, rows, rows // 40 + 1):  # refused rows in every workgroup's place
+            y = x.clone()
+            y[row:] = float("inf")
+            assert int(c.quantize_per_row(y)[3].item()) == hipq.INVALID_ARGUMENT
+            assert int(c.quantize_per_row(x)[3].item()) == 0
+        c.synchronize()
+    finally:
+        torch.cuda.synchronize()
+        c.close()
+
+
+@pytest.mark.parametrize("shape,axis", [((40, 64), 0), ((2, 40, 33), 1)])
+def test_status_word_of_a_captured_quantizer(stream_ctx, launched_kernels, shape, axis):
+    """A recorded quantizer keeps no state with its context, which may be at work when it is replayed: its status is cleared ahead."""
+    x = torch.randn(shape, device="cuda")
+    torch.cuda.synchronize()
+    names = launched_kernels(stream_ctx, lambda: stream_ctx.quantize_per_channel_auto(x, axis))
+    assert len(names) == 2 and "fill_i32_kernel" in names[0], names
+
+
+def test_captured_quantizers_beside_calls_of_their_context(hipq):
+    """Replays of recorded row and channel quantizers on another stream, while the context quantizes by tensor, by row and by channel."""
+    c, other = hipq.Context(0, own_stream=True), torch.cuda.Stream()
+    side = torch.cuda.ExternalStream(c.stream_handle)
+    try:
+        g = torch.Generator(device="cuda").manual_seed(3)
+        good = torch.randn(600, 500, generator=g, device="cuda")
+        bad = good.clone()
+        bad[599, 499] = float("inf")
+        torch.cuda.synchronize()
+        calls = lambda x: [c.quantize_per_row(x), c.quantize_per_channel_auto(x.view(2, 300, 500), 1)]
+        with torch.cuda.stream(side):
+            want = {id(x): calls(x) for x in (good, bad)}
+            tensor = c.quantize_dynamic_per_tensor(good)
+            graphs = []
+            for x in (good, bad):
+                graph = torch.cuda.CUDAGraph()
+                with torch.cuda.graph(graph, stream=side):
+                    out = calls(x)
+                graphs.append((graph, x, out))
+        torch.cuda.synchronize()
+        for rep in range(20):
+            with torch.cuda.stream(other):
+                for graph, _, _ in graphs:
+                    graph.replay()
+            with torch.cuda.stream(side):
+                eager = [(x, calls(x)) for x in (bad, good, good)]
+                q, params = c.quantize_dynamic_per_tensor(good)
+            torch.cuda.synchronize()
+            for x, got in eager + [(x, out) for _, x, out in graphs]:
+                for a, b in zip(got, want[id(x)]):
+                    assert int(a[3].item()) == int(b[3].item()) == (0 if x is good else hipq.INVALID_ARGUMENT), rep
+                    if x is good:
+                        assert all(torch.equal(t, u) for t, u in zip(a, b)), rep
+            assert torch.equal(q, tensor[0]) and torch.equal(params, tensor[1]), rep
+        c.synchronize()
+    finally:
+        torch.cuda.synchronize()
+        c.close()

@@ -32,10 +32,14 @@ int32_t enter(hipq_ctx *ctx) {
     return HIPQ_SUCCESS;
 }
 
+bool stream_is_capturing(const hipq_ctx *ctx) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(ctx->stream, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone;
+}
+
 int32_t scratch(hipq_ctx *ctx, size_t bytes, void **out) {
     // Kernels recorded under stream capture keep pointers into the block of that moment.
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    const bool capturing = hipStreamIsCapturing(ctx->stream, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone;
+    const bool capturing = stream_is_capturing(ctx);
     if (capturing) ctx->scratch_captured = true;
     if (bytes > ctx->scratch_bytes) {
         if (capturing)
@@ -68,8 +72,7 @@ int32_t scratch(hipq_ctx *ctx, size_t bytes, void **out) {
 }
 
 int32_t pair_area(hipq_ctx *ctx, size_t flag_bytes, size_t buf_bytes, uint32_t **flags, int8_t **buf) {
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    const bool capturing = hipStreamIsCapturing(ctx->stream, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone;
+    const bool capturing = stream_is_capturing(ctx);
     if (capturing) ctx->scratch_captured = true;
     const size_t flags_up = (flag_bytes + 255) & ~size_t(255);
     if (flags_up > ctx->pair_flag_bytes || flags_up + buf_bytes > ctx->pair_bytes) {

@@ -663,53 +663,35 @@ __global__ __launch_bounds__(kBlock) void dequantize_kernel(const InT *__restric
         out[i] = (static_cast<float>(q[i]) - zpf) * scale;
 }
 
-// The word that says whether a range was refused.  Nobody has cleared it: with `words` (up to kStatusItems rows or groups, a word each) every
-// row leaves its status in a tagged word of the context (hipq_meeting.h) and workgroup 0, when it is done with its own, waits for
-// the others' - nobody waits for it - and writes the word; without, the host has cleared the word with a launch of its own and a refused
-// range is written over that.  us, cleared by a launch / this: quantize + dequantize per channel of 1025 x 64 / 1024 x 64 floats 15.9 /
-// 12.7.
-constexpr size_t kStatusItems = 2 * kCtxSlots;
+// The word that says whether a range was refused.  Nobody has cleared it: workgroup 0 clears it, and the two words that may be written,
+// the cleared one and the refusal, are put in order by a word of the context: it rises to 2 `launch` once the status has been
+// cleared and to 2 `launch` + 1 with the first refusal.  Whoever finds the other there already writes the refusal, once; nobody waits,
+// and a launch without a refusal has one workgroup that looks.  The number comes from the host, so a launch that is recorded to be
+// replayed has no `word`: its status has been cleared by a launch of its own, and a refusal is written over that.  us, cleared by a
+// launch / this: quantize + dequantize per channel of 1025 x 64 floats 15.9 / 12.7.
 struct StatusWord {
     int32_t *out = nullptr;
-    uint32_t *words = nullptr;
-    int spin_limit = 0;
-    __device__ __forceinline__ unsigned long long *item(size_t i) const {
-        return reinterpret_cast<unsigned long long *>(words + kCtxRangeWord) + i;
+    unsigned long long *word = nullptr;
+    unsigned long long launch = 0;
+    __device__ __forceinline__ void write(int32_t st) const {
+        __hip_atomic_store(out, st, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    __device__ __forceinline__ uint32_t begin() const { return words ? meeting_number(words) : 0; }
-    __device__ __forceinline__ void report(uint32_t gen, size_t i, int st) const {  // one thread per item
-        if (words)
-            publish_tagged(item(i), gen, static_cast<uint32_t>(st));
-        else if (out && st != HIPQ_SUCCESS)
-            *out = st;
+    __device__ __forceinline__ void begin() const {  // all threads
+        if (word && blockIdx.x == 0 && threadIdx.x == 0) write(HIPQ_SUCCESS);
     }
-    __device__ __forceinline__ void finish(uint32_t gen, size_t items) const {  // all threads
-        if (!words || blockIdx.x != 0) return;
-        bool refused = false, lost = false;
-        constexpr int kLooks = 4;  // in flight together
-        for (size_t first = threadIdx.x; first < items; first += kLooks * kBlock) {
-            unsigned long long seen[kLooks];
-#pragma unroll
-            for (int u = 0; u < kLooks; ++u) {
-                const size_t i = first + u * kBlock;
-                seen[u] = __hip_atomic_load(item(i < items ? i : first), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
-#pragma unroll
-            for (int u = 0; u < kLooks; ++u) {
-                const size_t i = first + u * kBlock;
-                uint32_t st = static_cast<uint32_t>(seen[u]);
-                if (static_cast<uint32_t>(seen[u] >> 32) != gen && !poll_tagged(item(i < items ? i : first), gen, spin_limit, &st)) lost = true;
-                refused |= st != 0;
-            }
-        }
-        const bool any_refused = __syncthreads_or(refused) != 0, any_lost = __syncthreads_or(lost) != 0;
-        if (threadIdx.x == 0) {
-            meeting_mark_ready(words, gen);
-            *out = any_lost ? HIPQ_DEVICE_ERROR : any_refused ? HIPQ_INVALID_ARGUMENT : HIPQ_SUCCESS;
-        }
-        meeting_close(words, gen, any_lost);
+    __device__ __forceinline__ void report(int st) const {  // one thread per row or group
+        if (!out || st == HIPQ_SUCCESS) return;
+        if (!word || __hip_atomic_fetch_max(word, 2 * launch + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 2 * launch) write(st);
+    }
+    __device__ __forceinline__ void finish() const {  // all threads, behind begin
+        if (!word || blockIdx.x != 0 || threadIdx.x != 0) return;
+        asm volatile("" ::: "memory");
+        wait_vmcnt<0>();  // the cleared word is where the others' would go
+        asm volatile("" ::: "memory");
+        if (__hip_atomic_fetch_max(word, 2 * launch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 2 * launch + 1) write(HIPQ_INVALID_ARGUMENT);
     }
 };
+
 // Per-row (axis 0 of [rows, cols]) dynamic quantize: TPR threads own one row,
 // read it once (rows up to TPR*16 floats stay in registers), reduce min/max
 // across the row with wave shuffles, derive the row's parameters and quantize
@@ -865,11 +847,11 @@ __global__ __launch_bounds__(kBlock) void quantize_per_row_kernel(const float *_
                                                                   int flavor, int qmin, int qmax, int8_t *__restrict__ out,
                                                                   float *__restrict__ out_scales, int32_t *__restrict__ out_zps,
                                                                   StatusWord status, int poison) {
-    const uint32_t gen = status.begin();
+    status.begin();
     const int st = quantize_row<TPR, EVEN, PACKED, KC, STREAM>(x, rows, cols, ld, flavor, qmin, qmax, out, out_scales, out_zps, poison);
     const size_t row = size_t(blockIdx.x) * (kBlock / TPR) + threadIdx.x / TPR;
-    if (threadIdx.x % TPR == 0 && row < rows) status.report(gen, row, st);
-    status.finish(gen, rows);
+    if (threadIdx.x % TPR == 0 && row < rows) status.report(st);
+    status.finish();
 }
 
 // quantize_per_channel_auto for a channel axis that is not the leading one, and its group-wise
@@ -879,8 +861,8 @@ template <bool EVEN>
 __global__ __launch_bounds__(kBlock) void quantize_per_channel_auto_kernel(
     const float *__restrict__ x, size_t outer, size_t channels, size_t inner, size_t group, int flavor, int qmin,
     int qmax, int8_t *__restrict__ out, float *__restrict__ out_scales, int32_t *__restrict__ out_zps,
-    StatusWord status, size_t groups) {
-    const uint32_t gen = status.begin();
+    StatusWord status) {
+    status.begin();
     __shared__ float lds[2 * kBlock / kWave];
     const size_t g = blockIdx.x;
     const size_t c0 = g * group;
@@ -899,10 +881,10 @@ __global__ __launch_bounds__(kBlock) void quantize_per_channel_auto_kernel(
     if (threadIdx.x == 0) {
         if (out_scales) out_scales[g] = scale;
         if (out_zps) out_zps[g] = zp;
-        status.report(gen, g, st);
+        status.report(st);
     }
     if (st != HIPQ_SUCCESS) {
-        status.finish(gen, groups);
+        status.finish();
         return;
     }
     const float zpf = static_cast<float>(zp), lo = static_cast<float>(qmin), hi = static_cast<float>(qmax);
@@ -915,7 +897,7 @@ __global__ __launch_bounds__(kBlock) void quantize_per_channel_auto_kernel(
                                            ? quantize_int_cast<EVEN>(x[idx], scale, inv, zp, qmin, qmax)
                                            : to_int_nan0(quantize_value<true, EVEN>(x[idx], scale, inv, zpf, lo, hi)));
     }
-    status.finish(gen, groups);
+    status.finish();
 }
 
 // ---- the same over many workgroups: [outer, channels, inner] read as the matrix [outer, period = channels * inner],
@@ -1973,11 +1955,12 @@ int32_t hipq_dequantize_with_params_i8_f32(hipq_ctx *ctx, const int8_t *q, size_
 
 }  // extern "C"
 
-// The status word of a quantizer of `items` rows or groups (0: none will run), `elements` in all: found by its own kernel, or cleared
-// ahead of it, which nobody notices where the kernel is bound by memory: 1 x 500 x 12000 21.1 / 19.3 us, 1 x 4096 x 4000 34.0 / 34.5.
-static StatusWord status_word(hipq_ctx *ctx, int32_t *out_status, size_t items, size_t elements) {
+// The status word of a quantizer; `runs`: its kernel will be launched.  In a captured call, whose launch may run again with the same
+// arguments and beside other calls of the context, it is cleared ahead.
+static StatusWord status_word(hipq_ctx *ctx, int32_t *out_status, bool runs) {
     if (!out_status) return StatusWord{};
-    if (items != 0 && items <= kStatusItems && elements <= (size_t(1) << 23)) return StatusWord{out_status, ctx->wait_error, ctx->wait_spin_limit};
+    if (runs && !stream_is_capturing(ctx))
+        return StatusWord{out_status, reinterpret_cast<unsigned long long *>(ctx->wait_error + kCtxStatusWord), ++ctx->status_launches};
     hipLaunchKernelGGL(fill_i32_kernel, dim3(1), dim3(64), 0, ctx->stream, out_status, 0, size_t(1));
     return StatusWord{out_status, nullptr, 0};
 }
@@ -1991,7 +1974,7 @@ static int32_t quantize_rows(const char *fn, hipq_ctx *ctx, const float *x, size
     int32_t rc = any_flavor ? HIPQ_SUCCESS : check_row_flavor(fn, flavor);
     if (rc) return rc;
     if ((rc = check_mode(fn, mode))) return rc;
-    const StatusWord status = status_word(ctx, out_status, cols != 0 && ld >= cols && x && out ? rows : 0, rows * cols);
+    const StatusWord status = status_word(ctx, out_status, rows != 0 && !(rows >> 31) && cols != 0 && ld >= cols && x && out);
     if (rows == 0) return check_launch(fn);
     if (cols == 0) return fail(HIPQ_INVALID_ARGUMENT, "%s: rows of zero length have no range", fn);
     if (ld < cols) return fail(HIPQ_INVALID_ARGUMENT, "%s: row stride %zu smaller than the row length %zu", fn, ld, cols);
@@ -2096,7 +2079,8 @@ static int32_t quantize_channels(const char *fn, hipq_ctx *ctx, const float *x, 
     // with a stride where their runs are short, and works element by element.  Small tensors stay with its one launch.
     const bool spread = x && out && !(groups >> 31) && outer * period >= kSpreadMinElems && period >= 16;
     // (the spread form clears the status word in its first kernel)
-    const StatusWord status = spread ? StatusWord{} : status_word(ctx, out_status, outer != 0 && inner != 0 && x && out ? groups : 0, outer * channels * inner);
+    const StatusWord status =
+        spread ? StatusWord{} : status_word(ctx, out_status, channels != 0 && !(groups >> 31) && outer != 0 && inner != 0 && x && out);
     if (channels == 0) return check_launch(fn);
     if (outer == 0 || inner == 0) return fail(HIPQ_INVALID_ARGUMENT, "%s: channels of zero length have no range", fn);
     HIPQ_REQUIRE_PTR(x);
@@ -2185,11 +2169,11 @@ static int32_t quantize_channels(const char *fn, hipq_ctx *ctx, const float *x, 
     const int grid = static_cast<int>(groups);
     if (even)
         hipLaunchKernelGGL((quantize_per_channel_auto_kernel<true>), dim3(grid), dim3(kBlock), 0, ctx->stream, x, outer,
-                           channels, inner, group, flavor, qmin, qmax, out, out_scales, out_zero_points, status, groups);
+                           channels, inner, group, flavor, qmin, qmax, out, out_scales, out_zero_points, status);
     else
         hipLaunchKernelGGL((quantize_per_channel_auto_kernel<false>), dim3(grid), dim3(kBlock), 0, ctx->stream, x,
                            outer, channels, inner, group, flavor, qmin, qmax, out, out_scales, out_zero_points,
-                           status, groups);
+                           status);
     return check_launch(fn);
 }
 

@@ -367,13 +367,6 @@ static __device__ const v4i kZeroPiece = {0, 0, 0, 0};
 // Integer addition is associative, so the result is bit-identical for every WK.
 typedef int v16i __attribute__((ext_vector_type(16)));
 
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-    // gfx9 s_waitcnt encoding: vmcnt[3:0] | expcnt[6:4] | lgkmcnt[11:8] | vmcnt[5:4] at [15:14]
-    static_assert(N >= 0 && N < 64, "vmcnt is a 6-bit counter");
-    __builtin_amdgcn_s_waitcnt((N & 0xF) | ((N >> 4) << 14) | (0x7 << 4) | (0xF << 8));
-}
-
 __device__ __forceinline__ void wait_lgkmcnt0() {
     __builtin_amdgcn_s_waitcnt(0xF | (0x3 << 14) | (0x7 << 4) | (0x0 << 8));
 }

@@ -44,6 +44,8 @@ struct hipq_ctx {
     // Device words of the context (kCtxWordsBytes of them, laid out as the kCtx* constants below say).  Word 0 is
     // set by a kernel whose bounded wait gave up; hipq_ctx_synchronize reads and clears it.
     uint32_t *wait_error = nullptr;
+    // How many quantizers have put their status in order by the context's word; only launches that run once do.
+    unsigned long long status_launches = 0;
     // Test and tuning hooks, per context (torsh_hipq_testing.h): forced GEMM kernel form (0 = automatic) and the
     // spin limit of the kernels' bounded waits.
     int gemm_variant = 0;
@@ -73,7 +75,9 @@ constexpr size_t kCtxSlots = 2048;  // workgroups that can meet
 // launch; on a line of their own, the phase that each workgroup has finished.
 constexpr size_t kCtxTeamWord = kCtxRangeWord + kCtxSlots * 4;
 constexpr size_t kCtxTeams = 8, kCtxTeamWords = 64, kCtxTeamFlags = 32;
-constexpr size_t kCtxWordsBytes = (kCtxTeamWord + kCtxTeams * kCtxTeamWords) * 4;
+// 64 bits that order a quantizer's status word (StatusWord, hipq_elementwise.hip); on a line of their own.
+constexpr size_t kCtxStatusWord = kCtxTeamWord + kCtxTeams * kCtxTeamWords;
+constexpr size_t kCtxWordsBytes = (kCtxStatusWord + 32) * 4;
 // Number the first meeting of a context gets, a few launches before the counter wraps, so that the wrap (which
 // wipes the slots) is a path every context takes early, not once in 2^32 launches.
 constexpr uint32_t kCtxFirstEpoch = 0xfffffff0u;
@@ -96,6 +100,8 @@ void clear_error();
 
 // Makes the context's device current; returns HIPQ_SUCCESS or a recorded error.
 int32_t enter(hipq_ctx *ctx);
+// Whether calls of this context are being recorded into a graph.
+bool stream_is_capturing(const hipq_ctx *ctx);
 // Ensures ctx->scratch holds at least `bytes`; returns pointer via out.
 int32_t scratch(hipq_ctx *ctx, size_t bytes, void **out);
 // Ensures the pair-exchange area holds `flag_bytes` of zeroed flag words followed (256-byte aligned) by

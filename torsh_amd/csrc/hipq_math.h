@@ -15,6 +15,14 @@ namespace hipq {
 
 constexpr int kWave = 64;
 
+// Waits until at most N of the wave's vector memory operations are under way.
+template <int N>
+__device__ __forceinline__ void wait_vmcnt() {
+    // gfx9 s_waitcnt encoding: vmcnt[3:0] | expcnt[6:4] | lgkmcnt[11:8] | vmcnt[5:4] at [15:14]
+    static_assert(N >= 0 && N < 64, "vmcnt is a 6-bit counter");
+    __builtin_amdgcn_s_waitcnt((N & 0xF) | ((N >> 4) << 14) | (0x7 << 4) | (0xF << 8));
+}
+
 // Streaming (non-temporal) 16-byte and 4-byte accesses for data touched once.  Measured on
 // MI355X over 16 Mi elements: quantize (64 MiB read, 16 MiB written) 19.8 us with ordinary
 // accesses, 17.6 us with both streams non-temporal; dequantize (16 MiB read, 64 MiB written)
