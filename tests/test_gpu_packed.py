@@ -1036,3 +1036,28 @@ def test_gemm_three_rounds_of_tiles(hipq, m, n):
     finally:
         torch.cuda.synchronize()
         c.close()
+
+
+# Three rounds of 128 x 64 tiles on long rows.  Dealt evenly to eight dies: those tiles.  Not evenly: an odd number of row tiles, an odd
+# number of steps of K (1152), a tall matrix, and int8 results of any of them, through LDS; an even number of both, those tiles.
+@pytest.mark.parametrize("tiles_m,tiles_n,k,lds,lds_i8", [(24, 22, 1100, False, False), (23, 25, 1100, True, True), (22, 26, 1100, True, True),
+                                                          (22, 26, 1250, False, True), (34, 17, 1250, True, True), (33, 17, 1250, True, True)])
+def test_gemm_form_of_three_rounds_of_tiles(stream_ctx, launched_kernels, hipq, tiles_m, tiles_n, k, lds, lds_i8):
+    c, m, n = stream_ctx, tiles_m * 128 - 5, tiles_n * 64 - 3
+    try:
+        g = torch.Generator(device="cuda").manual_seed(m + n)
+        pa = c.pack_rows(torch.randint(-128, 128, (m, k), generator=g, device="cuda", dtype=torch.int8))
+        pw = c.pack_rows(torch.randint(-128, 128, (n, k), generator=g, device="cuda", dtype=torch.int8))
+        sa, sw = torch.ones(1, device="cuda"), torch.ones(n, device="cuda")
+        torch.cuda.synchronize()
+        for call, through_lds in ((lambda: c.gemm_packed_i8_i32(pa, pw, m, n, k), lds),
+                                  (lambda: c.linear_packed_i8_i8(pa, sa, pw, sw, None, m, n, k, 1e4, 0), lds_i8)):
+            assert any("packed_lds_kernel" in name for name in launched_kernels(c, call)) == through_lds
+            got = call()
+            c.set_gemm_kernel_variant(9)
+            want = call()
+            c.set_gemm_kernel_variant(0)
+            torch.cuda.synchronize()
+            assert torch.equal(got, want)
+    finally:
+        torch.cuda.synchronize()

@@ -972,7 +972,7 @@ static int32_t launch_gemm_packed(hipq_ctx *ctx, const int8_t *pa, const int8_t 
     }
     {
         // Tiles of 128 x 256 or 256 x 128 staged through LDS (hipq_gemm_big.hip; the shape that covers the matrix with
-        // fewer of them) once the 128 x 64 tiles make four rounds over the compute units, or three with K <= 1024.
+        // fewer of them) once the 128 x 64 tiles make four rounds over the compute units, or three with K <= 1024 or by the rule below.
         // 128 x 64 tiles / LDS in us: four rounds: 2048 x 4096 x 4096 43 / 38, 1800 x 4096 x 4096 45 / 36, 600 x 11008 x 4096
         // 49 / 33, 8192 x 1024 x 128 10.8 / 8.6, 2816 x 2304 x 768 13.4 / 11.5; three: 2000 x 3072 x 768 14.5 / 11.7,
         // 20000 x 256 x 256 9.8 / 7.7, but 1536 x 4096 x 4096 31.8 / 33.7, 768 x 8192 x 2048 18.4 / 19.1, 8192 x 768 x 3072
@@ -980,12 +980,16 @@ static int32_t launch_gemm_packed(hipq_ctx *ctx, const int8_t *pa, const int8_t 
         const size_t rbA = packed_row_blocks(m), rbW = packed_row_blocks(n), cus = size_t(ctx->num_cus);
         const size_t rounds = (((rbA + 3) / 4) * ((rbW + 1) / 2) + cus - 1) / cus;
         const bool forced = ctx->gemm_variant == 7 || ctx->gemm_variant == 8;
-        // Three rounds on longer rows: the 128 x 64 tiles where they are dealt to the eight dies evenly, else these: 6424 x 704 x
-        // 12992 148 / 98, 3608 x 1344 x 14592 175 / 107, 5210 x 1088 x 3520 52 / 33, 803 x 6016 x 2624 31 / 26, 1128 x 3840 x 9216 79 /
-        // 73, 1113 x 3840 x 2752 27.0 / 26.3, 1230 x 4160 x 2816 25.9 / 27.1; evenly: 5050 x 832 x 7616 54 / 59, 1400 x 4096 x 4096 34 / 36.
         const size_t tiles_m = (rbA + 3) / 4, tiles_n = (rbW + 1) / 2;
+        // Three rounds on longer rows: the 128 x 64 tiles where they are dealt to the eight dies evenly (5050 x 832 x 7616 54 / 59,
+        // 1400 x 4096 x 4096 34 / 36) or, with two workgroups a compute unit, an even number of row tiles meets an even number of
+        // steps (two stages in flight) and the matrix is not tall: medians over 77, 71 and 42 shapes 1.04 (1232 x 3456 x 8448 62 / 66,
+        // 1789 x 2688 x 2752 25.5 / 29.6), with odd steps 0.95, with odd row tiles 0.8 (6424 x 704 x 12992 148 / 98, 5210 x 1088 x 3520
+        // 52 / 33, 803 x 6016 x 2624 31 / 26, 1128 x 3840 x 9216 79 / 73); tall ones of the first kind 0.59 to 0.90 (7903 x 736 x 8704 117 /
+        // 69, 4785 x 1216 x 3776 40 / 35, but 12782 x 384 x 2048 21.5 / 22.9).
+        const bool even = EPI != EPI_I8 && tiles_m % 2 == 0 && steps % 2 == 0 && tiles_m < 2 * tiles_n;
         // (With a residual, which these tiles add in their checked epilogue: not measured to gain, left as it is.)
-        const bool third = rounds == 3 && (K <= 1024 || (tiles_m % 8 != 0 && tiles_n % 8 != 0 && !ep.residual));
+        const bool third = rounds == 3 && (K <= 1024 || (tiles_m % 8 != 0 && tiles_n % 8 != 0 && !even && !ep.residual));
         if (forced || (ctx->gemm_variant != 9 && !ctx->trace && (rounds >= 4 || third))) {
             const bool tall = forced ? ctx->gemm_variant == 7
                                      : ((rbA + 7) / 8) * ((rbW + 3) / 4) < ((rbA + 3) / 4) * ((rbW + 7) / 8);
