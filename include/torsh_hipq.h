@@ -670,9 +670,11 @@ HIPQ_API int32_t hipq_transformer_stack_forward_f32(hipq_ctx *ctx, const hipq_bl
  * (hipq_linear_residual_layer_norm_quantize_packed_i8, hipq_linear_gelu_quantize_packed_i8), the out-projection
  * quantizes the fp32 value slice itself (hipq_linear_from_f32_residual_layer_norm_quantize_packed_i8), and int8
  * activations stay packed between them.  Up to there the products are split over their columns and the row operations
- * are kernels of their own (eight kernels per layer), with the same bits.  x is what hipq_transformer_stack_forward_f32
+ * are kernels of their own (eight kernels per layer), and up to 128 tokens on rows of up to 768 floats all layers are one
+ * launch, whose workgroups meet by device words of the context or, in a call that is being captured, by 2 KB at the end of
+ * the workspace (without them: the kernels of their own); with the same bits.  x is what hipq_transformer_stack_forward_f32
  * computes up to the fold order of the LayerNorm sums (see those entry points).  d_model and d_ff: multiples of 128, at
- * most 3072 (else HIPQ_SHAPE_ERROR: use the form above).  The forward uses no memory but the workspace (and, where panels
+ * most 3072 (else HIPQ_SHAPE_ERROR: use the form above).  The forward takes no memory but the workspace (and, where panels
  * of rows are shared by two workgroups, their exchange area).  A workspace that holds the packed activations, the scales
  * and the qkv product but not, for up to 5120 tokens and d_ff > 3 d_model, fc1's fp32 output in its place is taken too:
  * the four kernels per layer then run at any number of tokens. */

@@ -694,6 +694,57 @@ def test_prepared_stack_by_teams(hipq, tokens, d, dff, layers):
         c.close()
 
 
+def test_captured_stack_of_few_tokens_meets_by_its_workspace(stream_ctx, launched_kernels, hipq):
+    """A recorded stack may be replayed while its context is at work: its teams meet by words of the workspace, cleared by the call.  A
+    workspace from before it had them runs the separate kernels.  Eager calls meet by the context's and clear nothing."""
+    tokens, d, dff = 19, 256, 512
+    g = torch.Generator(device="cuda").manual_seed(4)
+    prepared = stream_ctx.stack_prepare(_random_blocks(stream_ctx, g, d, dff, 2))
+    x, ws = torch.randn(tokens, d, generator=g, device="cuda"), stream_ctx.stack_workspace_prepared(tokens, d, dff)
+    torch.cuda.synchronize()
+    for w, teams in ((ws, True), (ws[:-1], False), (ws[:-2048], False)):
+        names = launched_kernels(stream_ctx, lambda: stream_ctx.stack_forward(prepared, x, dff, w, prepared=True))
+        assert sum("team_words_clear_kernel" in n for n in names) == sum("stack_team_kernel" in n for n in names) == teams, names
+
+
+def test_captured_stacks_beside_calls_of_their_context(hipq):
+    """Replays on another stream, from two workspaces and two inputs, beside eager stacks of the same context: the bits of a call alone."""
+    d, dff, layers = 256, 1024, 3
+    c, other = hipq.Context(0, own_stream=True), torch.cuda.Stream()
+    side = torch.cuda.ExternalStream(c.stream_handle)
+    try:
+        g = torch.Generator(device="cuda").manual_seed(8)
+        with torch.cuda.stream(side):
+            prepared = c.stack_prepare(_random_blocks(c, g, d, dff, layers))
+            x0 = [torch.randn(n, d, generator=g, device="cuda") for n in (40, 8, 77)]
+            ws = [c.stack_workspace_prepared(x.shape[0], d, dff) for x in x0]
+            for w in ws:
+                w.fill_(171)  # (whatever the workspace held)
+            run = lambda i, x: c.stack_forward(prepared, x, dff, ws[i], prepared=True)
+            want = [run(i, x.clone()) for i, x in enumerate(x0)]
+            xs = [torch.empty_like(x) for x in x0]
+            graphs = [torch.cuda.CUDAGraph() for _ in range(2)]
+            for i, graph in enumerate(graphs):
+                with torch.cuda.graph(graph, stream=side):
+                    run(i, xs[i])
+        torch.cuda.synchronize()
+        for rep in range(12):
+            for i in range(2):
+                xs[i].copy_(x0[i])
+            torch.cuda.synchronize()
+            with torch.cuda.stream(other):
+                for graph in graphs:
+                    graph.replay()
+            with torch.cuda.stream(side):
+                eager = [run(2, x0[2].clone()) for _ in range(3)]
+            torch.cuda.synchronize()
+            assert all(torch.equal(xs[i], want[i]) for i in range(2)) and all(torch.equal(y, want[2]) for y in eager), rep
+        c.synchronize()
+    finally:
+        torch.cuda.synchronize()
+        c.close()
+
+
 def test_prepared_stacks_of_two_streams_at_once(hipq):
     """Two contexts on streams of their own, each with stacks of few tokens queued, and nobody has said that they share the
     device: teams that cannot assemble leave their rows to one workgroup each, so every call gives the bits of a call alone."""

@@ -161,13 +161,16 @@ struct RowOpLinear {
 };
 // The layers of the prepared stack on few tokens in one launch (hipq_stack_team.hip), behind the first layer's qkv product
 // (q, k, v rows of 3 d floats in `qkv`).  maxima: room for tokens rounded up to a multiple of 8, times d_ff / 16 floats; codes:
-// as many rows of d_ff bytes.
+// as many rows of d_ff bytes; words: kTeamWordsBytes for the teams to meet by, cleared by the call, or null for the context's, which only
+// launches that run once on its stream may use.
+constexpr size_t kTeamTokens = 128, kTeamWordsBytes = kCtxTeams * kCtxTeamWords * 4;
 struct TeamStackCall {
     const hipq_block_weights *blocks;
     size_t layers, tokens, d, d_ff;
     float eps;
     float *x, *qkv, *maxima;
     int8_t *codes;
+    uint32_t *words;
 };
 bool team_stack_fits(const hipq_ctx *ctx, const float *x, size_t tokens, size_t d, size_t d_ff, PanelFold after_out,
                      PanelFold after_fc2);

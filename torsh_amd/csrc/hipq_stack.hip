@@ -18,6 +18,7 @@ struct StackBuffers {
     float *sa, *sb;   // their per-token scales
     float *qkv;
     float *hidden;  // fc1 output of the tiled form; lies where qkv does, which is used up by then
+    uint32_t *words;  // kTeamWordsBytes for the teams of a captured call, or null where the workspace has none
 };
 
 // Whether the value slice's quantizer runs inside the out-projection (row panels: a workgroup holds its rows' codes).
@@ -52,7 +53,9 @@ int32_t stack_tiled(hipq_ctx *ctx, const hipq_block_weights *blocks, size_t n_la
         return rc ? rc : linear_packed_rows_f32(ctx, b.qb, b.sb, w.w_out, w.s_out, w.b_out, x, tokens, d_model, d_model, x);
     };
     int32_t rc = HIPQ_SUCCESS;
-    const bool teams = team_stack_fits(ctx, x, tokens, d_model, d_ff, after_out, after_fc2);
+    // A captured call may be replayed beside other calls of its context, so its teams do not meet by the context's words.
+    const bool captured = stream_is_capturing(ctx);
+    const bool teams = team_stack_fits(ctx, x, tokens, d_model, d_ff, after_out, after_fc2) && (!captured || b.words);
     for (size_t l = 0; l < n_layers && rc == HIPQ_SUCCESS; ++l) {
         const hipq_block_weights &w = blocks[l];
         if (l == 0) {  // (the one LayerNorm that folds as the row kernels do)
@@ -62,7 +65,7 @@ int32_t stack_tiled(hipq_ctx *ctx, const hipq_block_weights *blocks, size_t n_la
                 return rc;
             if (teams)
                 return team_stack(ctx, TeamStackCall{blocks, n_layers, tokens, d_model, d_ff, eps, x, b.qkv,
-                                                     reinterpret_cast<float *>(b.qa), b.qb}, mode);
+                                                     reinterpret_cast<float *>(b.qa), b.qb, captured ? b.words : nullptr}, mode);
         } else if ((rc = norm_linear(w.ln1_gamma, w.ln1_beta, after_fc2, w.w_qkv, w.s_qkv, w.b_qkv, 3 * d_model, b.qkv))) {
             return rc;
         }
@@ -155,15 +158,19 @@ int32_t hipq_transformer_stack_forward_f32(hipq_ctx *ctx, const hipq_block_weigh
 // layer's LayerNorm 1 + quantize.  Activations travel between them as packed int8; the only fp32 tensors that
 // touch memory are the stream x and the qkv output (which the attention outside this path would read).
 
+// Bytes of the qkv product; few tokens: or of fc1's output, when that is the wider.
+static size_t product_bytes(size_t tokens, size_t d_model, size_t d_ff) {
+    const size_t row = tokens <= kTiledTokens && d_ff > 3 * d_model ? d_ff : 3 * d_model;
+    return align256(tokens * row * sizeof(float));
+}
+
 size_t hipq_transformer_stack_prepared_workspace_bytes(size_t tokens, size_t d_model, size_t d_ff) {
     const size_t widest = d_model > d_ff ? d_model : d_ff;
     size_t a = 0, b = 0;
     if (hipq_packed_size(tokens, d_model, &a) || hipq_packed_size(tokens, widest, &b)) return 0;
-    // qkv; few tokens: or fc1's output, when that is the wider
-    const size_t row = tokens <= kTiledTokens && d_ff > 3 * d_model ? d_ff : 3 * d_model;
     return align256(a) + align256(b)                // packed int8 activations (two in flight)
            + 2 * align256(tokens * sizeof(float))   // their per-token scales
-           + align256(tokens * row * sizeof(float));
+           + product_bytes(tokens, d_model, d_ff) + (tokens <= hipq::kTeamTokens ? hipq::kTeamWordsBytes : 0);
 }
 
 int32_t hipq_transformer_stack_forward_prepared_f32(hipq_ctx *ctx, const hipq_block_weights *blocks, size_t n_layers,
@@ -215,9 +222,12 @@ int32_t hipq_transformer_stack_forward_prepared_f32(hipq_ctx *ctx, const hipq_bl
     // so the panels are taken when they fill five eighths of the device, and where a workspace sized for them alone has no
     // room for fc1's output.  Both give the same bits.  (Test hook 15: panels always.)
     const bool room = workspace_bytes - ahead >= tokens * d_ff * sizeof(float);
+    const size_t words_at = product_bytes(tokens, d_model, d_ff);
     if (room && tokens <= kTiledTokens && tokens <= size_t(ctx->num_cus) * 20 && ctx->gemm_variant != 15)
         return stack_tiled(ctx, blocks, n_layers, tokens, d_model, d_ff, eps, round_bits, x,
-                           StackBuffers{qa, qb, sa, sb, qkv, qkv});
+                           StackBuffers{qa, qb, sa, sb, qkv, qkv,
+                                        workspace_bytes - ahead >= words_at + hipq::kTeamWordsBytes
+                                            ? reinterpret_cast<uint32_t *>(p + words_at) : nullptr});
     // quant(LN1(x)) of the first layer: the row kernel, then the packing pass (row-major codes parked in qb)
     rc = hipq_layer_norm_quantize_f32_i8(ctx, x, tokens, d_model, blocks[0].ln1_gamma, blocks[0].ln1_beta, eps,
                                          round_bits, qb, sa);

@@ -30,6 +30,7 @@ constexpr int kTeamWaves = 16;    // waves of a workgroup: the first multiply, t
 constexpr int kTeamProducts = 6;  // waves that multiply
 constexpr int kTeamRowWaves = kTeamWaves - kTeamProducts;
 constexpr int kTeamRows = 16;     // rows of a team at most
+static_assert(kTeamTokens == size_t(kTeams) * kTeamRows, "tokens of all teams");
 constexpr int kTeamLayers = 24;   // layers of one launch (their pointers are kernel arguments)
 constexpr int kTeamFloats = 3;    // float4 a lane per row: d_model <= 768
 constexpr int kTeamColumns = 3;   // column blocks of 32 a workgroup: N <= 3072
@@ -628,6 +629,8 @@ __global__ __launch_bounds__(1024) void stack_alone_kernel(StackTeam p) {
     }
 }
 
+__global__ void team_words_clear_kernel(uint32_t *words) { words[blockIdx.x * blockDim.x + threadIdx.x] = 0; }
+
 }  // namespace
 
 // Up to 128 tokens of rows of up to 768 floats (16 rows a team, three float4 a lane).  Separate kernels / this, us: 12 layers of d 768,
@@ -639,7 +642,7 @@ bool team_stack_fits(const hipq_ctx *ctx, const float *x, size_t tokens, size_t 
     const int share = ctx->resident_share > 0 ? ctx->resident_share : 1;
     auto folds = [](PanelFold f) { return !f.pair && f.wave_blocks == kTeamFloats; };
     return ctx->pair_ok && share == 1 && ctx->num_cus >= kTeams * kTeamSize && folds(after_out) && folds(after_fc2) &&
-           tokens <= size_t(kTeams) * kTeamRows && d % 128 == 0 && d <= size_t(kTeamFloats) * 256 && d_ff % 128 == 0 &&
+           tokens <= kTeamTokens && d % 128 == 0 && d <= size_t(kTeamFloats) * 256 && d_ff % 128 == 0 &&
            d_ff <= size_t(kTeamColumns) * kTeamSize * 32 && d_ff <= 4 * d && (reinterpret_cast<uintptr_t>(x) & 15u) == 0;
 }
 
@@ -649,7 +652,8 @@ int32_t team_stack(hipq_ctx *ctx, const TeamStackCall &call, int32_t mode) {
     p.qkv = call.qkv;
     p.maxima = call.maxima;
     p.codes = call.codes;
-    p.words = ctx->wait_error + kCtxTeamWord;
+    p.words = call.words ? call.words : ctx->wait_error + kCtxTeamWord;
+    if (call.words) hipLaunchKernelGGL(team_words_clear_kernel, dim3(kTeams), dim3(kCtxTeamWords), 0, ctx->stream, call.words);
     p.wait_error = ctx->wait_error;
     p.tokens = static_cast<int>(call.tokens);
     p.rows = static_cast<int>((call.tokens + kTeams - 1) / kTeams);
