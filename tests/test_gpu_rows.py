@@ -707,6 +707,35 @@ def test_captured_stack_of_few_tokens_meets_by_its_workspace(stream_ctx, launche
         assert sum("team_words_clear_kernel" in n for n in names) == sum("stack_team_kernel" in n for n in names) == teams, names
 
 
+@pytest.mark.parametrize("tokens,layers", [(19, 2), (128, 25)])
+def test_every_launch_leaves_its_number_in_the_flags_of_its_teams(hipq, tokens, layers):
+    """Flags are compared by their distance in launches, so a launch whose teams do not assemble renews them too.  Seen in the words of
+    a captured call: per team 64 of 32 bits, the flags from the 32nd on."""
+    d, dff = 128, 128
+    c = hipq.Context(0, own_stream=True)
+    side = torch.cuda.ExternalStream(c.stream_handle)
+    try:
+        g = torch.Generator(device="cuda").manual_seed(2)
+        with torch.cuda.stream(side):
+            prepared = c.stack_prepare(_random_blocks(c, g, d, dff, layers))
+            x, ws = torch.randn(tokens, d, generator=g, device="cuda"), c.stack_workspace_prepared(tokens, d, dff)
+            for limit, least in ((-1, 1), (0, 0)):  # meetings of the last launch, at least
+                c.set_wait_spin_limit(limit)
+                graph = torch.cuda.CUDAGraph()
+                with torch.cuda.graph(graph, stream=side):
+                    c.stack_forward(prepared, x, dff, ws, prepared=True)
+                graph.replay()
+                graph.replay()
+                side.synchronize()
+                teams = -(-tokens // -(-tokens // 8))
+                flags = ws[-2048:].view(torch.int32).view(8, 64)[:teams, 32:].cpu()
+                assert (flags // 4096 == (layers - 1) // 24).all(), limit  # launch 0, or 1 where there are two
+                assert (flags % 4096 // 16 >= least).all(), limit
+    finally:
+        torch.cuda.synchronize()
+        c.close()
+
+
 def test_captured_stacks_beside_calls_of_their_context(hipq):
     """Replays on another stream, from two workspaces and two inputs, beside eager stacks of the same context: the bits of a call alone."""
     d, dff, layers = 256, 1024, 3

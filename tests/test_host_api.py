@@ -125,6 +125,14 @@ def test_rules_of_the_per_channel_quantizer_that_reads_once():
     assert proc.returncode == 0, proc.stdout + proc.stderr
 
 
+def test_numbers_by_which_the_teams_of_the_stack_meet():
+    """Flags of a team over its meetings, launches and their wrap, on the CPU."""
+    subprocess.run(["make", "-C", os.path.join(ROOT, "tests", "host"), "bin/team_words_check"], check=True, capture_output=True)
+    proc = subprocess.run([os.path.join(ROOT, "tests", "host", "bin", "team_words_check")], capture_output=True, text=True,
+                          timeout=60)
+    assert proc.returncode == 0, proc.stdout + proc.stderr
+
+
 def test_every_kernel_that_must_be_resident_at_once_is_asked_about():
     """The kernels of the quantizers that are built for four workgroups per compute unit, because their workgroups wait for each
     other, are the ones whose occupancy decides whether they are taken."""

@@ -20,6 +20,7 @@
 #include "hipq_internal.h"
 #include "hipq_panel_norm.h"
 #include "hipq_quantize_rows.h"
+#include "hipq_team_words.h"
 
 namespace hipq {
 namespace {
@@ -36,8 +37,7 @@ constexpr int kTeamFloats = 3;    // float4 a lane per row: d_model <= 768
 constexpr int kTeamColumns = 3;   // column blocks of 32 a workgroup: N <= 3072
 constexpr int kTeamSteps = 8;     // pairs of k blocks a wave: K <= 3072
 constexpr int kTeamRowSteps = 2;  // the same where K is d_model
-constexpr uint32_t kTeamPhases = 256;  // numbers a launch may use: five meetings a layer
-static_assert(kTeamLayers * 5 < int(kTeamPhases), "phase numbers");
+static_assert(kTeamLayers * 5 < int(kTeamPhases), "five meetings a layer");
 constexpr int kPastL1 = /*sc1*/ 16;
 
 // Looks at the verdict before a workgroup stops waiting for its team, some 0.4 us each: a team that other work keeps from
@@ -248,7 +248,7 @@ __global__ __launch_bounds__(1024) void stack_team_kernel(StackTeam p) {
         uint32_t launch = 0;
         const bool go = lane == 0 && team_assembles(words, p.assembly_limit, &launch);
         if (lane == 0) together = go;
-        phase = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(launch))) * (kTeamPhases * 16);
+        phase = team_flag(static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(launch))), 0);
     }
     bool lost = false;  // (of the wave that polls)
     auto acknowledged = [] {  // this wave's stores have reached the L2
@@ -257,7 +257,7 @@ __global__ __launch_bounds__(1024) void stack_team_kernel(StackTeam p) {
         asm volatile("" ::: "memory");
     };
     auto meet = [&] {
-        phase += 16;
+        phase += team_flag(0, 1);
         __syncthreads();
         if (wave == kTeamWaves - 1 && !lost) {
             if (lane == 0) __builtin_amdgcn_raw_buffer_store_b32(static_cast<int>(phase | xcc), rflags, me * 4, 0, 0);
@@ -266,7 +266,7 @@ __global__ __launch_bounds__(1024) void stack_team_kernel(StackTeam p) {
             for (int spin = 0; spin <= p.spin_limit && !all; ++spin) {
                 asm volatile("" ::: "memory");
                 seen = static_cast<uint32_t>(__builtin_amdgcn_raw_buffer_load_b32(rflags, lane % kTeamSize * 4, 0, kPastL1));
-                all = __all(static_cast<int32_t>(seen - phase) >= 0);
+                all = __all(team_flag_reached(seen, phase));
             }
             lost = !all || !__all((seen & 15u) == xcc);
         }
@@ -521,7 +521,10 @@ __global__ __launch_bounds__(1024) void stack_alone_kernel(StackTeam p) {
     __shared__ uint32_t row_max[kTeamRows];
     const int team = static_cast<int>(blockIdx.x), T = p.rows, row0 = team * T;
     if (row0 >= p.tokens) return;
-    if ((p.words[team * kCtxTeamWords + kTeamVerdict] & 3u) != kTeamAlone) return;
+    uint32_t *words = p.words + team * kCtxTeamWords;
+    const uint32_t verdict = words[kTeamVerdict];
+    if ((verdict & 3u) != kTeamAlone) return;
+    if (threadIdx.x < kTeamSize) words[kCtxTeamFlags + threadIdx.x] = team_flag(verdict >> 2, 0);  // (the team has left them as they were)
     const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int R = T < p.tokens - row0 ? T : p.tokens - row0;
     const int d = p.d, dblocks = d / 32, fblocks = p.d_ff / 32, mine = 4 * (lane / 16);
