@@ -977,6 +977,31 @@ def test_linear_of_small_sizes_leaves_calls_over_their_input(stream_ctx, launche
         assert any("linear_small_kernel" in name for name in launched_kernels(stream_ctx, call)) == small
 
 
+# The last sizes of each form and the first past them; 256 compute units.
+@pytest.mark.parametrize("form,m,n,k,small", [
+    ("tensor", 64, 32, 1024, True), ("tensor", 65, 32, 1024, False), ("tensor", 32, 64, 2048, True), ("tensor", 31, 64, 2049, False),
+    ("tensor", 9, 8192, 64, True), ("tensor", 9, 8193, 64, False), ("tensor", 9, 40, 16, True), ("tensor", 9, 40, 15, False),
+    ("token", 64, 32, 1024, True), ("token", 64, 32, 1025, False), ("token", 4096, 32, 64, True), ("token", 4097, 32, 64, False),
+    ("static", 64, 32, 1024, True), ("static", 64, 32, 1025, False), ("static", 8192, 32, 64, True), ("static", 8193, 32, 64, False),
+    ("tensor packed", 64, 32, 1024, True), ("tensor packed", 32, 64, 2048, True), ("tensor packed", 9, 40, 15, True),
+    ("token packed", 64, 32, 1024, True), ("token packed", 64, 32, 1025, False),
+    ("static packed", 64, 32, 2048, True), ("static packed", 64, 32, 2049, False), ("static packed", 4096, 32, 1025, True),
+    ("static packed", 4097, 32, 1025, False)])
+def test_linears_that_run_in_one_launch(stream_ctx, launched_kernels, form, m, n, k, small):
+    c = stream_ctx
+    x, sw = torch.zeros(m, k, device="cuda"), torch.ones(n, device="cuda")
+    w = torch.ones(n, k, dtype=torch.int8, device="cuda")
+    if "packed" in form:
+        w = c.pack_rows(w)
+    torch.cuda.synchronize()
+    call = {"tensor": lambda: c.linear_dynamic(x, w, sw), "token": lambda: c.linear_dynamic(x, w, sw, per_token=True),
+            "static": lambda: c.linear_static(x, 0.1, w, sw), "tensor packed": lambda: c.linear_dynamic_packed(x, w, sw),
+            "token packed": lambda: c.linear_dynamic_packed(x, w, sw, per_token=True),
+            "static packed": lambda: c.linear_static_packed(x, 0.1, w, sw)}[form]
+    names = launched_kernels(c, call)
+    assert ["linear_small_kernel" in name for name in names] == ([True] if small else [False] * len(names)), names
+
+
 def test_linear_of_small_sizes_keeps_its_errors(hipq):
     c = hipq.Context(0)
     try:

@@ -664,8 +664,8 @@ def test_prepared_stack_first_call_in_a_graph(hipq):
                                                  (5, 128, 256, 24), (21, 128, 384, 25), (66, 256, 128, 26)])
 def test_prepared_stack_by_teams(hipq, tokens, d, dff, layers):
     """Up to 128 tokens, rows of up to 768 floats: the workgroups of an XCD take an eighth of the rows through all layers.  The
-    bits of the row panels (hook 15), also where no team assembles (a spin limit of 0: one workgroup a team instead) and where
-    the context has a share of the device only; a row that is not finite stays alone."""
+    bits of the row panels (hook 15), also where no team assembles (a spin limit of 0: the first workgroups to come instead) and
+    where the context has a share of the device only; a row that is not finite stays alone."""
     c = hipq.Context(0)
     try:
         g = torch.Generator(device="cuda").manual_seed(tokens + d + layers)
@@ -692,6 +692,58 @@ def test_prepared_stack_by_teams(hipq, tokens, d, dff, layers):
     finally:
         torch.cuda.synchronize()
         c.close()
+
+
+# GELU's results in the rows of qkv and beside them, by workgroups with one column half a wave and with many; every row count of a
+# last team; the layers of one launch and more; vectors that are not there.
+@pytest.mark.parametrize("tokens,d,dff,layers,absent", [(77, 768, 3072, 2, ()), (1, 768, 2304, 2, ("b_",)), (16, 128, 512, 2, ("_gamma",)),
+                                                        (128, 640, 2048, 1, ("_beta",)), (30, 256, 896, 3, ("b_", "_gamma", "_beta")),
+                                                        (11, 128, 128, 26, ())])
+def test_prepared_stack_by_the_workgroups_that_are_there(hipq, tokens, d, dff, layers, absent):
+    """Teams that do not assemble (limits of 0 and 1 looks): the first workgroups to come, and all that come within a few
+    microseconds, take the rows.  The bits of the row panels, with and without biases, gains and offsets, as for whole teams."""
+    c = hipq.Context(0)
+    try:
+        g = torch.Generator(device="cuda").manual_seed(tokens + d + layers)
+        blocks = [{k: None if any(a in k for a in absent) else v for k, v in blk.items()} for blk in _random_blocks(c, g, d, dff, layers)]
+        prepared = c.stack_prepare(blocks)
+        x0 = torch.randn(tokens, d, generator=g, device="cuda")
+        x0[tokens // 2, d // 3] = float("inf")
+        ws = c.stack_workspace_prepared(tokens, d, dff)
+        for mode in (0, hipq.ROUND_HALF_EVEN):
+            run = lambda: c.stack_forward(prepared, x0.clone(), dff, ws, mode=mode, prepared=True)
+            c.set_gemm_kernel_variant(15)
+            want = torch.nan_to_num(run(), nan=-77.0)
+            c.set_gemm_kernel_variant(0)
+            for limit in (-1, 0, 1, 0, 1, -1):
+                c.set_wait_spin_limit(limit)
+                assert torch.equal(torch.nan_to_num(run(), nan=-77.0), want), (mode, limit)
+        c.synchronize()  # nothing gave up
+    finally:
+        torch.cuda.synchronize()
+        c.close()
+
+
+@pytest.mark.parametrize("tokens,d,dff,teams", [(1, 128, 128, True), (128, 768, 3072, True), (129, 768, 3072, False), (128, 896, 1024, False),
+                                                (20, 128, 640, False), (20, 768, 128, True)])
+def test_prepared_stacks_that_run_by_teams(stream_ctx, launched_kernels, hipq, tokens, d, dff, teams):
+    """The sizes whose layers are one launch and the first past them; not on a share of the device, nor where panels are forced."""
+    g = torch.Generator(device="cuda").manual_seed(1)
+    prepared = stream_ctx.stack_prepare(_random_blocks(stream_ctx, g, d, dff, 2))
+    x, ws = torch.zeros(tokens, d, device="cuda"), stream_ctx.stack_workspace_prepared(tokens, d, dff)
+    torch.cuda.synchronize()
+    by_teams = lambda: ["stack_team_kernel" in n for n in launched_kernels(
+        stream_ctx, lambda: stream_ctx.stack_forward(prepared, x, dff, ws, prepared=True))].count(True)
+    try:
+        assert by_teams() == teams
+        stream_ctx.set_resident_share(2)
+        assert by_teams() == 0
+        stream_ctx.set_resident_share(1)
+        stream_ctx.set_gemm_kernel_variant(15)
+        assert by_teams() == 0
+    finally:
+        stream_ctx.set_resident_share(1)
+        stream_ctx.set_gemm_kernel_variant(0)
 
 
 def test_captured_stack_of_few_tokens_meets_by_its_workspace(stream_ctx, launched_kernels, hipq):
@@ -776,7 +828,7 @@ def test_captured_stacks_beside_calls_of_their_context(hipq):
 
 def test_prepared_stacks_of_two_streams_at_once(hipq):
     """Two contexts on streams of their own, each with stacks of few tokens queued, and nobody has said that they share the
-    device: teams that cannot assemble leave their rows to one workgroup each, so every call gives the bits of a call alone."""
+    device: teams that cannot assemble leave their rows to those that are there, so every call gives the bits of a call alone."""
     d, dff, layers = 256, 1024, 4
     contexts = [hipq.Context(0, own_stream=True) for _ in range(2)]
     maker = hipq.Context(0)

@@ -15,7 +15,7 @@
 // A team needs all its workgroups on the device at once, which other work may prevent (another stream's team is enough).
 // So it first counts itself: either the last workgroup to arrive finds that nobody has stopped waiting, and all 32 go on and
 // wait for nothing but each other from there on; or somebody stops waiting first, all of them leave without having touched
-// anything, and the kernel behind this one takes the team's rows through the layers with one workgroup that waits for nobody.
+// anything, and the kernel behind this one takes the team's rows through the layers with those of its workgroups that are there.
 #include "hipq_gemm_kernels.h"
 #include "hipq_internal.h"
 #include "hipq_panel_norm.h"
@@ -40,16 +40,19 @@ constexpr int kTeamRowSteps = 2;  // the same where K is d_model
 static_assert(kTeamLayers * 5 < int(kTeamPhases), "five meetings a layer");
 constexpr int kPastL1 = /*sc1*/ 16;
 
-// Looks at the verdict before a workgroup stops waiting for its team, some 0.4 us each: a team that other work keeps from
-// assembling for longer than a millisecond or two is better off with the one workgroup.
-constexpr int kAssemblyLimit = 4096;
+// Looks at the verdict before a workgroup stops waiting for its team, some 0.1 us each.  Beside ordinary kernels, whose workgroups make
+// room one after the other, a team assembles within that and then has its compute units: 77 tokens, d 768, us by 64 / 512 / 4096 looks
+// beside bf16 products of 4096^3 603 / 604 / 603 (separate kernels 5400: each waits again), an addition over 512 MB 922 / 448 / 447
+// (1170), Linears of 4096 x 11008 x 4096 602 / 401 / 401 (2450).  Where a workgroup that holds 128 KB of LDS for milliseconds sits on
+// every XCD, waiting is in vain: 1 / 256 / 1024 / 4096 looks 460 / 490 / 572 / 900 (separate kernels 345 to 365).
+constexpr int kAssemblyLimit = 512;
 
 struct StackTeam {
     hipq_block_weights blocks[kTeamLayers];
     float *x, *qkv, *maxima;
     int8_t *codes;
     uint32_t *words, *wait_error;
-    int layers, qkv_done, tokens, rows, d, d_ff, spin_limit, assembly_limit;
+    int layers, qkv_done, tokens, rows, d, d_ff, spin_limit, assembly_limit, gather_looks;
     float eps;
 };
 static_assert(sizeof(StackTeam) <= 4096, "kernel arguments");
@@ -58,15 +61,16 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t team_buffer(const void *base, 
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, bytes, 0x00020000);
 }
 
-// Words of a team: how many workgroups have ever arrived (32 a launch) and what was decided about the last launch: its number
-// and whether the team goes on.
-constexpr int kTeamArrivals = 0, kTeamVerdict = 1, kTeamGo = 1, kTeamAlone = 2;
+// Words of a team: how many workgroups have ever arrived (32 a launch), what was decided about the last launch - its number and
+// whether the team goes on - and, where it does not, who has come to the kernel behind this one.
+constexpr int kTeamArrivals = 0, kTeamVerdict = 1, kTeamGather = 2, kTeamGo = 1, kTeamApart = 2;
 
 // One lane of a workgroup: arrives and waits for the verdict on this launch, whose number is left in `launch`.
 __device__ __forceinline__ bool team_assembles(uint32_t *words, int spin_limit, uint32_t *launch) {
     const uint32_t before = __hip_atomic_fetch_add(words + kTeamArrivals, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const uint32_t n = before / kTeamSize;
     *launch = n;
+    if (before % kTeamSize == 0) __hip_atomic_store(words + kTeamGather, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     uint32_t *verdict = words + kTeamVerdict, seen = 0;
     auto decided = [&] { return seen != 0 && (seen >> 2) == n; };
     auto decide = [&](uint32_t v) {  // unless it has been decided already
@@ -83,7 +87,7 @@ __device__ __forceinline__ bool team_assembles(uint32_t *words, int spin_limit, 
             __builtin_amdgcn_s_sleep(1);
             seen = __hip_atomic_load(verdict, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
-        if (!decided()) decide(kTeamAlone);
+        if (!decided()) decide(kTeamApart);
     }
     return (seen & 3u) == kTeamGo;
 }
@@ -511,125 +515,245 @@ __global__ __launch_bounds__(1024) void stack_team_kernel(StackTeam p) {
         __hip_atomic_store(p.wait_error, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// The same layers of a team's rows by one workgroup that waits for nobody, where the team did not assemble: 16 columns at a time
-// per wave, fc1 once for the rows' maxima and once more for the codes (its results have no room here).
+// The same layers of a team's rows by the workgroups that are there, where the team did not assemble: half the registers and a
+// third of the LDS of a compute unit each, so they fit beside other work, and however many have arrived after a few looks, one at
+// least, share the columns, 16 at a time per wave; who comes later leaves.  So again they wait for nobody but each other.  GELU's
+// results are handed on in fp32, in the rows of qkv, which are used up by then, and the codes' room (3 d + d_ff / 4 >= d_ff floats), and
+// every workgroup makes the codes of all rows.  77 tokens, d 768, 12 layers: 426 us with all members, 1046 with one or two (one
+// workgroup of 16 waves that ran fc1 twice took 2120).
+constexpr int kPresentWaves = 8;
+constexpr int kPresentChunk = 12;  // pairs of k blocks in flight
+constexpr int kGatherLooks = 256;  // some 15 us
+constexpr uint32_t kGatherClosed = 0x80;
+
+// One lane: joins, and waits until it is settled who takes part.  The first to come settles it, and until then the flags are its own.
+__device__ __forceinline__ bool present_join(uint32_t *words, uint32_t launch, int looks, int spin_limit, int *rank, int *members) {
+    uint32_t *gather = words + kTeamGather;
+    uint32_t seen = __hip_atomic_load(gather, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    do {
+        if (seen & kGatherClosed) return false;
+    } while (!__hip_atomic_compare_exchange_strong(gather, &seen, seen + 1, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    *rank = static_cast<int>(seen++);
+    if (*rank == 0) {
+        for (int i = 0; i < kTeamSize; ++i) words[kCtxTeamFlags + i] = team_flag(launch, 0);  // (the team has left them as they were)
+        for (int look = 0; look < looks && seen < uint32_t(kTeamSize); ++look) {
+            __builtin_amdgcn_s_sleep(1);
+            seen = __hip_atomic_load(gather, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        asm volatile("" ::: "memory");
+        wait_vmcnt<0>();  // the flags have reached the L2
+        asm volatile("" ::: "memory");
+        seen = __hip_atomic_fetch_or(gather, kGatherClosed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) | kGatherClosed;
+    }
+    for (int spin = 0; spin <= spin_limit && !(seen & kGatherClosed); ++spin) {
+        __builtin_amdgcn_s_sleep(1);
+        seen = __hip_atomic_load(gather, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    *members = static_cast<int>(seen & ~kGatherClosed);
+    return (seen & kGatherClosed) != 0;
+}
+
 template <bool EVEN>
-__global__ __launch_bounds__(1024) void stack_alone_kernel(StackTeam p) {
-    constexpr int RC = kTeamFloats, kPiece = kTeamRows + 1;
-    __shared__ __attribute__((aligned(16))) v4i codes[RC * 8 * 2 * kPiece], hidden[kTeamColumns * kTeamSize * 2 * kPiece];
-    __shared__ float row_scale[kTeamRows], hidden_scale[kTeamRows], hidden_inv[kTeamRows];
-    __shared__ uint32_t row_max[kTeamRows];
-    const int team = static_cast<int>(blockIdx.x), T = p.rows, row0 = team * T;
+__global__ __launch_bounds__(kPresentWaves *kWave, 2) void stack_present_kernel(StackTeam p) {
+    constexpr int RC = kTeamFloats, kPiece = kTeamRows + 1, HC = kTeamColumns * kTeamSize * 32 / 256;  // (HC: float4 a lane of d_ff)
+    __shared__ __attribute__((aligned(16))) v4i codes[kTeamColumns * kTeamSize * 2 * kPiece];
+    __shared__ float row_scale[kTeamRows];
+    __shared__ int joined, my_rank, all_members;
+    const int team = static_cast<int>(blockIdx.x) % kTeams, T = p.rows, row0 = team * T;
     if (row0 >= p.tokens) return;
     uint32_t *words = p.words + team * kCtxTeamWords;
-    const uint32_t verdict = words[kTeamVerdict];
-    if ((verdict & 3u) != kTeamAlone) return;
-    if (threadIdx.x < kTeamSize) words[kCtxTeamFlags + threadIdx.x] = team_flag(verdict >> 2, 0);  // (the team has left them as they were)
-    const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const uint32_t verdict = words[kTeamVerdict], launch = verdict >> 2;
+    if ((verdict & 3u) != kTeamApart) return;
+    if (threadIdx.x == 0) {
+        int rank = 0, members = 0;
+        joined = present_join(words, launch, p.gather_looks, p.spin_limit, &rank, &members);
+        my_rank = rank;
+        all_members = members;
+    }
+    __syncthreads();
+    if (!joined) return;
+    int lane = threadIdx.x % kWave;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int rank = __builtin_amdgcn_readfirstlane(my_rank), members = __builtin_amdgcn_readfirstlane(all_members);
     const int R = T < p.tokens - row0 ? T : p.tokens - row0;
-    const int d = p.d, dblocks = d / 32, fblocks = p.d_ff / 32, mine = 4 * (lane / 16);
+    const int d = p.d, d_ff = p.d_ff, dblocks = d / 32, fblocks = d_ff / 32, mine = 4 * (lane / 16);
+    const int beside = d_ff > 3 * d ? d_ff - 3 * d : 0;  // of GELU's results of a row, those that lie where the codes would
+    const __amdgpu_buffer_rsrc_t rflags = team_buffer(words + kCtxTeamFlags, kTeamSize * 4);
     const __amdgpu_buffer_rsrc_t rx = team_buffer(p.x + size_t(row0) * d, R * d * 4);
     const __amdgpu_buffer_rsrc_t rqkv = team_buffer(p.qkv + size_t(row0) * 3 * d, R * 3 * d * 4);
-    auto row_codes = [&](auto norm, const __amdgpu_buffer_rsrc_t &rows, int ld, int first, const float *gamma, const float *beta) {
-        __syncthreads();
-        if (wave < R) {
-            const PanelColumns<RC, false> c(lane, dblocks);
-            float4 v[RC];
-#pragma unroll
-            for (int i = 0; i < RC; ++i)
-                v[i] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(
-                                                      rows, c.real[i] ? c.at(i) * 4 : 0x7fffffff, (wave * ld + first) * 4, kPastL1));
-            uint32_t q[RC];
-            float scale;
-            if constexpr (decltype(norm)::value)
-                scale = panel_norm_quantize<EVEN>(v, c, PanelAffine<RC>(c, gamma, beta), p.eps, q);
-            else
-                scale = row_range_quantize<EVEN>(v, c, q);
-            if (lane == 0) row_scale[wave] = scale;
-            uint32_t *dword = reinterpret_cast<uint32_t *>(codes);
-#pragma unroll
-            for (int i = 0; i < RC; ++i)
-                if (c.real[i]) dword[((c.block[i] * 2 + c.part / 4) * kPiece + wave) * 4 + c.part % 4] = q[i];
-        }
-        __syncthreads();
-    };
-    auto product = [&](const v4i *operand, const float *row_scales, const int8_t *w, const float *scales, const float *biases,
-                       int nblocks, int kblocks, auto use) {
-        const __amdgpu_buffer_rsrc_t rw = team_buffer(w, nblocks * kblocks * 1024);
-#pragma unroll 1
-        for (int half = wave; half < 2 * nblocks; half += kTeamWaves) {
-            v4i acc{0, 0, 0, 0};
-            for (int kb = 0; kb < kblocks; kb += 2)
-                acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(
-                    operand[(kb * 2 + lane / 16) * kPiece + lane % kTeamRows],
-                    __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(
-                                                rw, lane / 16 * 512 + lane % 16 * 16, (half / 2 * kblocks + kb) * 1024 + half % 2 * 256, 0)),
-                    acc, 0, 0, 0);
-            const int n = half * 16 + lane % 16;
-            const float sw = scales[n], bias = biases ? biases[n] : 0.0f;
-            float o[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                o[i] = static_cast<float>(acc[i]) * (row_scales[mine + i] * sw);
-                o[i] = o[i] + bias;
-            }
-            use(half, n, o);
-        }
+    const __amdgpu_buffer_rsrc_t rbeside = team_buffer(p.codes + size_t(team) * T * d_ff, R * beside * 4);
+    constexpr int kNowhere = 0x7fffffff;
+
+    uint32_t phase = team_flag(launch, 0);
+    const uint32_t xcc = team_xcc_id();
+    bool lost = false;  // (of wave 0)
+    auto acknowledged = [] {
         asm volatile("" ::: "memory");
         wait_vmcnt<0>();
         asm volatile("" ::: "memory");
     };
+    auto meet = [&] {  // behind `acknowledged` of every wave
+        phase += team_flag(0, 1);
+        __syncthreads();
+        if (wave == 0 && !lost) {
+            if (lane == 0) __builtin_amdgcn_raw_buffer_store_b32(static_cast<int>(phase | xcc), rflags, rank * 4, 0, 0);
+            bool all = false;
+            uint32_t seen = 0;
+            const bool looks = lane < members;
+            for (int spin = 0; spin <= p.spin_limit && !all; ++spin) {
+                asm volatile("" ::: "memory");
+                seen = static_cast<uint32_t>(__builtin_amdgcn_raw_buffer_load_b32(rflags, lane % kTeamSize * 4, 0, kPastL1));
+                all = __all(!looks || team_flag_reached(seen, phase));
+            }
+            lost = !all || !__all(!looks || (seen & 15u) == xcc);
+        }
+        __syncthreads();
+        asm volatile("" : "+v"(lane)::"memory");
+    };
+    // The codes of the team's rows into LDS, a row per wave.
+    auto row_codes = [&](auto norm, const __amdgpu_buffer_rsrc_t &rows, int ld, int first, const float *gamma, const float *beta) {
+        constexpr int kRounds = kTeamRows / kPresentWaves;
+        const PanelColumns<RC, false> c(lane, dblocks);
+        float4 v[kRounds][RC];
+#pragma unroll
+        for (int u = 0; u < kRounds; ++u) {
+            const int row = wave + u * kPresentWaves;
+            if (row < R) {
+#pragma unroll
+                for (int i = 0; i < RC; ++i)
+                    v[u][i] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                             rows, c.real[i] ? c.at(i) * 4 : kNowhere, (row * ld + first) * 4, kPastL1));
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < kRounds; ++u) {
+            const int row = wave + u * kPresentWaves;
+            if (row >= R) break;
+            uint32_t q[RC];
+            float scale;
+            if constexpr (decltype(norm)::value)
+                scale = panel_norm_quantize<EVEN>(v[u], c, PanelAffine<RC>(c, gamma, beta), p.eps, q);
+            else
+                scale = row_range_quantize<EVEN>(v[u], c, q);
+            if (lane == 0) row_scale[row] = scale;
+            uint32_t *dword = reinterpret_cast<uint32_t *>(codes);
+#pragma unroll
+            for (int i = 0; i < RC; ++i)
+                if (c.real[i]) dword[((c.block[i] * 2 + c.part / 4) * kPiece + row) * 4 + c.part % 4] = q[i];
+        }
+        __syncthreads();
+    };
+    // The same of GELU's results.
+    auto hidden_codes = [&] {
+#pragma unroll 1
+        for (int row = wave; row < R; row += kPresentWaves) {
+            v4i raw[HC];
+#pragma unroll
+            for (int i = 0; i < HC; ++i) {
+                const int col = 4 * (lane + kWave * i);
+                raw[i] = __builtin_amdgcn_raw_buffer_load_b128(rqkv, col < d_ff && col < 3 * d ? (row * 3 * d + col) * 4 : kNowhere, 0, kPastL1);
+                if (256 * i + 256 > 3 * d)  // (one of the two is out of range, which reads as zeros)
+                    raw[i] |= __builtin_amdgcn_raw_buffer_load_b128(
+                        rbeside, col < d_ff && col >= 3 * d ? (row * beside + col - 3 * d) * 4 : kNowhere, 0, kPastL1);
+            }
+            auto value = [&](int i, int e) {
+                const int bits = raw[i][e];
+                return __builtin_bit_cast(float, bits);
+            };
+            float am = 0.0f;  // (a NaN is no maximum)
+#pragma unroll
+            for (int i = 0; i < HC; ++i)
+                am = fmaxf(am, fmaxf(fmaxf(fabsf(value(i, 0)), fabsf(value(i, 1))), fmaxf(fabsf(value(i, 2)), fabsf(value(i, 3)))));
+            am = wave_max(am);
+            const float scale = am < FLT_EPSILON ? 1.0f : am / 127.0f, inv = recip_for_div(scale);
+            const bool good = am <= FLT_MAX;
+            if (lane == 0) row_scale[row] = good ? scale : NAN;
+            uint32_t *dword = reinterpret_cast<uint32_t *>(codes);
+#pragma unroll
+            for (int i = 0; i < HC; ++i) {
+                const int col = 4 * (lane + kWave * i);
+                if (col < d_ff)
+                    dword[(col / 16 * kPiece + row) * 4 + col % 16 / 4] =
+                        good ? pack4(quantize_int_sym<EVEN>(value(i, 0), scale, inv), quantize_int_sym<EVEN>(value(i, 1), scale, inv),
+                                     quantize_int_sym<EVEN>(value(i, 2), scale, inv), quantize_int_sym<EVEN>(value(i, 3), scale, inv))
+                             : 0u;
+            }
+        }
+        __syncthreads();
+    };
+    auto product = [&](const int8_t *w, const float *scales, const float *biases, int nblocks, int kblocks, auto use) {
+        const __amdgpu_buffer_rsrc_t rw = team_buffer(w, nblocks * kblocks * 1024);
+        const int fragment = lane / 16 * 512 + lane % 16 * 16;
+#pragma unroll 1
+        for (int half = wave * members + rank; half < 2 * nblocks; half += members * kPresentWaves) {
+            v4i acc{0, 0, 0, 0};
+            const int n = half * 16 + lane % 16, from = half / 2 * kblocks * 1024 + half % 2 * 256;
+            const float sw = scales[n], bias = biases ? biases[n] : 0.0f;
+#pragma unroll 1
+            for (int kb0 = 0; kb0 < kblocks; kb0 += 2 * kPresentChunk) {
+                v4i fw[kPresentChunk];
+#pragma unroll
+                for (int u = 0; u < kPresentChunk; ++u)
+                    if (kb0 + 2 * u < kblocks)
+                        fw[u] = __builtin_amdgcn_raw_buffer_load_b128(rw, fragment, from + (kb0 + 2 * u) * 1024, 0);
+#pragma unroll
+                for (int u = 0; u < kPresentChunk; ++u)
+                    if (kb0 + 2 * u < kblocks)
+                        acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(codes[((kb0 + 2 * u) * 2 + lane / 16) * kPiece + lane % kTeamRows], fw[u], acc, 0, 0, 0);
+            }
+            float o[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                o[i] = static_cast<float>(acc[i]) * (row_scale[mine + i] * sw);
+                o[i] = o[i] + bias;
+            }
+            use(half, n, o);
+        }
+        acknowledged();
+    };
+    auto store = [&](float v, const __amdgpu_buffer_rsrc_t &to, int at, int i) {  // result i of this lane, if its row is one of the team's
+        if (mine + i < R) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, v), to, at * 4, 0, 0);
+    };
     auto add_to_stream = [&](int, int n, float(&o)[4]) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-            if (mine + i < R) {
-                const int at = ((mine + i) * d + n) * 4;
-                const float x = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rx, at, 0, kPastL1));
-                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, o[i] + x), rx, at, 0, 0);
-            }
+        for (int i = 0; i < 4; ++i) {
+            const int at = (mine + i) * d + n;
+            const float x = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rx, mine + i < R ? at * 4 : kNowhere, 0, kPastL1));
+            store(o[i] + x, rx, at, i);
+        }
     };
 #pragma unroll 1
     for (int l = 0; l < p.layers; ++l) {
         const hipq_block_weights &b = p.blocks[l];
         if (l > 0 || !p.qkv_done) {
             row_codes(std::true_type{}, rx, d, 0, b.ln1_gamma, b.ln1_beta);
-            product(codes, row_scale, b.w_qkv, b.s_qkv, b.b_qkv, 3 * dblocks, dblocks, [&](int, int n, float(&o)[4]) {
+            product(b.w_qkv, b.s_qkv, b.b_qkv, 3 * dblocks, dblocks, [&](int, int n, float(&o)[4]) {
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    if (mine + i < R)
-                        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, o[i]), rqkv, ((mine + i) * 3 * d + n) * 4, 0, 0);
+                for (int i = 0; i < 4; ++i) store(o[i], rqkv, (mine + i) * 3 * d + n, i);
             });
+            meet();
         }
         row_codes(std::false_type{}, rqkv, 3 * d, 2 * d, nullptr, nullptr);
-        product(codes, row_scale, b.w_out, b.s_out, b.b_out, dblocks, dblocks, add_to_stream);
-        if (threadIdx.x < kTeamRows) row_max[threadIdx.x] = 0;
+        product(b.w_out, b.s_out, b.b_out, dblocks, dblocks, add_to_stream);
+        meet();
         row_codes(std::true_type{}, rx, d, 0, b.ln2_gamma, b.ln2_beta);
-        product(codes, row_scale, b.w_fc1, b.s_fc1, b.b_fc1, fblocks, dblocks, [&](int, int, float(&o)[4]) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {  // (not negative, so ordered as the bits are; a NaN is no maximum)
-                const float m = lane_row_max(fmaxf(fabsf(gelu_tanh(o[i])), 0.0f));
-                if (lane % 16 == 0) atomicMax(&row_max[mine + i], __builtin_bit_cast(uint32_t, m));
-            }
-        });
-        __syncthreads();
-        if (threadIdx.x < kTeamRows) {
-            const float am = __builtin_bit_cast(float, row_max[threadIdx.x]);
-            const float scale = am < FLT_EPSILON ? 1.0f : am / 127.0f;
-            hidden_scale[threadIdx.x] = am <= FLT_MAX ? scale : NAN;
-            hidden_inv[threadIdx.x] = recip_for_div(scale);
-        }
-        __syncthreads();
-        product(codes, row_scale, b.w_fc1, b.s_fc1, b.b_fc1, fblocks, dblocks, [&](int half, int, float(&o)[4]) {
+        product(b.w_fc1, b.s_fc1, b.b_fc1, fblocks, dblocks, [&](int half, int n, float(&o)[4]) {
+            const bool in_rows = half * 16 < 3 * d;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const float scale = hidden_scale[mine + i];
-                const int q = scale == scale ? quantize_int_sym<EVEN>(gelu_tanh(o[i]), scale, hidden_inv[mine + i]) : 0;
-                reinterpret_cast<int8_t *>(hidden)[(half * kPiece + mine + i) * 16 + lane % 16] = static_cast<int8_t>(q);
+                const float h = gelu_tanh(o[i]);
+                if (in_rows)
+                    store(h, rqkv, (mine + i) * 3 * d + n, i);
+                else
+                    store(h, rbeside, (mine + i) * beside + n - 3 * d, i);
             }
         });
-        __syncthreads();
-        product(hidden, hidden_scale, b.w_fc2, b.s_fc2, b.b_fc2, dblocks, fblocks, add_to_stream);
+        meet();
+        hidden_codes();
+        product(b.w_fc2, b.s_fc2, b.b_fc2, dblocks, fblocks, add_to_stream);
+        if (l + 1 < p.layers) meet();
     }
+    if (wave == 0 && lane == 0 && lost) __hip_atomic_store(p.wait_error, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 __global__ void team_words_clear_kernel(uint32_t *words) { words[blockIdx.x * blockDim.x + threadIdx.x] = 0; }
@@ -664,6 +788,7 @@ int32_t team_stack(hipq_ctx *ctx, const TeamStackCall &call, int32_t mode) {
     p.d_ff = static_cast<int>(call.d_ff);
     p.spin_limit = ctx->wait_spin_limit < 1024 ? 1 << 20 : ctx->wait_spin_limit;  // (a small one, a test's, is for the assembly)
     p.assembly_limit = ctx->wait_spin_limit < kAssemblyLimit ? ctx->wait_spin_limit : kAssemblyLimit;
+    p.gather_looks = ctx->wait_spin_limit == 0 ? 0 : kGatherLooks;
     p.eps = call.eps;
     for (size_t l = 0; l < call.layers; l += kTeamLayers) {
         p.layers = static_cast<int>(call.layers - l < size_t(kTeamLayers) ? call.layers - l : size_t(kTeamLayers));
@@ -671,10 +796,10 @@ int32_t team_stack(hipq_ctx *ctx, const TeamStackCall &call, int32_t mode) {
         for (int i = 0; i < p.layers; ++i) p.blocks[i] = call.blocks[l + i];
         if (mode & HIPQ_ROUND_HALF_EVEN) {
             hipLaunchKernelGGL(stack_team_kernel<true>, dim3(kTeams * kTeamSize), dim3(1024), 0, ctx->stream, p);
-            hipLaunchKernelGGL(stack_alone_kernel<true>, dim3(kTeams), dim3(1024), 0, ctx->stream, p);
+            hipLaunchKernelGGL(stack_present_kernel<true>, dim3(kTeams * kTeamSize), dim3(kPresentWaves * kWave), 0, ctx->stream, p);
         } else {
             hipLaunchKernelGGL(stack_team_kernel<false>, dim3(kTeams * kTeamSize), dim3(1024), 0, ctx->stream, p);
-            hipLaunchKernelGGL(stack_alone_kernel<false>, dim3(kTeams), dim3(1024), 0, ctx->stream, p);
+            hipLaunchKernelGGL(stack_present_kernel<false>, dim3(kTeams * kTeamSize), dim3(kPresentWaves * kWave), 0, ctx->stream, p);
         }
         const int32_t rc = check_launch("transformer stack (teams)");
         if (rc) return rc;
