@@ -68,3 +68,28 @@ def test_addresses_of_blocks(native):
         native.pointers(3, ("a",))
     with pytest.raises(AttributeError):
         native.pointers([{"a": "text"}], ("a",))
+
+
+def test_the_module_is_built_again_for_another_torch(monkeypatch, tmp_path):
+    """An incremental build leaves the module alone only where it was built against the python and the torch that are there."""
+    from torsh_amd import build
+
+    runs = []
+    monkeypatch.setattr(build, "PYTHON_PATH", str(tmp_path / "_hipq_python.so"))
+    monkeypatch.setattr(build, "PYTHON_STAMP", str(tmp_path / "_hipq_python.stamp"))
+
+    def run(cmd, **kwargs):
+        runs.append(cmd)
+        open(cmd[cmd.index("-o") + 1], "w").close()
+        return types.SimpleNamespace(returncode=0, stdout="", stderr="")
+
+    monkeypatch.setattr(build.subprocess, "run", run)
+    for expected in (1, 1):  # nothing there; all there
+        build._build_python(False)
+        assert len(runs) == expected
+    monkeypatch.setattr(torch, "__version__", "0.0.1")
+    for expected in (2, 2):
+        build._build_python(False)
+        assert len(runs) == expected
+    build._build_python(True)
+    assert len(runs) == 3

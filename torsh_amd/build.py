@@ -18,6 +18,7 @@ CSRC = os.path.join(PKG, "csrc")
 OBJ_DIR = os.path.join(PKG, "lib", "obj")
 LIB_PATH = os.path.join(PKG, "lib", "libtorsh_hipq.so")
 PYTHON_PATH = os.path.join(PKG, "lib", "_hipq_python.so")
+PYTHON_STAMP = os.path.join(OBJ_DIR, "_hipq_python.stamp")  # what the module was built against
 
 ARCH = "gfx950"
 
@@ -82,8 +83,11 @@ def _build_python(force: bool) -> None:
 
     src = os.path.join(CSRC, "hipq_python.cpp")
     newest = max(os.path.getmtime(src), os.path.getmtime(os.path.join(ROOT, "include", "torsh_hipq.h")))
-    if not force and os.path.exists(PYTHON_PATH) and os.path.getmtime(PYTHON_PATH) >= newest:
-        return
+    against = f"python {sys.version}\ntorch {torch.__version__} {torch.__file__}\n"
+    if not force and os.path.exists(PYTHON_PATH) and os.path.getmtime(PYTHON_PATH) >= newest and os.path.exists(PYTHON_STAMP):
+        with open(PYTHON_STAMP) as f:
+            if f.read() == against:
+                return
     cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-I", os.path.join(ROOT, "include"),
            "-isystem", sysconfig.get_paths()["include"]]
@@ -96,6 +100,8 @@ def _build_python(force: bool) -> None:
     proc = subprocess.run(cmd, capture_output=True, text=True)
     if proc.returncode != 0:
         raise RuntimeError(f"building {src} failed:\n{proc.stdout}\n{proc.stderr}")
+    with open(PYTHON_STAMP, "w") as f:
+        f.write(against)
 
 
 def build(force: bool = True, jobs: int = 8) -> str:
