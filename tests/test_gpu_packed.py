@@ -977,6 +977,26 @@ def test_linear_of_small_sizes_leaves_calls_over_their_input(stream_ctx, launche
         assert any("linear_small_kernel" in name for name in launched_kernels(stream_ctx, call)) == small
 
 
+@pytest.mark.parametrize("m,k", [(1, 512), (2, 2048), (4, 1024)])
+def test_decode_over_its_input(stream_ctx, launched_kernels, hipq, m, k):
+    """Linears of a few rows on prepared weights whose every workgroup quantizes the rows itself: a result over the input is right too."""
+    c = stream_ctx
+    side = torch.cuda.ExternalStream(c.stream_handle)
+    with torch.cuda.stream(side):
+        g = torch.Generator(device="cuda").manual_seed(m + k)
+        x0 = torch.randn(m, k, generator=g, device="cuda")
+        pw = c.pack_rows(torch.randint(-128, 128, (k, k), generator=g, device="cuda", dtype=torch.int8))
+        sw = torch.rand(k, generator=g, device="cuda") * 1e-3
+        for call in (lambda x, out: c.linear_dynamic_packed(x, pw, sw, per_token=True, out=out),
+                     lambda x, out: c.linear_static_packed(x, 0.02, pw, sw, out=out)):
+            want = call(x0, torch.empty_like(x0))
+            x = x0.clone()
+            side.synchronize()
+            names = launched_kernels(c, lambda: call(x, x))
+            assert len(names) > 1 and not any("gemv_i8_packed_from_f32" in name for name in names), names
+            assert torch.equal(call(x, x), want)
+
+
 # The last sizes of each form and the first past them; 256 compute units.
 @pytest.mark.parametrize("form,m,n,k,small", [
     ("tensor", 64, 32, 1024, True), ("tensor", 65, 32, 1024, False), ("tensor", 32, 64, 2048, True), ("tensor", 31, 64, 2049, False),

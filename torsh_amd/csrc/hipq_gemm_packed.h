@@ -660,6 +660,7 @@ static bool launch_gemv_packed_from_f32(hipq_ctx *ctx, const float *x, const int
     const size_t chunks = (KB * 2 + 255) / 256;  // 16-float groups per thread and row
     const size_t most_rows = STATIC ? 4 : 2;
     if (m == 0 || m > most_rows || k % 16 != 0 || (reinterpret_cast<uintptr_t>(x) & 15u) != 0 || KB < 16) return false;
+    if (memory_meets(x, m * k * sizeof(float), ep.out, m * n * sizeof(float))) return false;  // (others read x while one stores)
     const int mrows = m <= 2 ? static_cast<int>(m) : 4, ch = chunks <= 1 ? 1 : (chunks == 2 ? 2 : 4);
     if (chunks > 4 || mrows * ch > 4) return false;
     const int M = static_cast<int>(m), N = static_cast<int>(n), K = static_cast<int>(k);

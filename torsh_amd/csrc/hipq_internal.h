@@ -196,6 +196,12 @@ int32_t linear_noalloc_setup(int device);
 // the runtime once per device and remembered).
 bool four_wide_workgroups_fit(const hipq_ctx *ctx);
 
+// Whether two pieces of memory share a byte.
+inline bool memory_meets(const void *a, size_t a_bytes, const void *b, size_t b_bytes) {
+    const uintptr_t p = reinterpret_cast<uintptr_t>(a), q = reinterpret_cast<uintptr_t>(b);
+    return p < q + b_bytes && q < p + a_bytes;
+}
+
 // Bytes reserved at the head of the context scratch for small device records
 // (hipq_qparams, min/max pairs, status words); bulk scratch starts after it.
 constexpr size_t kScratchHeader = 4096;

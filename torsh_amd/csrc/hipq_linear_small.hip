@@ -228,8 +228,7 @@ bool linear_small(hipq_ctx *ctx, LinearRange range, const float *x, float scale,
     if (range == LINEAR_PER_TENSOR && m * k > 65536) return false;
     // A result over its input (an in-place call): a workgroup would store into rows that others have not read.  The quantizer has read
     // all of x before the product stores anything.
-    const uintptr_t in = reinterpret_cast<uintptr_t>(x), to = reinterpret_cast<uintptr_t>(out);
-    if (in < to + m * n * sizeof(float) && to < in + m * k * sizeof(float)) return false;
+    if (memory_meets(x, m * k * sizeof(float), out, m * n * sizeof(float))) return false;
     const LinearSmall p{x, w, w_scales, bias, out, scale, range, static_cast<int>(m), static_cast<int>(n), static_cast<int>(k),
                         k % 16 == 0 && (reinterpret_cast<uintptr_t>(w) & 15u) == 0};
     const bool div = range == LINEAR_PER_TOKEN || (mode & HIPQ_FORM_DIV), even = (mode & HIPQ_ROUND_HALF_EVEN) != 0;
