@@ -213,7 +213,7 @@ HIPQ_API int32_t hipq_dequantize_with_params_i8_f32(hipq_ctx *ctx, const int8_t 
  * HIPQ_PARAMS_SYMMETRIC or HIPQ_PARAMS_AFFINE) -> clamp(round(x / s) + zp,
  * qmin, qmax).  Used per output channel for weights and per token for
  * activations.  out_scales[rows], out_zero_points[rows] (may be NULL).
- * out_status: device int32, set non-zero if any row had a non-finite range. */
+ * out_status: device int32, set non-zero if any row had a non-finite range (no wait: nothing else sets it). */
 HIPQ_API int32_t hipq_quantize_per_row_f32_i8(hipq_ctx *ctx, const float *x, size_t rows, size_t cols,
                                               int32_t flavor, int32_t mode, int8_t *out, float *out_scales,
                                               int32_t *out_zero_points, int32_t *out_status);
@@ -391,8 +391,8 @@ HIPQ_API int32_t hipq_linear_packed_i8_i8(hipq_ctx *ctx, const int8_t *a_packed,
  * otherwise `scale` is used (quantize_per_tensor_affine, algorithms.rs:277-315).  Codes are those of
  * hipq_quantize_dynamic_per_tensor_f32 / hipq_quantize_per_tensor_f32_i8; a range that is not finite
  * gives status HIPQ_INVALID_ARGUMENT in out_params, a NaN scale and zero codes.
- * A dynamic call on up to 65536 * (compute units) elements (16 Mi on MI355X), cols % 16 == 0, x 16-byte aligned, is
- * one kernel: every wave holds its one or four fragments of 16 x 64 floats in registers while the workgroups agree on the range
+ * A dynamic call on up to 65536 * (compute units) elements (16 Mi on MI355X), rows of any length at any float, is one kernel:
+ * every wave holds its one, two or four fragments of 16 x 64 floats in registers while the workgroups agree on the range
  * through device words of the context (see hipq_ctx_set_wait_spin_limit), so x is read once.  It keeps no
  * host state per launch and can be captured and replayed.  Two such calls on one context must not overlap
  * (they cannot: a context has one stream). */

@@ -39,14 +39,18 @@ extern "C" {
 HIPQ_API int32_t hipq_set_gemm_kernel_variant(hipq_ctx *ctx, int32_t variant);
 /* Some kernels couple their waves through device memory: the persistent GEMM kernel (counters
  * between producer and consumer waves), the one-launch dynamic quantizers (their workgroups meet to
- * agree on the range), the GEMM form whose workgroup pairs exchange partial sums and the row-panel
- * forwards whose workgroup pairs exchange row maxima and sums.  All bound
+ * agree on the range), the GEMM form whose workgroup pairs exchange partial sums, the row-panel
+ * forwards whose workgroup pairs exchange row maxima and sums, and the prepared stack of few tokens, whose teams of
+ * workgroups meet between its products.  All bound
  * every wait, so that a grid always drains; a wait that gives up marks the context, and the next
  * hipq_ctx_synchronize returns HIPQ_DEVICE_ERROR once instead of handing back a wrong result
  * silently (the quantizers also leave zero codes, a NaN scale and status HIPQ_DEVICE_ERROR in
  * out_params).  `limit` is the number of polls after the first look (negative = the default, 2^20);
  * 0 lets a test see the error path without hanging anything.  The per-channel quantizer over a middle axis waits
- * at most 2^13 polls, and a few once that was in vain, and then reads its channel's range itself: no error there. */
+ * at most 2^13 polls, and a few once that was in vain, and then reads its channel's range itself: no error there.  A
+ * team of the stack waits at most 2^9 polls for all its workgroups to be there and then leaves its rows to those that come to
+ * the kernel behind it within a few microseconds (with a limit of 0: to the first), no error either; meetings are bounded by
+ * `limit`, or by the default where it is below 2^10. */
 HIPQ_API int32_t hipq_ctx_set_wait_spin_limit(hipq_ctx *ctx, int32_t limit);
 /* While a device buffer is set, hipq_linear_packed_i8_f32 (and the forwards built on it) run a
  * form of the packed GEMM kernel in which every wave records the shader clock at six points -

@@ -224,8 +224,8 @@ int32_t hipq_ctx_synchronize(hipq_ctx *ctx) {
         const int32_t rc = hipq::reset_ctx_words(ctx);
         if (rc) return rc;
         return hipq::fail(HIPQ_DEVICE_ERROR,
-                          "hipq_ctx_synchronize: a bounded wait inside a kernel (persistent GEMM or one-launch "
-                          "dynamic quantize) gave up (spin limit %d); results of the calls since the last "
+                          "hipq_ctx_synchronize: a bounded wait inside a kernel (persistent GEMM, one-launch dynamic "
+                          "quantize, or workgroups that share rows of a panel or a stack) gave up (spin limit %d); results of the calls since the last "
                           "synchronize are invalid",
                           ctx->wait_spin_limit);
     }

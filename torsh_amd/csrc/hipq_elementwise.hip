@@ -667,8 +667,9 @@ __global__ __launch_bounds__(kBlock) void dequantize_kernel(const InT *__restric
 // the cleared one and the refusal, are put in order by a word of the context: it rises to 2 `launch` once the status has been
 // cleared and to 2 `launch` + 1 with the first refusal.  Whoever finds the other there already writes the refusal, once; nobody waits,
 // and a launch without a refusal has one workgroup that looks.  The number comes from the host, so a launch that is recorded to be
-// replayed has no `word`: its status has been cleared by a launch of its own, and a refusal is written over that.  us, cleared by a
-// launch / this: quantize + dequantize per channel of 1025 x 64 floats 15.9 / 12.7.
+// replayed has no `word`: its status has been cleared by a launch of its own, and a refusal is written over that.  Quantize per row, us,
+// cleared by a launch / this: 16000 x 300 12.2 / 10.3, 4096 x 4000 16.4 / 14.6; collected by a meeting of all workgroups / this: 1024 x 64
+// 8.3 / 8.3, 4096 x 2000 12.4 / 10.6, 500 x 12000 10.9 / 8.8.
 struct StatusWord {
     int32_t *out = nullptr;
     unsigned long long *word = nullptr;

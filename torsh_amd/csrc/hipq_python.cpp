@@ -7,8 +7,8 @@
 // given.  As with ctypes, the interpreter lock is not held during the call.
 //
 // us a pass of small calls, which the host bounds or nearly does, ctypes / this: a quantize and a dequantize per channel with five
-// outputs 21.0 / 17.5, per tensor with three 13.9 / 11.5, a convolution 11.75 / 9.9, a Linear into a given output 9.1 / 8.4 (its two
-// launches follow one another in 8).
+// outputs 21.0 / 17.5, per tensor with three 13.9 / 11.5, a convolution 11.75 / 9.9, a Linear of two launches into a given output 9.1 / 8.4
+// (the two follow one another in 8).
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -26,7 +26,7 @@ namespace {
 
 PyObject *g_error_handler = nullptr;
 
-// The address of a tensor's data, or -1 with an exception set.  Subclasses other than Parameter answer for themselves.
+// Leaves the address of a tensor's data in `out`; false with an exception set.  Subclasses other than Parameter answer for themselves.
 bool tensor_address(PyObject *o, bool dense, void **out) {
     if (THPVariable_CheckExact(o)) {
         const at::Tensor &t = THPVariable_Unpack(o);
