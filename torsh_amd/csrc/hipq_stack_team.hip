@@ -764,6 +764,8 @@ __global__ void team_words_clear_kernel(uint32_t *words) { words[blockIdx.x * bl
 // d_ff 3072 1 token 303 / 191, 16 313 / 217, 77 334 / 240, 128 368 / 281; d 384, d_ff 1152, 10 layers, 3 tokens 231 / 118; d 256,
 // d_ff 1024, 6 layers, 40 tokens 140 / 82.  What is left is 2.3 us a phase (rows 0.5, LayerNorm and codes 1.1, product 0.3, results
 // and their acknowledgement 0.9, meeting 0.35) and, at d 768, 7 MB of weights a layer through each XCD's port, at some 0.7 TB/s.
+// Rows of up to 1024 floats would need three steps of K times three column blocks of weights in the registers of a wave that multiplies,
+// where there is room for eight (115 of 128 are taken), or eight such waves and eight for the rows: not tried.
 bool team_stack_fits(const hipq_ctx *ctx, const float *x, size_t tokens, size_t d, size_t d_ff, PanelFold after_out,
                      PanelFold after_fc2) {
     const int share = ctx->resident_share > 0 ? ctx->resident_share : 1;
