@@ -682,7 +682,13 @@ struct StatusWord {
     }
     __device__ __forceinline__ void report(int st) const {  // one thread per row or group
         if (!out || st == HIPQ_SUCCESS) return;
-        if (!word || __hip_atomic_fetch_max(word, 2 * launch + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 2 * launch) write(st);
+        if (!word) return write(st);
+        // Refusals of many rows would follow one another at the one word, 12 ns each: the first of a sixty-fourth of the workgroups
+        // goes there.  16000 x 300 without a finite range, one word / 64 of them in front: 184 / 9.2 us; 4096 x 64 49 / 7.7.
+        unsigned long long *front = word + (1 + blockIdx.x % kCtxStatusFronts) * kCtxStatusStep;
+        if (__hip_atomic_load(front, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == launch) return;
+        if (__hip_atomic_fetch_max(front, launch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == launch) return;
+        if (__hip_atomic_fetch_max(word, 2 * launch + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 2 * launch) write(st);
     }
     __device__ __forceinline__ void finish() const {  // all threads, behind begin
         if (!word || blockIdx.x != 0 || threadIdx.x != 0) return;

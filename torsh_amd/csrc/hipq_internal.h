@@ -75,9 +75,10 @@ constexpr size_t kCtxSlots = 2048;  // workgroups that can meet
 // launch; on a line of their own, the phase that each workgroup has finished.
 constexpr size_t kCtxTeamWord = kCtxRangeWord + kCtxSlots * 4;
 constexpr size_t kCtxTeams = 8, kCtxTeamWords = 64, kCtxTeamFlags = 32;
-// 64 bits that order a quantizer's status word (StatusWord, hipq_elementwise.hip); on a line of their own.
+// 64 bits that order a quantizer's status word (StatusWord, hipq_elementwise.hip) and those in front of it, each on a line of its own.
 constexpr size_t kCtxStatusWord = kCtxTeamWord + kCtxTeams * kCtxTeamWords;
-constexpr size_t kCtxWordsBytes = (kCtxStatusWord + 32) * 4;
+constexpr size_t kCtxStatusFronts = 64, kCtxStatusStep = 16;
+constexpr size_t kCtxWordsBytes = kCtxStatusWord * 4 + (1 + kCtxStatusFronts) * kCtxStatusStep * 8;
 // Number the first meeting of a context gets, a few launches before the counter wraps, so that the wrap (which
 // wipes the slots) is a path every context takes early, not once in 2^32 launches.
 constexpr uint32_t kCtxFirstEpoch = 0xfffffff0u;
